@@ -32,7 +32,7 @@
 extern "C" {
 #endif
 
-#define SVDQ_ABI_VERSION 9
+#define SVDQ_ABI_VERSION 10
 
 enum { SVDQ_BF16 = 0, SVDQ_FP16 = 1 };
 enum { SVDQ_PRE_NONE = 0, SVDQ_PRE_GLU = 1, SVDQ_PRE_GELU = 2 }; /* svdq_quantize_args.prologue */
@@ -310,6 +310,14 @@ int svdq_awq_gemv_w4a16_batched(const svdq_awq_gemv_args *first, const svdq_awq_
  */
 int svdq_awq_dequantize(const void *qweight, const void *scales, const void *zeros, void *out, int32_t N, int32_t K,
                         int32_t group_size, int32_t ld_scales, int32_t ld_out, int32_t dtype, void *stream);
+
+/*
+ * AWQ W4A16 GEMM: out = x . T(q * s + z)^T with the weight of svdq_awq_dequantize decoded inside the kernel
+ * (nunchaku/ops/triton/awq.py:232-251 awq_gemm_w4a16, there a dense decode and a library product).  `args` as for the
+ * GEMV, with any M, N % 4 == 0, scales / zeros (K / group_size, N), group_size a multiple of 32 that divides K; out rows
+ * 8-byte aligned.
+ */
+int svdq_awq_gemm_w4a16(const svdq_awq_gemv_args *args, int32_t group_size, void *stream);
 
 /*
  * Unmasked scaled-dot-product attention, head dimension D = 128 or 64 (nunchaku/ops/dispatch.py:67-99 attention_fp16 /

@@ -14,7 +14,7 @@ import torch
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libsvdq_mi355x.so")
-ABI_VERSION = 9
+ABI_VERSION = 10
 
 BF16, FP16 = 0, 1
 EPI_PLAIN, EPI_QK_NORM_ROPE, EPI_GELU_QUANT, EPI_SWIGLU_QUANT = 0, 1, 2, 3
@@ -42,6 +42,7 @@ EXPORTS = (
     "svdq_awq_gemv_w4a16",
     "svdq_awq_gemv_w4a16_batched",
     "svdq_awq_dequantize",
+    "svdq_awq_gemm_w4a16",
     "svdq_attention_fp16",
     "svdq_unpack_mma_weight",
     "svdq_unpack_mma_scale",
@@ -146,6 +147,7 @@ def load() -> ctypes.CDLL:
     lib.svdq_awq_gemv_w4a16.argtypes = [ctypes.POINTER(AwqGemvArgs), _vp]
     lib.svdq_awq_gemv_w4a16_batched.argtypes = [ctypes.POINTER(AwqGemvArgs), _vp, _i32, _vp]
     lib.svdq_awq_dequantize.argtypes = [_vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32, _vp]
+    lib.svdq_awq_gemm_w4a16.argtypes = [ctypes.POINTER(AwqGemvArgs), _i32, _vp]
     lib.svdq_attention_fp16.argtypes = [ctypes.POINTER(AttentionArgs), _vp]
     lib.svdq_unpack_mma_weight.argtypes = [_vp, _vp, _i32, _i32, _i32, _vp]
     lib.svdq_unpack_mma_scale.argtypes = [_vp, _vp, _i32, _i32, _i32, _vp]

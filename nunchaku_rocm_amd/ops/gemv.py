@@ -23,19 +23,16 @@ def awq_gemv_w4a16_cuda(
     """
     ``out = in_feats @ (q * scaling_factors + zeros).T`` with ``q`` the TinyChat-packed uint4 weight
     (``kernel`` ``(n // 4, k // 2)`` int32).  Group size 64 runs the fused GEMV kernel (weights read once for all ``m``
-    rows).  Two cases take the reference's own route for everything but group size 64 (ops/triton/awq.py:226-228), still
-    on the GPU: :func:`awq_dequantize` to a dense ``(n, k)`` 16-bit weight (``2 n k`` bytes, allocated per call), then a
-    library matmul -- other group sizes or ``n % 32 != 0``, and shapes whose per-group tables do not fit the kernel's
-    64 KB of LDS (``k = 12288`` with more than 16 rows; no FLUX shape).  Weights of 4 GiB and more are refused
-    (``RuntimeError``): the kernels address them with 32-bit offsets.  Returns ``in_feats.shape[:-1] + (n,)`` in the
-    input dtype.
+    rows).  Two cases take :func:`awq_gemm_w4a16` (the weight rounded to 16 bits, the reference's own route for everything
+    but group size 64, ops/triton/awq.py:226-228): other group sizes or ``n % 32 != 0``, and shapes whose per-group tables
+    do not fit the kernel's 64 KB of LDS (``k = 12288`` with more than 16 rows; no FLUX shape).  Weights of 4 GiB and more
+    are refused (``RuntimeError``): the kernels address them with 32-bit offsets.  Returns ``in_feats.shape[:-1] + (n,)``
+    in the input dtype.
     """
     _lib.require_cuda(in_feats, kernel, scaling_factors, zeros)
     x = in_feats.reshape(m, k)
     if group_size != 64 or n % 32:
-        # as the reference (ops/triton/awq.py:226-228): decode to a dense weight, then a library matmul
-        w = awq_dequantize(kernel, scaling_factors, zeros, n, k, group_size, x.dtype)
-        return torch.matmul(x, w.t()).reshape(*in_feats.shape[:-1], n)
+        return _product(x, kernel, scaling_factors, zeros, n, k, group_size).reshape(*in_feats.shape[:-1], n)
     if x.stride(1) != 1 or x.stride(0) % 8 or x.data_ptr() % 16:
         x = x.contiguous()
     if kernel.element_size() * kernel.numel() != n * k // 2 or not kernel.is_contiguous():
@@ -68,10 +65,8 @@ def awq_gemv_w4a16_cuda(
             rc = lib.svdq_awq_gemv_w4a16(args, _lib.stream_of(x))
             if rc == _lib.E_UNSUPPORTED:
                 # the kernel's per-group tables do not fit LDS (K = 12288 with more than 16 rows, longer K with fewer):
-                # decode the weight and multiply on the GPU, the reference's route for everything but group size 64 (the
-                # other refusal, a weight of 4 GiB and more, was raised above)
-                w = awq_dequantize(kernel, scaling_factors, zeros, n, k, group_size, x.dtype)
-                return torch.matmul(x, w.t()).reshape(*in_feats.shape[:-1], n)
+                # the GEMM, as for other group sizes (the other refusal, a weight of 4 GiB and more, was raised above)
+                return _product(x, kernel, scaling_factors, zeros, n, k, group_size).reshape(*in_feats.shape[:-1], n)
             _lib.check(rc)
     return out.reshape(*in_feats.shape[:-1], n)
 
@@ -123,6 +118,48 @@ class AwqGemvBatch:
         return self.out
 
 
+def _check_weight(kernel, scaling_factors, zeros, n: int, k: int, group_size: int, dtype: torch.dtype):
+    _lib.require_cuda(kernel, scaling_factors, zeros)
+    if kernel.element_size() * kernel.numel() != n * k // 2 or not kernel.is_contiguous():
+        raise ValueError(f"unexpected packed AWQ weight shape {tuple(kernel.shape)} for n={n}, k={k}")
+    if group_size <= 0 or k % group_size:
+        raise ValueError(f"group_size={group_size} does not divide k={k}")
+    groups = k // group_size
+    if scaling_factors.shape != (groups, n) or zeros.shape != (groups, n):
+        raise ValueError(f"scaling_factors / zeros must be ({groups}, {n})")
+    if scaling_factors.dtype != dtype or zeros.dtype != dtype:
+        raise ValueError("scaling_factors / zeros must have the output dtype")
+    if scaling_factors.stride(1) != 1 or zeros.stride() != scaling_factors.stride():
+        scaling_factors, zeros = scaling_factors.contiguous(), zeros.contiguous()
+    return scaling_factors, zeros
+
+
+# More rows than this: the weight is decoded to memory once and a library product reads it (K = 4096, bf16: N = 10240
+# 169 us in the kernel against 173 at 2048 rows, 241 against 200 at 3000; N = 4096 63 against 73, 108 against 91).
+_GEMM_MAX_ROWS = 2048
+
+
+def _product(x: torch.Tensor, kernel, scaling_factors, zeros, n: int, k: int, group_size: int) -> torch.Tensor:
+    """``x @ T(q * s + z).T`` for a 2-D ``x``: the weight decoded inside the GEMM (``svdq_awq_gemm_w4a16``), or decoded to
+    memory first where many rows share it."""
+    scaling_factors, zeros = _check_weight(kernel, scaling_factors, zeros, n, k, group_size, x.dtype)
+    m = x.shape[0]
+    if 0 < m <= _GEMM_MAX_ROWS and x.shape[1] == k:
+        if x.stride(1) != 1 or x.stride(0) % 8 or x.stride(0) < k or x.data_ptr() % 16:
+            x = x.contiguous()
+        out = torch.empty(m, n, dtype=x.dtype, device=x.device)
+        args = _lib.AwqGemvArgs(x=x.data_ptr(), qweight=kernel.data_ptr(), scales=scaling_factors.data_ptr(), zeros=zeros.data_ptr(),
+                                out=out.data_ptr(), M=m, N=n, K=k, ld_x=x.stride(0), ld_scales=scaling_factors.stride(0), ld_out=n,
+                                dtype=_lib.dtype_code(x.dtype))  # fmt: skip
+        with torch.cuda.device(x.device):
+            rc = _lib.load().svdq_awq_gemm_w4a16(args, group_size, _lib.stream_of(x))
+        if rc != _lib.E_UNSUPPORTED:  # tensors too large for its 32-bit offsets
+            _lib.check(rc)
+            return out
+    w = awq_dequantize(kernel, scaling_factors, zeros, n, k, group_size, x.dtype)
+    return torch.matmul(x, w.t())
+
+
 def awq_dequantize(
     kernel: torch.Tensor,
     scaling_factors: torch.Tensor,
@@ -136,18 +173,7 @@ def awq_dequantize(
     Unpack a TinyChat-packed AWQ W4 weight to a dense ``(n, k)`` tensor ``q * scaling_factors + zeros`` of ``dtype``
     (reference: nunchaku/ops/triton/awq.py:83-118).
     """
-    _lib.require_cuda(kernel, scaling_factors, zeros)
-    if kernel.element_size() * kernel.numel() != n * k // 2 or not kernel.is_contiguous():
-        raise ValueError(f"unexpected packed AWQ weight shape {tuple(kernel.shape)} for n={n}, k={k}")
-    if group_size <= 0 or k % group_size:
-        raise ValueError(f"group_size={group_size} does not divide k={k}")
-    groups = k // group_size
-    if scaling_factors.shape != (groups, n) or zeros.shape != (groups, n):
-        raise ValueError(f"scaling_factors / zeros must be ({groups}, {n})")
-    if scaling_factors.dtype != dtype or zeros.dtype != dtype:
-        raise ValueError("scaling_factors / zeros must have the output dtype")
-    if scaling_factors.stride(1) != 1 or zeros.stride() != scaling_factors.stride():
-        scaling_factors, zeros = scaling_factors.contiguous(), zeros.contiguous()
+    scaling_factors, zeros = _check_weight(kernel, scaling_factors, zeros, n, k, group_size, dtype)
     out = torch.empty(n, k, dtype=dtype, device=kernel.device)
     with torch.cuda.device(kernel.device):
         _lib.check(_lib.load().svdq_awq_dequantize(kernel.data_ptr(), scaling_factors.data_ptr(), zeros.data_ptr(),
@@ -164,15 +190,16 @@ def awq_gemm_w4a16(
     group_size: int = 128,
 ) -> torch.Tensor:
     """
-    AWQ W4A16 GEMM for larger batches (reference: nunchaku/ops/triton/awq.py:232-251): the weight is decoded once by
-    :func:`awq_dequantize`, the product is a dense library matmul.
+    AWQ W4A16 GEMM for larger batches (reference: nunchaku/ops/triton/awq.py:232-251, there a dense decode and a library
+    product): up to 2048 rows the weight is decoded, and rounded to the input dtype, inside the GEMM; with more it is
+    decoded to memory once by :func:`awq_dequantize` for a library product.
     """
+    _lib.require_cuda(in_feats, kernel, scaling_factors, zeros)
     shape = in_feats.shape
     k = shape[-1]
     x = in_feats.reshape(-1, k)
     n = scaling_factors.shape[-1]
-    w = awq_dequantize(kernel, scaling_factors, zeros, n, k, group_size, x.dtype)
-    return torch.matmul(x, w.t()).reshape(*shape[:-1], n)
+    return _product(x, kernel, scaling_factors, zeros, n, k, group_size).reshape(*shape[:-1], n)
 
 
 def gemv_awq(in_feats, kernel, scaling_factors, zeros, m: int, n: int, k: int, group_size: int) -> torch.Tensor:

@@ -215,7 +215,9 @@ size_t svdq_lora_down_blocked_bytes(int32_t N, int32_t R2);
 /* The fp8 main loop exists in two builds: three workgroups per CU (fills a loaded CU best) and two per CU with
  * software-pipelined steps (a workgroup on its own runs faster); svdq_gemm_w4a4 picks by the number of 128x128 tiles and
  * CUs.  This overrides the choice for the whole process: -1 = by tile count (default), 0 = three per CU, 1 = two per CU.
- * For tuning and tests; results of the two are bit-identical.  No counterpart in the reference. */
+ * For tuning and tests; results of the two are bit-identical.  By default launches with few rows (unsigned activations or
+ * fp6 codes) go to a third kernel that splits K over wavefronts and adds the groups up in another order; forced builds do
+ * not.  No counterpart in the reference. */
 int svdq_gemm_w4a4_set_variant(int32_t variant);
 
 /*

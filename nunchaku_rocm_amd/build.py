@@ -10,17 +10,18 @@ import os
 import shutil
 import subprocess
 import sys
+import tempfile
+from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libsvdq_mi355x.so")
-SOURCES = ["common.hip", "quantize.hip", "gemm_w4a4.hip", "awq_gemv.hip", "awq_gemm.hip", "attention.hip", "layout.hip"]
+SOURCES = ["common.hip", "quantize.hip", "gemm_w4a4.hip", "gemm_w4a4_split.hip", "awq_gemv.hip", "awq_gemm.hip", "attention.hip", "layout.hip"]
 FLAGS = [
     "--offload-arch=gfx950",
     "-O3",
     "-std=c++17",
     "-fPIC",
-    "-shared",
     # packed fp32 VALU ops stay off: plain v_fma_f32 / v_mul_f32 only
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wno-unused-command-line-argument",
@@ -35,15 +36,21 @@ def hipcc() -> str:
 
 
 def build(verbose: bool = False) -> str:
-    cmd = [hipcc(), *FLAGS, *[os.path.join(CSRC, s) for s in SOURCES], "-o", LIB + ".tmp"]
-    if verbose:
-        print(" ".join(cmd), flush=True)
-    proc = subprocess.run(cmd, capture_output=True, text=True)
-    err = "\n".join(ln for ln in proc.stderr.splitlines() if "not a recognized feature" not in ln)
-    if proc.returncode != 0:
-        raise RuntimeError(f"hipcc failed ({proc.returncode}):\n{err}")
-    if verbose and err.strip():
-        print(err, file=sys.stderr)
+    def run(cmd: list[str]) -> None:
+        if verbose:
+            print(" ".join(cmd), flush=True)
+        proc = subprocess.run(cmd, capture_output=True, text=True)
+        err = "\n".join(ln for ln in proc.stderr.splitlines() if "not a recognized feature" not in ln)
+        if proc.returncode != 0:
+            raise RuntimeError(f"hipcc failed ({proc.returncode}):\n{err}")
+        if verbose and err.strip():
+            print(err, file=sys.stderr)
+
+    # one compiler process per source file: the kernels' instantiations are what takes the time
+    with tempfile.TemporaryDirectory() as tmp, ThreadPoolExecutor(min(len(SOURCES), os.cpu_count() or 1)) as pool:
+        objs = [os.path.join(tmp, s + ".o") for s in SOURCES]
+        list(pool.map(run, [[hipcc(), *FLAGS, "-c", os.path.join(CSRC, s), "-o", o] for s, o in zip(SOURCES, objs)]))
+        run([hipcc(), *FLAGS, "-shared", *objs, "-o", LIB + ".tmp"])
     os.replace(LIB + ".tmp", LIB)
     return LIB
 

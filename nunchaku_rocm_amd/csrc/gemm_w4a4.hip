@@ -54,6 +54,7 @@
 #include <atomic>
 #include <type_traits>
 
+#include "gemm_w4a4_split.h"
 #include "gemm_w4a4_tile.h"
 
 namespace svdq {
@@ -766,6 +767,8 @@ static void launch_gemm_f8p(const svdq_gemm_args &a, hipStream_t s) {
 template <typename T, bool U>
 static void launch_gemm_f8(const svdq_gemm_args &a, hipStream_t s) {
     const bool two = two_workgroups_per_cu((long)((a.M + BM - 1) / BM) * ((a.N + BN - 1) / BN));
+    // few rows: K split over the wavefronts of smaller workgroups (a forced build of this loop means this loop)
+    if ((U || a.act_blocked == 2) && g_f8_variant.load(std::memory_order_relaxed) < 0 && launch_gemm_split(a, cu_count(), s)) return;
     if (a.act_blocked == 2) {  // fp6 codes carry their sign: one instantiation for signed and unsigned activations
         if (a.ascales_blocked) {
             if (two)

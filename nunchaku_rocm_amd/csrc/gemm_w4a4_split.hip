@@ -1,0 +1,244 @@
+// W4A4 GEMM for launches with few rows: a workgroup owns 32 rows x 128 columns and its eight or four wavefronts split K.
+//
+// F6ACT: activations as fp6 codes (act_blocked == 2), signed or not; otherwise unsigned nibbles, as the (M, K / 2) matrix or
+// in lane order, unpacked to fp8 codes: the same integers and the same sums, so that all hand-over forms of unsigned
+// activations give the same bits.  (Signed nibbles need the offset correction and stay with the tiles.)  Same arithmetic as gemm_w4a4_f8_kernel (per group one fp6 x fp6 or fp6 x fp8 matrix
+// instruction = the exact integer dot product, one 16-bit matrix instruction = the product of the two scales, one fp32
+// FMA per output); only the order of the fp32 sums over groups differs (a partial sum per wavefront).
+//
+// Why: with 128 x 128 tiles a prompt's 512 rows give a 3072-wide layer 96 workgroups on 256 CUs, each alone on its CU with
+// one wavefront per SIMD and a barrier per 128 k.  Here the same layer has 384 workgroups and a wavefront runs a quarter of
+// K (an eighth where no CU gets a second workgroup: two wavefronts per SIMD either way).  What bounds it: every workgroup streams its own copy of the weight tile from L2 (there is no second row block in the
+// workgroup to share it with), 64 bytes per clock and CU at best, which is why large launches stay with the tiles.
+//
+//  * Nothing is shared between the wavefronts of a workgroup inside the loop, so weights go straight to registers (they lie
+//    in the matrix instruction's lane order) and there is neither LDS nor a barrier in it; a stage (two groups) is
+//    requested one stage ahead: 16 KB in flight per wavefront.
+//  * Wavefront w takes stages w, w + WAVES, ...: the workgroup reads a contiguous stretch of the weight at a time.
+//  * The partial tiles meet in LDS: wavefront w < 4 adds up column block w in a fixed order (the result does not depend on
+//    timing), the sums go to wavefront 0, which owns the whole 32 x 128 tile for the epilogue as in the other kernels.
+//  * Workgroups of one column tile are neighbours on one XCD, so that a weight tile is fetched into one L2.
+#include <type_traits>
+
+#include "gemm_w4a4_split.h"
+#include "gemm_w4a4_tile.h"
+
+namespace svdq {
+
+constexpr int SK_BLOCK_BYTES = 16 * 64 * 4;  // one 32 x 32 fp32 block, 16 registers of 64 lanes
+
+template <typename T, int EPI, int WAVES, bool F6ACT>
+__global__ __launch_bounds__(WAVES * 64, 2) void gemm_w4a4_split_kernel(svdq_gemm_args a, int tiles_m) {
+    static_assert(WAVES >= NBN && NBN == NWAVES, "wavefront w < 4 adds up column block w");
+    __shared__ __align__(16) uint8_t sred[NBN * (WAVES - 1) * SK_BLOCK_BYTES];  // [column block][the other wavefronts]
+    __shared__ __align__(16) uint8_t sepi[EPI_LDS_BYTES];
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l32 = lane & 31, half = lane >> 5;
+
+    // XCD-contiguous renumbering (ids are dealt round-robin over the XCDs), then the row blocks of a column tile in a row
+    const int nb = gridDim.x, xcd = blockIdx.x % NUM_XCD, loc = blockIdx.x / NUM_XCD;
+    const int per = (nb + NUM_XCD - 1) / NUM_XCD, rem = nb % NUM_XCD;
+    const int id = ((rem == 0 || xcd < rem) ? xcd * per : rem * per + (xcd - rem) * (per - 1)) + loc;
+    const int pid_m = id % tiles_m, pid_n = id / tiles_m;
+    const int m0 = pid_m * 32, n0 = pid_n * BN;
+    const int G = a.K / GROUP, nst = (G + 1) / 2;
+    const int count = (nst - wave + WAVES - 1) / WAVES;  // this wavefront's stages (none where K is short)
+
+    // operands, all through raw buffers: base in SGPRs + per-lane offset + scalar offset of block and stage.  A column block
+    // past N re-reads the last one (its outputs are never stored).
+    const int b0 = n0 / 32, blast = (a.N + 31) / 32 - 1;
+    const __amdgpu_buffer_rsrc_t rW = g_buffer((const uint8_t *)a.wgt_planes + (size_t)b0 * nst * (WPL_BLOCKS * BLK_BYTES));
+    const __amdgpu_buffer_rsrc_t rX =
+        g_buffer((const uint8_t *)a.wgt_planes + planes_code_bytes(a.N, a.K) + (size_t)b0 * (nst + 1) * AUX_BLK);
+    const bool ablk = F6ACT || a.act_blocked != 0;
+    const uint32_t sA = F6ACT ? 1536u : ablk ? 1024u : 32u;  // a step of one group
+    const int mrow = min(m0 + l32, a.M - 1);
+    const __amdgpu_buffer_rsrc_t rA = g_buffer((const uint8_t *)a.act + (ablk ? (size_t)pid_m * G * sA : (size_t)m0 * a.ld_act));
+    const uint32_t oA = ablk ? (uint32_t)lane * 16u : (uint32_t)(mrow - m0) * (uint32_t)a.ld_act + half * 16;
+    // activation scales: with ascales_blocked eight groups of a row lie side by side, 512 bytes per 32 rows
+    const bool sblk = a.ascales_blocked != 0;
+    const __amdgpu_buffer_rsrc_t rS = g_buffer((const uint8_t *)a.ascales + (sblk ? (size_t)pid_m * (G >> 3) * 512 : 0));
+    const uint32_t s1 = sblk ? 2u : 2u * (uint32_t)a.ld_ascales, s8 = sblk ? 512u : 8u * s1;  // steps of one and of eight groups
+    const uint32_t oS = sblk ? (uint32_t)l32 * 16u : 2u * (uint32_t)mrow;
+    uint32_t wblk[NBN], xblk[NBN];
+#pragma unroll
+    for (int bn = 0; bn < NBN; bn++) {
+        const uint32_t b = (uint32_t)(min(b0 + bn, blast) - b0);
+        wblk[bn] = b * (uint32_t)nst * (uint32_t)(WPL_BLOCKS * BLK_BYTES);
+        xblk[bn] = b * (uint32_t)(nst + 1) * (uint32_t)AUX_BLK;
+    }
+    const uint32_t l16 = (uint32_t)lane * 16u, l8 = 1024u + (uint32_t)lane * 8u;
+    const uint32_t oX = (uint32_t)l32 * AUX_ROW + 8u;
+
+    v4i w[2][NBN][WPL_BLOCKS], alo[2][2];
+    v2i ahi[2][2];
+    int ws[2][NBN];
+    uint16_t as[2][2];
+    auto load = [&](auto set_tag, int i) {  // the wavefront's i-th stage
+        constexpr int S = decltype(set_tag)::value;
+        const uint32_t s = (uint32_t)(i * WAVES + wave);
+#pragma unroll
+        for (int gg = 0; gg < 2; gg++) {  // a group past the end (K / 64 odd) re-reads the last one: its weights are zeros
+            const uint32_t g = min(2 * s + gg, (uint32_t)G - 1);
+            alo[S][gg] = g_load128(rA, oA, g * sA);
+            if constexpr (F6ACT) ahi[S][gg] = g_load64(rA, l8, g * sA);
+            as[S][gg] = g_load16(rS, oS, (g >> 3) * s8 + (g & 7) * s1);
+        }
+#pragma unroll
+        for (int bn = 0; bn < NBN; bn++) ws[S][bn] = __builtin_amdgcn_raw_buffer_load_b32(rX, (int)oX, (int)(xblk[bn] + s * AUX_BLK), 0);
+#pragma unroll
+        for (int bn = 0; bn < NBN; bn++)
+#pragma unroll
+            for (int p = 0; p < WPL_BLOCKS; p++)
+                w[S][bn][p] = g_load128(rW, l16, wblk[bn] + s * (uint32_t)(WPL_BLOCKS * BLK_BYTES) + (uint32_t)(p * BLK_BYTES));
+        __builtin_amdgcn_sched_barrier(0);
+    };
+
+    v16f acc[NBN];
+#pragma unroll
+    for (int bn = 0; bn < NBN; bn++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) acc[bn][i] = 0.0f;
+    const v16f z16 = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+    auto compute = [&](auto set_tag) {
+        constexpr int S = decltype(set_tag)::value;
+        // scale product of group gg: the activation side carries its scale in that group's K slot and zeros elsewhere
+        const v2i sa[2] = {(v2i){half ? 0 : (int)as[S][0], 0}, (v2i){half ? 0 : (int)((uint32_t)as[S][1] << 16), 0}};
+        v8i am[2];
+#pragma unroll
+        for (int gg = 0; gg < 2; gg++) {
+            if constexpr (F6ACT) {
+                am[gg] = (v8i){alo[S][gg][0], alo[S][gg][1], alo[S][gg][2], alo[S][gg][3], ahi[S][gg][0], ahi[S][gg][1], 0, 0};
+            } else {  // even nibbles, then odd ones, as in gemm_w4a4_f8_kernel
+                const v4i e = alo[S][gg] & 0x0F0F0F0F, o = (alo[S][gg] >> 4) & 0x0F0F0F0F;
+                am[gg] = (v8i){e[0], e[1], e[2], e[3], o[0], o[1], o[2], o[3]};
+            }
+        }
+#pragma unroll
+        for (int b = 0; b < 2 * NBN; b++) {
+            const int gg = b & 1, bn = b >> 1;
+            const v8i w6 = {w[S][bn][gg][0], w[S][bn][gg][1], w[S][bn][gg][2], w[S][bn][gg][3], w[S][bn][2][2 * gg], w[S][bn][2][2 * gg + 1], 0, 0};
+            const v16f sc = mfma32_16bit_k8<T>((v2i){ws[S][bn], 0}, sa[gg], z16);
+            v16f p;
+            if constexpr (F6ACT)
+                p = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(w6, am[gg], z16, 2, 2, 0, F6_SCALE, 0, F6_SCALE);
+            else
+                p = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(w6, am[gg], z16, 2, 0, 0, F6_SCALE, 0, F8_SCALE);
+#pragma unroll
+            for (int i = 0; i < 16; i++) acc[bn][i] = __builtin_fmaf(p[i], sc[i], acc[bn][i]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    const std::integral_constant<int, 0> S0;
+    const std::integral_constant<int, 1> S1;
+    if (count > 0) load(S0, 0);
+    if (wave < NWAVES) fetch_epilogue_operands<EPI>(a, sepi, n0, wave, lane);
+    int i = 0;
+    for (; i + 1 < count; i += 2) {  // past the end: the last stage again
+        load(S1, i + 1);
+        compute(S0);
+        load(S0, min(i + 2, count - 1));
+        compute(S1);
+    }
+    if (i < count) compute(S0);
+
+    // ---- partial sums: block bn of wavefront v lands at slot (bn, v < bn ? v : v - 1) ----------------------------------
+#pragma unroll
+    for (int bn = 0; bn < NBN; bn++)
+        if (bn != wave) {
+            uint8_t *p = sred + (bn * (WAVES - 1) + (wave < bn ? wave : wave - 1)) * SK_BLOCK_BYTES + lane * 16;
+#pragma unroll
+            for (int j = 0; j < 4; j++) *(v4f *)(p + j * 1024) = (v4f){acc[bn][4 * j], acc[bn][4 * j + 1], acc[bn][4 * j + 2], acc[bn][4 * j + 3]};
+        }
+    __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, 0));  // (also: this wavefront's share of the epilogue operands has landed)
+    __syncthreads();
+    if (wave < NBN) {
+        v16f mine = acc[0];
+#pragma unroll
+        for (int bn = 1; bn < NBN; bn++)
+            if (bn == wave) mine = acc[bn];
+        uint8_t *p = sred + wave * (WAVES - 1) * SK_BLOCK_BYTES + lane * 16;
+#pragma unroll
+        for (int v = 0; v < WAVES - 1; v++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const v4f t = *(const v4f *)(p + v * SK_BLOCK_BYTES + j * 1024);
+#pragma unroll
+                for (int e = 0; e < 4; e++) mine[4 * j + e] += t[e];
+            }
+        if (wave != 0) {
+#pragma unroll
+            for (int j = 0; j < 4; j++) *(v4f *)(p + j * 1024) = (v4f){mine[4 * j], mine[4 * j + 1], mine[4 * j + 2], mine[4 * j + 3]};
+        } else {
+            acc[0] = mine;
+        }
+    }
+    __syncthreads();
+    if (wave != 0) return;
+#pragma unroll
+    for (int bn = 1; bn < NBN; bn++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const v4f t = *(const v4f *)(sred + bn * (WAVES - 1) * SK_BLOCK_BYTES + lane * 16 + j * 1024);
+#pragma unroll
+            for (int e = 0; e < 4; e++) acc[bn][4 * j + e] = t[e];
+        }
+    // block 0's slots (12 KB or more) were read before the second barrier: wavefront 0's private epilogue memory
+    static_assert(PRIV_BYTES <= (WAVES - 1) * SK_BLOCK_BYTES, "the epilogue's private memory must not reach the sums of block 1");
+    tile_epilogue<T, EPI, true>(a, acc, sred, sepi, m0, n0, pid_n, 0, lane);
+}
+
+template <typename T, int WAVES, bool F6ACT>
+static void launch_split(const svdq_gemm_args &a, int tiles_m, hipStream_t s) {
+    const dim3 grid((unsigned)tiles_m * (unsigned)((a.N + BN - 1) / BN)), block(WAVES * 64);
+    switch (a.epilogue) {
+        case SVDQ_EPI_PLAIN:
+            hipLaunchKernelGGL((gemm_w4a4_split_kernel<T, SVDQ_EPI_PLAIN, WAVES, F6ACT>), grid, block, 0, s, a, tiles_m);
+            break;
+        case SVDQ_EPI_QK_NORM_ROPE:
+            hipLaunchKernelGGL((gemm_w4a4_split_kernel<T, SVDQ_EPI_QK_NORM_ROPE, WAVES, F6ACT>), grid, block, 0, s, a, tiles_m);
+            break;
+        case SVDQ_EPI_GELU_QUANT:
+            hipLaunchKernelGGL((gemm_w4a4_split_kernel<T, SVDQ_EPI_GELU_QUANT, WAVES, F6ACT>), grid, block, 0, s, a, tiles_m);
+            break;
+        case SVDQ_EPI_SWIGLU_QUANT:
+            hipLaunchKernelGGL((gemm_w4a4_split_kernel<T, SVDQ_EPI_SWIGLU_QUANT, WAVES, F6ACT>), grid, block, 0, s, a, tiles_m);
+            break;
+    }
+}
+
+template <typename T>
+static void launch_split_type(const svdq_gemm_args &a, int tiles_m, bool wide, hipStream_t s) {
+    if (a.act_blocked == 2)
+        wide ? launch_split<T, 8, true>(a, tiles_m, s) : launch_split<T, 4, true>(a, tiles_m, s);
+    else
+        wide ? launch_split<T, 8, false>(a, tiles_m, s) : launch_split<T, 4, false>(a, tiles_m, s);
+}
+
+// Row blocks a launch has to run: the requantizing epilogues write all M rows, the others those below actual_m only.
+static int row_blocks(const svdq_gemm_args &a) {
+    const bool quant = a.epilogue == SVDQ_EPI_GELU_QUANT || a.epilogue == SVDQ_EPI_SWIGLU_QUANT;
+    return ((quant ? a.M : a.actual_m) + 31) / 32;
+}
+
+// Two workgroups fit a CU (256 registers a wavefront).  Up to that many the split is faster than the tiles, beyond it each
+// further round streams the weight tiles again.  PLAIN launch in us, this kernel / the faster tile build (bf16, rank 32):
+//   K = 3072,  N = 3072:  512 rows (384 workgroups) 16.4 / 18.3;  768 rows (576) 24.2 / 18.5
+//   K = 12288, N = 3072:  512 rows 45.2 / 63.4;  768 rows 70.7 / 63.5
+//   K = 2048,  N = 2048:  1024 rows (512) 13.5 / 13.7;  1536 rows (768) 20.0 / 14.0
+// With at most one workgroup per CU eight wavefronts share its K, so that every SIMD still has two (K = 12288, N = 3072, 256
+// rows: 27.8 us with eight, 32.9 with four, 64.0 as tiles; K = 6144, N = 1536, 512 rows: 17.3, 19.1, 32.6).
+bool launch_gemm_split(const svdq_gemm_args &a, int cus, hipStream_t s) {
+    const int tiles_m = row_blocks(a);
+    const long wgs = (long)tiles_m * ((a.N + BN - 1) / BN);
+    if (wgs > 2L * cus || (uint64_t)NBN * (a.K / 128 + 1) * (WPL_BLOCKS * BLK_BYTES) >= (1ull << 32)) return false;
+    if (a.dtype == SVDQ_BF16)
+        launch_split_type<BF16>(a, tiles_m, wgs <= cus, s);
+    else
+        launch_split_type<FP16>(a, tiles_m, wgs <= cus, s);
+    return true;
+}
+
+}  // namespace svdq

@@ -7,6 +7,7 @@ goes on torch's current HIP stream of the tensor's device, as the reference's na
 
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import os
 
@@ -194,11 +195,31 @@ def ptr(t: torch.Tensor | None):
     return None if t is None else t.data_ptr()
 
 
-def stream_of(t: torch.Tensor):
-    return torch.cuda.current_stream(t.device).cuda_stream
+def stream_of(t: torch.Tensor) -> int:
+    """The handle of the stream that is current on ``t``'s device (without the ``torch.cuda.Stream`` object, whose
+    construction costs more than the launch it is for)."""
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
+
+
+_CURRENT = contextlib.nullcontext()
+
+
+def on_device(device: torch.device):
+    """``torch.cuda.device(device)``, which switches twice per call, only where another device is current."""
+    return _CURRENT if torch.cuda.current_device() == device.index else torch.cuda.device(device)
 
 
 def require_cuda(*tensors: torch.Tensor | None) -> torch.device:
+    first, same = None, True
+    for t in tensors:
+        if t is None:
+            continue
+        if first is None:
+            first, index = t, t.get_device()
+        elif t.get_device() != index:
+            same = False
+    if same and first is not None and first.is_cuda:
+        return first.device
     devs = {t.device for t in tensors if t is not None}
     if len(devs) != 1:
         raise ValueError(f"tensors on different devices: {sorted(map(str, devs))}")

@@ -47,14 +47,14 @@ class _Ready:
 
 
 def _source_of(t: torch.Tensor) -> tuple:
-    """What identifies the bytes a copy was derived from: version counter, the storage (kept alive) and the view."""
-    return (t._version, t.untyped_storage(), t.storage_offset(), tuple(t.shape), tuple(t.stride()))
+    """What identifies the bytes a copy was derived from: version counter, first element's address, the view, and the
+    storage, held so that its address is not given to another tensor."""
+    return (t._version, t.data_ptr(), t.storage_offset(), t.shape, t.stride(), t.untyped_storage())
 
 
 def _same_source(src: tuple, t: torch.Tensor) -> bool:
-    version, storage, offset, shape, stride = src
-    return (version == t._version and storage.data_ptr() == t.untyped_storage().data_ptr() and offset == t.storage_offset()
-            and shape == tuple(t.shape) and stride == tuple(t.stride()))  # fmt: skip
+    # (equal first elements at equal offsets are equal storages; asking for the storage itself builds an object each time)
+    return src[1] == t.data_ptr() and src[0] == t._version and src[2] == t.storage_offset() and src[3] == t.shape and src[4] == t.stride()
 
 
 def invalidate(t: torch.Tensor) -> None:

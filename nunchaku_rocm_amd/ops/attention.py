@@ -37,7 +37,7 @@ def attention_fp16(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: torch.T
         sob=o.stride(0), som=o.stride(1),
         B=B, H=H, Tq=Tq, Tkv=Tkv, D=D, dtype=_lib.dtype_code(q.dtype), scale=float(scale),
     )  # fmt: skip
-    with torch.cuda.device(q.device):
+    with _lib.on_device(q.device):
         _lib.check(lib.svdq_attention_fp16(args, _lib.stream_of(q)))
 
 

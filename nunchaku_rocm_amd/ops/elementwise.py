@@ -47,7 +47,7 @@ def gated_residual(
     if gate.stride(1) < 1 or (gate.stride(1) == 1 and (gate.stride(0) % 8 or gate.data_ptr() % 16)):
         gate = gate.contiguous()
     stats = torch.empty(B * S, 2, dtype=torch.float32, device=x.device) if want_stats else None
-    with torch.cuda.device(x.device):
+    with _lib.on_device(x.device):
         _lib.check(_lib.load().svdq_gated_residual(
             x2.data_ptr(), gate.data_ptr(), ya.data_ptr(), _lib.ptr(yb), o2.data_ptr(), _lib.ptr(stats), B * S, C,
             x2.stride(0), ya.stride(0), o2.stride(0), S if B > 1 else 0, gate.stride(0), gate.stride(1),

@@ -335,7 +335,7 @@ def svdq_gemm_w4a4_cuda(
                 args.oscales_blocked = 1
         args.shift = 0.0 if fuse_swiglu else GELU_SHIFT
 
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         entry = lib.svdq_gemm_w4a4_static_scratch if STATIC_SCRATCH else lib.svdq_gemm_w4a4
         _lib.check(entry(args, _lib.stream_of(act)))
     return None
@@ -348,7 +348,7 @@ def group_acc_i32(act: torch.Tensor, wgt: torch.Tensor, group: int, act_unsigned
     dev = _lib.require_cuda(act, wgt)
     M, K, N = act.shape[0], act.shape[1] * 2, wgt.shape[0]
     out = torch.empty(M, N, dtype=torch.int32, device=dev)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         _lib.check(
             _lib.load().svdq_group_acc_i32(
                 act.data_ptr(), wgt.data_ptr(), out.data_ptr(), M, N, K, act.stride(0), wgt.stride(0), group,

@@ -45,7 +45,7 @@ def awq_gemv_w4a16_cuda(
         raise RuntimeError(f"AWQ weight of {n * k // 2} bytes: 4 GiB and more are not supported (32-bit offsets)")
     out = torch.empty(m, n, dtype=x.dtype, device=x.device)
     lib = _lib.load()
-    with torch.cuda.device(x.device):
+    with _lib.on_device(x.device):
         for r0 in range(0, m, _MAX_ROWS):
             rows = min(_MAX_ROWS, m - r0)
             args = _lib.AwqGemvArgs(
@@ -113,7 +113,7 @@ class AwqGemvBatch:
 
     def __call__(self, in_feats: torch.Tensor) -> torch.Tensor:
         self.x.copy_(in_feats.reshape(self.m, self.k))
-        with torch.cuda.device(self.x.device):
+        with _lib.on_device(self.x.device):
             _lib.check(_lib.load().svdq_awq_gemv_w4a16_batched(self._first, self._table.data_ptr(), self.count, _lib.stream_of(self.x)))
         return self.out
 
@@ -151,7 +151,7 @@ def _product(x: torch.Tensor, kernel, scaling_factors, zeros, n: int, k: int, gr
         args = _lib.AwqGemvArgs(x=x.data_ptr(), qweight=kernel.data_ptr(), scales=scaling_factors.data_ptr(), zeros=zeros.data_ptr(),
                                 out=out.data_ptr(), M=m, N=n, K=k, ld_x=x.stride(0), ld_scales=scaling_factors.stride(0), ld_out=n,
                                 dtype=_lib.dtype_code(x.dtype))  # fmt: skip
-        with torch.cuda.device(x.device):
+        with _lib.on_device(x.device):
             rc = _lib.load().svdq_awq_gemm_w4a16(args, group_size, _lib.stream_of(x))
         if rc != _lib.E_UNSUPPORTED:  # tensors too large for its 32-bit offsets
             _lib.check(rc)
@@ -175,7 +175,7 @@ def awq_dequantize(
     """
     scaling_factors, zeros = _check_weight(kernel, scaling_factors, zeros, n, k, group_size, dtype)
     out = torch.empty(n, k, dtype=dtype, device=kernel.device)
-    with torch.cuda.device(kernel.device):
+    with _lib.on_device(kernel.device):
         _lib.check(_lib.load().svdq_awq_dequantize(kernel.data_ptr(), scaling_factors.data_ptr(), zeros.data_ptr(),
                                                    out.data_ptr(), n, k, group_size, scaling_factors.stride(0),
                                                    out.stride(0), _lib.dtype_code(dtype), _lib.stream_of(kernel)))  # fmt: skip

@@ -21,7 +21,7 @@ def layer_norm_stats(input: torch.Tensor, eps: float = 1e-6) -> torch.Tensor:
     if inp.stride(1) != 1 or inp.stride(0) % 8 or inp.data_ptr() % 16:
         inp = inp.contiguous()
     stats = torch.empty(inp.shape[0], 2, dtype=torch.float32, device=inp.device)
-    with torch.cuda.device(inp.device):
+    with _lib.on_device(inp.device):
         _lib.check(_lib.load().svdq_row_stats(inp.data_ptr(), stats.data_ptr(), inp.shape[0], inp.shape[1], inp.stride(0),
                                               _lib.dtype_code(inp.dtype), float(eps), _lib.stream_of(inp)))  # fmt: skip
     return stats
@@ -152,7 +152,7 @@ def quantize_w4a4_act_fuse_lora(
         out_blocked=min(out_blocked, 2),
         scales_blocked=int(out_blocked == 3),
     )
-    with torch.cuda.device(inp.device):
+    with _lib.on_device(inp.device):
         _lib.check(_lib.load().svdq_quantize_act(args, _lib.stream_of(inp)))
     return output, oscales, lora_act_out
 

@@ -32,7 +32,7 @@
 extern "C" {
 #endif
 
-#define SVDQ_ABI_VERSION 10
+#define SVDQ_ABI_VERSION 11
 
 enum { SVDQ_BF16 = 0, SVDQ_FP16 = 1 };
 enum { SVDQ_PRE_NONE = 0, SVDQ_PRE_GLU = 1, SVDQ_PRE_GELU = 2 }; /* svdq_quantize_args.prologue */
@@ -289,6 +289,9 @@ typedef struct {
 } svdq_awq_gemv_args;
 
 int svdq_awq_gemv_w4a16(const svdq_awq_gemv_args *args, void *stream);
+/* ... plus `bias` (N values of T, or NULL) on every row: the product is rounded to T, then the sum with the bias, as when the
+ * bias is added to the finished output (models/linear.py:392-399). */
+int svdq_awq_gemv_w4a16_bias(const svdq_awq_gemv_args *args, const void *bias, void *stream);
 
 /*
  * The same GEMV for `count` weights of one shape in a single launch (M <= 8).  The adaLN projections of a diffusion

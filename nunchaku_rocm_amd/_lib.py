@@ -15,7 +15,7 @@ import torch
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libsvdq_mi355x.so")
-ABI_VERSION = 10
+ABI_VERSION = 11
 
 BF16, FP16 = 0, 1
 EPI_PLAIN, EPI_QK_NORM_ROPE, EPI_GELU_QUANT, EPI_SWIGLU_QUANT = 0, 1, 2, 3
@@ -41,6 +41,7 @@ EXPORTS = (
     "svdq_weight_planes_bytes",
     "svdq_group_acc_i32",
     "svdq_awq_gemv_w4a16",
+    "svdq_awq_gemv_w4a16_bias",
     "svdq_awq_gemv_w4a16_batched",
     "svdq_awq_dequantize",
     "svdq_awq_gemm_w4a16",
@@ -146,6 +147,7 @@ def load() -> ctypes.CDLL:
     lib.svdq_gemm_w4a4_static_scratch_capacity.argtypes = []
     lib.svdq_gemm_w4a4_static_scratch_prepare.argtypes = []
     lib.svdq_awq_gemv_w4a16.argtypes = [ctypes.POINTER(AwqGemvArgs), _vp]
+    lib.svdq_awq_gemv_w4a16_bias.argtypes = [ctypes.POINTER(AwqGemvArgs), _vp, _vp]
     lib.svdq_awq_gemv_w4a16_batched.argtypes = [ctypes.POINTER(AwqGemvArgs), _vp, _i32, _vp]
     lib.svdq_awq_dequantize.argtypes = [_vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32, _vp]
     lib.svdq_awq_gemm_w4a16.argtypes = [ctypes.POINTER(AwqGemvArgs), _i32, _vp]

@@ -8,7 +8,7 @@ import torch
 from torch import nn
 
 from .ops.gemm import svdq_gemm_w4a4_cuda
-from .ops.gemv import awq_gemv_w4a16_cuda
+from .ops.gemv import awq_gemv_bias
 from .ops.quantize import svdq_quantize_w4a4_act_fuse_lora_cuda
 
 
@@ -173,12 +173,8 @@ class AWQW4A16Linear(nn.Module):
         self.wzeros = nn.Parameter(torch.empty(in_features // group_size, out_features, dtype=torch_dtype, device=device), requires_grad=False)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        output = awq_gemv_w4a16_cuda(in_feats=x, kernel=self.qweight, scaling_factors=self.wscales, zeros=self.wzeros,
-                                     m=x.shape[0], n=self.out_features, k=self.in_features, group_size=self.group_size)  # fmt: skip
-        if self.bias is not None:
-            view_shape = [1] * (output.ndim - 1) + [-1]
-            output.add_(self.bias.view(view_shape))
-        return output
+        return awq_gemv_bias(x, self.qweight, self.wscales, self.wzeros, self.bias, m=x.shape[0], n=self.out_features,
+                             k=self.in_features, group_size=self.group_size)  # fmt: skip
 
     @classmethod
     def from_linear(cls, linear: nn.Linear, group_size: int = 64, torch_dtype: torch.dtype = torch.bfloat16,

@@ -29,10 +29,16 @@ def awq_gemv_w4a16_cuda(
     are refused (``RuntimeError``): the kernels address them with 32-bit offsets.  Returns ``in_feats.shape[:-1] + (n,)``
     in the input dtype.
     """
+    return awq_gemv_bias(in_feats, kernel, scaling_factors, zeros, None, m, n, k, group_size)
+
+
+def awq_gemv_bias(in_feats, kernel, scaling_factors, zeros, bias: torch.Tensor | None, m: int, n: int, k: int, group_size: int = 64) -> torch.Tensor:
+    """:func:`awq_gemv_w4a16_cuda`, then ``+ bias`` (``(n,)``, rounded again as an addition of its own would) in the kernel's
+    last step where the fused kernel runs and the bias is a contiguous tensor of the output dtype that needs no gradient."""
     _lib.require_cuda(in_feats, kernel, scaling_factors, zeros)
     x = in_feats.reshape(m, k)
     if group_size != 64 or n % 32:
-        return _product(x, kernel, scaling_factors, zeros, n, k, group_size).reshape(*in_feats.shape[:-1], n)
+        return _plus_bias(_product(x, kernel, scaling_factors, zeros, n, k, group_size).reshape(*in_feats.shape[:-1], n), bias)
     if x.stride(1) != 1 or x.stride(0) % 8 or x.data_ptr() % 16:
         x = x.contiguous()
     if kernel.element_size() * kernel.numel() != n * k // 2 or not kernel.is_contiguous():
@@ -44,6 +50,10 @@ def awq_gemv_w4a16_cuda(
     if n * k // 2 >= 1 << 32:
         raise RuntimeError(f"AWQ weight of {n * k // 2} bytes: 4 GiB and more are not supported (32-bit offsets)")
     out = torch.empty(m, n, dtype=x.dtype, device=x.device)
+    fused = None  # the bias' address where the kernel adds it
+    if bias is not None and bias.dtype == x.dtype and bias.device == x.device and bias.shape == (n,) and bias.is_contiguous():
+        if not (bias.requires_grad and torch.is_grad_enabled()):
+            fused = bias.data_ptr()
     lib = _lib.load()
     with _lib.on_device(x.device):
         for r0 in range(0, m, _MAX_ROWS):
@@ -62,13 +72,18 @@ def awq_gemv_w4a16_cuda(
                 ld_out=out.stride(0),
                 dtype=_lib.dtype_code(x.dtype),
             )
-            rc = lib.svdq_awq_gemv_w4a16(args, _lib.stream_of(x))
+            rc = lib.svdq_awq_gemv_w4a16_bias(args, fused, _lib.stream_of(x))
             if rc == _lib.E_UNSUPPORTED:
                 # the kernel's per-group tables do not fit LDS (K = 12288 with more than 16 rows, longer K with fewer):
                 # the GEMM, as for other group sizes (the other refusal, a weight of 4 GiB and more, was raised above)
-                return _product(x, kernel, scaling_factors, zeros, n, k, group_size).reshape(*in_feats.shape[:-1], n)
+                return _plus_bias(_product(x, kernel, scaling_factors, zeros, n, k, group_size).reshape(*in_feats.shape[:-1], n), bias)
             _lib.check(rc)
-    return out.reshape(*in_feats.shape[:-1], n)
+    out = out.reshape(*in_feats.shape[:-1], n)
+    return out if fused else _plus_bias(out, bias)
+
+
+def _plus_bias(out: torch.Tensor, bias: torch.Tensor | None) -> torch.Tensor:
+    return out if bias is None else out.add_(bias.view([1] * (out.ndim - 1) + [-1]))
 
 
 class AwqGemvBatch:

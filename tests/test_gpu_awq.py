@@ -214,3 +214,29 @@ def test_dequantize_inverts_the_packing(dev, dtype, N, K, group_size):
     assert torch.equal(out.float().cpu(), q.float())
     out32 = ops.awq_dequantize(packed.view(torch.int32), ones, torch.zeros_like(ones), N, K, group_size, dtype)
     assert torch.equal(out32, out)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m,N,K", [(1, 64, 128), (2, 96, 3072), (4, 32, 64), (7, 64, 448), (9, 96, 320), (25, 32, 192), (40, 64, 128)])
+def test_module_bias_has_the_bits_of_an_addition(dev, m, N, K, dtype):
+    """The bias the kernels add in their last step: the bits of ``output.add_(bias)``; a bias the kernel does not take (a
+    strided one, one that wants its gradient) is added as before."""
+    from nunchaku_rocm_amd import ops
+    from nunchaku_rocm_amd.linear import AWQW4A16Linear
+
+    print(f"case m={m} N={N} K={K} {dtype}", flush=True)
+    lin = {k: v.to(dev) for k, v in O.make_awq_linear(K, N, dtype=dtype).items()}
+    mod = AWQW4A16Linear(K, N, torch_dtype=dtype, device=dev)
+    mod.qweight.data, mod.wscales.data, mod.wzeros.data = lin["qweight"].view(torch.int32).reshape(N // 4, K // 2), lin["wscales"], lin["wzeros"]
+    g = torch.Generator().manual_seed(m)
+    x = torch.randn(m, K, generator=g).to(dtype).to(dev)
+    bias = torch.randn(2 * N, generator=g).to(dtype).to(dev)
+    plain = ops.awq_gemv_w4a16_cuda(x, mod.qweight, mod.wscales, mod.wzeros, m, N, K)
+    for b in (bias[:N], bias[::2], bias[1 : N + 1]):
+        mod.bias.data = b
+        with torch.no_grad():
+            assert torch.equal(mod(x), plain + b)
+    out = mod(x)
+    assert out.requires_grad and torch.equal(out.detach(), plain + mod.bias.detach())
+    out.float().sum().backward()
+    assert torch.equal(mod.bias.grad, torch.full((N,), m, dtype=dtype, device=dev))

@@ -7,7 +7,8 @@ kept for as long as the weight tensor lives, is not modified in place and keeps 
 A cache entry holds a reference to the storage it was made from.  Assigning ``param.data = other`` changes neither the
 parameter object nor its version counter, and without that reference the allocator could hand the freed block to the
 next tensor of the same size, which would then look like the cached source; with it, an equal storage address means
-the same storage.
+the same storage, as long as the storage's address is looked up at each use (a held storage can still be resized to
+nothing, which gives its block back).
 
 A copy is made on the stream that is current at its first use.  A later use on another stream waits for the event
 recorded behind that launch (until it has completed once); the copy itself stays allocated while it is cached.
@@ -47,14 +48,18 @@ class _Ready:
 
 
 def _source_of(t: torch.Tensor) -> tuple:
-    """What identifies the bytes a copy was derived from: version counter, first element's address, the view, and the
-    storage, held so that its address is not given to another tensor."""
-    return (t._version, t.data_ptr(), t.storage_offset(), t.shape, t.stride(), t.untyped_storage())
+    """What identifies the bytes a copy was derived from: version counter, the storage (kept alive), the first element's place
+    in it, and the view."""
+    storage = t.untyped_storage()
+    return (t._version, storage, t.data_ptr() - storage.data_ptr(), t.shape, t.stride())
 
 
 def _same_source(src: tuple, t: torch.Tensor) -> bool:
-    # (equal first elements at equal offsets are equal storages; asking for the storage itself builds an object each time)
-    return src[1] == t.data_ptr() and src[0] == t._version and src[2] == t.storage_offset() and src[3] == t.shape and src[4] == t.stride()
+    # The held storage is asked where it is now: one that was resized to nothing gave its block back, and an address noted when
+    # the copy was made would fit the next tensor that got the block.  While it has its block, an address in it is in no
+    # other storage.  (``t``'s own storage is not asked for: that builds an object at each use.)
+    version, storage, place, shape, stride = src
+    return storage.data_ptr() + place == t.data_ptr() and version == t._version and shape == t.shape and stride == t.stride()
 
 
 def invalidate(t: torch.Tensor) -> None:

@@ -4,6 +4,7 @@ nunchaku/ops/gemv.py:10-56, nunchaku/ops/dispatch.py:19-49, nunchaku/ops/triton/
 from __future__ import annotations
 
 import torch
+from torch.autograd import forward_ad
 
 from .. import _lib
 
@@ -154,12 +155,23 @@ def _check_weight(kernel, scaling_factors, zeros, n: int, k: int, group_size: in
 _GEMM_MAX_ROWS = 2048
 
 
+def _is_plain(t: torch.Tensor) -> bool:
+    """Whether ``t`` is no more than the values in its memory: a kernel that is handed an address carries no gradient, tangent,
+    batch dimension of a transform, subclass or pending negation along."""
+    if t.requires_grad and torch.is_grad_enabled():
+        return False
+    if type(t) not in (torch.Tensor, torch.nn.Parameter) or t.is_neg() or torch._C._functorch.is_functorch_wrapped_tensor(t):
+        return False
+    return forward_ad._current_level < 0 or forward_ad.unpack_dual(t).tangent is None
+
+
 def _product(x: torch.Tensor, kernel, scaling_factors, zeros, n: int, k: int, group_size: int) -> torch.Tensor:
     """``x @ T(q * s + z).T`` for a 2-D ``x``: the weight decoded inside the GEMM (``svdq_awq_gemm_w4a16``), or decoded to
-    memory first where many rows share it."""
+    memory first for a library product where many rows share it or where ``x`` is more than its values: the product is
+    differentiable in ``x``, forward and backward, and can be mapped over it."""
     scaling_factors, zeros = _check_weight(kernel, scaling_factors, zeros, n, k, group_size, x.dtype)
     m = x.shape[0]
-    if 0 < m <= _GEMM_MAX_ROWS and x.shape[1] == k:
+    if 0 < m <= _GEMM_MAX_ROWS and x.shape[1] == k and _is_plain(x):
         if x.stride(1) != 1 or x.stride(0) % 8 or x.stride(0) < k or x.data_ptr() % 16:
             x = x.contiguous()
         out = torch.empty(m, n, dtype=x.dtype, device=x.device)
@@ -206,8 +218,9 @@ def awq_gemm_w4a16(
 ) -> torch.Tensor:
     """
     AWQ W4A16 GEMM for larger batches (reference: nunchaku/ops/triton/awq.py:232-251, there a dense decode and a library
-    product): up to 2048 rows the weight is decoded, and rounded to the input dtype, inside the GEMM; with more it is
-    decoded to memory once by :func:`awq_dequantize` for a library product.
+    product): up to 2048 rows the weight is decoded, and rounded to the input dtype, inside the GEMM; with more, or where
+    ``in_feats`` wants a gradient or is under a transform, it is decoded to memory once by :func:`awq_dequantize` for a
+    library product.
     """
     _lib.require_cuda(in_feats, kernel, scaling_factors, zeros)
     shape = in_feats.shape

@@ -1,0 +1,113 @@
+"""Which route a call of the AWQ product takes: the kernel that decodes the weight inside, or the decode to memory and a library
+product, which carries gradients, tangents, transforms and subclasses of the activations along."""
+
+import pytest
+import torch
+from torch.autograd import forward_ad
+
+from oracle import svdq_oracle as O
+
+N, K, GROUP = 64, 256, 128
+
+
+class _Marked(torch.Tensor):
+    pass
+
+
+def _weight(n=N, k=K, group=GROUP, dtype=torch.float16, seed=0):
+    g = torch.Generator().manual_seed(seed)
+    q = torch.randint(0, 16, (n, k), generator=g, dtype=torch.int32)
+    s = (torch.rand(k // group, n, generator=g) * 0.015 + 0.005).to(dtype)
+    z = (-torch.randint(0, 16, s.shape, generator=g).float() * s.float()).to(dtype)
+    packed = O.awq_pack(q)
+    return packed.view(torch.int32), s, z, O.awq_dequantize(packed, s, z, group)
+
+
+@pytest.fixture
+def routes(monkeypatch):
+    """The operators on CPU tensors: the decode by the oracle, the kernel's launch noted instead of made."""
+    from nunchaku_rocm_amd import _lib
+    from nunchaku_rocm_amd.ops import gemv
+
+    launches = []
+
+    class Stub:
+        def svdq_awq_gemm_w4a16(self, args, group, stream):
+            launches.append(args)
+            return 0
+
+        def svdq_awq_gemv_w4a16_bias(self, args, bias, stream):
+            launches.append((args, bias))
+            return 0
+
+    import contextlib
+
+    monkeypatch.setattr(_lib, "load", Stub)
+    monkeypatch.setattr(_lib, "require_cuda", lambda *t: torch.device("cpu"))
+    monkeypatch.setattr(_lib, "stream_of", lambda t: 0)
+    monkeypatch.setattr(_lib, "on_device", lambda d: contextlib.nullcontext())
+    monkeypatch.setattr(gemv, "awq_dequantize", lambda kernel, s, z, n, k, group, dtype: O.awq_dequantize(kernel.view(torch.int16), s, z, group))
+    return launches
+
+
+def test_plain_activations_take_the_kernel(routes):
+    from nunchaku_rocm_amd import ops
+
+    qw, s, z, _ = _weight()
+    x = torch.randn(5, K).half()
+    ops.awq_gemm_w4a16(x, qw, s, z, group_size=GROUP)
+    with torch.no_grad():  # nobody will ask for the gradient
+        ops.awq_gemm_w4a16(x.clone().requires_grad_(), qw, s, z, group_size=GROUP)
+    ops.awq_gemv_w4a16_cuda(x, qw, s, z, 5, N, K, group_size=GROUP)
+    with forward_ad.dual_level():  # a level is open, the activations have no part in it
+        ops.awq_gemm_w4a16(x, qw, s, z, group_size=GROUP)
+    assert len(routes) == 4
+
+
+def test_what_the_kernel_does_not_carry_is_carried_on(routes):
+    from nunchaku_rocm_amd import ops
+
+    qw, s, z, w = _weight()
+    x, t = torch.randn(5, K).half(), torch.randn(5, K).half()
+    call = lambda a: ops.awq_gemm_w4a16(a, qw, s, z, group_size=GROUP)  # noqa: E731
+    # the same product up to the order of K fp32 additions and the rounding to fp16
+    close = lambda a, b: torch.testing.assert_close(a.float(), b.float(), rtol=2.0**-9, atol=2e-2)  # noqa: E731
+
+    a = x.clone().requires_grad_()
+    call(a).backward(t[:, :N])
+    close(a.grad, t[:, :N] @ w)
+    with forward_ad.dual_level():
+        out = forward_ad.unpack_dual(call(forward_ad.make_dual(x, t)))
+        close(out.primal, x @ w.t())
+        close(out.tangent, t @ w.t())
+    close(torch.func.jvp(call, (x,), (t,))[1], t @ w.t())
+    close(torch.func.vmap(call)(torch.stack([x, t])), torch.stack([x, t]) @ w.t())
+    close(call(torch._neg_view(x)), -x @ w.t())
+    assert type(call(x.as_subclass(_Marked))) is _Marked
+    assert not routes
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m", [3, 300, 2048, 2049])
+def test_gradients_on_both_sides_of_the_row_limit(dev, m):
+    from nunchaku_rocm_amd.linear import AWQW4A16Linear
+
+    dtype = torch.bfloat16
+    qw, s, z, w = _weight(dtype=dtype)
+    mod = AWQW4A16Linear(K, N, group_size=GROUP, torch_dtype=dtype, device=dev)
+    mod.qweight.data, mod.wscales.data, mod.wzeros.data = qw.to(dev), s.to(dev), z.to(dev)
+    mod.bias.data.fill_(0.5)
+    g = torch.Generator().manual_seed(m)
+    x, grad = torch.randn(m, K, generator=g).to(dtype), torch.randn(m, N, generator=g).to(dtype)
+    a = x.to(dev).requires_grad_()
+    out = mod(a)
+    out.backward(grad.to(dev))
+    ref = grad.double() @ w.double()
+    # one rounding to bf16, and N fp32 additions of exact products in any order
+    bound = ref.abs() * 2.0**-8 + N * 2.0**-24 * (grad.double().abs() @ w.double().abs()) + 1e-6
+    assert ((a.grad.cpu().double() - ref).abs() <= bound).all()
+    with torch.no_grad():  # the kernel, where it runs: the same product before the bias within two roundings
+        plain = mod(a)
+    ref = x.double() @ w.double().t() + 0.5
+    bound = (ref.abs() + 1) * 2.0**-7 + K * 2.0**-24 * (x.double().abs() @ w.double().abs().t())
+    assert ((plain.cpu().double() - ref).abs() <= bound).all() and ((out.detach().cpu().double() - ref).abs() <= bound).all()

@@ -165,13 +165,17 @@ def _is_plain(t: torch.Tensor) -> bool:
     return forward_ad._current_level < 0 or forward_ad.unpack_dual(t).tangent is None
 
 
+def _cast_by_autocast(x: torch.Tensor) -> bool:
+    return torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") != x.dtype
+
+
 def _product(x: torch.Tensor, kernel, scaling_factors, zeros, n: int, k: int, group_size: int) -> torch.Tensor:
     """``x @ T(q * s + z).T`` for a 2-D ``x``: the weight decoded inside the GEMM (``svdq_awq_gemm_w4a16``), or decoded to
     memory first for a library product where many rows share it or where ``x`` is more than its values: the product is
-    differentiable in ``x``, forward and backward, and can be mapped over it."""
+    differentiable in ``x``, forward and backward, can be mapped over it, and follows an enclosing autocast."""
     scaling_factors, zeros = _check_weight(kernel, scaling_factors, zeros, n, k, group_size, x.dtype)
     m = x.shape[0]
-    if 0 < m <= _GEMM_MAX_ROWS and x.shape[1] == k and _is_plain(x):
+    if 0 < m <= _GEMM_MAX_ROWS and x.shape[1] == k and _is_plain(x) and not _cast_by_autocast(x):
         if x.stride(1) != 1 or x.stride(0) % 8 or x.stride(0) < k or x.data_ptr() % 16:
             x = x.contiguous()
         out = torch.empty(m, n, dtype=x.dtype, device=x.device)

@@ -111,3 +111,17 @@ def test_gradients_on_both_sides_of_the_row_limit(dev, m):
     ref = x.double() @ w.double().t() + 0.5
     bound = (ref.abs() + 1) * 2.0**-7 + K * 2.0**-24 * (x.double().abs() @ w.double().abs().t())
     assert ((plain.cpu().double() - ref).abs() <= bound).all() and ((out.detach().cpu().double() - ref).abs() <= bound).all()
+
+
+@pytest.mark.gpu
+def test_autocast_decides_on_the_type(dev):
+    from nunchaku_rocm_amd import ops
+
+    qw, s, z, w = (t.to(dev) for t in _weight(dtype=torch.bfloat16))
+    x = torch.randn(5, K, generator=torch.Generator().manual_seed(1)).to(torch.bfloat16).to(dev)
+    with torch.autocast("cuda", torch.float16):
+        out = ops.awq_gemm_w4a16(x, qw, s, z, group_size=GROUP)
+    assert out.dtype == torch.float16 and torch.equal(out, x.half() @ w.half().t())
+    with torch.autocast("cuda", torch.bfloat16):
+        assert torch.equal(ops.awq_gemm_w4a16(x, qw, s, z, group_size=GROUP), ops.awq_gemm_w4a16(x, qw, s, z, group_size=GROUP))
+    assert ops.awq_gemm_w4a16(x, qw, s, z, group_size=GROUP).dtype == torch.bfloat16

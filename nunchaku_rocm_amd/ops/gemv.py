@@ -169,6 +169,16 @@ def _cast_by_autocast(x: torch.Tensor) -> bool:
     return torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") != x.dtype
 
 
+def _aligned_rows(x: torch.Tensor) -> tuple[torch.Tensor, int]:
+    """The 2-D ``x`` with 16-byte aligned rows of unit stride, and the distance of its rows: itself, or a copy (``contiguous()``
+    makes none of a tensor that lies in one piece at an odd address).  The stride of a lone row means nothing."""
+    m, k = x.shape
+    ld = x.stride(0) if m > 1 else k
+    if x.stride(1) == 1 and ld >= k and ld % 8 == 0 and x.data_ptr() % 16 == 0:
+        return x, ld
+    return x.clone(memory_format=torch.contiguous_format), k
+
+
 def _product(x: torch.Tensor, kernel, scaling_factors, zeros, n: int, k: int, group_size: int) -> torch.Tensor:
     """``x @ T(q * s + z).T`` for a 2-D ``x``: the weight decoded inside the GEMM (``svdq_awq_gemm_w4a16``), or decoded to
     memory first for a library product where many rows share it or where ``x`` is more than its values: the product is
@@ -176,11 +186,10 @@ def _product(x: torch.Tensor, kernel, scaling_factors, zeros, n: int, k: int, gr
     scaling_factors, zeros = _check_weight(kernel, scaling_factors, zeros, n, k, group_size, x.dtype)
     m = x.shape[0]
     if 0 < m <= _GEMM_MAX_ROWS and x.shape[1] == k and _is_plain(x) and not _cast_by_autocast(x):
-        if x.stride(1) != 1 or x.stride(0) % 8 or x.stride(0) < k or x.data_ptr() % 16:
-            x = x.contiguous()
+        x, ld_x = _aligned_rows(x)
         out = torch.empty(m, n, dtype=x.dtype, device=x.device)
         args = _lib.AwqGemvArgs(x=x.data_ptr(), qweight=kernel.data_ptr(), scales=scaling_factors.data_ptr(), zeros=zeros.data_ptr(),
-                                out=out.data_ptr(), M=m, N=n, K=k, ld_x=x.stride(0), ld_scales=scaling_factors.stride(0), ld_out=n,
+                                out=out.data_ptr(), M=m, N=n, K=k, ld_x=ld_x, ld_scales=scaling_factors.stride(0), ld_out=n,
                                 dtype=_lib.dtype_code(x.dtype))  # fmt: skip
         with _lib.on_device(x.device):
             rc = _lib.load().svdq_awq_gemm_w4a16(args, group_size, _lib.stream_of(x))

@@ -125,3 +125,44 @@ def test_autocast_decides_on_the_type(dev):
     with torch.autocast("cuda", torch.bfloat16):
         assert torch.equal(ops.awq_gemm_w4a16(x, qw, s, z, group_size=GROUP), ops.awq_gemm_w4a16(x, qw, s, z, group_size=GROUP))
     assert ops.awq_gemm_w4a16(x, qw, s, z, group_size=GROUP).dtype == torch.bfloat16
+
+
+def _laid_out(x: torch.Tensor) -> dict:
+    """The values of ``x`` in the layouts the library product takes."""
+    m, k = x.shape
+    odd = torch.empty(1 + m * k, dtype=x.dtype, device=x.device)[1:].view(m, k)
+    wide = torch.empty(m, k + 4, dtype=x.dtype, device=x.device)[:, 2 : 2 + k]
+    padded = torch.empty(m, k + 8, dtype=x.dtype, device=x.device)[:, :k]
+    turned = torch.empty(k, m, dtype=x.dtype, device=x.device).t()
+    views = {"one piece at an odd address": odd, "odd columns": wide, "aligned rows apart": padded, "transposed": turned}
+    for v in views.values():
+        v.copy_(x)
+    views["one row over and over"] = x[:1].expand(m, k)
+    return views
+
+
+@pytest.mark.parametrize("m", [1, 2, 5])
+def test_rows_are_handed_over_aligned(routes, m):
+    from nunchaku_rocm_amd import ops
+
+    qw, s, z, _ = _weight()
+    views = _laid_out(torch.randn(m, K).half())
+    for name, x in views.items():
+        ops.awq_gemm_w4a16(x, qw, s, z, group_size=GROUP)
+        args = routes[-1]
+        assert args.x % 16 == 0 and args.ld_x >= K and args.ld_x % 8 == 0, name
+        if name == "aligned rows apart":
+            assert args.x == x.data_ptr() and (m == 1 or args.ld_x == K + 8)
+    assert len(routes) == len(views)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m", [1, 2, 40])
+def test_layouts_of_the_activations(dev, m):
+    from nunchaku_rocm_amd import ops
+
+    qw, s, z, _ = (t.to(dev) for t in _weight())
+    x = torch.randn(m, K, generator=torch.Generator().manual_seed(m)).half().to(dev)
+    for name, v in _laid_out(x).items():
+        print(f"case m={m} {name}", flush=True)
+        assert torch.equal(ops.awq_gemm_w4a16(v, qw, s, z, group_size=GROUP), ops.awq_gemm_w4a16(v.clone(memory_format=torch.contiguous_format), qw, s, z, group_size=GROUP))

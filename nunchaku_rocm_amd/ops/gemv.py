@@ -35,7 +35,8 @@ def awq_gemv_w4a16_cuda(
 
 def awq_gemv_bias(in_feats, kernel, scaling_factors, zeros, bias: torch.Tensor | None, m: int, n: int, k: int, group_size: int = 64) -> torch.Tensor:
     """:func:`awq_gemv_w4a16_cuda`, then ``+ bias`` (``(n,)``, rounded again as an addition of its own would) in the kernel's
-    last step where the fused kernel runs and the bias is a contiguous tensor of the output dtype that needs no gradient."""
+    last step where the fused kernel runs and the bias is a contiguous tensor of the output dtype and no more than its values
+    (a gradient or a tangent wanted through it: an addition of its own)."""
     _lib.require_cuda(in_feats, kernel, scaling_factors, zeros)
     x = in_feats.reshape(m, k)
     if group_size != 64 or n % 32:
@@ -52,9 +53,8 @@ def awq_gemv_bias(in_feats, kernel, scaling_factors, zeros, bias: torch.Tensor |
         raise RuntimeError(f"AWQ weight of {n * k // 2} bytes: 4 GiB and more are not supported (32-bit offsets)")
     out = torch.empty(m, n, dtype=x.dtype, device=x.device)
     fused = None  # the bias' address where the kernel adds it
-    if bias is not None and bias.dtype == x.dtype and bias.device == x.device and bias.shape == (n,) and bias.is_contiguous():
-        if not (bias.requires_grad and torch.is_grad_enabled()):
-            fused = bias.data_ptr()
+    if bias is not None and _is_plain(bias) and bias.dtype == x.dtype and bias.device == x.device and bias.shape == (n,) and bias.is_contiguous():
+        fused = bias.data_ptr()
     lib = _lib.load()
     with _lib.on_device(x.device):
         for r0 in range(0, m, _MAX_ROWS):

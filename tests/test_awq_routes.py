@@ -127,6 +127,24 @@ def test_autocast_decides_on_the_type(dev):
     assert ops.awq_gemm_w4a16(x, qw, s, z, group_size=GROUP).dtype == torch.bfloat16
 
 
+def test_a_bias_the_kernel_cannot_carry_is_added_behind_it(routes):
+    from nunchaku_rocm_amd.ops.gemv import awq_gemv_bias
+
+    qw, s, z, _ = _weight(group=64)
+    x, bias, tangent = torch.zeros(2, K).half(), torch.randn(N).half(), torch.randn(N).half()
+    call = lambda b: awq_gemv_bias(x, qw, s, z, b, 2, N, K)  # noqa: E731
+    call(bias)
+    assert routes[-1][1] == bias.data_ptr()
+    with forward_ad.dual_level():
+        call(bias)
+        assert routes[-1][1] == bias.data_ptr()
+        out = call(forward_ad.make_dual(bias, tangent))
+        assert torch.equal(forward_ad.unpack_dual(out).tangent, tangent.expand(2, N)) and routes[-1][1] is None
+    assert call(bias.clone().requires_grad_()).requires_grad and routes[-1][1] is None
+    call(torch._neg_view(bias))
+    assert routes[-1][1] is None
+
+
 def _laid_out(x: torch.Tensor) -> dict:
     """The values of ``x`` in the layouts the library product takes."""
     m, k = x.shape

@@ -157,11 +157,12 @@ __global__ __launch_bounds__(NS * 128, MB == 4 && NS == 2 ? 1 : 2) void awq_gemm
             const int par = u >> 2, pi = (u >> 1) & 1, b = u & 1;
             __builtin_amdgcn_sched_barrier(0);
             if (u == 4) {
+                // this wavefront's activations of stage s + 1 have landed: nothing younger is outstanding.  (The weights are asked
+                // for behind the wait.  A wait that leaves their six loads out would count loads that the compiler may drop or
+                // move; asked for before or after, a launch takes the same time.)  Behind the barrier everybody's have landed, and
+                // nobody reads stage s - 1 any more: its buffer takes stage s + 2 (past the end: the last stage again)
+                __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, 15));
                 load_w(min(s + 2, slast), w);  // all of them decoded: their registers take the stage after next
-                // this wavefront's activations of stage s + 1 have landed (its own new weight loads may not); behind the barrier
-                // everybody's have, and nobody reads stage s - 1 any more: its buffer takes stage s + 2 (past the end: the last
-                // stage again)
-                __builtin_amdgcn_s_waitcnt(waitcnt_imm(6, 15));
                 __builtin_amdgcn_s_barrier();
                 issue_x(min(s + 2, slast), fill);
             }
@@ -174,11 +175,14 @@ __global__ __launch_bounds__(NS * 128, MB == 4 && NS == 2 ? 1 : 2) void awq_gemm
         }
         __builtin_amdgcn_sched_barrier(0);
     };
+    // The first wait leaves out the block loads of stage 1 and nothing else: they are kept, and kept the youngest.
     issue_x(0, smem0);
     load_w(0, wa);
-    issue_x(min(1, slast), smem1);
     load_w(min(1, slast), wb);
-    __builtin_amdgcn_s_waitcnt(waitcnt_imm(XLOADS + 6, 15));
+    __builtin_amdgcn_sched_barrier(0);
+    issue_x(min(1, slast), smem1);
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(waitcnt_imm(XLOADS, 15));
     __builtin_amdgcn_s_barrier();
 #pragma unroll
     for (int m = 0; m < MB; m++) read_x(smem0, 0, m);

@@ -32,7 +32,7 @@
 extern "C" {
 #endif
 
-#define SVDQ_ABI_VERSION 11
+#define SVDQ_ABI_VERSION 12
 
 enum { SVDQ_BF16 = 0, SVDQ_FP16 = 1 };
 enum { SVDQ_PRE_NONE = 0, SVDQ_PRE_GLU = 1, SVDQ_PRE_GELU = 2 }; /* svdq_quantize_args.prologue */
@@ -216,9 +216,13 @@ size_t svdq_lora_down_blocked_bytes(int32_t N, int32_t R2);
  * software-pipelined steps (a workgroup on its own runs faster); svdq_gemm_w4a4 picks by the number of 128x128 tiles and
  * CUs.  This overrides the choice for the whole process: -1 = by tile count (default), 0 = three per CU, 1 = two per CU.
  * For tuning and tests; results of the two are bit-identical.  By default launches with few rows (unsigned activations or
- * fp6 codes) go to a third kernel that splits K over wavefronts and adds the groups up in another order; forced builds do
- * not.  No counterpart in the reference. */
+ * fp6 codes) go to a third kernel that splits K over wavefronts and adds the groups up in another order, so the last bit of
+ * a row's output may depend on how many rows the launch has (the same launch gives the same bits every time); forced
+ * builds do not.  No counterpart in the reference. */
 int svdq_gemm_w4a4_set_variant(int32_t variant);
+/* Over how many wavefronts (8 or 4) svdq_gemm_w4a4 splits K for `args` on a device of `cus` compute units (0: this one's);
+ * 0 = not split.  Host arithmetic on the sizes; for tests.  No counterpart in the reference. */
+int svdq_gemm_w4a4_split_wavefronts(const svdq_gemm_args *args, int32_t cus);
 
 /*
  * One-time re-layout of a weight for the GEMM.  Every (32-row block, pair of scale groups = one stage of the main

@@ -15,7 +15,7 @@ import torch
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libsvdq_mi355x.so")
-ABI_VERSION = 11
+ABI_VERSION = 12
 
 BF16, FP16 = 0, 1
 EPI_PLAIN, EPI_QK_NORM_ROPE, EPI_GELU_QUANT, EPI_SWIGLU_QUANT = 0, 1, 2, 3
@@ -29,6 +29,7 @@ EXPORTS = (
     "svdq_transpose_lora_down",
     "svdq_gemm_w4a4",
     "svdq_gemm_w4a4_set_variant",
+    "svdq_gemm_w4a4_split_wavefronts",
     "svdq_block_rotary",
     "svdq_rotary_blocked_bytes",
     "svdq_block_lora_down",
@@ -136,6 +137,7 @@ def load() -> ctypes.CDLL:
     lib.svdq_quantize_act.argtypes = [ctypes.POINTER(QuantizeArgs), _vp]
     lib.svdq_gemm_w4a4.argtypes = [ctypes.POINTER(GemmArgs), _vp]
     lib.svdq_gemm_w4a4_set_variant.argtypes = [_i32]
+    lib.svdq_gemm_w4a4_split_wavefronts.argtypes = [ctypes.POINTER(GemmArgs), _i32]
     lib.svdq_block_rotary.argtypes = [_vp, _vp, _i32, _i32, _vp]
     lib.svdq_rotary_blocked_bytes.restype = ctypes.c_size_t
     lib.svdq_rotary_blocked_bytes.argtypes = [_i32]

@@ -2,6 +2,8 @@
 #include <stdarg.h>
 #include <stdio.h>
 
+#include <atomic>
+
 #include "svdq_common.h"
 
 namespace svdq {
@@ -22,6 +24,17 @@ int check_launch(const char *what) {
         return SVDQ_E_LAUNCH;
     }
     return SVDQ_OK;
+}
+
+int cu_count() {
+    static std::atomic<int> cached{0};
+    int n = cached.load(std::memory_order_relaxed);
+    if (n > 0) return n;
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
+        n = 256;
+    cached.store(n, std::memory_order_relaxed);
+    return n;
 }
 
 }  // namespace svdq

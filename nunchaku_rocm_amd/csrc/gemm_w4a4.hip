@@ -722,16 +722,6 @@ static void launch_gemm_i8(const svdq_gemm_args &a, hipStream_t s) {
 // 1.4 / 2 (k = 1 / 2).  The constants are measured (K = 3072, N = 9216: M = 512 -> 288 tiles, M = 1024 -> 576, M = 4608 -> 2592;
 // K = 12288, N = 3072, M = 4608 -> 864), and the model picks as the measurements do: 2592, 3456, 4608 and 576 tiles -> three per
 // CU; 864 and 288 tiles -> two.
-static int cu_count() {
-    static std::atomic<int> cached{0};
-    int n = cached.load(std::memory_order_relaxed);
-    if (n > 0) return n;
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
-        n = 256;
-    cached.store(n, std::memory_order_relaxed);
-    return n;
-}
 static std::atomic<int> g_f8_variant{-1};  // svdq_gemm_w4a4_set_variant
 static bool two_workgroups_per_cu(long tiles) {
     const int forced = g_f8_variant.load(std::memory_order_relaxed);
@@ -743,6 +733,12 @@ static bool two_workgroups_per_cu(long tiles) {
     };
     const double last3[3] = {1.75, 2.15, 3.0}, last2[3] = {1.4, 2.0, 2.0};
     return cost(2, 2.16, last2) < cost(3, 3.0, last3);
+}
+
+// Few rows: K split over the wavefronts of smaller workgroups (a forced build of this loop means this loop).
+static int split_of(const svdq_gemm_args &a, int cus) {
+    if (!a.wgt_planes || !(a.act_unsigned || a.act_blocked == 2) || g_f8_variant.load(std::memory_order_relaxed) >= 0) return 0;
+    return split_wavefronts(a, cus);
 }
 
 template <typename T, bool U, bool PIPE, bool F6ACT, bool SB = false>
@@ -767,8 +763,10 @@ static void launch_gemm_f8p(const svdq_gemm_args &a, hipStream_t s) {
 template <typename T, bool U>
 static void launch_gemm_f8(const svdq_gemm_args &a, hipStream_t s) {
     const bool two = two_workgroups_per_cu((long)((a.M + BM - 1) / BM) * ((a.N + BN - 1) / BN));
-    // few rows: K split over the wavefronts of smaller workgroups (a forced build of this loop means this loop)
-    if ((U || a.act_blocked == 2) && g_f8_variant.load(std::memory_order_relaxed) < 0 && launch_gemm_split(a, cu_count(), s)) return;
+    if (const int wavefronts = split_of(a, cu_count())) {
+        launch_gemm_split(a, wavefronts, s);
+        return;
+    }
     if (a.act_blocked == 2) {  // fp6 codes carry their sign: one instantiation for signed and unsigned activations
         if (a.ascales_blocked) {
             if (two)
@@ -899,6 +897,10 @@ extern "C" int svdq_split_weight_planes(const void *wgt, const void *wscales, vo
         hipLaunchKernelGGL(weight_aux_kernel<FP16>, dim3((unsigned)((nd + 255) / 256)), dim3(256), 0, st,
                            (const uint8_t *)wgt, (const uint16_t *)wscales, (uint16_t *)aux, status, N, G, ld_wgt, ld_wscales);
     return check_launch("svdq_split_weight_planes (scales and offset terms)");
+}
+
+extern "C" int svdq_gemm_w4a4_split_wavefronts(const svdq_gemm_args *args, int32_t cus) {
+    return args && args->K > 0 && args->N > 0 ? split_of(*args, cus > 0 ? cus : cu_count()) : 0;
 }
 
 extern "C" size_t svdq_gemm_w4a4_scratch_bytes(int32_t M, int32_t N, int32_t R2, int32_t epilogue) {

@@ -209,36 +209,51 @@ static void launch_split(const svdq_gemm_args &a, int tiles_m, hipStream_t s) {
     }
 }
 
-template <typename T>
-static void launch_split_type(const svdq_gemm_args &a, int tiles_m, bool wide, hipStream_t s) {
-    if (a.act_blocked == 2)
-        wide ? launch_split<T, 8, true>(a, tiles_m, s) : launch_split<T, 4, true>(a, tiles_m, s);
-    else
-        wide ? launch_split<T, 8, false>(a, tiles_m, s) : launch_split<T, 4, false>(a, tiles_m, s);
-}
-
 // Row blocks a launch has to run: the requantizing epilogues write all M rows, the others those below actual_m only.
 static int row_blocks(const svdq_gemm_args &a) {
     const bool quant = a.epilogue == SVDQ_EPI_GELU_QUANT || a.epilogue == SVDQ_EPI_SWIGLU_QUANT;
     return ((quant ? a.M : a.actual_m) + 31) / 32;
 }
 
-// Two workgroups fit a CU (256 registers a wavefront).  Up to that many the split is faster than the tiles, beyond it each
-// further round streams the weight tiles again.  PLAIN launch in us, this kernel / the faster tile build (bf16, rank 32):
+template <typename T>
+static void launch_split_type(const svdq_gemm_args &a, int wavefronts, hipStream_t s) {
+    const int tiles_m = row_blocks(a);
+    if (a.act_blocked == 2)
+        wavefronts == 8 ? launch_split<T, 8, true>(a, tiles_m, s) : launch_split<T, 4, true>(a, tiles_m, s);
+    else
+        wavefronts == 8 ? launch_split<T, 8, false>(a, tiles_m, s) : launch_split<T, 4, false>(a, tiles_m, s);
+}
+
+// Rows and columns: two workgroups fit a CU (256 registers a wavefront).  Up to that many the split is faster than the tiles,
+// beyond it each further round streams the weight tiles again.  PLAIN launch in us, this kernel / the faster tile build (bf16,
+// rank 32):
 //   K = 3072,  N = 3072:  512 rows (384 workgroups) 16.4 / 18.3;  768 rows (576) 24.2 / 18.5
 //   K = 12288, N = 3072:  512 rows 45.2 / 63.4;  768 rows 70.7 / 63.5
 //   K = 2048,  N = 2048:  1024 rows (512) 13.5 / 13.7;  1536 rows (768) 20.0 / 14.0
 // With at most one workgroup per CU eight wavefronts share its K, so that every SIMD still has two (K = 12288, N = 3072, 256
 // rows: 27.8 us with eight, 32.9 with four, 64.0 as tiles; K = 6144, N = 1536, 512 rows: 17.3, 19.1, 32.6).
-bool launch_gemm_split(const svdq_gemm_args &a, int cus, hipStream_t s) {
-    const int tiles_m = row_blocks(a);
-    const long wgs = (long)tiles_m * ((a.N + BN - 1) / BN);
-    if (wgs > 2L * cus || (uint64_t)NBN * (a.K / 128 + 1) * (WPL_BLOCKS * BLK_BYTES) >= (1ull << 32)) return false;
+//
+// K: the exchange of the partial tiles costs 0.6 us, the epilogue on one wavefront as much, so the split has to save that on the
+// loop.  With eight wavefronts it does from three stages (K = 320) on (300 x 3072: K = 128 6.1 us against 5.5, 256 6.3 against
+// 6.2, 384 6.5 against 6.8).  With four, which run more stages each beside a second workgroup, it does later.  512 x 3072, PLAIN:
+// K = 640 8.3 against 7.9, 1152 10.6 against 10.3, 1280 10.8 against 11.1, 1536 11.5 against 11.9.  The other epilogues do more on their
+// one wavefront (704 x 1536, GELU: K = 1280 17.9 against 17.5, 1408 17.7 against 18.1), and at K = 2048, where the four column
+// blocks of a weight tile lie 48 KB apart, do not win at all (1344 x 1536, Q/K norm + RoPE: 17.1 against 16.0; 1920 and 2304 win
+// 1 and 4 %); at 1024, where PLAIN dips as well (10.9 against 9.6), the rule on K says tiles already.
+int split_wavefronts(const svdq_gemm_args &a, int cus) {
+    const long wgs = (long)row_blocks(a) * ((a.N + BN - 1) / BN);
+    if (wgs > 2L * cus || (uint64_t)NBN * (a.K / 128 + 1) * (WPL_BLOCKS * BLK_BYTES) >= (1ull << 32)) return 0;
+    const int stages = (a.K / GROUP + 1) / 2;
+    if (wgs <= cus) return stages >= 3 ? 8 : 0;
+    if (a.epilogue == SVDQ_EPI_PLAIN) return stages >= 10 ? 4 : 0;
+    return stages >= 11 && stages != 16 ? 4 : 0;
+}
+
+void launch_gemm_split(const svdq_gemm_args &a, int wavefronts, hipStream_t s) {
     if (a.dtype == SVDQ_BF16)
-        launch_split_type<BF16>(a, tiles_m, wgs <= cus, s);
+        launch_split_type<BF16>(a, wavefronts, s);
     else
-        launch_split_type<FP16>(a, tiles_m, wgs <= cus, s);
-    return true;
+        launch_split_type<FP16>(a, wavefronts, s);
 }
 
 }  // namespace svdq

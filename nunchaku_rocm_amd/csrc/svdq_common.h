@@ -147,5 +147,6 @@ __device__ inline float silu(float x) { return x / (1.0f + __expf(-x)); }
 // ---- host side ------------------------------------------------------------------------------------
 void set_error(const char *fmt, ...);
 int check_launch(const char *what);
+int cu_count();  // compute units of the device (256 on MI355X)
 
 }  // namespace svdq

@@ -6,11 +6,30 @@ import torch
 
 from oracle import svdq_oracle as O
 
-pytestmark = pytest.mark.gpu
 
 
-def _both(call):
-    """``call()`` by the tile kernel and, twice, as the rule chooses."""
+@pytest.fixture
+def splits(monkeypatch):
+    """Over how many wavefronts each GEMM launched so far split K (0: the tile kernel)."""
+    from nunchaku_rocm_amd import _lib
+
+    lib, seen = _lib.load(), []
+
+    class Watched:
+        def __getattr__(self, name):
+            return getattr(lib, name)
+
+        def svdq_gemm_w4a4(self, args, stream):
+            seen.append(lib.svdq_gemm_w4a4_split_wavefronts(args, 0))
+            return lib.svdq_gemm_w4a4(args, stream)
+
+    watched = Watched()
+    monkeypatch.setattr(_lib, "load", lambda: watched)
+    return seen
+
+
+def _both(call, splits, expected):
+    """``call()`` by the tile kernel and, twice, as the rule chooses: its GEMMs split over the ``expected`` wavefronts."""
     from nunchaku_rocm_amd.ops import gemm as gemm_mod
 
     gemm_mod.set_fp8_loop_variant(1)
@@ -18,7 +37,32 @@ def _both(call):
         tiles = call()
     finally:
         gemm_mod.set_fp8_loop_variant(-1)
-    return tiles, call(), call()
+    assert splits == [0] * len(expected)
+    splits.clear()
+    results = tiles, call(), call()
+    assert splits == 2 * list(expected)
+    return results
+
+
+@pytest.mark.parametrize("epilogue,quant", [(0, False), (1, False), (2, True), (3, True)])
+def test_lines_of_the_rule(epilogue, quant):
+    """Where the split begins and ends, in rows, columns and K, on 256 CUs; forms that it does not take."""
+    from nunchaku_rocm_amd import _lib
+
+    def wavefronts(rows, n, k, **more):
+        m = -(-rows // 256) * 256
+        args = dict(wgt_planes=16, M=rows if quant else m, actual_m=rows, N=n, K=k, epilogue=epilogue, act_blocked=2)
+        return _lib.load().svdq_gemm_w4a4_split_wavefronts(_lib.GemmArgs(**{**args, **more}), 256)
+
+    assert wavefronts(32, 8, 256) == 0 and wavefronts(32, 8, 320) == 8
+    assert wavefronts(256, 4096, 320) == 8 and wavefronts(256, 4096, 12288) == 8  # 256 workgroups
+    last = 1216 if epilogue == 0 else 1344
+    assert wavefronts(288, 4096, last - 64) == 0 and wavefronts(288, 4096, last) == 4  # 288
+    assert wavefronts(512, 4096, 2048) == (4 if epilogue == 0 else 0) and wavefronts(512, 4096, 2112) == 4  # 512
+    assert wavefronts(544, 4096, 3072) == 0  # 544
+    assert wavefronts(32, 8, 1024, wgt_planes=None) == 0
+    assert wavefronts(32, 8, 1024, act_blocked=1) == 0 and wavefronts(32, 8, 1024, act_blocked=0) == 0
+    assert wavefronts(32, 8, 1024, act_blocked=1, act_unsigned=1) == 8 and wavefronts(32, 8, 1024, act_blocked=0, act_unsigned=1) == 8
 
 
 def _module(dev, K, N, R, dtype, unsigned=False):
@@ -31,26 +75,31 @@ def _module(dev, K, N, R, dtype, unsigned=False):
     return mod
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize(
-    "M,K,N,R",
+    "M,K,N,R,wavefronts",
     [
-        (1, 64, 8, 16),  # one group: most wavefronts have no stage
-        (31, 192, 136, 16),  # odd number of groups, a column block past N
-        (33, 512, 128, 32),  # half the wavefronts without a stage
-        (100, 1088, 264, 48),  # nine stages over eight wavefronts
-        (333, 1536, 1544, 64),  # 8 wavefronts, one column block of eight rows
-        (333, 1216, 4096, 32),  # 352 workgroups: 4 wavefronts, an odd number of groups
-        (512, 3072, 4096, 32),  # the last launch that is split: 512 workgroups
+        (1, 64, 8, 16, 0),  # one group: left to the tiles
+        (31, 192, 136, 16, 0),
+        (1, 320, 8, 16, 8),  # three stages, the last one half: five wavefronts have none
+        (31, 448, 136, 16, 8),  # odd number of groups, a column block past N
+        (33, 512, 128, 32, 8),  # half the wavefronts without a stage
+        (100, 1088, 264, 48, 8),  # nine stages over eight wavefronts
+        (333, 1536, 1544, 64, 8),  # one column block of eight rows
+        (333, 1216, 4096, 32, 4),  # 352 workgroups, an odd number of groups
+        (333, 1408, 4104, 128, 4),  # 363 workgroups, eleven stages over four wavefronts
+        (512, 3072, 4096, 32, 4),  # the last launch that is split: 512 workgroups
+        (513, 3072, 4096, 32, 0),  # 544
     ],
 )
-def test_split_against_tiles(dev, M, K, N, R, dtype):
+def test_split_against_tiles(dev, splits, M, K, N, R, wavefronts, dtype):
     print(f"case M={M} K={K} N={N} R={R} {dtype}", flush=True)
     mod = _module(dev, K, N, R, dtype)
     x = O.make_activations(M, K, seed=M, dtype=dtype).to(dev)[None]
     canary = torch.full((M + 8, N), 7.0, dtype=dtype, device=dev)
     with torch.no_grad():
-        tiles, a, b = _both(lambda: mod(x, output=canary[:M]).clone())
+        tiles, a, b = _both(lambda: mod(x, output=canary[:M]).clone(), splits, [wavefronts])
     assert torch.equal(a, b)  # the same bits every time
     assert (canary[M:] == 7.0).all()
     # fp32 sums of the K / 64 group terms in another order, then one rounding to the 16-bit type on either side
@@ -69,31 +118,45 @@ def _abs_terms(mod, x):
     return (act.reshape(M, K) @ wgt.reshape(-1, K).t() + lora + mod.bias.float().cpu().abs()).to(x.device)[None]
 
 
-@pytest.mark.parametrize("blocked", [0, 1, 2, 3])
-@pytest.mark.parametrize("M,N,K", [(40, 136, 512), (333, 4104, 1024)])
-def test_unsigned_hand_over_forms_at_unit_scales(dev, M, N, K, blocked):
-    """Every form of unsigned activations through the split: integers below 2^24, exact in any order."""
+@pytest.mark.gpu
+@pytest.mark.parametrize("form", ["matrix", "lane order", "fp6", "fp6 and scales", "signed fp6", "signed fp6 and scales"])
+@pytest.mark.parametrize("M,N,K,wavefronts", [(40, 136, 512, 8), (333, 4104, 1536, 4)])
+def test_hand_over_forms_at_unit_scales(dev, splits, M, N, K, wavefronts, form):
+    """Every form of activations that the split takes: integers below 2^24, exact in any order."""
     from nunchaku_rocm_amd import ops
     from nunchaku_rocm_amd.layout import block_activations, block_activations_f6, block_scales
 
-    print(f"case M={M} N={N} K={K} blocked={blocked}", flush=True)
+    print(f"case M={M} N={N} K={K} {form}", flush=True)
+    unsigned = "signed" not in form
     rows = -(-M // 32) * 32
-    g = torch.Generator().manual_seed(M + blocked)
+    g = torch.Generator().manual_seed(M)
     act = torch.randint(0, 256, (rows, K // 2), dtype=torch.uint8, generator=g)
     wgt = torch.randint(0, 256, (N, K // 2), dtype=torch.uint8, generator=g).view(torch.int8)
     one = lambda n: torch.ones(K // 64, n, dtype=torch.float16, device=dev)  # noqa: E731
-    ref = O.unpack_int4(act[:M], False).double() @ O.unpack_int4(wgt, True).double().t()
-    sent = {0: lambda: act, 1: lambda: block_activations(act), 2: lambda: block_activations_f6(act, True), 3: lambda: block_activations_f6(act, True)}[blocked]()
+    ref = O.unpack_int4(act[:M], not unsigned).double() @ O.unpack_int4(wgt, True).double().t()
+    sent, blocked = {"matrix": (lambda: act, 0), "lane order": (lambda: block_activations(act), 1)}.get(
+        form, (lambda: block_activations_f6(act, unsigned), 3 if "scales" in form else 2)
+    )
     scales = block_scales(one(rows)) if blocked == 3 else one(rows)
     out = torch.empty(M, N, dtype=torch.float16, device=dev)
     param = torch.nn.Parameter(wgt.to(dev), requires_grad=False)
-    ops.svdq_gemm_w4a4_cuda(act=sent.to(dev), wgt=param, out=out, ascales=scales, wscales=one(N), act_unsigned=True, act_blocked=blocked)
+    ops.svdq_gemm_w4a4_cuda(act=sent().to(dev), wgt=param, out=out, ascales=scales, wscales=one(N), act_unsigned=unsigned, act_blocked=blocked)
+    assert splits == [wavefronts]
     assert torch.equal(out.cpu(), ref.to(torch.float16))
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype,rel", [(torch.bfloat16, 1.5e-3), (torch.float16, 3.5e-4)])
-@pytest.mark.parametrize("tokens,K,hidden", [(1, 512, 512), (130, 1024, 4096), (333, 1536, 2048)])
-def test_requantizing_epilogues(dev, tokens, K, hidden, dtype, rel):
+@pytest.mark.parametrize(
+    "tokens,K,hidden,gelu_split,glu_split",  # of the two GEMMs: the first has its rows padded to 256 and, for SwiGLU, twice the columns
+    [
+        (1, 512, 512, [8, 8], [8, 8]),
+        (130, 1024, 4096, [8, 8], [0, 8]),
+        (333, 1536, 2048, [8, 8], [4, 8]),
+        (600, 1536, 2048, [4, 8], [0, 8]),
+    ],
+)
+def test_requantizing_epilogues(dev, splits, tokens, K, hidden, gelu_split, glu_split, dtype, rel):
     """GELU and SwiGLU feed-forwards; a last-bit difference may move a code by one step: the bound on the result is the one
     for two correct orders of the sums (measured between the tile kernel's two main loops, times four)."""
     from nunchaku_rocm_amd import ops
@@ -103,26 +166,28 @@ def test_requantizing_epilogues(dev, tokens, K, hidden, dtype, rel):
     gelu = _module(dev, K, hidden, 32, dtype), _module(dev, hidden, K, 32, dtype, unsigned=True)
     glu = _module(dev, K, 2 * hidden, 32, dtype), _module(dev, hidden, K, 32, dtype)
     ops.interleave_swiglu_linear_(glu[0])
-    for fn, (fc1, fc2), bar in ((ops.fused_gelu_mlp, gelu, rel), (ops.fused_swiglu_mlp, glu, 3 * rel)):
+    for fn, (fc1, fc2), bar, expected in ((ops.fused_gelu_mlp, gelu, rel, gelu_split), (ops.fused_swiglu_mlp, glu, 3 * rel, glu_split)):
+        splits.clear()
         with torch.no_grad():
-            tiles, a, b = _both(lambda: fn(x, fc1, fc2))
+            tiles, a, b = _both(lambda: fn(x, fc1, fc2), splits, expected)
         assert torch.equal(a, b)
         assert ((a.double() - tiles.double()).norm() / tiles.double().norm()).item() <= bar
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("tokens,heads", [(7, 1), (257, 3), (300, 12)])
-def test_qk_norm_rope(dev, tokens, heads, dtype):
+@pytest.mark.parametrize("tokens,heads,K,wavefronts", [(7, 1, 512, 8), (257, 3, 512, 8), (300, 12, 512, 0), (300, 12, 1536, 4)])
+def test_qk_norm_rope(dev, splits, tokens, heads, K, wavefronts, dtype):
     from nunchaku_rocm_amd import ops
     from nunchaku_rocm_amd.flux_shaped import flux_ids, rope_table
 
-    print(f"case tokens={tokens} heads={heads} {dtype}", flush=True)
-    mod = _module(dev, 512, 3 * heads * 128, 32, dtype)
+    print(f"case tokens={tokens} heads={heads} K={K} {dtype}", flush=True)
+    mod = _module(dev, K, 3 * heads * 128, 32, dtype)
     norm = torch.nn.RMSNorm(128, eps=1e-6, device=dev, dtype=dtype).requires_grad_(False)
     rot = rope_table(flux_ids(0, 1, tokens, device=dev), (16, 56, 56), 10000.0)
-    x = O.make_activations(tokens, 512, seed=tokens, dtype=dtype).to(dev)[None]
+    x = O.make_activations(tokens, K, seed=tokens, dtype=dtype).to(dev)[None]
     with torch.no_grad():
-        tiles, a, b = _both(lambda: ops.fused_qkv_norm_rottary(x, mod, norm, norm, rot))
+        tiles, a, b = _both(lambda: ops.fused_qkv_norm_rottary(x, mod, norm, norm, rot), splits, [wavefronts])
     assert torch.equal(a, b)
-    # each side within one rounding of values that differ in the order of eight group terms
+    # each side within one rounding of values that differ in the order of the K / 64 group terms
     assert ((a.float() - tiles.float()).abs() <= tiles.float().abs() * (2.0**-7 if dtype == torch.bfloat16 else 2.0**-10) + 1e-4).all()

@@ -327,6 +327,9 @@ int svdq_awq_dequantize(const void *qweight, const void *scales, const void *zer
  * 8-byte aligned.
  */
 int svdq_awq_gemm_w4a16(const svdq_awq_gemv_args *args, int32_t group_size, void *stream);
+/* The tile of a workgroup of that launch on a device of `cus` compute units (0: this one's): rows << 16 | channels.  Host
+ * arithmetic on the sizes; for tests.  No counterpart in the reference. */
+int svdq_awq_gemm_tile(int32_t M, int32_t N, int32_t cus);
 
 /*
  * Unmasked scaled-dot-product attention, head dimension D = 128 or 64 (nunchaku/ops/dispatch.py:67-99 attention_fp16 /

@@ -46,6 +46,7 @@ EXPORTS = (
     "svdq_awq_gemv_w4a16_batched",
     "svdq_awq_dequantize",
     "svdq_awq_gemm_w4a16",
+    "svdq_awq_gemm_tile",
     "svdq_attention_fp16",
     "svdq_unpack_mma_weight",
     "svdq_unpack_mma_scale",
@@ -153,6 +154,7 @@ def load() -> ctypes.CDLL:
     lib.svdq_awq_gemv_w4a16_batched.argtypes = [ctypes.POINTER(AwqGemvArgs), _vp, _i32, _vp]
     lib.svdq_awq_dequantize.argtypes = [_vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32, _vp]
     lib.svdq_awq_gemm_w4a16.argtypes = [ctypes.POINTER(AwqGemvArgs), _i32, _vp]
+    lib.svdq_awq_gemm_tile.argtypes = [_i32, _i32, _i32]
     lib.svdq_attention_fp16.argtypes = [ctypes.POINTER(AttentionArgs), _vp]
     lib.svdq_unpack_mma_weight.argtypes = [_vp, _vp, _i32, _i32, _i32, _vp]
     lib.svdq_unpack_mma_scale.argtypes = [_vp, _vp, _i32, _i32, _i32, _vp]

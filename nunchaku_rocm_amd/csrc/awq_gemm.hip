@@ -20,8 +20,6 @@
 // Activations: rows x 128 k of T per stage, [row][256 bytes] with the row's sixteen 16-byte chunks XOR-swizzled by
 // row % 16 (operand reads are conflict free), fetched memory -> LDS directly, two stages ahead (one stage ahead the same
 // launch waited 9 us for them); weights into registers two stages ahead.
-#include <algorithm>
-
 #include "svdq_common.h"
 
 namespace svdq {
@@ -260,6 +258,30 @@ __global__ __launch_bounds__(NS * 128, MB == 4 && NS == 2 ? 1 : 2) void awq_gemm
     }
 }
 
+// Rows and channels of a workgroup's tile, by the workgroups of the most loaded CU: microseconds of one such workgroup at
+// K = 4096 (alone on its CU, each further one), measured on 80 to 1280 workgroups.  Tall and wide tiles decode a weight for
+// more rows; small ones keep CUs from idling (M = 512: N = 4096 23.6 us with 64 x 128 tiles against 43.9 with 128 x 256,
+// N = 10240 53.9 against 46.5; M = 1024, N = 4096 36.4 with 128 x 128).
+struct AwqTile {
+    int rows, channels;
+};
+static AwqTile awq_gemm_tile(int M, int N, int cus) {
+    auto cost = [&](AwqTile t, double first, double next) {
+        const long wgs = (long)((M + t.rows - 1) / t.rows) * ((N + t.channels - 1) / t.channels), per_cu = (wgs + cus - 1) / cus;
+        return first + (double)(per_cu - 1) * next;
+    };
+    AwqTile best = {128, 256};
+    double least = cost(best, 42, 50);
+    auto consider = [&](AwqTile t, double first, double next) {
+        const double c = cost(t, first, next);
+        if (c < least) best = t, least = c;
+    };
+    consider({128, 128}, 28, 34);
+    consider({64, 128}, 21, 16.5);
+    consider({32, 128}, 19, 12.5);
+    return best;
+}
+
 template <typename T>
 static void launch_awq_gemm(const svdq_awq_gemv_args &a, int group, hipStream_t s) {
     auto go = [&](auto mtag, auto ntag) {
@@ -272,21 +294,12 @@ static void launch_awq_gemm(const svdq_awq_gemv_args &a, int group, hipStream_t 
     constexpr std::integral_constant<int, 1> c1{};
     constexpr std::integral_constant<int, 2> c2{};
     constexpr std::integral_constant<int, 4> c4{};
-    // Tile by the workgroups of the most loaded CU: microseconds of one such workgroup at K = 4096 (alone on its CU, each
-    // further one), measured on 80 to 1280 workgroups.  Tall and wide tiles decode a weight for more rows; small ones
-    // keep CUs from idling (M = 512: N = 4096 23.6 us with 64 x 128 tiles against 43.9 with 128 x 256, N = 10240 53.9
-    // against 46.5; M = 1024, N = 4096 36.4 with 128 x 128).
-    auto cost = [&](int rows, int cols, double first, double next) {
-        const long wgs = (long)((a.M + rows - 1) / rows) * ((a.N + cols - 1) / cols), per_cu = (wgs + 255) / 256;
-        return first + (double)(per_cu - 1) * next;
-    };
-    const double t44 = cost(128, 256, 42, 50), t42 = cost(128, 128, 28, 34), t22 = cost(64, 128, 21, 16.5), t12 = cost(32, 128, 19, 12.5);
-    const double best = std::min(std::min(t44, t42), std::min(t22, t12));
-    if (best == t44)
+    const AwqTile t = awq_gemm_tile(a.M, a.N, cu_count());
+    if (t.channels == 256)
         go(c4, c4);
-    else if (best == t42)
+    else if (t.rows == 128)
         go(c4, c2);
-    else if (best == t22)
+    else if (t.rows == 64)
         go(c2, c2);
     else
         go(c1, c2);
@@ -295,6 +308,12 @@ static void launch_awq_gemm(const svdq_awq_gemv_args &a, int group, hipStream_t 
 }  // namespace svdq
 
 using namespace svdq;
+
+extern "C" int svdq_awq_gemm_tile(int32_t M, int32_t N, int32_t cus) {
+    if (M <= 0 || N <= 0) return 0;
+    const AwqTile t = awq_gemm_tile(M, N, cus > 0 ? cus : cu_count());
+    return t.rows << 16 | t.channels;
+}
 
 extern "C" int svdq_awq_gemm_w4a16(const svdq_awq_gemv_args *args, int32_t group_size, void *stream) {
     if (!args) {

@@ -28,3 +28,14 @@ def dev():
     import torch
 
     return torch.device("cuda", 0)
+
+
+@pytest.fixture(params=[-1, 0, 1], ids=["chosen-build", "three-per-cu", "two-per-cu"])
+def fp8_build(request):
+    """Every test that asks for it runs with the GEMM's kernel chosen by size (for small launches the one that splits K)
+    and with each build of the fp8 main loop, which serve the large launches."""
+    from nunchaku_rocm_amd.ops import gemm as G
+
+    G.set_fp8_loop_variant(request.param)
+    yield request.param
+    G.set_fp8_loop_variant(-1)

@@ -106,6 +106,7 @@ def test_scale_layout_helpers_invert_each_other():
     assert b.reshape(-1)[((m // 32) * 2 + g // 8) * 256 + (m % 32) * 8 + g % 8] == a[g, m]
 
 
+@pytest.mark.usefixtures("fp8_build")
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("M,K,N,R,norm", [(300, 512, 264, 16, False), (4608, 3072, 384, 32, False), (1000, 1536, 256, 32, True), (96, 1024, 128, 0, False)])
 def test_scales_in_the_gemms_order(dev, M, K, N, R, norm, dtype):
@@ -167,6 +168,7 @@ def test_scales_in_the_gemms_order_need_k_of_512(dev):
         gemm_mod.USE_WEIGHT_PLANES = old
 
 
+@pytest.mark.usefixtures("fp8_build")
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_quantizer_then_gemm_through_fp6_codes(dev, dtype):
     """The pair as the modules run it: quantizer (out_blocked=2) -> GEMM (act_blocked=2) against the pair through the
@@ -195,6 +197,7 @@ def test_quantizer_then_gemm_through_fp6_codes(dev, dtype):
     assert err < (4e-3 if dtype == torch.bfloat16 else 1e-3), err
 
 
+@pytest.mark.usefixtures("fp8_build")
 @pytest.mark.parametrize("unsigned", [False, True])
 @pytest.mark.parametrize("M,N,K,R", [(256, 264, 256, 16), (96, 128, 320, 0), (4608, 3072, 3072, 32)])
 def test_gemm_reads_either_order(dev, M, N, K, R, unsigned):
@@ -248,6 +251,7 @@ def test_fp6_layout_helpers_invert_each_other():
     assert code == (32 - v if v < 0 else v)
 
 
+@pytest.mark.usefixtures("fp8_build")
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("unsigned", [False, True])
 @pytest.mark.parametrize("M,N,K,R", [(256, 264, 256, 16), (96, 128, 320, 0), (4608, 3072, 3072, 32), (1024, 640, 1216, 32)])
@@ -299,6 +303,7 @@ def test_gemm_takes_fp6_codes(dev, M, N, K, R, unsigned, dtype):
         gemm_mod.USE_WEIGHT_PLANES = old
 
 
+@pytest.mark.usefixtures("fp8_build")
 @pytest.mark.parametrize("swiglu", [False, True])
 def test_requantizing_epilogues_write_either_order(dev, swiglu):
     from nunchaku_rocm_amd import ops
@@ -333,6 +338,7 @@ def test_requantizing_epilogues_write_either_order(dev, swiglu):
     assert (res[0][0] != 0xEE).any()
 
 
+@pytest.mark.usefixtures("fp8_build")
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_modules_compute_the_same_bits_either_way(dev, dtype):
     """SVDQW4A4Linear.forward, fused_gelu_mlp, fused_qkv_norm_rottary and fused_swiglu_mlp with the hand-over switched

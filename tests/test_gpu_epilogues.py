@@ -10,13 +10,18 @@ from parity_bars import assert_requantized_like_the_reference
 pytestmark = pytest.mark.gpu
 
 
-@pytest.fixture(autouse=True, params=["none", "all"], ids=["int8-loop", "fp8-loop"])
+@pytest.fixture(autouse=True, params=[("none", -1), ("all", -1), ("all", 0), ("all", 1)],
+                ids=["int8-loop", "fp8-loop", "fp8-loop-three-per-cu", "fp8-loop-two-per-cu"])  # fmt: skip
 def main_loop(request):
-    """Every test runs through both GEMM main loops: packed weights (int8 MFMA) and pre-split weights (fp8 MFMA)."""
+    """Every test runs through both GEMM main loops: packed weights (int8 MFMA) and pre-split weights (fp8 MFMA: the kernel
+    chosen by size, which for small launches may be the one that splits K, and each build of the tile kernel)."""
     from nunchaku_rocm_amd.ops import gemm as G
 
-    old, G.USE_WEIGHT_PLANES = G.USE_WEIGHT_PLANES, request.param
-    yield request.param
+    planes, build = request.param
+    old, G.USE_WEIGHT_PLANES = G.USE_WEIGHT_PLANES, planes
+    G.set_fp8_loop_variant(build)
+    yield planes
+    G.set_fp8_loop_variant(-1)
     G.USE_WEIGHT_PLANES = old
 TOL = 1e-2
 

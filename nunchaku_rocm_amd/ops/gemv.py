@@ -150,9 +150,18 @@ def _check_weight(kernel, scaling_factors, zeros, n: int, k: int, group_size: in
     return scaling_factors, zeros
 
 
-# More rows than this: the weight is decoded to memory once and a library product reads it (K = 4096, bf16: N = 10240
-# 169 us in the kernel against 173 at 2048 rows, 241 against 200 at 3000; N = 4096 63 against 73, 108 against 91).
-_GEMM_MAX_ROWS = 2048
+def _decodes_inside(m: int, n: int, k: int) -> bool:
+    """Whether the GEMM that decodes the weight inside is the faster one, or a decode to memory and a library product is.
+
+    Rows: beyond 2048 the decode to memory is paid once for many (K = 4096: N = 10240 169 us in the kernel against 173 at 2048
+    rows, 241 against 200 at 3000; N = 4096 63 against 73, 108 against 91).
+    Columns and K: a workgroup of the kernel walks all of K, 3.7 us per 1024 of it however few workgroups there are, while the
+    decode costs by the weight's size and the library product may split K.  So it needs columns (and, less, rows) for its K.  The
+    line is a fit to 1098 sizes (K 1024 to 24576, N 128 to 10240, 1 to 2048 rows) on which it takes no size that is more than 2 %
+    slower in the kernel.  Kernel against library, us, 32 rows: K = 12288, N = 512 50 against 28, 1024 50 against 36, 4096 50
+    against 58; K = 4096, N = 512 19 against 14, 1536 20 against 22; K = 2048, N = 128 11.5 against 11.6.  Past 12288 the library
+    product slows down by more than K."""
+    return 0 < m <= 2048 and (k <= 2048 or n * (512 + m) >= 128 * (2400 + min(k, 12288)))
 
 
 def _is_plain(t: torch.Tensor) -> bool:
@@ -181,11 +190,11 @@ def _aligned_rows(x: torch.Tensor) -> tuple[torch.Tensor, int]:
 
 def _product(x: torch.Tensor, kernel, scaling_factors, zeros, n: int, k: int, group_size: int) -> torch.Tensor:
     """``x @ T(q * s + z).T`` for a 2-D ``x``: the weight decoded inside the GEMM (``svdq_awq_gemm_w4a16``), or decoded to
-    memory first for a library product where many rows share it or where ``x`` is more than its values: the product is
+    memory first for a library product where that is faster or where ``x`` is more than its values: the product is
     differentiable in ``x``, forward and backward, can be mapped over it, and follows an enclosing autocast."""
     scaling_factors, zeros = _check_weight(kernel, scaling_factors, zeros, n, k, group_size, x.dtype)
     m = x.shape[0]
-    if 0 < m <= _GEMM_MAX_ROWS and x.shape[1] == k and _is_plain(x) and not _cast_by_autocast(x):
+    if _decodes_inside(m, n, k) and x.shape[1] == k and _is_plain(x) and not _cast_by_autocast(x):
         x, ld_x = _aligned_rows(x)
         out = torch.empty(m, n, dtype=x.dtype, device=x.device)
         args = _lib.AwqGemvArgs(x=x.data_ptr(), qweight=kernel.data_ptr(), scales=scaling_factors.data_ptr(), zeros=zeros.data_ptr(),
@@ -231,9 +240,9 @@ def awq_gemm_w4a16(
 ) -> torch.Tensor:
     """
     AWQ W4A16 GEMM for larger batches (reference: nunchaku/ops/triton/awq.py:232-251, there a dense decode and a library
-    product): up to 2048 rows the weight is decoded, and rounded to the input dtype, inside the GEMM; with more, or where
-    ``in_feats`` wants a gradient or is under a transform, it is decoded to memory once by :func:`awq_dequantize` for a
-    library product.
+    product): the weight is decoded, and rounded to the input dtype, inside the GEMM; with more than 2048 rows, too few columns
+    for a long ``k``, or where ``in_feats`` wants a gradient or is under a transform, it is decoded to memory once by
+    :func:`awq_dequantize` for a library product.
     """
     _lib.require_cuda(in_feats, kernel, scaling_factors, zeros)
     shape = in_feats.shape

@@ -64,6 +64,21 @@ def test_plain_activations_take_the_kernel(routes):
     assert len(routes) == 4
 
 
+def test_too_few_columns_for_a_long_k_take_the_library_product(routes):
+    """A workgroup of the kernel walks all of K; sizes on either side of the line, with what was measured (kernel, library)."""
+    from nunchaku_rocm_amd import ops
+    from nunchaku_rocm_amd.ops.gemv import _decodes_inside
+
+    for m, n, k in [(1, 512, 12288), (17, 1024, 12288), (32, 2048, 12288), (1024, 512, 12288), (1, 512, 4096), (2049, 10240, 4096), (0, 4096, 4096)]:
+        assert not _decodes_inside(m, n, k)  # 49 / 24, 50 / 31, 50 / 41, 51 / 45, 19 / 16 us
+    for m, n, k in [(1, 4096, 12288), (256, 4096, 12288), (77, 4096, 4096), (2048, 10240, 4096), (1, 4, 64), (2048, 128, 2048), (1024, 2048, 12288)]:
+        assert _decodes_inside(m, n, k)  # 50 / 55, 54 / 79, 20 / 36, 171 / 175 us, ..., 70 / 92
+    qw, s, z, w = _weight(k=2304)
+    x = torch.randn(5, 2304).half()
+    out = ops.awq_gemm_w4a16(x, qw, s, z, group_size=GROUP)
+    assert not routes and torch.equal(out, x @ w.t())
+
+
 def test_what_the_kernel_does_not_carry_is_carried_on(routes):
     from nunchaku_rocm_amd import ops
 

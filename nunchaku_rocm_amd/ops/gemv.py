@@ -164,12 +164,14 @@ def _decodes_inside(m: int, n: int, k: int) -> bool:
     return 0 < m <= 2048 and (k <= 2048 or n * (512 + m) >= 128 * (2400 + min(k, 12288)))
 
 
+_PLAIN_TYPES = frozenset((torch.Tensor, torch.nn.Parameter))
+_is_wrapped = torch._C._functorch.is_functorch_wrapped_tensor
+
+
 def _is_plain(t: torch.Tensor) -> bool:
     """Whether ``t`` is no more than the values in its memory: a kernel that is handed an address carries no gradient, tangent,
     batch dimension of a transform, subclass or pending negation along."""
-    if t.requires_grad and torch.is_grad_enabled():
-        return False
-    if type(t) not in (torch.Tensor, torch.nn.Parameter) or t.is_neg() or torch._C._functorch.is_functorch_wrapped_tensor(t):
+    if type(t) not in _PLAIN_TYPES or (t.requires_grad and torch.is_grad_enabled()) or t.is_neg() or _is_wrapped(t):
         return False
     return forward_ad._current_level < 0 or forward_ad.unpack_dual(t).tangent is None
 

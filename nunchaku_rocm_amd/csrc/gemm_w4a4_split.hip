@@ -2,14 +2,21 @@
 //
 // F6ACT: activations as fp6 codes (act_blocked == 2), signed or not; otherwise unsigned nibbles, as the (M, K / 2) matrix or
 // in lane order, unpacked to fp8 codes: the same integers and the same sums, so that all hand-over forms of unsigned
-// activations give the same bits.  (Signed nibbles need the offset correction and stay with the tiles.)  Same arithmetic as gemm_w4a4_f8_kernel (per group one fp6 x fp6 or fp6 x fp8 matrix
-// instruction = the exact integer dot product, one 16-bit matrix instruction = the product of the two scales, one fp32
-// FMA per output); only the order of the fp32 sums over groups differs (a partial sum per wavefront).
+// activations give the same bits.  (Signed nibbles need the offset correction and stay with the tiles.)  Same arithmetic as
+// gemm_w4a4_f8_kernel (per group one fp6 x fp6 or fp6 x fp8 matrix instruction = the exact integer dot product, one 16-bit
+// matrix instruction = the product of the two scales, one fp32 FMA per output); only the order of the fp32 sums over groups
+// differs (a partial sum per wavefront).  Against 64-bit sums it is the closer one: of 512 x 3072 outputs in fp16 (K = 3072)
+// 989 are not the correctly rounded value, 1086 with the tiles; K = 12288, 333 rows: 1053 and 1366.
 //
 // Why: with 128 x 128 tiles a prompt's 512 rows give a 3072-wide layer 96 workgroups on 256 CUs, each alone on its CU with
 // one wavefront per SIMD and a barrier per 128 k.  Here the same layer has 384 workgroups and a wavefront runs a quarter of
-// K (an eighth where no CU gets a second workgroup: two wavefronts per SIMD either way).  What bounds it: every workgroup streams its own copy of the weight tile from L2 (there is no second row block in the
-// workgroup to share it with), 64 bytes per clock and CU at best, which is why large launches stay with the tiles.
+// K (an eighth where no CU gets a second workgroup).  A CU with two workgroups, or with one of eight wavefronts, has two
+// wavefronts per SIMD; between one and two workgroups per CU those CUs that get one of four wavefronts have one (333 rows x
+// 3072, K = 12288: 264 workgroups, 248 CUs with one, 43 us; 256 rows 28 us).
+// What bounds it: every workgroup streams its own copy of the weight tile from L2 (there is no second row block in the
+// workgroup to share it with), in all about 11 TB/s at K = 12288 and 512 rows, the rate the tiles' loop is delivered at too and
+// less than half of 64 bytes per clock and CU.  That is why large launches stay with the tiles.  The epilogue is wavefront
+// 0's alone; the others have ended.
 //
 //  * Nothing is shared between the wavefronts of a workgroup inside the loop, so weights go straight to registers (they lie
 //    in the matrix instruction's lane order) and there is neither LDS nor a barrier in it; a stage (two groups) is
@@ -18,6 +25,7 @@
 //  * The partial tiles meet in LDS: wavefront w < 4 adds up column block w in a fixed order (the result does not depend on
 //    timing), the sums go to wavefront 0, which owns the whole 32 x 128 tile for the epilogue as in the other kernels.
 //  * Workgroups of one column tile are neighbours on one XCD, so that a weight tile is fetched into one L2.
+#include <algorithm>
 #include <type_traits>
 
 #include "gemm_w4a4_split.h"
@@ -233,20 +241,25 @@ static void launch_split_type(const svdq_gemm_args &a, int wavefronts, hipStream
 // With at most one workgroup per CU eight wavefronts share its K, so that every SIMD still has two (K = 12288, N = 3072, 256
 // rows: 27.8 us with eight, 32.9 with four, 64.0 as tiles; K = 6144, N = 1536, 512 rows: 17.3, 19.1, 32.6).
 //
-// K: the exchange of the partial tiles costs 0.6 us, the epilogue on one wavefront as much, so the split has to save that on the
-// loop.  With eight wavefronts it does from three stages (K = 320) on (300 x 3072: K = 128 6.1 us against 5.5, 256 6.3 against
-// 6.2, 384 6.5 against 6.8).  With four, which run more stages each beside a second workgroup, it does later.  512 x 3072, PLAIN:
-// K = 640 8.3 against 7.9, 1152 10.6 against 10.3, 1280 10.8 against 11.1, 1536 11.5 against 11.9.  The other epilogues do more on their
-// one wavefront (704 x 1536, GELU: K = 1280 17.9 against 17.5, 1408 17.7 against 18.1), and at K = 2048, where the four column
-// blocks of a weight tile lie 48 KB apart, do not win at all (1344 x 1536, Q/K norm + RoPE: 17.1 against 16.0; 1920 and 2304 win
-// 1 and 4 %); at 1024, where PLAIN dips as well (10.9 against 9.6), the rule on K says tiles already.
+// K and rank: the exchange of the partial tiles costs 0.6 us, which the split has to save elsewhere: on the loop, where K is
+// long, or on the low-rank product, whose serial steps over 16 ranks each more and smaller workgroups run faster.  Time against
+// the tiles, PLAIN, 256 x 3072 (eight wavefronts) | 512 x 3072 (four, which run more stages each beside a second workgroup):
+//   rank 32:  K = 128 1.10 | 1.11;  256 1.01 | 1.08;  512 0.92 | 1.01;  1024 0.78 | 1.14;  1280 0.75 | 0.99;  2048 0.77 | 0.96
+//   rank 64:  K = 128 0.97 | 1.05;  256 0.91 | 1.00;  512 0.85 | 0.93;  1024 0.74 | 1.06;  1280 0.72 | 0.94;  2048 0.74 | 0.94
+//   rank 128: K = 128 0.82 | 0.91;  256 0.79 | 0.88;  512 0.75 | 0.84;  1024 0.68 | 0.95;  1280 0.67 | 0.86;  2048 0.69 | 0.89
+// The other epilogues lie within 0.1 of these.  At rank 32 and four wavefronts SwiGLU wins from K = 1280 on (0.97), Q/K norm +
+// RoPE from 1344 (0.95; 1280 1.01), GELU from 1600 (0.98; 1536 1.02, and 1.04 at rank 16).  The dips at K = 1024 and 2048 lie at
+// column blocks of a weight tile 24 and 48 KB apart; the second one counts for Q/K norm + RoPE (1.05) and GELU (1.03) only.
 int split_wavefronts(const svdq_gemm_args &a, int cus) {
     const long wgs = (long)row_blocks(a) * ((a.N + BN - 1) / BN);
     if (wgs > 2L * cus || (uint64_t)NBN * (a.K / 128 + 1) * (WPL_BLOCKS * BLK_BYTES) >= (1ull << 32)) return 0;
     const int stages = (a.K / GROUP + 1) / 2;
-    if (wgs <= cus) return stages >= 3 ? 8 : 0;
-    if (a.epilogue == SVDQ_EPI_PLAIN) return stages >= 10 ? 4 : 0;
-    return stages >= 11 && stages != 16 ? 4 : 0;
+    const bool gelu = a.epilogue == SVDQ_EPI_GELU_QUANT, swiglu = a.epilogue == SVDQ_EPI_SWIGLU_QUANT, qk = a.epilogue == SVDQ_EPI_QK_NORM_ROPE;
+    const int rank = gelu || swiglu ? std::min(a.R, a.R2) : a.R;
+    if (wgs <= cus) return stages >= 3 || rank >= 64 ? 8 : 0;
+    if (rank >= 128) return 4;
+    const int from = rank >= 64 ? 3 : gelu ? 13 : qk ? 11 : 10;
+    return stages >= from && stages != 8 && !(stages == 16 && (gelu || qk)) ? 4 : 0;
 }
 
 void launch_gemm_split(const svdq_gemm_args &a, int wavefronts, hipStream_t s) {

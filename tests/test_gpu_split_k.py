@@ -44,22 +44,26 @@ def _both(call, splits, expected):
     return results
 
 
-@pytest.mark.parametrize("epilogue,quant", [(0, False), (1, False), (2, True), (3, True)])
-def test_lines_of_the_rule(epilogue, quant):
-    """Where the split begins and ends, in rows, columns and K, on 256 CUs; forms that it does not take."""
+@pytest.mark.parametrize("epilogue,quant,first,at_2048", [(0, False, 1216, 4), (1, False, 1344, 0), (2, True, 1600, 0), (3, True, 1216, 4)])
+def test_lines_of_the_rule(epilogue, quant, first, at_2048):
+    """Where the split begins and ends, in rows, columns, K and rank, on 256 CUs; forms that it does not take.  ``first``: the
+    shortest K of a launch with more workgroups than CUs and a rank below 64."""
     from nunchaku_rocm_amd import _lib
 
-    def wavefronts(rows, n, k, **more):
+    def wavefronts(rows, n, k, rank=32, **more):
         m = -(-rows // 256) * 256
-        args = dict(wgt_planes=16, M=rows if quant else m, actual_m=rows, N=n, K=k, epilogue=epilogue, act_blocked=2)
+        args = dict(wgt_planes=16, M=rows if quant else m, actual_m=rows, N=n, K=k, epilogue=epilogue, act_blocked=2, R=rank, R2=rank)
         return _lib.load().svdq_gemm_w4a4_split_wavefronts(_lib.GemmArgs(**{**args, **more}), 256)
 
     assert wavefronts(32, 8, 256) == 0 and wavefronts(32, 8, 320) == 8
     assert wavefronts(256, 4096, 320) == 8 and wavefronts(256, 4096, 12288) == 8  # 256 workgroups
-    last = 1216 if epilogue == 0 else 1344
-    assert wavefronts(288, 4096, last - 64) == 0 and wavefronts(288, 4096, last) == 4  # 288
-    assert wavefronts(512, 4096, 2048) == (4 if epilogue == 0 else 0) and wavefronts(512, 4096, 2112) == 4  # 512
-    assert wavefronts(544, 4096, 3072) == 0  # 544
+    assert wavefronts(288, 4096, first - 64) == 0 and wavefronts(288, 4096, first) == 4  # 288
+    assert wavefronts(512, 4096, 2048) == at_2048 and wavefronts(512, 4096, 2112) == 4  # 512
+    assert wavefronts(32, 8, 64, 48) == 0 and wavefronts(32, 8, 64, 64) == 8
+    assert wavefronts(288, 4096, 256, 64) == 0 and wavefronts(288, 4096, 320, 64) == 4 and wavefronts(288, 4096, 1024, 112) == 0
+    assert wavefronts(288, 4096, 64, 128) == 4 and wavefronts(512, 4096, 1024, 128) == 4
+    assert wavefronts(288, 4096, 320, 64, R2=16) == (0 if quant else 4)
+    assert wavefronts(544, 4096, 3072) == 0 and wavefronts(544, 4096, 3072, 256) == 0  # 544
     assert wavefronts(32, 8, 1024, wgt_planes=None) == 0
     assert wavefronts(32, 8, 1024, act_blocked=1) == 0 and wavefronts(32, 8, 1024, act_blocked=0) == 0
     assert wavefronts(32, 8, 1024, act_blocked=1, act_unsigned=1) == 8 and wavefronts(32, 8, 1024, act_blocked=0, act_unsigned=1) == 8
@@ -82,6 +86,8 @@ def _module(dev, K, N, R, dtype, unsigned=False):
     [
         (1, 64, 8, 16, 0),  # one group: left to the tiles
         (31, 192, 136, 16, 0),
+        (40, 64, 136, 64, 8),  # one group, half a stage: seven wavefronts have none
+        (333, 128, 4104, 128, 4),  # one stage: three have none
         (1, 320, 8, 16, 8),  # three stages, the last one half: five wavefronts have none
         (31, 448, 136, 16, 8),  # odd number of groups, a column block past N
         (33, 512, 128, 32, 8),  # half the wavefronts without a stage
@@ -153,7 +159,7 @@ def test_hand_over_forms_at_unit_scales(dev, splits, M, N, K, wavefronts, form):
         (1, 512, 512, [8, 8], [8, 8]),
         (130, 1024, 4096, [8, 8], [0, 8]),
         (333, 1536, 2048, [8, 8], [4, 8]),
-        (600, 1536, 2048, [4, 8], [0, 8]),
+        (600, 1600, 2048, [4, 8], [0, 8]),
     ],
 )
 def test_requantizing_epilogues(dev, splits, tokens, K, hidden, gelu_split, glu_split, dtype, rel):

@@ -16,7 +16,7 @@ from concurrent.futures import ThreadPoolExecutor
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libsvdq_mi355x.so")
-SOURCES = ["common.hip", "quantize.hip", "gemm_w4a4.hip", "gemm_w4a4_split.hip", "awq_gemv.hip", "awq_gemm.hip", "attention.hip", "layout.hip"]
+SOURCES = ["common.hip", "quantize.hip", "gemm_w4a4.hip", "gemm_w4a4_split.hip", "gemm_w4a4_wide.hip", "awq_gemv.hip", "awq_gemm.hip", "attention.hip", "layout.hip"]
 FLAGS = [
     "--offload-arch=gfx950",
     "-O3",

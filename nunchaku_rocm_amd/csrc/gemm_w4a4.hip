@@ -56,6 +56,7 @@
 
 #include "gemm_w4a4_split.h"
 #include "gemm_w4a4_tile.h"
+#include "gemm_w4a4_wide.h"
 
 namespace svdq {
 
@@ -715,7 +716,7 @@ static void launch_gemm_i8(const svdq_gemm_args &a, hipStream_t s) {
     }
 }
 
-// Workgroups per CU for the fp8 kernel.  Three (PIPE = false) keep a full CU about 8 % busier than two (PIPE = true), but a
+// Workgroups per CU for the fp8 kernel (with blocked activation scales gemm_w4a4_wide.hip serves full CUs).  Three (PIPE = false) keep a full CU about 8 % busier than two (PIPE = true), but a
 // workgroup of the two-per-CU kernel runs faster, which decides when the last round of tiles leaves most CUs with one or
 // two workgroups.  Cost model, in units of a tile's share of a fully loaded three-per-CU CU: whole rounds cost 3 (three per
 // CU) or 2 * 1.08 (two per CU); a last round whose fullest CU holds k tiles costs 1.75 / 2.15 / 3 (k = 1 / 2 / 3) or
@@ -769,10 +770,11 @@ static void launch_gemm_f8(const svdq_gemm_args &a, hipStream_t s) {
     }
     if (a.act_blocked == 2) {  // fp6 codes carry their sign: one instantiation for signed and unsigned activations
         if (a.ascales_blocked) {
-            if (two)
-                launch_gemm_f8p<T, true, true, true, true>(a, s);
+            const int forced = g_f8_variant.load(std::memory_order_relaxed);
+            if (wide_runs(a) && (forced == 0 || (forced < 0 && wide_takes(a, cu_count()))))
+                launch_gemm_wide(a, cu_count(), s);
             else
-                launch_gemm_f8p<T, true, false, true, true>(a, s);
+                launch_gemm_f8p<T, true, true, true, true>(a, s);
         } else if (two) {
             launch_gemm_f8p<T, true, true, true>(a, s);
         } else {
@@ -1086,7 +1088,7 @@ extern "C" int svdq_block_rotary(const float *rotary, float *blocked, int32_t ro
 
 extern "C" int svdq_gemm_w4a4_set_variant(int32_t variant) {
     if (variant < -1 || variant > 1) {
-        set_error("svdq_gemm_w4a4_set_variant: %d is not -1 (by tile count), 0 (three workgroups per CU) or 1 (two)", variant);
+        set_error("svdq_gemm_w4a4_set_variant: %d is not -1 (by tile count), 0 (for full CUs) or 1 (two workgroups per CU)", variant);
         return SVDQ_E_INVALID;
     }
     g_f8_variant.store(variant, std::memory_order_relaxed);

@@ -349,9 +349,11 @@ __device__ __forceinline__ void tile_epilogue(const svdq_gemm_args &a, v16f (&ac
         }
         if (a.out != nullptr) store_out();  // pre-GELU output, when asked for
 #pragma unroll
-        for (int bn = 0; bn < NBN; bn++)
+        for (int bn = 0; bn < NBN; bn++) {
 #pragma unroll
             for (int i = 0; i < 16; i++) acc[bn][i] = gelu_tanh(acc[bn][i]);
+            __builtin_amdgcn_sched_barrier(0);  // (all 64 at once spill where the wavefront owns a second row block)
+        }
 
         // next layer's LoRA-down on the un-shifted, un-smoothed GELU output rounded to T:
         // D[r][m] = sum_n ldT[r][n] * x[n][m] over the tile's 128 columns; registers [8 s, 8 s + 8) of a block are one

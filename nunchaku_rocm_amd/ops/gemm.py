@@ -58,8 +58,9 @@ def prepare_static_scratch(device=None) -> None:
 
 def set_fp8_loop_variant(variant: int) -> None:
     """Which build of the fp8 main loop every following GEMM on pre-split weights uses: -1 = chosen by the number of tiles
-    (default; launches with few rows go to the kernel that splits K), 0 = three workgroups per CU, 1 = two per CU with
-    software-pipelined steps.  The two give identical bits; the switch exists for tuning and for tests (``svdq_gemm_w4a4_set_variant``)."""
+    (default; launches with few rows go to the kernel that splits K), 0 = the build for full CUs (256 x 128 tiles for blocked fp6
+    codes and scales, otherwise three workgroups per CU), 1 = two per CU with software-pipelined steps.  The two give identical
+    bits; the switch exists for tuning and for tests (``svdq_gemm_w4a4_set_variant``)."""
     _lib.check(_lib.load().svdq_gemm_w4a4_set_variant(int(variant)))
 
 

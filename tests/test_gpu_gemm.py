@@ -414,9 +414,8 @@ def test_weight_planes_layout(dev, N, K):
 @pytest.mark.parametrize("unsigned", [False, True])
 @pytest.mark.parametrize("M,N,K,R", [(300, 520, 1152, 32), (129, 136, 320, 16), (2048, 1280, 512, 0)])
 def test_fp8_loop_builds_agree_bit_for_bit(dev, M, N, K, R, unsigned):
-    """The fp8 main loop is built twice (three workgroups per CU, steps in program order; two per CU, steps software
-    pipelined) and the library picks by tile count: both issue the same arithmetic in the same order, so every output bit
-    agrees, whichever one a shape gets."""
+    """The fp8 main loop is built twice (for full CUs; two workgroups per CU, steps software pipelined) and the library picks
+    by tile count: both issue the same arithmetic in the same order, so every output bit agrees, whichever one a shape gets."""
     from nunchaku_rocm_amd.ops import gemm as gemm_mod
 
     print(f"case M={M} N={N} K={K} R={R} unsigned={unsigned}", flush=True)

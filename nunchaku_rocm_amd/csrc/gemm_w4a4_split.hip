@@ -12,7 +12,7 @@
 // one wavefront per SIMD and a barrier per 128 k.  Here the same layer has 384 workgroups and a wavefront runs a quarter of
 // K (an eighth where no CU gets a second workgroup).  A CU with two workgroups, or with one of eight wavefronts, has two
 // wavefronts per SIMD; between one and two workgroups per CU those CUs that get one of four wavefronts have one (333 rows x
-// 3072, K = 12288: 264 workgroups, 248 CUs with one, 43 us; 256 rows 28 us).
+// 3072, K = 12288: 264 workgroups, 248 CUs with one, 41 us; 256 rows 26 us).
 // What bounds it: every workgroup streams its own copy of the weight tile from L2 (there is no second row block in the
 // workgroup to share it with), in all about 11 TB/s at K = 12288 and 512 rows, the rate the tiles' loop is delivered at too and
 // less than half of 64 bytes per clock and CU.  That is why large launches stay with the tiles.  The epilogue is wavefront
@@ -235,11 +235,11 @@ static void launch_split_type(const svdq_gemm_args &a, int wavefronts, hipStream
 // Rows and columns: two workgroups fit a CU (256 registers a wavefront).  Up to that many the split is faster than the tiles,
 // beyond it each further round streams the weight tiles again.  PLAIN launch in us, this kernel / the faster tile build (bf16,
 // rank 32):
-//   K = 3072,  N = 3072:  512 rows (384 workgroups) 16.4 / 18.3;  768 rows (576) 24.2 / 18.5
-//   K = 12288, N = 3072:  512 rows 45.2 / 63.4;  768 rows 70.7 / 63.5
+//   K = 3072,  N = 3072:  512 rows (384 workgroups) 15.5 / 18.3;  768 rows (576) 24.2 / 18.5
+//   K = 12288, N = 3072:  512 rows 42.1 / 63.4;  768 rows 70.7 / 63.5
 //   K = 2048,  N = 2048:  1024 rows (512) 13.5 / 13.7;  1536 rows (768) 20.0 / 14.0
 // With at most one workgroup per CU eight wavefronts share its K, so that every SIMD still has two (K = 12288, N = 3072, 256
-// rows: 27.8 us with eight, 32.9 with four, 64.0 as tiles; K = 6144, N = 1536, 512 rows: 17.3, 19.1, 32.6).
+// rows: 26.2 us with eight, 32.9 with four, 64.0 as tiles; K = 6144, N = 1536, 512 rows: 16.5, 19.1, 32.6).
 //
 // K and rank: the exchange of the partial tiles costs 0.6 us, which the split has to save elsewhere: on the loop, where K is
 // long, or on the low-rank product, whose serial steps over 16 ranks each more and smaller workgroups run faster.  Time against

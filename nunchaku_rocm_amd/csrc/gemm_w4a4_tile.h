@@ -74,6 +74,9 @@ __device__ inline v2i g_load64(__amdgpu_buffer_rsrc_t r, uint32_t lane_off, uint
 __device__ inline void g_load16_lds(__amdgpu_buffer_rsrc_t r, uint8_t *lds, uint32_t lane_off, uint32_t uniform_off) {
     __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (SVDQ_AS3 void *)lds, 16, (int)lane_off, (int)uniform_off, 0, 0);
 }
+__device__ inline void g_load4_lds(__amdgpu_buffer_rsrc_t r, uint8_t *lds, uint32_t lane_off, uint32_t uniform_off) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (SVDQ_AS3 void *)lds, 4, (int)lane_off, (int)uniform_off, 0, 0);
+}
 __device__ inline void g_load12_lds(__amdgpu_buffer_rsrc_t r, uint8_t *lds, uint32_t lane_off, uint32_t uniform_off) {
     __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (SVDQ_AS3 void *)lds, 12, (int)lane_off, (int)uniform_off, 0, 0);
 }
@@ -95,27 +98,26 @@ __device__ inline void tile_ids(int tiles_m, int tiles_n, int &pid_m, int &pid_n
 
 // Epilogue operands every wavefront of the tile needs, fetched global -> LDS next to stage 0: the tile's 128 bias
 // values, the first 32 ranks of lora_up and (Q/K norm + RoPE epilogue, Q and K tiles) the head's 128 norm weights.
+// (Buffer loads: next to a global_load_lds in flight the compiler waits for every load before the first register load's
+// use in a loop that follows.)
 template <int EPI>
 __device__ inline void fetch_epilogue_operands(const svdq_gemm_args &a, uint8_t *sepi, int n0, int wm, int lane) {
     const int l32 = lane & 31, half = lane >> 5;
     if constexpr (EPI == SVDQ_EPI_QK_NORM_ROPE) {
         const int part = n0 / (a.N / 3);
-        if (part < 2 && wm == 2) {  // 64 lanes x 4 bytes
-            const uint8_t *src = (const uint8_t *)(part == 0 ? a.norm_q : a.norm_k) + 4 * lane;
-            __builtin_amdgcn_global_load_lds((const SVDQ_AS1 void *)src, (SVDQ_AS3 void *)(sepi + EPI_NORM_OFF), 4, 0, 0);
-        }
+        if (part < 2 && wm == 2)  // 64 lanes x 4 bytes
+            g_load4_lds(g_buffer(part == 0 ? a.norm_q : a.norm_k), sepi + EPI_NORM_OFF, 4u * (uint32_t)lane, 0);
     }
-    if (a.bias != nullptr && wm == 3) {  // 64 lanes x 4 bytes = the tile's 128 bias values
-        const uint8_t *src = (const uint8_t *)a.bias + (size_t)min(n0 + 2 * lane, a.N - 2) * 2;
-        __builtin_amdgcn_global_load_lds((const SVDQ_AS1 void *)src, (SVDQ_AS3 void *)(sepi + LORA_UP_BYTES), 4, 0, 0);
-    }
+    if (a.bias != nullptr && wm == 3)  // 64 lanes x 4 bytes = the tile's 128 bias values
+        g_load4_lds(g_buffer((const uint16_t *)a.bias + n0), sepi + LORA_UP_BYTES, 2u * (uint32_t)min(2 * lane, a.N - 2 - n0), 0);
     if (a.R > 0) {
 #pragma unroll
         for (int i = 0; i < 2; i++) {
             const int q = wm * 2 + i, c = q >> 2, blk = q & 3;  // wave-uniform
-            const uint8_t *src = (const uint8_t *)a.lora_up + ((size_t)min(n0 + blk * 32 + l32, a.N - 1) * a.ld_lora_up + 16 * c + 8 * half) * 2;
-            if (16 * c < a.R)
-                __builtin_amdgcn_global_load_lds((const SVDQ_AS1 void *)src, (SVDQ_AS3 void *)(sepi + q * BLK_BYTES), 16, 0, 0);
+            const int r0 = min(n0 + blk * 32, a.N - 1);         // the block's first row: its rows are 32-bit offsets from there
+            const __amdgpu_buffer_rsrc_t r = g_buffer((const uint16_t *)a.lora_up + (size_t)r0 * a.ld_lora_up);
+            const uint32_t row = (uint32_t)(min(n0 + blk * 32 + l32, a.N - 1) - r0);
+            if (16 * c < a.R) g_load16_lds(r, sepi + q * BLK_BYTES, row * 2u * (uint32_t)a.ld_lora_up + (uint32_t)(32 * c + 16 * half), 0);
         }
     }
 }

@@ -32,7 +32,7 @@
 extern "C" {
 #endif
 
-#define SVDQ_ABI_VERSION 12
+#define SVDQ_ABI_VERSION 13
 
 enum { SVDQ_BF16 = 0, SVDQ_FP16 = 1 };
 enum { SVDQ_PRE_NONE = 0, SVDQ_PRE_GLU = 1, SVDQ_PRE_GELU = 2 }; /* svdq_quantize_args.prologue */
@@ -72,7 +72,7 @@ typedef struct {
                               * x[:, :K] * silu(x[:, K:]) (fuse_glu); SVDQ_PRE_GELU: tanh-GELU of x (fuse_gelu,
                               * ops/triton/gemm_w4a4.py:1403-1408): the LoRA-down sees the result rounded to T */
     float shift;             /* added before smoothing (0.171875 after GELU, else 0)                        */
-    /* Optional norm prologue (NULL norm_stats = off; only with SVDQ_PRE_NONE): the quantized and LoRA-projected value is
+    /* Optional norm prologue (NULL norm_stats and norm_eps 0 = off; only with SVDQ_PRE_NONE): the quantized and LoRA-projected value is
      * T(T(T((x - mean[m]) * rstd[m]) * norm_scale[k]) + norm_shift[k]), i.e. LayerNorm without affine followed by the
      * adaLN modulate, each step rounded to T as separate elementwise kernels would
      * (nunchaku/models/normalization.py:97-104, models/transformers/transformer_flux_v2.py:236-237). */
@@ -99,6 +99,9 @@ typedef struct {
     /* 512; the buffer holds ceil(M / 32) * 32 * (K / 64) elements, 16-byte aligned; ld_scales is not used).  No          */
     /* counterpart in the reference.                                                                                      */
     int32_t scales_blocked;
+    /* norm prologue with norm_stats == NULL: > 0 = the statistics are computed by this call, bit for bit as svdq_row_stats     */
+    /* would with this eps (one launch less); 0 = norm_stats decides                                                            */
+    float norm_eps;
 } svdq_quantize_args;
 
 int svdq_quantize_act(const svdq_quantize_args *args, void *stream);

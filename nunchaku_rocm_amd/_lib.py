@@ -15,7 +15,7 @@ import torch
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libsvdq_mi355x.so")
-ABI_VERSION = 12
+ABI_VERSION = 13
 
 BF16, FP16 = 0, 1
 EPI_PLAIN, EPI_QK_NORM_ROPE, EPI_GELU_QUANT, EPI_SWIGLU_QUANT = 0, 1, 2, 3
@@ -67,6 +67,7 @@ class QuantizeArgs(ctypes.Structure):
         + [("shift", _f32)]
         + [(n, _vp) for n in ("norm_stats", "norm_scale", "norm_shift")]
         + [(n, _i32) for n in ("norm_rows_per_batch", "norm_ld", "norm_stride", "out_blocked", "scales_blocked")]
+        + [("norm_eps", _f32)]
     )  # fmt: skip
 
 

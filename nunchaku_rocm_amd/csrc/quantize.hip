@@ -47,6 +47,76 @@ struct QVecs {
     uint16_t sm, ns, nh;  // smooth factor, norm scale, norm shift
 };
 
+template <int CTRL>
+__device__ inline float q_dpp(float x) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xF, 0xF, false));
+}
+// Sum over the wavefront, the same value in every lane, fixed order: pairs, quads, octets, rows of sixteen lanes (data
+// parallel primitives, no LDS round trips), then the four rows in order.
+__device__ inline float wave_sum(float s) {
+    s += q_dpp<0xB1>(s);   // quad_perm [1, 0, 3, 2]
+    s += q_dpp<0x4E>(s);   // quad_perm [2, 3, 0, 1]
+    s += q_dpp<0x141>(s);  // row_half_mirror
+    s += q_dpp<0x140>(s);  // row_mirror
+    const int b = __builtin_bit_cast(int, s);
+    const float r0 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(b, 0)), r1 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(b, 16));
+    const float r2 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(b, 32)), r3 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(b, 48));
+    return ((r0 + r1) + r2) + r3;
+}
+
+// (mean, 1 / sqrt(var + eps)) of NR rows by one wavefront: mean, then the centred sum of squares, in an order of sums that
+// depends on K alone.  Rows of up to 512 * MAXC values are read once and kept in registers, the loads of all rows issued
+// eight to a row at a time without branches (offsets past the end of the row are clamped and those chunks not used), so that a
+// wavefront has 8 KB and more in flight instead of 1; longer rows are read twice, the second time from cache.
+template <typename T, int NR, int MAXC>
+__device__ __forceinline__ void row_moments(const uint16_t *const (&row)[NR], int K, float eps, int lane, float2 (&out)[NR]) {
+    constexpr int BATCH = 8;  // 16-byte chunks of a row: loads in flight
+    float s[NR], q[NR], mean[NR];
+#pragma unroll
+    for (int n = 0; n < NR; n++) s[n] = q[n] = 0.0f;
+    auto add = [&](int n, v4i w) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) s[n] += T::lo_f32((uint32_t)w[e]) + T::hi_f32((uint32_t)w[e]);
+    };
+    auto add_squares = [&](int n, v4i w) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const float d0 = T::lo_f32((uint32_t)w[e]) - mean[n], d1 = T::hi_f32((uint32_t)w[e]) - mean[n];
+            q[n] += d0 * d0 + d1 * d1;
+        }
+    };
+    if (K <= 512 * MAXC) {
+        v4i r[NR][MAXC];
+#pragma unroll
+        for (int c0 = 0; c0 < MAXC; c0 += BATCH)
+            if (512 * c0 < K) {
+#pragma unroll
+                for (int n = 0; n < NR; n++)
+#pragma unroll
+                    for (int u = 0; u < BATCH; u++) r[n][c0 + u] = *(const v4i *)(row[n] + min(8 * lane + 512 * (c0 + u), K - 8));
+            }
+#pragma unroll
+        for (int n = 0; n < NR; n++) {
+#pragma unroll
+            for (int c = 0; c < MAXC; c++)
+                if (8 * lane + 512 * c < K) add(n, r[n][c]);
+            mean[n] = wave_sum(s[n]) / (float)K;
+#pragma unroll
+            for (int c = 0; c < MAXC; c++)
+                if (8 * lane + 512 * c < K) add_squares(n, r[n][c]);
+        }
+    } else {
+#pragma unroll
+        for (int n = 0; n < NR; n++) {
+            for (int k = 8 * lane; k < K; k += 512) add(n, *(const v4i *)(row[n] + k));
+            mean[n] = wave_sum(s[n]) / (float)K;
+            for (int k = 8 * lane; k < K; k += 512) add_squares(n, *(const v4i *)(row[n] + k));
+        }
+    }
+#pragma unroll
+    for (int n = 0; n < NR; n++) out[n] = make_float2(mean[n], 1.0f / sqrtf(wave_sum(q[n]) / (float)K + eps));
+}
+
 template <typename T, bool UNSIGNED, int PRE, bool HAS_LORA, bool HAS_SMOOTH, bool NORM, int QR>
 __global__ __launch_bounds__(Q_WAVES * 64, QR == 32 ? 1 : (NORM ? 4 : 2)) void quantize_act_kernel(svdq_quantize_args a) {
     constexpr bool GLU = PRE == SVDQ_PRE_GLU, GELU = PRE == SVDQ_PRE_GELU;
@@ -60,6 +130,7 @@ __global__ __launch_bounds__(Q_WAVES * 64, QR == 32 ? 1 : (NORM ? 4 : 2)) void q
     static_assert(!HAS_LORA || Q_RCHUNK * (QR + 1) * 4 <= WAVE_BYTES, "partial products do not fit the wavefront's stages");
     __shared__ __align__(16) uint8_t smem[Q_WAVES * WAVE_BYTES];
     __shared__ float lds_rs[Q_WAVES][64];
+    __shared__ float2 lds_st[NORM ? QR : 1];  // (mean, rstd) of the workgroup's rows
     __shared__ float lds_ns[NORM ? Q_WAVES : 1][64], lds_nh[NORM ? Q_WAVES : 1][64];
     auto lds_acc = [&](int w) { return (float (*)[QR + 1])(smem + w * WAVE_BYTES); };  // [Q_RCHUNK][QR + 1] of wavefront w
 
@@ -129,11 +200,28 @@ __global__ __launch_bounds__(Q_WAVES * 64, QR == 32 ? 1 : (NORM ? 4 : 2)) void q
     float n_mean[NH], n_rstd[NH];
     const uint16_t *__restrict__ nscale = nullptr, *__restrict__ nshift = nullptr;
     if (NORM) {
+        if (a.norm_stats == nullptr) {
+            // the statistics of the workgroup's own rows, two to a wavefront, by the code (and with the bits) of
+            // row_stats_kernel: the rows are about to be read anyway, the second time from L2 (K = 3072, both launches / this one:
+            // 4096 rows 20.6 / 17.0 us, 8192 32.2 / 28.5, 512 equal)
+            static_assert(Q_ROWS == 2 * Q_WAVES, "two rows of a half to a wavefront");
+#pragma unroll
+            for (int h = 0; h < NH; h++) {
+                const uint16_t *row[2];
+                float2 st[2];
+#pragma unroll
+                for (int n = 0; n < 2; n++) row[n] = (const uint16_t *)a.x + (size_t)min(m0 + Q_ROWS * h + 2 * wave + n, a.M - 1) * a.ld_x;
+                row_moments<T, 2, 8>(row, a.K, a.norm_eps, lane, st);
+                if (lane == 0) lds_st[Q_ROWS * h + 2 * wave] = st[0], lds_st[Q_ROWS * h + 2 * wave + 1] = st[1];
+            }
+            __syncthreads();
+        }
 #pragma unroll
         for (int h = 0; h < NH; h++) {
             const int mr = min(m0 + Q_ROWS * h + ml, a.M - 1);
-            n_mean[h] = a.norm_stats[2 * mr];
-            n_rstd[h] = a.norm_stats[2 * mr + 1];
+            const float2 st = a.norm_stats ? *(const float2 *)(a.norm_stats + 2 * mr) : lds_st[Q_ROWS * h + ml];
+            n_mean[h] = st.x;
+            n_rstd[h] = st.y;
         }
         const size_t voff = a.norm_rows_per_batch > 0 ? (size_t)(m0 / a.norm_rows_per_batch) * a.norm_ld : 0;
         nscale = (const uint16_t *)a.norm_scale + voff;
@@ -440,79 +528,15 @@ __global__ __launch_bounds__(Q_WAVES * 64, QR == 32 ? 1 : (NORM ? 4 : 2)) void q
     }
 }
 
-template <int CTRL>
-__device__ inline float q_dpp(float x) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xF, 0xF, false));
-}
-// Sum over the wavefront, the same value in every lane, fixed order: pairs, quads, octets, rows of sixteen lanes (data
-// parallel primitives, no LDS round trips), then the four rows in order.
-__device__ inline float wave_sum(float s) {
-    s += q_dpp<0xB1>(s);   // quad_perm [1, 0, 3, 2]
-    s += q_dpp<0x4E>(s);   // quad_perm [2, 3, 0, 1]
-    s += q_dpp<0x141>(s);  // row_half_mirror
-    s += q_dpp<0x140>(s);  // row_mirror
-    const int b = __builtin_bit_cast(int, s);
-    const float r0 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(b, 0)), r1 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(b, 16));
-    const float r2 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(b, 32)), r3 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(b, 48));
-    return ((r0 + r1) + r2) + r3;
-}
-
-// one wavefront per row: mean, then the centred sum of squares, fixed reduction order.  Rows of up to 8192 values are
-// read once and kept in registers, their loads issued eight at a time without branches (offsets past the end of the
-// row are clamped and those chunks not used), so that a wavefront has 8 KB in flight instead of 1; longer rows are read
-// twice, the second time from cache.
+// one wavefront per row
 template <typename T>
 __global__ __launch_bounds__(256) void row_stats_kernel(const uint16_t *x, float *stats, int M, int K, long ld_x, float eps) {
-    constexpr int MAXC = 16, BATCH = 8;  // 16-byte chunks per lane kept in registers; loads in flight
     const int lane = threadIdx.x & 63, m = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (m >= M) return;
-    const uint16_t *row = x + (long)m * ld_x;
-    float s = 0.0f, q = 0.0f, mean;
-    if (K <= 512 * MAXC) {
-        v4i r[MAXC];
-#pragma unroll
-        for (int c0 = 0; c0 < MAXC; c0 += BATCH)
-            if (512 * c0 < K) {
-#pragma unroll
-                for (int u = 0; u < BATCH; u++) r[c0 + u] = *(const v4i *)(row + min(8 * lane + 512 * (c0 + u), K - 8));
-            }
-#pragma unroll
-        for (int c = 0; c < MAXC; c++)
-            if (8 * lane + 512 * c < K) {
-#pragma unroll
-                for (int e = 0; e < 4; e++) s += T::lo_f32((uint32_t)r[c][e]) + T::hi_f32((uint32_t)r[c][e]);
-            }
-        mean = wave_sum(s) / (float)K;
-#pragma unroll
-        for (int c = 0; c < MAXC; c++)
-            if (8 * lane + 512 * c < K) {
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    const float d0 = T::lo_f32((uint32_t)r[c][e]) - mean, d1 = T::hi_f32((uint32_t)r[c][e]) - mean;
-                    q += d0 * d0 + d1 * d1;
-                }
-            }
-    } else {
-        for (int k = 8 * lane; k < K; k += 512) {
-            const v4i w = *(const v4i *)(row + k);
-#pragma unroll
-            for (int e = 0; e < 4; e++) s += T::lo_f32((uint32_t)w[e]) + T::hi_f32((uint32_t)w[e]);
-        }
-        mean = wave_sum(s) / (float)K;
-        for (int k = 8 * lane; k < K; k += 512) {
-            const v4i w = *(const v4i *)(row + k);
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const float d0 = T::lo_f32((uint32_t)w[e]) - mean, d1 = T::hi_f32((uint32_t)w[e]) - mean;
-                q += d0 * d0 + d1 * d1;
-            }
-        }
-    }
-    const float var = wave_sum(q) / (float)K;
-    if (lane == 0) {
-        stats[2 * m] = mean;
-        stats[2 * m + 1] = 1.0f / sqrtf(var + eps);
-    }
+    const uint16_t *row[1] = {x + (long)m * ld_x};
+    float2 st[1];
+    row_moments<T, 1, 16>(row, K, eps, lane, st);
+    if (lane == 0) *(float2 *)(stats + 2 * m) = st[0];
 }
 
 // one wavefront per row; the rounded results stay in registers (packed) for the statistics, so the row is read once
@@ -604,6 +628,8 @@ __global__ void transpose_kr_kernel(const uint16_t *in, uint16_t *out, int K, in
     out[idx] = in[(size_t)k * ld_in + r];
 }
 
+static bool has_norm(const svdq_quantize_args &a) { return a.norm_stats || a.norm_eps > 0.0f; }
+
 // Rows per workgroup.  A workgroup streams 4 KB of LoRA-down weight per group whatever its number of rows, and the
 // vector memory pipe of a CU is what that traffic is bound by: with 16-row workgroups, M = 4608 puts two of them on 32 of
 // the 256 CUs and the launch waits for those.  32-row workgroups (one LoRA-down tile read for two MFMA passes; a longer
@@ -612,7 +638,7 @@ __global__ void transpose_kr_kernel(const uint16_t *in, uint16_t *out, int K, in
 // R = 32); below and above that range the 16-row kernel wins.
 static int quantize_rows_per_workgroup(const svdq_quantize_args &a) {
     if (a.R == 0 || a.prologue != SVDQ_PRE_NONE) return Q_ROWS;
-    if (a.norm_stats) return Q_ROWS;  // twice the arithmetic per value: 19.0 against 19.9 us at M = 4608, 20.6 against 21.7 at 8192
+    if (has_norm(a)) return Q_ROWS;  // twice the arithmetic per value: 19.0 against 19.9 us at M = 4608, 20.6 against 21.7 at 8192
     const int wg16 = (a.M + 15) / 16;
     return (wg16 > Q32_ABOVE && wg16 <= Q32_UPTO) ? 32 : Q_ROWS;
 }
@@ -638,7 +664,7 @@ static int quantize_grid_y(const svdq_quantize_args &a, int row_blocks, int rows
     const int chunks = (a.R + Q_RCHUNK - 1) / Q_RCHUNK, cus = device_cus();
     // (with a prologue the workgroups that only project compute it a second time: only where half the CUs would idle
     // anyway; norm prologue, M = 512: 10.4 against 11.8 us, M = 4608: 25.5 against 20.7)
-    const bool prologue = a.norm_stats || a.prologue != SVDQ_PRE_NONE;
+    const bool prologue = has_norm(a) || a.prologue != SVDQ_PRE_NONE;
     const int limit = prologue ? cus / 2 : cus + (rows == 32 ? cus / 8 : 0);
     if (row_blocks * (chunks + 1) > limit) return chunks;
     const int nq = std::min({3, limit / row_blocks - chunks, a.K / GROUP});
@@ -673,7 +699,7 @@ static void launch_quantize3(const svdq_quantize_args &a, hipStream_t s) {
 template <typename T, bool U, int G>
 static void launch_quantize2(const svdq_quantize_args &a, hipStream_t s) {
     if constexpr (G == SVDQ_PRE_NONE) {
-        if (a.norm_stats) {
+        if (has_norm(a)) {
             launch_quantize3<T, U, SVDQ_PRE_NONE, true>(a, s);
             return;
         }
@@ -753,7 +779,7 @@ extern "C" int svdq_quantize_act(const svdq_quantize_args *args, void *stream) {
         set_error("svdq_quantize_act: dtype %d", a.dtype);
         return SVDQ_E_INVALID;
     }
-    if (a.norm_stats) {
+    if (has_norm(a)) {
         if (a.prologue != SVDQ_PRE_NONE) {
             set_error("svdq_quantize_act: the norm prologue cannot be combined with the GLU / GELU prologue");
             return SVDQ_E_UNSUPPORTED;

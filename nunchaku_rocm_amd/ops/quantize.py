@@ -28,10 +28,13 @@ def layer_norm_stats(input: torch.Tensor, eps: float = 1e-6) -> torch.Tensor:
 
 
 def _norm_args(norm, inp: torch.Tensor, M: int, K: int, eps: float):
-    """``norm = (scale, shift[, stats])`` -> (stats, scale, shift, rows_per_batch, ld, stride) for the C call.  scale
-    and shift are used where they lie when they share their strides (as the slices of one adaLN projection do)."""
+    """``norm = (scale, shift[, stats])`` -> (stats, scale, shift, rows_per_batch, ld, stride) for the C call; no stats: the
+    quantizer computes them itself (except for an ``eps`` of 0, which the C call reads as none).  scale and shift are used
+    where they lie when they share their strides (as the slices of one adaLN projection do)."""
     scale, shift = norm[0], norm[1]
-    stats = norm[2] if len(norm) > 2 and norm[2] is not None else layer_norm_stats(inp, eps)
+    stats = norm[2] if len(norm) > 2 else None
+    if stats is None and not eps > 0:
+        stats = layer_norm_stats(inp, eps)
     if scale.dim() == 1:
         scale, shift = scale[None], shift[None]
     batches = scale.shape[0]
@@ -39,7 +42,7 @@ def _norm_args(norm, inp: torch.Tensor, M: int, K: int, eps: float):
         raise ValueError("norm scale and shift must both be (K,) or (batches, K) of the input dtype")
     if M % batches or (batches > 1 and (M // batches) % 16):
         raise ValueError(f"{M} rows do not split into {batches} batches of a multiple of 16 rows")
-    if stats.dtype != torch.float32 or stats.shape != (M, 2) or not stats.is_contiguous():
+    if stats is not None and (stats.dtype != torch.float32 or stats.shape != (M, 2) or not stats.is_contiguous()):
         raise ValueError("norm stats must be a contiguous (M, 2) float32 tensor")
     if scale.stride() != shift.stride() or scale.stride(1) < 1 or (batches > 1 and scale.stride(0) < 0):
         scale, shift = scale.contiguous(), shift.contiguous()
@@ -151,6 +154,7 @@ def quantize_w4a4_act_fuse_lora(
         shift=float(shift_value),
         out_blocked=min(out_blocked, 2),
         scales_blocked=int(out_blocked == 3),
+        norm_eps=float(norm_eps) if norm is not None and nstats is None else 0.0,
     )
     with _lib.on_device(inp.device):
         _lib.check(_lib.load().svdq_quantize_act(args, _lib.stream_of(inp)))

@@ -196,6 +196,25 @@ def test_norm_modulate_prologue(dev, M, K, R, batches, dtype):
     assert torch.equal(q3[:M], q[:M]) and torch.equal(s3[:, :M].view(torch.int16), s[:, :M].view(torch.int16))
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,K,R", [(1, 64, 16), (17, 512, 32), (33, 4096, 48), (16, 4160, 16), (31, 8192, 0), (18, 8256, 32), (4100, 128, 16)])
+def test_statistics_inside_the_quantizer(dev, M, K, R, dtype):
+    """The row statistics a norm prologue computes for itself are layer_norm_stats' own, bit for bit: rows kept in registers
+    up to K = 4096 there and 8192 here, read twice beyond; ends of the row blocks; one and several workgroups to a row block."""
+    from nunchaku_rocm_amd import ops
+
+    g = torch.Generator(device=dev).manual_seed(M + K)
+    x = (torch.randn(M, K, generator=g, device=dev) * 1.7 + 0.3).to(dtype)
+    scale, shift = (1 + 0.3 * torch.randn(K, generator=g, device=dev)).to(dtype), (0.2 * torch.randn(K, generator=g, device=dev)).to(dtype)
+    down = torch.randn(K, R, generator=g, device=dev).to(dtype) if R else None
+    for eps in (1e-6, 0.25, 0.0):
+        own = ops.svdq_quantize_w4a4_act_fuse_lora_cuda(x, lora_down=down, norm=(scale, shift), norm_eps=eps)
+        given = ops.svdq_quantize_w4a4_act_fuse_lora_cuda(x, lora_down=down, norm=(scale, shift, ops.layer_norm_stats(x, eps)), norm_eps=eps)
+        torch.cuda.synchronize()
+        assert torch.equal(own[0][:M], given[0][:M]) and torch.equal(own[1][:, :M].view(torch.int16), given[1][:, :M].view(torch.int16))
+        assert torch.equal(own[2][:M], given[2][:M])
+
+
 def test_plain_aliases_and_quantized_product(dev):
     """quantize_w4a4_act / quantize_w4a4_wgt (no smoothing, no LoRA): bit-equal to the oracle, and their outputs are the
     GEMM's natural-layout operands: the int4 product tracks the dense one within the quantization noise."""

@@ -15,6 +15,7 @@ import torch
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libsvdq_mi355x.so")
+HOST_PATH = os.path.join(_HERE, "_host.so")
 ABI_VERSION = 13
 
 BF16, FP16 = 0, 1
@@ -108,6 +109,7 @@ class AttentionArgs(ctypes.Structure):
 
 
 _lib = None
+_host = None  # the extension with the operators' checks in native code (csrc/host.cpp)
 
 
 def load() -> ctypes.CDLL:
@@ -164,8 +166,23 @@ def load() -> ctypes.CDLL:
     lib.svdq_group_acc_i32.argtypes = [_vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _vp]
     if lib.svdq_abi_version() != ABI_VERSION:
         raise RuntimeError(f"{LIB_PATH} has ABI version {lib.svdq_abi_version()}, expected {ABI_VERSION}: rebuild it")
+    host()
     _lib = lib
     return lib
+
+
+def host():
+    """The extension that checks an operator's ordinary call and fills its argument block (see ``csrc/host.cpp``)."""
+    global _host
+    if _host is None:
+        try:
+            from . import _host as native
+        except ImportError as e:
+            raise RuntimeError(f"{HOST_PATH} is missing or does not load ({e}): build it with `python -m nunchaku_rocm_amd.build`") from e
+        if native.ABI_VERSION != ABI_VERSION:
+            raise RuntimeError(f"{HOST_PATH} has ABI version {native.ABI_VERSION}, expected {ABI_VERSION}: rebuild it")
+        _host = native
+    return _host
 
 
 def hip_runtimes_mapped() -> list[str]:

@@ -58,8 +58,38 @@ def _same_source(src: tuple, t: torch.Tensor) -> bool:
     # The held storage is asked where it is now: one that was resized to nothing gave its block back, and an address noted when
     # the copy was made would fit the next tensor that got the block.  While it has its block, an address in it is in no
     # other storage.  (``t``'s own storage is not asked for: that builds an object at each use.)
+    if _lib._host is not None:
+        same = _lib._host.same_source(src, t)
+        if same is not None:  # (None: not a plain tensor on a GPU)
+            return same
     version, storage, place, shape, stride = src
     return storage.data_ptr() + place == t.data_ptr() and version == t._version and shape == t.shape and stride == t.stride()
+
+
+def _made(cache: dict, t: torch.Tensor) -> tuple | None:
+    """The entry of ``t`` in one of the caches below if its copy is there and valid, and was complete at an earlier use (else
+    the function that makes and orders copies has to look)."""
+    hit = cache.get(id(t))
+    return hit if hit is not None and hit[0]() is t and hit[3].event is None and _same_source(hit[1], t) else None
+
+
+def made_lora_down(lora_down: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor | None] | None:
+    """What :func:`lora_down_t` and, where made, :func:`lora_down_blocked` have; ``None`` where the former has to look."""
+    t, b = _made(_cache, lora_down), _made(_ldb_cache, lora_down)
+    return None if t is None else (t[2], None if b is None else b[2])
+
+
+def made_rotary(rotary_emb: torch.Tensor) -> torch.Tensor | None:
+    hit = _made(_rotary_cache, rotary_emb)
+    return None if hit is None or hit[4] * 128 != rotary_emb.numel() else hit[2]
+
+
+def made_weight_planes(qweight: torch.Tensor, wscales: torch.Tensor) -> torch.Tensor | None:
+    hit = _pinned.get(id(qweight))
+    if hit is not None and hit[0]() is qweight:
+        return hit[1]
+    hit = _made(_planes_cache, qweight)
+    return None if hit is None or not _same_source(hit[4], wscales) else hit[2]
 
 
 def invalidate(t: torch.Tensor) -> None:
@@ -187,7 +217,7 @@ def weight_planes(qweight: torch.Tensor, wscales: torch.Tensor) -> torch.Tensor 
     key = id(qweight)
     hit = _planes_cache.get(key)
     if hit is not None:
-        ref, src, src_s, t, ready = hit
+        ref, src, t, ready, src_s = hit
         if ref() is qweight and _same_source(src, qweight) and _same_source(src_s, wscales):
             if t is not None:
                 ready.wait(t.device)
@@ -203,7 +233,7 @@ def weight_planes(qweight: torch.Tensor, wscales: torch.Tensor) -> torch.Tensor 
             t = None
     try:
         ref = weakref.ref(qweight, lambda _r, k=key: _planes_cache.pop(k, None))
-        _planes_cache[key] = (ref, _source_of(qweight), _source_of(wscales), t, ready)
+        _planes_cache[key] = (ref, _source_of(qweight), t, ready, _source_of(wscales))
     except TypeError:
         pass
     return t

@@ -60,6 +60,13 @@ def scaled_dot_product_attention(
     fp16 / bf16 attention with head dimension 128 or 64 runs on the HIP kernel; what the kernel does not cover (a mask,
     fp32, another head dimension, a strided head dimension) goes to torch, as in the reference.
     """
+    if attn_mask is None:  # the ordinary call, checked in native code; anything else is left to what follows
+        args = _lib.AttentionArgs()
+        out = _lib.host().attention(args, query, key, value) if query.is_cuda else False
+        if out is not False:
+            _lib.check(_lib.load().svdq_attention_fp16(args, _lib.stream_of(query)))
+            B, H, T, D = query.shape
+            return out.view(B, T, H, D).transpose(1, 2)
     if attn_mask is not None or not _covered(query, key, value):
         return F.scaled_dot_product_attention(query, key, value, attn_mask=attn_mask, dropout_p=0.0, is_causal=False)
     B, H, T, D = query.shape

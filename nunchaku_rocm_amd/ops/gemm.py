@@ -5,6 +5,7 @@ from __future__ import annotations
 import torch
 
 from .. import _lib
+from . import _prep
 from ._prep import lora_down_blocked as _lora_down_blocked
 from ._prep import lora_down_t as _lora_down_t
 from ._prep import pinned_weight_planes as _pinned_weight_planes
@@ -149,6 +150,32 @@ def svdq_gemm_w4a4_cuda(
     ``out_vk``, ``out_linearattn``, ``out_q/k/v``) and for the NVFP4-only ones (``fp4``, ``wcscales``, ``alpha != 1``,
     ``fuse_silu``).  ``lora_scales`` is accepted and ignored, as in the reference's ROCm backend.  Returns ``None``.
     """
+    if (
+        poolout is None and out_vk is None and out_linearattn is None and out_q is None and out_k is None and out_v is None
+        and wcscales is None and not fp4 and not fuse_silu and (alpha is None or alpha == 1.0) and not STATIC_SCRATCH
+        and (USE_WEIGHT_PLANES == "all" or (USE_WEIGHT_PLANES == "parameters" and type(wgt) is torch.nn.Parameter))
+    ):  # fmt: skip
+        # the ordinary call, checked in native code: every copy it reads is made (see _prep); anything else is left to what follows
+        planes = _prep.made_weight_planes(wgt, wscales)
+        if planes is not None:
+            down, rot = (None, None), None
+            if lora_down is not None:
+                down = _prep.made_lora_down(lora_down)
+                if down is not None and (fuse_swiglu or not USE_BLOCKED_LORA_DOWN):
+                    down = (down[0], None)
+                elif down is not None and down[1] is None:
+                    down = None
+            if rotary_emb is not None:
+                rot = _prep.made_rotary(rotary_emb) if USE_BLOCKED_ROTARY else None
+            if down is not None:
+                args = _lib.GemmArgs()
+                # (a tensor: the scratch memory of the launch)
+                ready = _lib.host().gemm(args, act, wgt, planes, out, qout, ascales, wscales, oscales, lora_act_in, lora_up, lora_down,
+                                         down[0], down[1], lora_act_out, norm_q, norm_k, rotary_emb, rot, bias, smooth_factor,
+                                         int(act_unsigned), int(fuse_swiglu), int(act_blocked), int(qout_blocked))  # fmt: skip
+                if ready is not False:
+                    _lib.check(_lib.load().svdq_gemm_w4a4(args, _lib.stream_of(act)))
+                    return None
     unsupported = {
         "poolout": poolout,
         "out_vk": out_vk,

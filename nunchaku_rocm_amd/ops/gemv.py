@@ -37,6 +37,14 @@ def awq_gemv_bias(in_feats, kernel, scaling_factors, zeros, bias: torch.Tensor |
     """:func:`awq_gemv_w4a16_cuda`, then ``+ bias`` (``(n,)``, rounded again as an addition of its own would) in the kernel's
     last step where the fused kernel runs and the bias is a contiguous tensor of the output dtype and no more than its values
     (a gradient or a tangent wanted through it: an addition of its own)."""
+    if group_size == 64:  # the ordinary call, checked in native code; anything else is left to what follows
+        args = _lib.AwqGemvArgs()
+        ready = _lib.host().gemv(args, in_feats, kernel, scaling_factors, zeros, bias, m, n, k)
+        if ready:
+            rc = _lib.load().svdq_awq_gemv_w4a16_bias(args, ready[1], _lib.stream_of(in_feats))
+            if rc != _lib.E_UNSUPPORTED:
+                _lib.check(rc)
+                return ready[0]
     _lib.require_cuda(in_feats, kernel, scaling_factors, zeros)
     x = in_feats.reshape(m, k)
     if group_size != 64 or n % 32:

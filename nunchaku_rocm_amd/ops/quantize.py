@@ -5,6 +5,7 @@ from __future__ import annotations
 import torch
 
 from .. import _lib
+from . import _prep
 from ._prep import lora_down_t as _lora_down_t
 
 
@@ -85,6 +86,16 @@ def quantize_w4a4_act_fuse_lora(
     32 -- holds the scales in the GEMM's own order too (``svdq_quantize_args.scales_blocked``, for ``act_blocked=3``;
     :func:`nunchaku_rocm_amd.layout.unblock_scales`).
     """
+    if output is not None and oscales is not None and not (fuse_glu or fp4 or fuse_gelu or shift_value or unsigned):
+        # the ordinary call, checked in native code; anything else is left to what follows
+        down = (None, None) if lora_down is None else _prep.made_lora_down(lora_down)
+        if down is not None:
+            scale, shift, stats = (None, None, None) if norm is None else (norm[0], norm[1], norm[2] if len(norm) > 2 else None)
+            args = _lib.QuantizeArgs()
+            if _lib.host().quantize(args, input, output, oscales, lora_down, down[0], lora_act_out, smooth, stats, scale, shift,
+                                    norm_eps, int(out_blocked)):  # fmt: skip
+                _lib.check(_lib.load().svdq_quantize_act(args, _lib.stream_of(input)))
+                return output, oscales, lora_act_out
     if fp4:
         raise NotImplementedError("NVFP4 quantization is not implemented (int4 only)")
     if fuse_gelu and fuse_glu:
@@ -218,6 +229,10 @@ def svdq_quantize_w4a4_act_fuse_lora_cuda(
         raise NotImplementedError("NVFP4 quantization is not implemented (int4 only)")
     if input.dim() != 2:
         raise ValueError(f"input must be 2-D (M, K), got {tuple(input.shape)}")
+    if output is None and oscales is None and lora_act_out is None and lora_down is not None and not fuse_glu:
+        buffers = _lib.host().quantize_buffers(input, lora_down.shape[1], pad_size, int(out_blocked))
+        if buffers:  # what the lines below allocate
+            output, oscales, lora_act_out = buffers
     batch_size, channels = input.shape
     rank = lora_down.shape[1] if lora_down is not None else 0
     batch_size_pad = _ceil_divide(batch_size, pad_size) * pad_size

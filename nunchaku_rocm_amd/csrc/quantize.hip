@@ -10,7 +10,8 @@
 // Work split: one workgroup = 16 (or 32) rows x all of K, eight wavefronts taking scale groups round-robin with two
 // groups in flight each; on the grid's second axis, one workgroup row per chunk of 32 LoRA ranks and, where CUs are
 // left over, up to three rows that only quantize a slice of the groups each.  A group's operands (16 rows x 128 bytes of activations, 32 ranks x 128 bytes of the transposed
-// LoRA-down weight (R, K)) are fetched straight into LDS (global_load_lds_dwordx4) by loads whose 64 lanes cover eight
+// LoRA-down weight (R, K)) are fetched straight into LDS (buffer_load_dwordx4 ... lds: with a 64-bit address per load, as
+// global_load_lds, the norm prologue's launch took 17.0 instead of 15.7 us at 4096 x 3072) by loads whose 64 lanes cover eight
 // full 128-byte rows -- read lane-per-row from global memory, the same bytes cost the memory pipeline four times as
 // many cycles -- and land in a tile whose 16-byte chunks are XOR-swizzled by the row so that the transposed read-back
 // is conflict free.  Lane (m = lane % 16, q = lane / 16) then owns the 16 consecutive channels [64 g + 16 q, +16)
@@ -40,6 +41,14 @@ constexpr uint32_t pack_bias() {
     uint32_t c = 0;
     for (int j = 0; j < 8; j++) c += (uint32_t)RNE_MAGIC_BITS << (4 * j);
     return c;
+}
+
+// 16 bytes per lane at base + lane offset + uniform offset -> lds + 16 * lane
+__device__ inline __amdgpu_buffer_rsrc_t q_buffer(const void *base) {
+    return __builtin_amdgcn_make_buffer_rsrc((void *)base, 0, (int)0xFFFFFFFFu, 0x00020000);  // raw buffer, 32-bit data format
+}
+__device__ inline void q_load16_lds(__amdgpu_buffer_rsrc_t r, uint8_t *lds, uint32_t lane_off, uint32_t uniform_off) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (SVDQ_AS3 void *)lds, 16, (int)lane_off, (int)uniform_off, 0, 0);
 }
 
 // per-group vectors a lane fetches for the group's 64 channels (one channel per lane), shared through LDS later
@@ -152,7 +161,8 @@ __global__ __launch_bounds__(Q_WAVES * 64, QR == 32 ? 1 : (NORM ? 4 : 2)) void q
     // load's 1 KB, i.e. tile[row][chunk ^ (row & 7)].  Rows >= M re-read row M - 1 and ranks >= R rank R - 1 (valid
     // memory; nothing is stored for them).  Addresses = uniform base + 32-bit lane offset (+ uniform group step).
     const int drow = lane >> 3, dchunk = (lane & 7) ^ drow;
-    const uint8_t *__restrict__ xbase = (const uint8_t *)a.x + (size_t)m0 * a.ld_x * 2;
+    const uint8_t *const xbase = (const uint8_t *)a.x + (size_t)m0 * a.ld_x * 2;
+    const __amdgpu_buffer_rsrc_t rx = q_buffer(xbase), rgate = q_buffer(xbase + (GLU ? (size_t)a.K * 2 : 0));
     uint32_t xdma[2 * NH];
 #pragma unroll
     for (int i = 0; i < 2 * NH; i++) xdma[i] = (uint32_t)(min(m0 + 8 * i + drow, a.M - 1) - m0) * a.ld_x * 2 + dchunk * 16;
@@ -241,7 +251,7 @@ __global__ __launch_bounds__(Q_WAVES * 64, QR == 32 ? 1 : (NORM ? 4 : 2)) void q
 #pragma unroll
         for (int h = 0; h < NH; h++) acc0[h] = acc1[h] = (v4f){0.f, 0.f, 0.f, 0.f};
         // ranks >= R re-read rank R - 1; their accumulator rows are never stored
-        const uint8_t *__restrict__ lbase = (const uint8_t *)a.lora_down_t;
+        const __amdgpu_buffer_rsrc_t rl = q_buffer(a.lora_down_t);
         uint32_t ldma[4] = {0, 0, 0, 0};
         if (HAS_LORA) {
 #pragma unroll
@@ -265,23 +275,17 @@ __global__ __launch_bounds__(Q_WAVES * 64, QR == 32 ? 1 : (NORM ? 4 : 2)) void q
                 qv.nh = nshift[((k0 >> 1) + lane) * a.norm_stride];
             }
 #pragma unroll
-            for (int j = 0; j < 2 * NH; j++)
-                __builtin_amdgcn_global_load_lds((const SVDQ_AS1 void *)(xbase + (xdma[j] + k0)),
-                                                 (SVDQ_AS3 void *)(dst + j * 1024), 16, 0, 0);
+            for (int j = 0; j < 2 * NH; j++) q_load16_lds(rx, dst + j * 1024, xdma[j], k0);
             if (GLU) {
 #pragma unroll
-                for (int j = 0; j < 2 * NH; j++)
-                    __builtin_amdgcn_global_load_lds((const SVDQ_AS1 void *)(xbase + (size_t)a.K * 2 + (xdma[j] + k0)),
-                                                     (SVDQ_AS3 void *)(dst + G_OFF + j * 1024), 16, 0, 0);
+                for (int j = 0; j < 2 * NH; j++) q_load16_lds(rgate, dst + G_OFF + j * 1024, xdma[j], k0);
             }
         };
         auto issue_l = [&](int i) {
             if (!do_lora) return;
             const uint32_t k0 = group_off(i);
 #pragma unroll
-            for (int j = 0; j < 4; j++)
-                __builtin_amdgcn_global_load_lds((const SVDQ_AS1 void *)(lbase + (ldma[j] + k0)),
-                                                 (SVDQ_AS3 void *)(wbase + L_OFF + j * 1024), 16, 0, 0);
+            for (int j = 0; j < 4; j++) q_load16_lds(rl, wbase + L_OFF + j * 1024, ldma[j], k0);
         };
 
         struct Ops {

@@ -602,15 +602,27 @@ __global__ __launch_bounds__(NTHREADS, PIPE ? 2 : 3) void gemm_w4a4_f8_kernel(sv
     tile_epilogue<T, EPI, true>(a, acc, priv, sepi, m0, n0, pid_n, wm, lane);
 }
 
-// lora_act_out[m, r] = sum over n-tiles of the partial LoRA-down products, in tile order (deterministic)
-__global__ __launch_bounds__(64) void lora_part_reduce_kernel(const float *part, float *out, int tiles, int M, int R2,
-                                                              int ld_out) {
-    const int idx = (blockIdx.x * 64 + threadIdx.x) * 4;  // four consecutive r of one row (R2 % 16 == 0)
-    if (idx >= M * R2) return;
+// lora_act_out[m, r] = sum over n-tiles of the partial LoRA-down products, in an order that depends on their number alone: four
+// wavefronts sum a quarter of the tiles each, in tile order, and the quarters are added in order.  (One wavefront for all tiles
+// has eight of them in flight and waits twelve times for 96 tiles: fc1 + GELU 64 x 12288 31.0 us, 28.8 with four.)
+constexpr int RED_PARTS = 4;
+__global__ __launch_bounds__(64 * RED_PARTS) void lora_part_reduce_kernel(const float *part, float *out, int tiles, int M, int R2,
+                                                                          int ld_out) {
+    __shared__ v4f quarter[RED_PARTS - 1][64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int idx = (blockIdx.x * 64 + lane) * 4;  // four consecutive r of one row (R2 % 16 == 0)
     const size_t stride = (size_t)M * R2;
+    const int per = (tiles + RED_PARTS - 1) / RED_PARTS, t1 = min((w + 1) * per, tiles);
     v4f s = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (idx < M * R2) {
 #pragma unroll 8
-    for (int t = 0; t < tiles; t++) s += *(const v4f *)(part + t * stride + idx);
+        for (int t = w * per; t < t1; t++) s += *(const v4f *)(part + t * stride + idx);
+    }
+    if (w > 0) quarter[w - 1][lane] = s;
+    __syncthreads();
+    if (w > 0 || idx >= M * R2) return;
+#pragma unroll
+    for (int q = 0; q < RED_PARTS - 1; q++) s += quarter[q][lane];
     *(v4f *)(out + (size_t)(idx / R2) * ld_out + idx % R2) = s;
 }
 
@@ -1055,7 +1067,7 @@ static int gemm_w4a4_checked(const svdq_gemm_args &a, void *stream) {
     if (rc) return rc;
     if (quant && a.R2 > 0) {
         const int n = a.M * a.R2;
-        hipLaunchKernelGGL(lora_part_reduce_kernel, dim3((n / 4 + 63) / 64), dim3(64), 0, s, a.scratch, a.lora_act_out,
+        hipLaunchKernelGGL(lora_part_reduce_kernel, dim3((n / 4 + 63) / 64), dim3(64 * RED_PARTS), 0, s, a.scratch, a.lora_act_out,
                            (a.N + BN - 1) / BN, a.M, a.R2, a.ld_lora_act_out);
         rc = check_launch("svdq_gemm_w4a4 (LoRA-down partial sum)");
     }

@@ -32,7 +32,7 @@
 extern "C" {
 #endif
 
-#define SVDQ_ABI_VERSION 13
+#define SVDQ_ABI_VERSION 14
 
 enum { SVDQ_BF16 = 0, SVDQ_FP16 = 1 };
 enum { SVDQ_PRE_NONE = 0, SVDQ_PRE_GLU = 1, SVDQ_PRE_GELU = 2 }; /* svdq_quantize_args.prologue */
@@ -188,9 +188,18 @@ typedef struct {
     int32_t ascales_blocked;
     /* non-zero: the requantizing epilogues write `oscales` in that layout (NQ a multiple of 512; ld_oscales unused)      */
     int32_t oscales_blocked;
+    /* svdq_gemm_w4a4_act_scratch_bytes(args) bytes, 16-byte aligned, or NULL: where a launch with act_blocked = 0 or 1 may   */
+    /* put its activations as fp6 codes with their scales (act_blocked = 2, ascales_blocked) and read them from               */
+    void *act_scratch;
 } svdq_gemm_args;
 
 int svdq_gemm_w4a4(const svdq_gemm_args *args, void *stream);
+
+/* How many bytes svdq_gemm_w4a4 wants behind args->act_scratch; 0 where it reads the activations as they are.  Not zero where
+ * the launch is long enough that re-laying-out its activations first (one pass over them) and running the fp6 x fp6 loop is
+ * the faster way.  Without the memory the launch runs all the same.  Host arithmetic on the sizes; no counterpart in the
+ * reference. */
+size_t svdq_gemm_w4a4_act_scratch_bytes(const svdq_gemm_args *args);
 
 /*
  * One-time re-layout of a rotary table for the Q/K RMSNorm + RoPE epilogue: (rows, 128) fp32 rows of (sin, cos) pairs,

@@ -16,7 +16,7 @@ import torch
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libsvdq_mi355x.so")
 HOST_PATH = os.path.join(_HERE, "_host.so")
-ABI_VERSION = 13
+ABI_VERSION = 14
 
 BF16, FP16 = 0, 1
 EPI_PLAIN, EPI_QK_NORM_ROPE, EPI_GELU_QUANT, EPI_SWIGLU_QUANT = 0, 1, 2, 3
@@ -36,6 +36,7 @@ EXPORTS = (
     "svdq_block_lora_down",
     "svdq_lora_down_blocked_bytes",
     "svdq_gemm_w4a4_scratch_bytes",
+    "svdq_gemm_w4a4_act_scratch_bytes",
     "svdq_gemm_w4a4_static_scratch",
     "svdq_gemm_w4a4_static_scratch_capacity",
     "svdq_gemm_w4a4_static_scratch_prepare",
@@ -84,7 +85,7 @@ class GemmArgs(ctypes.Structure):
         + [(n, _vp) for n in ("qout", "oscales", "smooth_next", "lora_down_t", "lora_act_out", "scratch")]
         + [(n, _i32) for n in ("R2", "ld_qout", "ld_oscales", "ld_lora_act_out")]
         + [("shift", _f32), ("rotary_blocked", _vp), ("lora_down_blocked", _vp), ("act_blocked", _i32), ("qout_blocked", _i32),
-           ("ascales_blocked", _i32), ("oscales_blocked", _i32)]
+           ("ascales_blocked", _i32), ("oscales_blocked", _i32), ("act_scratch", _vp)]
     )  # fmt: skip
 
 
@@ -133,6 +134,8 @@ def load() -> ctypes.CDLL:
     lib.svdq_last_error.restype = ctypes.c_char_p
     lib.svdq_gemm_w4a4_scratch_bytes.restype = ctypes.c_size_t
     lib.svdq_gemm_w4a4_scratch_bytes.argtypes = [_i32, _i32, _i32, _i32]
+    lib.svdq_gemm_w4a4_act_scratch_bytes.restype = ctypes.c_size_t
+    lib.svdq_gemm_w4a4_act_scratch_bytes.argtypes = [ctypes.POINTER(GemmArgs)]
     lib.svdq_weight_planes_bytes.restype = ctypes.c_size_t
     lib.svdq_weight_planes_bytes.argtypes = [_i32, _i32]
     lib.svdq_split_weight_planes.argtypes = [_vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _vp]

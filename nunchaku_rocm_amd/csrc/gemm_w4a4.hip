@@ -709,6 +709,43 @@ __global__ __launch_bounds__(256) void block_rotary_kernel(const float *rot, v4f
     out[o] = *(const v4f *)(rot + (size_t)(row < rows ? row : 0) * ld + d);
 }
 
+// Activations as nibbles -- the (M, K / 2) matrix, or its bytes in lane order -- and their scales as the fp6 codes and scales of
+// act_blocked = 2 with ascales_blocked.  Thread (32-row block, group, lane 32 h + r): nibble h of the 32 bytes of row r's group.
+// Two's complement nibbles become sign | magnitude four to a dword: t = sign, magnitude = (x ^ 15 t) + t.  Bound by its own launch
+// and latency (every thread one round of loads, work and stores): 4608 x 3072 moves 18 MB in about 5 us.
+template <bool SIGNED>
+__global__ __launch_bounds__(256) void act_to_f6_kernel(const uint8_t *act, const uint16_t *ascales, uint8_t *codes, uint16_t *scales, int rows,
+                                                        int G, int ld_act, int ld_ascales, int blocked) {
+    const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
+    const int g = blockIdx.x * 4 + (threadIdx.x >> 6), rb = blockIdx.y, m = rb * 32 + r;  // (G is a multiple of 8)
+    if (m >= rows) return;
+    const size_t bg = (size_t)rb * G + g;
+    const uint16_t sc = h == 0 ? ascales[(size_t)g * ld_ascales + m] : (uint16_t)0;
+    const uint8_t *src = blocked ? act + bg * 1024 + r * 16 : act + (size_t)m * ld_act + g * 32;
+    const v4i part[2] = {*(const v4i *)src, *(const v4i *)(src + (blocked ? 512 : 16))};
+    uint32_t p[8];  // four codes of six bits each
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        uint32_t c = ((uint32_t)part[i >> 2][i & 3] >> (4 * h)) & 0x0F0F0F0Fu;
+        if (SIGNED) {
+            const uint32_t t = (c >> 3) & 0x01010101u;
+            c = ((c ^ ((t << 4) - t)) + t) | (t << 5);
+        }
+        p[i] = (c & 0x3Fu) | ((c >> 2) & 0xFC0u) | ((c >> 4) & 0x3F000u) | ((c >> 6) & 0xFC0000u);
+    }
+    uint32_t d[6];
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        d[3 * i] = p[4 * i] | (p[4 * i + 1] << 24);
+        d[3 * i + 1] = (p[4 * i + 1] >> 8) | (p[4 * i + 2] << 16);
+        d[3 * i + 2] = (p[4 * i + 2] >> 16) | (p[4 * i + 3] << 8);
+    }
+    uint8_t *dst = codes + bg * 1536;
+    *(v4i *)(dst + 16 * lane) = (v4i){(int)d[0], (int)d[1], (int)d[2], (int)d[3]};
+    *(v2i *)(dst + 1024 + 8 * lane) = (v2i){(int)d[4], (int)d[5]};
+    if (h == 0) scales[((size_t)rb * (G >> 3) + (g >> 3)) * 256 + r * 8 + (g & 7)] = sc;
+}
+
 template <typename T, bool U, bool ODDG>
 static void launch_gemm_i8(const svdq_gemm_args &a, hipStream_t s) {
     const dim3 grid(((a.M + BM - 1) / BM) * ((a.N + BN - 1) / BN)), block(NTHREADS);
@@ -917,6 +954,32 @@ extern "C" int svdq_gemm_w4a4_split_wavefronts(const svdq_gemm_args *args, int32
     return args && args->K > 0 && args->N > 0 ? split_of(*args, cus > 0 ? cus : cu_count()) : 0;
 }
 
+// Bytes of the re-laid-out activations, where the launch gains by them.  The pass over the activations costs 3 us with its gap,
+// 8 us at 8192 x 3072; the fp6 x fp6 loops take 0.75 of the time of the nibble-fed one where tiles fill the CUs, and less than half where
+// few rows of signed codes otherwise run as 128-row tiles.  us as they are / re-laid-out (bf16, signed, rank 32):
+//   few rows (K split over wavefronts), eight of them: K = 1024, 256 x 3072 10.8 / 9.8;  K = 3072 22.4 / 14.1;  K = 512 7.9 / 8.8;
+//     four: K = 2048, 256 x 6144 16.8 / 15.7;  K = 3072, 512 x 3072 22.5 / 20.0;  K = 1024, 512 x 3072 10.9 / 12.2
+//   more than two 128-row tiles to a CU: K = 2048, 1536 x 6144 33.2 / 29.0;  K = 3072, 4608 x 9216 168 / 132;  K = 1536, 8192 x 1536
+//     29.6 / 31.7;  fewer: K = 3072, 1536 x 3072 32.1 / 31.4, 1024 x 3072 22.7 / 24.5, 2048 x 3072 32.3 / 32.7
+//   K = 6144, any rows: 768 x 3072 41.7 / 40.1, 1536 x 3072 58.0 / 51.3, 4608 x 3072 117 / 93;  K = 4096, 1024 x 4096 30.1 / 30.0
+// Unsigned activations of few rows split their K as they are (split_of); beyond those 1536 x 9216 at K = 3072 58.4 / 51.2.  (The
+// grid of the pass is two-dimensional: 2^20 rows keep it inside 65536.)
+static size_t act_scratch_bytes(const svdq_gemm_args &a, int cus) {
+    if (!a.wgt_planes || a.act_blocked == 2 || a.K <= 0 || a.K % 512 || a.M <= 0 || a.M > 1 << 20 || a.N <= 0 || a.actual_m < 0 ||
+        g_f8_variant.load(std::memory_order_relaxed) >= 0 || split_of(a, cus))
+        return 0;
+    svdq_gemm_args b = a;
+    b.act_blocked = 2, b.ascales_blocked = 1;
+    const bool quant = a.epilogue == SVDQ_EPI_GELU_QUANT || a.epilogue == SVDQ_EPI_SWIGLU_QUANT;
+    const long rows = quant ? a.M : a.actual_m, tiles = ((rows + BM - 1) / BM) * ((a.N + BN - 1) / BN);
+    const int split = split_wavefronts(b, cus);
+    if (!(a.K >= 6144 || (split == 8 && a.K >= 1024) || (split == 4 && a.K >= 2048) || (!split && tiles > 2L * cus && a.K >= 2048))) return 0;
+    const size_t padded = (size_t)((a.M + 31) / 32 * 32);
+    return padded * (size_t)(a.K / 4 * 3) + padded * (size_t)(a.K / GROUP) * 2;
+}
+
+extern "C" size_t svdq_gemm_w4a4_act_scratch_bytes(const svdq_gemm_args *args) { return args ? act_scratch_bytes(*args, cu_count()) : 0; }
+
 extern "C" size_t svdq_gemm_w4a4_scratch_bytes(int32_t M, int32_t N, int32_t R2, int32_t epilogue) {
     if (R2 <= 0 || (epilogue != SVDQ_EPI_GELU_QUANT && epilogue != SVDQ_EPI_SWIGLU_QUANT)) return 0;
     return (size_t)((N + BN - 1) / BN) * (size_t)M * (size_t)R2 * sizeof(float);
@@ -1050,8 +1113,28 @@ static int gemm_w4a4_checked(const svdq_gemm_args &a, void *stream) {
         set_error("svdq_gemm_w4a4: unknown epilogue %d", a.epilogue);
         return SVDQ_E_INVALID;
     }
+    if (a.act_scratch && !al16(a.act_scratch)) {
+        set_error("svdq_gemm_w4a4: act_scratch must be 16-byte aligned");
+        return SVDQ_E_INVALID;
+    }
     if (a.M == 0 || (a.actual_m == 0 && !quant)) return SVDQ_OK;  // nothing to write
     hipStream_t s = (hipStream_t)stream;
+    if (a.act_scratch && act_scratch_bytes(a, cu_count())) {
+        svdq_gemm_args b = a;
+        b.act = a.act_scratch;
+        b.ascales = (uint8_t *)a.act_scratch + (size_t)((a.M + 31) / 32 * 32) * (size_t)(a.K / 4 * 3);
+        b.act_blocked = 2, b.ascales_blocked = 1, b.act_scratch = nullptr;
+        const int rows = quant ? a.M : a.actual_m, G = a.K / GROUP;  // rows behind them are never stored
+        const dim3 grid((unsigned)G / 4, (unsigned)(rows + 31) / 32), block(256);
+        if (a.act_unsigned)
+            hipLaunchKernelGGL(act_to_f6_kernel<false>, grid, block, 0, s, (const uint8_t *)a.act, (const uint16_t *)a.ascales, (uint8_t *)b.act, (uint16_t *)b.ascales,
+                               rows, G, a.ld_act, a.ld_ascales, a.act_blocked);
+        else
+            hipLaunchKernelGGL(act_to_f6_kernel<true>, grid, block, 0, s, (const uint8_t *)a.act, (const uint16_t *)a.ascales, (uint8_t *)b.act, (uint16_t *)b.ascales,
+                               rows, G, a.ld_act, a.ld_ascales, a.act_blocked);
+        const int rc = check_launch("svdq_gemm_w4a4 (activations as fp6 codes)");
+        return rc ? rc : gemm_w4a4_checked(b, stream);
+    }
     if (a.dtype == SVDQ_BF16) {
         if (a.act_unsigned)
             launch_gemm_epi<BF16, true>(a, s);

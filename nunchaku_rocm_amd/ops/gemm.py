@@ -93,6 +93,19 @@ HEAD_DIM = 128
 GELU_SHIFT = 0.171875
 
 
+def _act_scratch(args, device: torch.device) -> torch.Tensor | None:
+    """Memory in which a long launch re-lays-out activations that arrive as nibbles, where it wants some (set in ``args``)."""
+    nbytes = _lib.load().svdq_gemm_w4a4_act_scratch_bytes(args)
+    if not nbytes:
+        return None
+    try:
+        t = torch.empty(nbytes, dtype=torch.uint8, device=device)
+    except torch.OutOfMemoryError:  # the launch runs without it
+        return None
+    args.act_scratch = t.data_ptr()
+    return t
+
+
 def svdq_gemm_w4a4_cuda(
     act: torch.Tensor,
     wgt: torch.Tensor,
@@ -174,6 +187,7 @@ def svdq_gemm_w4a4_cuda(
                                          down[0], down[1], lora_act_out, norm_q, norm_k, rotary_emb, rot, bias, smooth_factor,
                                          int(act_unsigned), int(fuse_swiglu), int(act_blocked), int(qout_blocked))  # fmt: skip
                 if ready is not False:
+                    codes = None if int(act_blocked) >= ACT_CODES_F6 else _act_scratch(args, act.device)  # noqa: F841 (kept until the launch)
                     _lib.check(_lib.load().svdq_gemm_w4a4(args, _lib.stream_of(act)))
                     return None
     unsupported = {
@@ -366,6 +380,8 @@ def svdq_gemm_w4a4_cuda(
         args.shift = 0.0 if fuse_swiglu else GELU_SHIFT
 
     with _lib.on_device(dev):
+        if planes is not None and act_blocked < ACT_CODES_F6 and not STATIC_SCRATCH:
+            keep.append(_act_scratch(args, dev))
         entry = lib.svdq_gemm_w4a4_static_scratch if STATIC_SCRATCH else lib.svdq_gemm_w4a4
         _lib.check(entry(args, _lib.stream_of(act)))
     return None

@@ -71,3 +71,54 @@ def test_wide_tiles_agree_bit_for_bit(dev, rows, k, n, rank, epilogue, dtype):
             continue
         for a, b in zip(_outputs(rows, k, n, rank, epilogue, dtype, dev, build), want):
             assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize(
+    "rows,k,n,rank,epilogue,unsigned",
+    [
+        (1, 1024, 128, 16, "plain", False), (33, 6144, 136, 0, "plain", False), (33, 6144, 136, 32, "plain", True), (257, 6144, 264, 48, "plain", False),
+        (289, 2048, 4096, 32, "plain", False), (65, 1024, 384, 32, "qkv", False), (40, 6144, 128, 32, "gelu", False), (300, 6144, 256, 16, "swiglu", False),
+        (2100, 2048, 4096, 32, "plain", False), (2100, 2048, 4096, 32, "plain", True),
+    ],
+)  # fmt: skip
+def test_nibbles_relaid_out_agree_with_fp6_codes(dev, rows, k, n, rank, epilogue, unsigned, dtype):
+    """Launches that turn the (M, K / 2) matrix, or its bytes in lane order, into fp6 codes first: the bits of the launch that was
+    handed the codes.  (Unsigned activations of few rows are not re-laid-out; their bits agree all the same.)"""
+    from nunchaku_rocm_amd import _lib, ops
+    from nunchaku_rocm_amd.layout import block_activations, block_activations_f6, block_scales
+    from nunchaku_rocm_amd.ops import gemm as G
+
+    print(f"case {rows} x {n}, K={k} R={rank} {epilogue} unsigned={unsigned} {dtype}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(rows + k)
+    lin = {name: t.to(dev) for name, t in O.make_svdq_linear(k, n, R=max(rank, 16), seed=k + n, dtype=dtype).items()}
+    M = -(-rows // 32) * 32
+    act = torch.randint(0, 256, (M, k // 2), generator=g, device=dev, dtype=torch.int16).to(torch.uint8)
+    asc = (torch.rand(k // 64, M, generator=g, device=dev) * 0.1 + 0.01).to(dtype)
+    kw = dict(wgt=lin["qweight"], wscales=lin["wscales"], lora_act_in=torch.randn(M, rank, generator=g, device=dev) if rank else None,
+              lora_up=lin["proj_up"][:, :rank].contiguous() if rank else None, bias=lin["bias"], act_unsigned=unsigned)  # fmt: skip
+    nq = n // 2 if epilogue == "swiglu" else n
+    if epilogue == "qkv":
+        kw.update(norm_q=torch.rand(128, generator=g, device=dev).to(dtype), norm_k=torch.rand(128, generator=g, device=dev).to(dtype),
+                  rotary_emb=torch.randn(rows, 128, generator=g, device=dev))  # fmt: skip
+    elif epilogue != "plain":
+        kw.update(lora_down=torch.randn(nq, 16, generator=g, device=dev).to(dtype), fuse_swiglu=epilogue == "swiglu")
+    wanted, real = [], G._act_scratch
+    old, G.USE_WEIGHT_PLANES = G.USE_WEIGHT_PLANES, "all"
+    G._act_scratch = lambda args, device: wanted.append(t := real(args, device)) or t
+    try:
+        results = []
+        for a, s, mode in ((act, asc, 0), (block_activations(act.cpu()).to(dev), asc, 1), (block_activations_f6(act.cpu(), unsigned).to(dev), block_scales(asc.cpu()).to(dev), 3)):
+            out = dict(out=torch.zeros(rows, n, dtype=dtype, device=dev)) if epilogue in ("plain", "qkv") else dict(
+                qout=torch.zeros(M, nq * 3 // 4, dtype=torch.uint8, device=dev), oscales=torch.zeros(nq // 64, M, dtype=dtype, device=dev),
+                lora_act_out=torch.zeros(M, 16, device=dev), qout_blocked=2)  # fmt: skip
+            for _ in range(2):  # the second call is the native one
+                ops.svdq_gemm_w4a4_cuda(act=a, ascales=s, act_blocked=mode, **kw, **out)
+                torch.cuda.synchronize()
+            results.append([t.view(torch.uint8).cpu() for t in out.values() if torch.is_tensor(t)])
+    finally:
+        G.USE_WEIGHT_PLANES, G._act_scratch = old, real
+    few_unsigned = unsigned and _lib.load().svdq_gemm_w4a4_split_wavefronts(_lib.GemmArgs(wgt_planes=16, M=M, actual_m=rows, N=n, K=k, act_unsigned=1, R=rank), 0)
+    assert len(wanted) == 4 and all((t is None) == bool(few_unsigned) for t in wanted)
+    for other in results[1:]:
+        assert all(torch.equal(x, y) for x, y in zip(results[0], other))

@@ -5,7 +5,7 @@ A step is one pass of the hot path over one batch of synthetic input: the FLUX.1
 (M=4608 tokens, K=3072, N=9216, group 64, LoRA rank 32) as activation quantizer + W4A4 GEMM, inputs resident in HBM.
 ``value`` is 2*M*N*K / step time in TOP/s (the reference's GEMM convention, tests/triton/bench_kernels.py:61, charged
 with the quantizer's time as well).  The step's two launches are recorded once into a HIP graph and the timed region
-replays it, so the figure is what the kernels take and not what Python needs to marshal two calls (about 15 us each,
+replays it, so the figure is what the kernels take and not what Python needs to marshal two calls (about 7 us each,
 more than the quantizer runs); ``--eager`` times the eager calls instead.  Every timed region follows at least 0.12 s
 of the same work without a pause (the W warm-up steps and as many more as that takes): the GPU's clocks need about
 50 ms of continuous work to settle, and the settled rate is the one a denoising loop sees.  The JSON line also carries the roofline of
@@ -31,11 +31,11 @@ INT8_MFMA_PEAK_TOPS = 5000.0  # MI355X dense int8 MFMA, published
 FP6_MFMA_PEAK_TOPS = 10100.0  # MI355X dense fp6 / fp4 MFMA, published
 BF16_MFMA_PEAK_TFLOPS = 2500.0  # MI355X dense bf16 / fp16 MFMA, published
 HBM_PEAK_GBS = 8000.0  # MI355X HBM3E, published
-# HBM bytes of one QKV GEMM launch: 2.00 x FETCH_SIZE + 1.00 x WRITE_SIZE (KiB per dispatch) of the grid-663552 launches
+# HBM bytes of one QKV GEMM launch: 2.00 x FETCH_SIZE + 1.00 x WRITE_SIZE (KiB per dispatch) of the grid-335872 launches
 # in profiles/bench_all_kernels_hbm_traffic.txt, the factors being what the same counters read on plain copy kernels of
 # known size in the same run (FETCH_SIZE reads half the bytes of 16-byte-per-lane loads); counters cannot be read from
 # inside this process
-GEMM_QKV_HBM_BYTES = (2.0 * 103184.3 + 82944.0) * 1024
+GEMM_QKV_HBM_BYTES = (2.0 * 105015.9 + 82944.0) * 1024
 
 
 def _events(n):
@@ -62,8 +62,8 @@ def _steady(run, seconds=STEADY_S):
 
 def _time_kernel(fn, iters=50, warmup=10, graph=False):
     """Average launch duration in ms at settled clocks: HIP events on the launch stream around ``iters`` back-to-back
-    launches.  ``graph=True`` records the launches into one HIP graph first, which takes the host's launch cost (about
-    15 us per call through ctypes, more than the small kernels run) out of the figure."""
+    launches.  ``graph=True`` records the launches into one HIP graph first, which takes the host's launch cost (7 to
+    15 us per call, more than some of the small kernels run) out of the figure."""
     import torch
 
     for _ in range(warmup):
@@ -390,7 +390,7 @@ def main():
                    "M": M, "K": K, "N": N, "rank": R, "group": 64},  # fmt: skip
         "roofline": {
             "bound": "mfma",
-            "kernel": "gemm_w4a4_f8_kernel<BF16, fp6 activation codes with their scales in the loop's order, plain epilogue, three workgroups per CU>",
+            "kernel": "gemm_w4a4_wide_kernel<BF16, plain epilogue>: fp6 activation codes with their scales in the loop's order, 256 x 128 tiles",
             "achieved": round(achieved, 2),
             "peak": INT8_MFMA_PEAK_TOPS,
             "unit": "TOP/s",
@@ -403,7 +403,7 @@ def main():
             "step_over_kernels": round(step_ms / (gemm_ms + quant_ms), 4),
             "frac_of_fp6_mfma_peak": round(achieved / FP6_MFMA_PEAK_TOPS, 4),
             "note": "2*M*N*K integer ops per launch against the int8 MFMA peak the target is stated in (5.0 POP/s); the group "
-                    "products run on the fp6 x fp6 form of v_mfma_scale_f32_32x32x64_f8f6f4 on int4-valued codes (exact integer "
+                    "products run on the fp6 x fp6 form of v_mfma_f32_32x32x64_f8f6f4 on int4-valued codes (exact integer "
                     "sums), whose own published dense peak is 10.1 POP/s (frac_of_fp6_mfma_peak), next to one 16-bit MFMA "
                     "and 16 fp32 FMAs per 32x32 block and group for the scales; avg_launch_ms = back-to-back launches "
                     "between HIP events on the launch stream",

@@ -30,7 +30,9 @@
 //    Fed by this library's own quantizer or requantizing epilogues (act_blocked = 2) the activations arrive as fp6 codes
 //    sign | magnitude in the loop's lane order and go into the matrix instruction as loaded: fp6 x fp6 (half the matrix
 //    time per group), no unpack, no offset, one instantiation for signed and unsigned activations; their scales can come
-//    in the loop's order too (ascales_blocked: one 16-byte load per lane every four stages).
+//    in the loop's order too (ascales_blocked: one 16-byte load per lane every four stages).  Such launches with more 128-row tiles than
+//    CUs are gemm_w4a4_wide.hip's, and those of few rows gemm_w4a4_split.hip's; the ones between run here with two workgroups to a CU.
+//    Long launches whose activations arrive as nibbles turn them into such codes first (act_to_f6_kernel, act_scratch_bytes).
 //  * gemm_w4a4_i8_kernel (packed weights): a 16-byte LDS read holds 32 nibbles; the even and the odd nibbles are split
 //    into two int8 planes with shift/mask only (signed values land in the high nibble of each byte, i.e. times 16;
 //    unsigned activations in the low nibble, times 1).  Both operands use the same split, so the K order inside a group
@@ -712,7 +714,8 @@ __global__ __launch_bounds__(256) void block_rotary_kernel(const float *rot, v4f
 // Activations as nibbles -- the (M, K / 2) matrix, or its bytes in lane order -- and their scales as the fp6 codes and scales of
 // act_blocked = 2 with ascales_blocked.  Thread (32-row block, group, lane 32 h + r): nibble h of the 32 bytes of row r's group.
 // Two's complement nibbles become sign | magnitude four to a dword: t = sign, magnitude = (x ^ 15 t) + t.  Bound by its own launch
-// and latency (every thread one round of loads, work and stores): 4608 x 3072 moves 18 MB in about 5 us.
+// and latency (every thread one round of loads, work and stores): 4608 x 3072 moves 18 MB in 9 us.  Whole rows loaded through
+// LDS and 16-byte stores of the scales were no faster (launches 0.3 to 1 us longer).
 template <bool SIGNED>
 __global__ __launch_bounds__(256) void act_to_f6_kernel(const uint8_t *act, const uint16_t *ascales, uint8_t *codes, uint16_t *scales, int rows,
                                                         int G, int ld_act, int ld_ascales, int blocked) {
@@ -955,7 +958,7 @@ extern "C" int svdq_gemm_w4a4_split_wavefronts(const svdq_gemm_args *args, int32
 }
 
 // Bytes of the re-laid-out activations, where the launch gains by them.  The pass over the activations costs 3 us with its gap,
-// 8 us at 8192 x 3072; the fp6 x fp6 loops take 0.75 of the time of the nibble-fed one where tiles fill the CUs, and less than half where
+// 9 us at 4608 x 3072; the fp6 x fp6 loops take 0.75 of the time of the nibble-fed one where tiles fill the CUs, and less than half where
 // few rows of signed codes otherwise run as 128-row tiles.  us as they are / re-laid-out (bf16, signed, rank 32):
 //   few rows (K split over wavefronts), eight of them: K = 1024, 256 x 3072 10.8 / 9.8;  K = 3072 22.4 / 14.1;  K = 512 7.9 / 8.8;
 //     four: K = 2048, 256 x 6144 16.8 / 15.7;  K = 3072, 512 x 3072 22.5 / 20.0;  K = 1024, 512 x 3072 10.9 / 12.2

@@ -13,8 +13,8 @@ from ._prep import rotary_blocked as _rotary_blocked
 from ._prep import weight_planes as _weight_planes
 
 # Which weights get the GEMM's working copy (fp6 codes in MFMA lane order with their scales and offset terms, cached per
-# tensor, see _prep.weight_planes; 0.84 bytes per weight next to the packed weight's 0.5; without it the GEMM is 36 %
-# slower, 240 against 176 us at the FLUX QKV shape): "parameters" = weights that are nn.Parameter (module weights, which
+# tensor, see _prep.weight_planes; 0.84 bytes per weight next to the packed weight's 0.5; without it the GEMM takes
+# 240 instead of 133 us at the FLUX QKV shape): "parameters" = weights that are nn.Parameter (module weights, which
 # live long), "all" = any weight tensor (a temporary pays the re-layout on every call), "none" = the GEMM unpacks the
 # packed weight itself (int8 main loop, no extra memory).
 USE_WEIGHT_PLANES = "parameters"

@@ -604,28 +604,38 @@ __global__ __launch_bounds__(NTHREADS, PIPE ? 2 : 3) void gemm_w4a4_f8_kernel(sv
     tile_epilogue<T, EPI, true>(a, acc, priv, sepi, m0, n0, pid_n, wm, lane);
 }
 
-// lora_act_out[m, r] = sum over n-tiles of the partial LoRA-down products, in an order that depends on their number alone: four
-// wavefronts sum a quarter of the tiles each, in tile order, and the quarters are added in order.  (One wavefront for all tiles
-// has eight of them in flight and waits twelve times for 96 tiles: fc1 + GELU 64 x 12288 31.0 us, 28.8 with four.)
-constexpr int RED_PARTS = 4;
-__global__ __launch_bounds__(64 * RED_PARTS) void lora_part_reduce_kernel(const float *part, float *out, int tiles, int M, int R2,
+// lora_act_out[m, r] = sum over n-tiles of the partial LoRA-down products, in tile order (deterministic).  What bounds it: latency.
+// The partials of RED_TILES tiles are fetched at once by four wavefronts, each a quarter of them for 256 columns, and laid down in LDS,
+// where every thread sums a column of its own; the next ones are on their way meanwhile.  (fc1 + GELU with its reduction, 64 x 12288:
+// 31.8 us with one wavefront that has eight tiles in flight, 30.2 so; 32 of them in flight per wavefront 35, 16 or 64 tiles in LDS as here.)
+constexpr int RED_WAVES = 4, RED_EACH = 8, RED_TILES = RED_WAVES * RED_EACH;
+__global__ __launch_bounds__(64 * RED_WAVES) void lora_part_reduce_kernel(const float *part, float *out, int tiles, int M, int R2,
                                                                           int ld_out) {
-    __shared__ v4f quarter[RED_PARTS - 1][64];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int idx = (blockIdx.x * 64 + lane) * 4;  // four consecutive r of one row (R2 % 16 == 0)
+    __shared__ __align__(16) float lds[RED_TILES][64 * RED_WAVES];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const size_t stride = (size_t)M * R2;
-    const int per = (tiles + RED_PARTS - 1) / RED_PARTS, t1 = min((w + 1) * per, tiles);
-    v4f s = {0.0f, 0.0f, 0.0f, 0.0f};
-    if (idx < M * R2) {
-#pragma unroll 8
-        for (int t = w * per; t < t1; t++) s += *(const v4f *)(part + t * stride + idx);
-    }
-    if (w > 0) quarter[w - 1][lane] = s;
-    __syncthreads();
-    if (w > 0 || idx >= M * R2) return;
+    const int base = blockIdx.x * 64 * RED_WAVES, last = M * R2 - 4;
+    const float *src = part + min(base + 4 * lane, last);  // (four consecutive r of one row: R2 % 16 == 0)
+    v4f p[RED_EACH];
+    auto fetch = [&](int t0) {
 #pragma unroll
-    for (int q = 0; q < RED_PARTS - 1; q++) s += quarter[q][lane];
-    *(v4f *)(out + (size_t)(idx / R2) * ld_out + idx % R2) = s;
+        for (int u = 0; u < RED_EACH; u++)
+            if (const int t = t0 + RED_WAVES * u + w; t < tiles) p[u] = *(const v4f *)(src + t * stride);
+    };
+    float s = 0.0f;
+    fetch(0);
+    for (int t0 = 0; t0 < tiles; t0 += RED_TILES) {
+#pragma unroll
+        for (int u = 0; u < RED_EACH; u++) *(v4f *)&lds[RED_WAVES * u + w][4 * lane] = p[u];  // (rows past the tiles: not summed)
+        __syncthreads();
+        fetch(t0 + RED_TILES);
+        const int n = min(tiles - t0, RED_TILES);
+#pragma unroll 8
+        for (int t = 0; t < n; t++) s += lds[t][threadIdx.x];
+        __syncthreads();
+    }
+    const int idx = base + threadIdx.x;
+    if (idx < M * R2) out[(size_t)(idx / R2) * ld_out + idx % R2] = s;
 }
 
 // Debug read-out of one group's exact int32 accumulators: one wavefront per 32x32 block, operands straight from
@@ -1153,7 +1163,7 @@ static int gemm_w4a4_checked(const svdq_gemm_args &a, void *stream) {
     if (rc) return rc;
     if (quant && a.R2 > 0) {
         const int n = a.M * a.R2;
-        hipLaunchKernelGGL(lora_part_reduce_kernel, dim3((n / 4 + 63) / 64), dim3(64 * RED_PARTS), 0, s, a.scratch, a.lora_act_out,
+        hipLaunchKernelGGL(lora_part_reduce_kernel, dim3((n / 4 + 63) / 64), dim3(64 * RED_WAVES), 0, s, a.scratch, a.lora_act_out,
                            (a.N + BN - 1) / BN, a.M, a.R2, a.ld_lora_act_out);
         rc = check_launch("svdq_gemm_w4a4 (LoRA-down partial sum)");
     }

@@ -32,7 +32,7 @@
 extern "C" {
 #endif
 
-#define SVDQ_ABI_VERSION 14
+#define SVDQ_ABI_VERSION 15
 
 enum { SVDQ_BF16 = 0, SVDQ_FP16 = 1 };
 enum { SVDQ_PRE_NONE = 0, SVDQ_PRE_GLU = 1, SVDQ_PRE_GELU = 2 }; /* svdq_quantize_args.prologue */
@@ -105,6 +105,10 @@ typedef struct {
 } svdq_quantize_args;
 
 int svdq_quantize_act(const svdq_quantize_args *args, void *stream);
+
+/* 1 where a call that computes its own statistics (norm_eps) is faster with norm_stats filled by svdq_row_stats first, else 0: the
+ * results are the same bits.  Host arithmetic on the sizes; no counterpart in the reference. */
+int svdq_quantize_stats_first(const svdq_quantize_args *args);
 
 /* Per-row mean and 1 / sqrt(biased variance + eps) of x (M, K) T in fp32: stats[m] = (mean, rstd).  The statistics
  * LayerNorm needs (nunchaku/models/normalization.py:97), for the quantizer's norm prologue. */

@@ -16,7 +16,7 @@ import torch
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libsvdq_mi355x.so")
 HOST_PATH = os.path.join(_HERE, "_host.so")
-ABI_VERSION = 14
+ABI_VERSION = 15
 
 BF16, FP16 = 0, 1
 EPI_PLAIN, EPI_QK_NORM_ROPE, EPI_GELU_QUANT, EPI_SWIGLU_QUANT = 0, 1, 2, 3
@@ -25,6 +25,7 @@ E_INVALID, E_UNSUPPORTED, E_LAUNCH = -1, -2, -3
 
 EXPORTS = (
     "svdq_quantize_act",
+    "svdq_quantize_stats_first",
     "svdq_row_stats",
     "svdq_gated_residual",
     "svdq_transpose_lora_down",
@@ -135,6 +136,7 @@ def load() -> ctypes.CDLL:
     lib.svdq_gemm_w4a4_scratch_bytes.restype = ctypes.c_size_t
     lib.svdq_gemm_w4a4_scratch_bytes.argtypes = [_i32, _i32, _i32, _i32]
     lib.svdq_gemm_w4a4_act_scratch_bytes.restype = ctypes.c_size_t
+    lib.svdq_quantize_stats_first.argtypes = [ctypes.POINTER(QuantizeArgs)]
     lib.svdq_gemm_w4a4_act_scratch_bytes.argtypes = [ctypes.POINTER(GemmArgs)]
     lib.svdq_weight_planes_bytes.restype = ctypes.c_size_t
     lib.svdq_weight_planes_bytes.argtypes = [_i32, _i32]

@@ -34,6 +34,7 @@ constexpr int Q_ROWS = 16;         // rows of one MFMA pass; a workgroup takes Q
 constexpr int Q_WAVES = 8;
 constexpr int Q_ROW_BYTES = 128;  // one scale group of one row (64 x 16 bit)
 constexpr int Q_RCHUNK = 32;  // LoRA ranks per pass over the row block
+constexpr int Q_STATS_K = 4096;  // longest row whose statistics the norm prologue computes from registers (two rows to a wavefront)
 constexpr int Q32_ABOVE = 256, Q32_UPTO = 512;  // number of 16-row workgroups for which 32-row workgroups are used instead
 
 // sum_j (0x4B400000 << 4 j) mod 2^32: what eight magic-biased codes add up to besides their nibbles
@@ -212,8 +213,7 @@ __global__ __launch_bounds__(Q_WAVES * 64, QR == 32 ? 1 : (NORM ? 4 : 2)) void q
     if (NORM) {
         if (a.norm_stats == nullptr) {
             // the statistics of the workgroup's own rows, two to a wavefront, by the code (and with the bits) of
-            // row_stats_kernel: the rows are about to be read anyway, the second time from L2 (K = 3072, both launches / this one:
-            // 4096 rows 20.6 / 17.0 us, 8192 32.2 / 28.5, 512 equal)
+            // row_stats_kernel: the rows are about to be read anyway, the second time from L2 (when it is the faster way: stats_first)
             static_assert(Q_ROWS == 2 * Q_WAVES, "two rows of a half to a wavefront");
 #pragma unroll
             for (int h = 0; h < NH; h++) {
@@ -221,7 +221,7 @@ __global__ __launch_bounds__(Q_WAVES * 64, QR == 32 ? 1 : (NORM ? 4 : 2)) void q
                 float2 st[2];
 #pragma unroll
                 for (int n = 0; n < 2; n++) row[n] = (const uint16_t *)a.x + (size_t)min(m0 + Q_ROWS * h + 2 * wave + n, a.M - 1) * a.ld_x;
-                row_moments<T, 2, 8>(row, a.K, a.norm_eps, lane, st);
+                row_moments<T, 2, Q_STATS_K / 512>(row, a.K, a.norm_eps, lane, st);
                 if (lane == 0) lds_st[Q_ROWS * h + 2 * wave] = st[0], lds_st[Q_ROWS * h + 2 * wave + 1] = st[1];
             }
             __syncthreads();
@@ -642,7 +642,7 @@ static bool has_norm(const svdq_quantize_args &a) { return a.norm_stats || a.nor
 // R = 32); below and above that range the 16-row kernel wins.
 static int quantize_rows_per_workgroup(const svdq_quantize_args &a) {
     if (a.R == 0 || a.prologue != SVDQ_PRE_NONE) return Q_ROWS;
-    if (has_norm(a)) return Q_ROWS;  // twice the arithmetic per value: 19.0 against 19.9 us at M = 4608, 20.6 against 21.7 at 8192
+    if (has_norm(a)) return Q_ROWS;  // twice the arithmetic per value: 23.2 against 25.2 us at M = 4608, 27.5 against 28.3 at 8192
     const int wg16 = (a.M + 15) / 16;
     return (wg16 > Q32_ABOVE && wg16 <= Q32_UPTO) ? 32 : Q_ROWS;
 }
@@ -667,12 +667,26 @@ static int quantize_grid_y(const svdq_quantize_args &a, int row_blocks, int rows
     if (a.R == 0) return 1;
     const int chunks = (a.R + Q_RCHUNK - 1) / Q_RCHUNK, cus = device_cus();
     // (with a prologue the workgroups that only project compute it a second time: only where half the CUs would idle
-    // anyway; norm prologue, M = 512: 10.4 against 11.8 us, M = 4608: 25.5 against 20.7)
+    // anyway.  Norm prologue, K = 3072, R = 32, with half of the CUs / all of them as the limit: M = 512 11.0 / 11.0 us, 1024 13.6 /
+    // 12.0, 2048 15.3 / 14.2, 4096 16.7 / 16.2, 4608 23.2 / 22.7)
     const bool prologue = has_norm(a) || a.prologue != SVDQ_PRE_NONE;
     const int limit = prologue ? cus / 2 : cus + (rows == 32 ? cus / 8 : 0);
     if (row_blocks * (chunks + 1) > limit) return chunks;
     const int nq = std::min({3, limit / row_blocks - chunks, a.K / GROUP});
     return chunks + std::max(nq, 1);
+}
+
+// Whether a norm prologue without statistics is faster with a launch of svdq_row_stats in front of it than with computing them
+// itself.  Its own cost a launch less, but every workgroup of the grid's second axis computes them again: with one chunk of ranks no
+// other does, with two it is hidden up to two workgroups to a CU, with more up to one.  Beyond 4096 values a row does not fit
+// the registers and is read twice for them.  us, its own / a launch in front (bf16):
+//   rank 32:  K = 3072, 512 rows 11.2 / 11.2, 4608 23.1 / 26.2, 8192 27.4 / 31.2;  K = 4608, 64 rows 16.4 / 13.1, 4608 37.0 / 35.3
+//   rank 64:  K = 3072, 4096 rows 19.8 / 22.3, 4608 28.6 / 28.4, 8192 44.5 / 38.5;  K = 1024, 4096 rows 11.5 / 12.3, 4608 16.7 / 15.3
+//   rank 128: K = 3072, 333 rows 11.0 / 11.2, 1201 18.9 / 17.8, 8192 75.1 / 59.5;  rank 256: 1201 rows 23.5 / 21.0, 8192 132 / 96
+static bool stats_first(const svdq_quantize_args &a) {
+    if (a.M <= 0 || a.norm_stats || !has_norm(a)) return false;
+    const int chunks = (a.R + Q_RCHUNK - 1) / Q_RCHUNK;
+    return a.K > Q_STATS_K || (chunks > 1 && (long)((a.M + Q_ROWS - 1) / Q_ROWS) * chunks > device_cus() * (chunks == 2 ? 2L : 1L));
 }
 
 template <typename T, bool U, int G, bool NORM>
@@ -802,6 +816,8 @@ extern "C" int svdq_quantize_act(const svdq_quantize_args *args, void *stream) {
         launch_quantize<FP16>(a, (hipStream_t)stream);
     return check_launch("svdq_quantize_act");
 }
+
+extern "C" int svdq_quantize_stats_first(const svdq_quantize_args *args) { return args && stats_first(*args); }
 
 extern "C" int svdq_row_stats(const void *x, float *stats, int32_t M, int32_t K, int32_t ld_x, int32_t dtype, float eps,
                               void *stream) {

@@ -30,7 +30,7 @@ def layer_norm_stats(input: torch.Tensor, eps: float = 1e-6) -> torch.Tensor:
 
 def _norm_args(norm, inp: torch.Tensor, M: int, K: int, eps: float):
     """``norm = (scale, shift[, stats])`` -> (stats, scale, shift, rows_per_batch, ld, stride) for the C call; no stats: the
-    quantizer computes them itself (except for an ``eps`` of 0, which the C call reads as none).  scale and shift are used
+    quantizer computes them itself or :func:`_stats_first` does (except for an ``eps`` of 0, which the C call reads as none).  scale and shift are used
     where they lie when they share their strides (as the slices of one adaLN projection do)."""
     scale, shift = norm[0], norm[1]
     stats = norm[2] if len(norm) > 2 else None
@@ -48,6 +48,18 @@ def _norm_args(norm, inp: torch.Tensor, M: int, K: int, eps: float):
     if scale.stride() != shift.stride() or scale.stride(1) < 1 or (batches > 1 and scale.stride(0) < 0):
         scale, shift = scale.contiguous(), shift.contiguous()
     return stats, scale, shift, (M // batches if batches > 1 else 0), scale.stride(0), scale.stride(1)
+
+
+def _stats_first(args, device: torch.device) -> torch.Tensor | None:
+    """The statistics of a norm prologue that would compute them itself, where a launch of their own in front of it is the faster
+    way (set in ``args``; the same bits)."""
+    lib = _lib.load()
+    if not args.norm_eps > 0 or not lib.svdq_quantize_stats_first(args):
+        return None
+    stats = torch.empty(args.M, 2, dtype=torch.float32, device=device)
+    _lib.check(lib.svdq_row_stats(args.x, stats.data_ptr(), args.M, args.K, args.ld_x, args.dtype, args.norm_eps, _lib.stream_of(stats)))
+    args.norm_stats, args.norm_eps = stats.data_ptr(), 0.0
+    return stats
 
 
 def quantize_w4a4_act_fuse_lora(
@@ -94,6 +106,7 @@ def quantize_w4a4_act_fuse_lora(
             args = _lib.QuantizeArgs()
             if _lib.host().quantize(args, input, output, oscales, lora_down, down[0], lora_act_out, smooth, stats, scale, shift,
                                     norm_eps, int(out_blocked)):  # fmt: skip
+                own = _stats_first(args, input.device)  # noqa: F841 (kept until the launch)
                 _lib.check(_lib.load().svdq_quantize_act(args, _lib.stream_of(input)))
                 return output, oscales, lora_act_out
     if fp4:
@@ -168,6 +181,7 @@ def quantize_w4a4_act_fuse_lora(
         norm_eps=float(norm_eps) if norm is not None and nstats is None else 0.0,
     )
     with _lib.on_device(inp.device):
+        own = _stats_first(args, inp.device)  # noqa: F841 (kept until the launch)
         _lib.check(_lib.load().svdq_quantize_act(args, _lib.stream_of(inp)))
     return output, oscales, lora_act_out
 

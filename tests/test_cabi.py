@@ -88,6 +88,21 @@ def test_invalid_arguments_are_rejected_without_launch(lib):
     assert lib.svdq_gemm_w4a4_scratch_bytes(256, 256, 32, _lib.EPI_PLAIN) == 0
 
 
+def test_when_statistics_have_a_launch_of_their_own(lib):
+    """256 CUs: more than one chunk of 32 ranks on more than two (two chunks) or one (more) workgroups to a CU, rows of more than
+    4096 values; never without a norm, or with statistics given."""
+    from nunchaku_rocm_amd import _lib
+
+    first = lambda M, K, R, **kw: lib.svdq_quantize_stats_first(_lib.QuantizeArgs(M=M, K=K, R=R, **({"norm_eps": 1e-6} | kw)))  # noqa: E731
+    for M, K, R, want in (
+        (1, 64, 16, 0), (8704, 4096, 32, 0), (8704, 4096, 0, 0), (1, 4160, 0, 1), (0, 8192, 32, 0), (4096, 3072, 33, 0), (4096, 3072, 64, 0),
+        (4097, 3072, 64, 1), (4097, 3072, 48, 1), (1360, 64, 96, 0), (1361, 64, 96, 1), (512, 3072, 256, 0), (513, 3072, 256, 1),
+    ):  # fmt: skip
+        assert first(M, K, R) == want, (M, K, R)
+        assert first(M, K, R, norm_eps=0.0) == 0 and first(M, K, R, norm_stats=16) == 0
+    assert lib.svdq_quantize_stats_first(None) == 0
+
+
 def test_ops_refuse_cpu_tensors_loudly():
     from nunchaku_rocm_amd import ops
 

@@ -215,6 +215,40 @@ def test_statistics_inside_the_quantizer(dev, M, K, R, dtype):
         assert torch.equal(own[2][:M], given[2][:M])
 
 
+@pytest.mark.parametrize("M,K,R,launches", [(4096, 128, 64, 1), (4097, 128, 64, 2), (17, 4096, 32, 1), (17, 4160, 32, 2), (512, 192, 256, 1), (530, 192, 256, 2)])
+def test_statistics_in_a_launch_of_their_own(dev, monkeypatch, M, K, R, launches):
+    """Where a statistics launch in front is the faster way it is made, by native and Python checks alike; the bits are the same."""
+    from nunchaku_rocm_amd import _lib, ops
+    from nunchaku_rocm_amd.ops import quantize as Q
+
+    g = torch.Generator(device=dev).manual_seed(M + K)
+    x = (torch.randn(M, K, generator=g, device=dev) * 1.7 + 0.3).to(torch.bfloat16)
+    scale, shift = (1 + 0.3 * torch.randn(K, generator=g, device=dev)).to(x.dtype), (0.2 * torch.randn(K, generator=g, device=dev)).to(x.dtype)
+    down = torch.randn(K, R, generator=g, device=dev).to(x.dtype)
+    lib, seen = _lib.load(), []
+
+    class Lib:
+        def __getattr__(self, name):
+            if name in ("svdq_row_stats", "svdq_quantize_act"):
+                seen.append(name)
+            return getattr(lib, name)
+
+    monkeypatch.setattr(_lib, "load", lambda: Lib())
+    run = lambda: ops.svdq_quantize_w4a4_act_fuse_lora_cuda(x, lora_down=down, norm=(scale, shift))  # noqa: E731
+    results = []
+    for _ in range(3):  # the third call finds its copy of the weight made and complete: the native checks
+        seen.clear()
+        results.append(run())
+        torch.cuda.synchronize()
+        assert seen == ["svdq_row_stats", "svdq_quantize_act"][2 - launches :]
+    monkeypatch.setattr(Q, "_stats_first", lambda args, device: None)
+    results.append(run())  # its own, whatever the size
+    torch.cuda.synchronize()
+    for r in results[1:]:
+        assert torch.equal(r[0][:M], results[0][0][:M]) and torch.equal(r[1][:, :M].view(torch.int16), results[0][1][:, :M].view(torch.int16))
+        assert torch.equal(r[2][:M], results[0][2][:M])
+
+
 def test_plain_aliases_and_quantized_product(dev):
     """quantize_w4a4_act / quantize_w4a4_wgt (no smoothing, no LoRA): bit-equal to the oracle, and their outputs are the
     GEMM's natural-layout operands: the int4 product tracks the dense one within the quantization noise."""

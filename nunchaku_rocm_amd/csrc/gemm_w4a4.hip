@@ -604,13 +604,26 @@ __global__ __launch_bounds__(NTHREADS, PIPE ? 2 : 3) void gemm_w4a4_f8_kernel(sv
     tile_epilogue<T, EPI, true>(a, acc, priv, sepi, m0, n0, pid_n, wm, lane);
 }
 
-// lora_act_out[m, r] = sum over n-tiles of the partial LoRA-down products, in tile order (deterministic).  What bounds it: latency.
-// The partials of RED_TILES tiles are fetched at once by four wavefronts, each a quarter of them for 256 columns, and laid down in LDS,
-// where every thread sums a column of its own; the next ones are on their way meanwhile.  (fc1 + GELU with its reduction, 64 x 12288:
-// 31.8 us with one wavefront that has eight tiles in flight, 30.2 so; 32 of them in flight per wavefront 35, 16 or 64 tiles in LDS as here.)
+// lora_act_out[m, r] = sum over n-tiles of the partial LoRA-down products, in tile order (deterministic): many columns
+// M * R2, four to a thread, eight tiles in flight.
+__global__ __launch_bounds__(64) void lora_part_reduce_kernel(const float *part, float *out, int tiles, int M, int R2,
+                                                              int ld_out) {
+    const int idx = (blockIdx.x * 64 + threadIdx.x) * 4;  // four consecutive r of one row (R2 % 16 == 0)
+    if (idx >= M * R2) return;
+    const size_t stride = (size_t)M * R2;
+    v4f s = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 8
+    for (int t = 0; t < tiles; t++) s += *(const v4f *)(part + t * stride + idx);
+    *(v4f *)(out + (size_t)(idx / R2) * ld_out + idx % R2) = s;
+}
+
+// The same sums for few columns, which leave the chip waiting for a few wavefronts' loads: the partials of RED_TILES tiles are fetched
+// at once by four wavefronts, each a quarter of them for 256 columns, and laid down in LDS, where every thread sums a column of its own;
+// the next ones are on their way meanwhile.  us, this kernel / four columns to a thread (R2 = 32): 96 tiles, 64 rows 4.2 / 5.4, 1024 4.4 / 5.2, 2048 (a
+// workgroup to a CU) 5.9 / 6.0, 4096 9.2 / 8.3;  12 tiles, 512 rows 2.8 / 3.4;  192 tiles, 64 rows 5.8 / 8.9, 4096 16.8 / 14.8.
 constexpr int RED_WAVES = 4, RED_EACH = 8, RED_TILES = RED_WAVES * RED_EACH;
-__global__ __launch_bounds__(64 * RED_WAVES) void lora_part_reduce_kernel(const float *part, float *out, int tiles, int M, int R2,
-                                                                          int ld_out) {
+__global__ __launch_bounds__(64 * RED_WAVES) void lora_part_reduce_few_kernel(const float *part, float *out, int tiles, int M, int R2,
+                                                                              int ld_out) {
     __shared__ __align__(16) float lds[RED_TILES][64 * RED_WAVES];
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const size_t stride = (size_t)M * R2;
@@ -1163,8 +1176,13 @@ static int gemm_w4a4_checked(const svdq_gemm_args &a, void *stream) {
     if (rc) return rc;
     if (quant && a.R2 > 0) {
         const int n = a.M * a.R2;
-        hipLaunchKernelGGL(lora_part_reduce_kernel, dim3((n / 4 + 63) / 64), dim3(64 * RED_WAVES), 0, s, a.scratch, a.lora_act_out,
-                           (a.N + BN - 1) / BN, a.M, a.R2, a.ld_lora_act_out);
+        const dim3 grid((n / 4 + 63) / 64);  // 256 columns to a workgroup in both kernels
+        if (grid.x <= (unsigned)cu_count())  // (both sides: lora_part_reduce_few_kernel)
+            hipLaunchKernelGGL(lora_part_reduce_few_kernel, grid, dim3(64 * RED_WAVES), 0, s, a.scratch, a.lora_act_out, (a.N + BN - 1) / BN, a.M,
+                               a.R2, a.ld_lora_act_out);
+        else
+            hipLaunchKernelGGL(lora_part_reduce_kernel, grid, dim3(64), 0, s, a.scratch, a.lora_act_out, (a.N + BN - 1) / BN, a.M, a.R2,
+                               a.ld_lora_act_out);
         rc = check_launch("svdq_gemm_w4a4 (LoRA-down partial sum)");
     }
     return rc;

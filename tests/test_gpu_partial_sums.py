@@ -8,7 +8,7 @@ pytestmark = pytest.mark.gpu
 
 # tiles: fewer than a batch of loads, whole batches, batches and a rest of eights, of eights and ones, of ones
 @pytest.mark.parametrize("n", [128, 896, 4096, 12288, 6144, 5376, 4352])
-@pytest.mark.parametrize("rows,rank", [(16, 16), (48, 32), (272, 48)])
+@pytest.mark.parametrize("rows,rank", [(16, 16), (48, 32), (272, 48), (2048, 32), (2064, 32)])  # up to, and beyond, a workgroup of 256 columns to a CU
 @pytest.mark.parametrize("epilogue", ["gelu", "swiglu"])
 def test_sum_in_tile_order(dev, monkeypatch, n, rows, rank, epilogue):
     from nunchaku_rocm_amd import _lib, ops

@@ -229,9 +229,9 @@ int svdq_block_lora_down(const void *lora_down_t, void *blocked, int32_t N, int3
 size_t svdq_lora_down_blocked_bytes(int32_t N, int32_t R2);
 
 /* The fp8 main loop exists in two builds: one that fills a loaded CU best (256 x 128 tiles with act_blocked = 2 and
- * ascales_blocked, otherwise three workgroups of 128 x 128 per CU) and one with two workgroups of 128 x 128 per CU and
- * software-pipelined steps (a workgroup on its own runs faster); svdq_gemm_w4a4 picks by the number of 128x128 tiles and
- * CUs.  This overrides the choice for the whole process: -1 = by tile count (default), 0 = for full CUs, 1 = two per CU.
+ * ascales_blocked where they are the faster ones, otherwise three workgroups of 128 x 128 per CU; 0 below forces the former) and one with two workgroups of 128 x 128 per CU and
+ * software-pipelined steps (a workgroup on its own runs faster); svdq_gemm_w4a4 picks by the number of tiles and CUs, K and
+ * the epilogue.  This overrides the choice for the whole process: -1 = by size (default), 0 = for full CUs, 1 = two per CU.
  * For tuning and tests; results of the two are bit-identical.  By default launches with few rows (unsigned activations or
  * fp6 codes) go to a third kernel that splits K over wavefronts and adds the groups up in another order, so the last bit of
  * a row's output may depend on how many rows the launch has (the same launch gives the same bits every time); forced

@@ -30,8 +30,8 @@
 //    Fed by this library's own quantizer or requantizing epilogues (act_blocked = 2) the activations arrive as fp6 codes
 //    sign | magnitude in the loop's lane order and go into the matrix instruction as loaded: fp6 x fp6 (half the matrix
 //    time per group), no unpack, no offset, one instantiation for signed and unsigned activations; their scales can come
-//    in the loop's order too (ascales_blocked: one 16-byte load per lane every four stages).  Such launches with more 128-row tiles than
-//    CUs are gemm_w4a4_wide.hip's, and those of few rows gemm_w4a4_split.hip's; the ones between run here with two workgroups to a CU.
+//    in the loop's order too (ascales_blocked: one 16-byte load per lane every four stages).  Such launches that have a 256-row tile for
+//    every CU and a K that is long for their epilogue are gemm_w4a4_wide.hip's, and those of few rows gemm_w4a4_split.hip's.
 //    Long launches whose activations arrive as nibbles turn them into such codes first (act_to_f6_kernel, act_scratch_bytes).
 //  * gemm_w4a4_i8_kernel (packed weights): a 16-byte LDS read holds 32 nibbles; the even and the odd nibbles are split
 //    into two int8 planes with shift/mask only (signed values land in the high nibble of each byte, i.e. times 16;
@@ -791,13 +791,13 @@ static void launch_gemm_i8(const svdq_gemm_args &a, hipStream_t s) {
     }
 }
 
-// Workgroups per CU for the fp8 kernel (with blocked activation scales gemm_w4a4_wide.hip serves full CUs).  Three (PIPE = false) keep a full CU about 8 % busier than two (PIPE = true), but a
-// workgroup of the two-per-CU kernel runs faster, which decides when the last round of tiles leaves most CUs with one or
+// Workgroups per CU for the fp8 kernel (with blocked activation scales most launches that fill the CUs are gemm_w4a4_wide.hip's:
+// wide_takes).  Three (PIPE = false) keep a full CU about 8 % busier than two (PIPE = true), but a workgroup of the two-per-CU kernel runs faster, which decides when the last round of tiles leaves most CUs with one or
 // two workgroups.  Cost model, in units of a tile's share of a fully loaded three-per-CU CU: whole rounds cost 3 (three per
 // CU) or 2 * 1.08 (two per CU); a last round whose fullest CU holds k tiles costs 1.75 / 2.15 / 3 (k = 1 / 2 / 3) or
 // 1.4 / 2 (k = 1 / 2).  The constants are measured (K = 3072, N = 9216: M = 512 -> 288 tiles, M = 1024 -> 576, M = 4608 -> 2592;
-// K = 12288, N = 3072, M = 4608 -> 864), and the model picks as the measurements do: 2592, 3456, 4608 and 576 tiles -> three per
-// CU; 864 and 288 tiles -> two.
+// K = 12288, N = 3072, M = 4608 -> 864), measured on nibbles and codes with scales in the matrix), and the model
+// picks as the measurements do: 2592, 3456, 4608 and 576 tiles -> three per CU; 864 and 288 tiles -> two.
 static std::atomic<int> g_f8_variant{-1};  // svdq_gemm_w4a4_set_variant
 static bool two_workgroups_per_cu(long tiles) {
     const int forced = g_f8_variant.load(std::memory_order_relaxed);
@@ -848,8 +848,10 @@ static void launch_gemm_f8(const svdq_gemm_args &a, hipStream_t s) {
             const int forced = g_f8_variant.load(std::memory_order_relaxed);
             if (wide_runs(a) && (forced == 0 || (forced < 0 && wide_takes(a, cu_count()))))
                 launch_gemm_wide(a, cu_count(), s);
-            else
+            else if (two)
                 launch_gemm_f8p<T, true, true, true, true>(a, s);
+            else
+                launch_gemm_f8p<T, true, false, true, true>(a, s);
         } else if (two) {
             launch_gemm_f8p<T, true, true, true>(a, s);
         } else {

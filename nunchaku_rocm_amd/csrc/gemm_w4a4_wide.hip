@@ -20,7 +20,7 @@
 //    without block scales (codes count as code / 8, so the sums are 1/64 of the result: an exact factor, put back at the end).
 //  * LDS objects are split so that nothing is read from one that a load in flight writes to: the compiler waits for every
 //    load before such a read (the scales of even and odd pairs of stages, with one object: 162 against 158 us at K = 12288).
-//  * Tiles of 128 rows (32 to a wavefront, same code) fill the last round: see the rule at wide_split.
+//  * Tiles of 128 rows (32 to a wavefront, same code) fill the last round: see the rule at wide_whole.
 #include <algorithm>
 #include <type_traits>
 
@@ -45,8 +45,8 @@ struct WideLds {  // the kernel's LDS objects
 // 27 us for one tile of K = 3072, then 21 more for each (288 tiles of 256 rows on 256 CUs 43 us, 504 49, 576 68).  Where the
 // last round has tiles for half of the CUs at most, halves take that round from 21 us to 11 (1152 tiles 111.5 / 105.6, 1296 131.9
 // / 121.7, 576 67.7 / 58.6); for more than half of them some CU has two halves and both are slower than a whole (432 tiles,
-// K = 12288: 184 with halves, 156 without).  With less than one tile to a CU all run as halves: nobody shares then
-// (216 tiles 28.1 / 25.9).
+// K = 12288: 184 with halves, 156 without).  An XCD with less than one tile to a CU (launches that the rule at wide_takes leaves to
+// the 128-row kernels, unless set_variant forces them here) has 128-row tiles only: 216 tiles 28.1 / 25.9.
 __host__ __device__ inline int wide_whole(int tiles, int cus_per_xcd) {
     const int whole = tiles / cus_per_xcd * cus_per_xcd;
     return whole == 0 || 2 * (tiles - whole) <= cus_per_xcd ? whole : tiles;
@@ -296,10 +296,27 @@ bool wide_runs(const svdq_gemm_args &a) {  // (offsets of a wavefront's two row 
     return a.act_blocked == 2 && a.ascales_blocked && (uint64_t)(a.K / GROUP) * 3072 < (1ull << 32);
 }
 
-// 64 rows to a wavefront pay from the first CU on that has more than one 128-row tile; below, the 128-row kernel's lone
-// workgroup is as fast or faster (K = 3072, 3072 columns: 240 tiles 20.3 here, 19.4 there; 504 tiles 30.9 / 37.2).
+// Tiles of 256 rows pay where there is one for every CU (below, every tile runs as two of 128 rows, and the kernel built for those is
+// the faster one) and where K is long for the epilogue: the loop gains 10 to 20 % of its time, but a wavefront takes its two row blocks
+// through the epilogue one after the other, with two workgroups on a CU where the 128-row kernel has three to hide it.  Between two
+// and three rounds of tiles (the 128-row kernel: about one and a half to two of its own) K has to be longer.  us, here / the faster
+// 128-row build (bf16):
+//   plain, rank 32, 3072 columns: K = 3072, 2560 rows (240 tiles) 29.4 / 28.7, 2688 (264) 34.0 / 39.0;  K = 12288 97.6 / 95.4 and
+//     110.8 / 132.9;  9216 columns, 2200 rows (648 tiles): K = 512 21.7 / 20.0, K = 1024 30.2 / 30.3;  3072 x 4608, K = 512 14.0 / 15.5
+//   Q/K norm + RoPE, 4608 columns: 3072 rows (432 tiles), K = 1024 rank 32 23.2 / 24.9, 128 37.5 / 38.7;  8192 rows, K = 512
+//     36.8 / 35.0;  4608 rows (648 tiles): rank 32 K = 1024 35.1 / 34.1, K = 1536 44.6 / 44.8, rank 128 K = 1536 64.2 / 63.2, K = 2048 73.2 / 73.5
+//   GELU, 6144 columns, 3072 rows: rank 32 K = 2048 60.4 / 59.4, K = 3072 75.8 / 76.6;  rank 128 K = 3072 121.5 / 117.2, K = 4608 144.3 / 143.2
+//   SwiGLU, 4096 columns, 4608 rows: rank 32 K = 1024 40.2 / 39.7, K = 2048 55.7 / 56.4;  rank 128 K = 1536 90.4 / 88.7, K = 2048 97.1 / 96.9
 bool wide_takes(const svdq_gemm_args &a, int cus) {
-    return (long)((wide_rows(a) + BM - 1) / BM) * ((a.N + BN - 1) / BN) > cus;
+    const long tiles = (long)((wide_rows(a) + WBM - 1) / WBM) * ((a.N + BN - 1) / BN);
+    if (tiles < cus) return false;
+    const bool between = tiles > 2L * cus && tiles < 3L * cus;
+    switch (a.epilogue) {
+        case SVDQ_EPI_QK_NORM_ROPE: return a.K >= 1024 + (between ? 8 * a.R : 0);
+        case SVDQ_EPI_GELU_QUANT: return a.K >= 1900 + 18 * a.R2;
+        case SVDQ_EPI_SWIGLU_QUANT: return a.K >= 1024 + 8 * a.R2;
+        default: return a.K >= 1024 || !between;
+    }
 }
 
 void launch_gemm_wide(const svdq_gemm_args &a, int cus, hipStream_t s) {

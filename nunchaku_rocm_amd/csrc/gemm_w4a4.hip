@@ -982,14 +982,19 @@ extern "C" int svdq_gemm_w4a4_split_wavefronts(const svdq_gemm_args *args, int32
     return args && args->K > 0 && args->N > 0 ? split_of(*args, cus > 0 ? cus : cu_count()) : 0;
 }
 
-// Bytes of the re-laid-out activations, where the launch gains by them.  The pass over the activations costs 3 us with its gap,
-// 9 us at 4608 x 3072; the fp6 x fp6 loops take 0.75 of the time of the nibble-fed one where tiles fill the CUs, and less than half where
-// few rows of signed codes otherwise run as 128-row tiles.  us as they are / re-laid-out (bf16, signed, rank 32):
-//   few rows (K split over wavefronts), eight of them: K = 1024, 256 x 3072 10.8 / 9.8;  K = 3072 22.4 / 14.1;  K = 512 7.9 / 8.8;
-//     four: K = 2048, 256 x 6144 16.8 / 15.7;  K = 3072, 512 x 3072 22.5 / 20.0;  K = 1024, 512 x 3072 10.9 / 12.2
-//   more than two 128-row tiles to a CU: K = 2048, 1536 x 6144 33.2 / 29.0;  K = 3072, 4608 x 9216 168 / 132;  K = 1536, 8192 x 1536
-//     29.6 / 31.7;  fewer: K = 3072, 1536 x 3072 32.1 / 31.4, 1024 x 3072 22.7 / 24.5, 2048 x 3072 32.3 / 32.7
-//   K = 6144, any rows: 768 x 3072 41.7 / 40.1, 1536 x 3072 58.0 / 51.3, 4608 x 3072 117 / 93;  K = 4096, 1024 x 4096 30.1 / 30.0
+// Bytes of the re-laid-out activations, where the launch gains by them.  The pass over the activations costs 3 us with its gap and about
+// 0.4 us for a million values, as much for a narrow output as for a wide one; the fp6 x fp6 loops take 0.75 of the time of the nibble-fed
+// one where tiles fill the CUs, and less than half where few rows of signed codes otherwise run as 128-row tiles, one after the other along K.
+// us as they are / re-laid-out (bf16, signed, rank 32):
+//   few rows (K split over wavefronts), eight of them: as long as there are fewer rows than K: 256 x 3072 K = 1024 10.8 / 9.8, K = 3072 22.4 /
+//     14.1, K = 512 7.9 / 8.8;  K = 1024, 1024 columns, 512 rows 11.3 / 10.6, 1024 rows 11.4 / 11.5;  K = 2048, 256 columns, 3072 rows 17.5 / 18.1
+//   four: up to K / 4 rows: K = 2048, 256 x 6144 16.8 / 15.7, 1024 x 1536 17.1 / 18.1;  K = 3072, 512 x 3072 22.5 / 20.0, 1344 x 1536 23.1 /
+//     23.8;  from K = 4096 up to 2 K / 3: K = 4608, 1344 x 1536 32.9 / 28.8, 8192 x 256 1.06 of the time
+//   more than two 128-row tiles to a CU: K = 2048, 1536 x 6144 33.2 / 29.0, 8192 x 1536 37.2 / 38.7;  K = 3072, 4608 x 9216 168 / 132, 8192 x 1536
+//     52.7 / 48.5, 16384 x 1024 0.92, 32768 x 512 1.04;  K = 1536, 8192 x 1536 29.6 / 31.7;  fewer: K = 3072, 1536 x 3072 32.1 / 31.4, 1024 x 3072
+//     22.7 / 24.5
+//   K = 6144: 768 x 3072 41.7 / 40.1, 4608 x 3072 117 / 93, 3072 x 1536 (288 tiles) 59.0 / 55.1, 2048 x 1536 (192) 42.4 / 43.8;  K = 12288, 2048 x
+//     1536 78.2 / 73.4
 // Unsigned activations of few rows split their K as they are (split_of); beyond those 1536 x 9216 at K = 3072 58.4 / 51.2.  (The
 // grid of the pass is two-dimensional: 2^20 rows keep it inside 65536.)
 static size_t act_scratch_bytes(const svdq_gemm_args &a, int cus) {
@@ -999,9 +1004,15 @@ static size_t act_scratch_bytes(const svdq_gemm_args &a, int cus) {
     svdq_gemm_args b = a;
     b.act_blocked = 2, b.ascales_blocked = 1;
     const bool quant = a.epilogue == SVDQ_EPI_GELU_QUANT || a.epilogue == SVDQ_EPI_SWIGLU_QUANT;
-    const long rows = quant ? a.M : a.actual_m, tiles = ((rows + BM - 1) / BM) * ((a.N + BN - 1) / BN);
-    const int split = split_wavefronts(b, cus);
-    if (!(a.K >= 6144 || (split == 8 && a.K >= 1024) || (split == 4 && a.K >= 2048) || (!split && tiles > 2L * cus && a.K >= 2048))) return 0;
+    const long rows = quant ? a.M : a.actual_m, tiles = ((rows + BM - 1) / BM) * ((a.N + BN - 1) / BN), K = a.K, N = a.N;
+    bool pays;
+    switch (split_wavefronts(b, cus)) {
+        case 8: pays = K >= 1024 && rows < K; break;
+        case 4: pays = K >= 2048 && (K >= 4096 ? 3 * rows <= 2 * K : 4 * rows <= K); break;
+        default:
+            pays = N >= 1024 && ((tiles > 2L * cus && K >= (N >= 2048 ? 2048 : 3072)) || (K >= 6144 && (tiles > cus || K * N >= 1 << 24)));
+    }
+    if (!pays) return 0;
     const size_t padded = (size_t)((a.M + 31) / 32 * 32);
     return padded * (size_t)(a.K / 4 * 3) + padded * (size_t)(a.K / GROUP) * 2;
 }

@@ -103,6 +103,23 @@ def test_when_statistics_have_a_launch_of_their_own(lib):
     assert lib.svdq_quantize_stats_first(None) == 0
 
 
+def test_when_nibbles_are_relaid_out(lib):
+    """256 CUs, signed codes: where the pass over the activations costs less than it saves.  Narrow outputs of very many rows, short K
+    and few tiles are read as they are."""
+    from nunchaku_rocm_amd import _lib
+
+    for rows, n, k, want in (
+        (256, 3072, 1024, 1), (256, 3072, 512, 0), (512, 1024, 1024, 1), (1024, 1024, 1024, 0), (2048, 512, 2048, 0), (3072, 256, 2048, 0), (8192, 128, 3072, 0),
+        (256, 6144, 2048, 1), (1024, 1536, 2048, 0), (512, 3072, 3072, 1), (1344, 1536, 3072, 0), (1344, 1536, 4608, 1), (8192, 256, 4608, 0), (16384, 128, 12288, 0),
+        (1536, 6144, 2048, 1), (8192, 1536, 2048, 0), (8192, 1536, 3072, 1), (32768, 512, 12288, 0), (1536, 3072, 3072, 0), (4608, 9216, 3072, 1),
+        (2048, 1536, 6144, 0), (3072, 1536, 6144, 1), (768, 3072, 6144, 1), (2048, 1536, 12288, 1), (1 << 20, 3072, 3072, 1), ((1 << 20) + 1, 3072, 3072, 0),
+    ):  # fmt: skip
+        nbytes = lib.svdq_gemm_w4a4_act_scratch_bytes(_lib.GemmArgs(wgt_planes=16, M=rows, actual_m=rows, N=n, K=k, R=32))
+        padded = -(-rows // 32) * 32
+        assert nbytes == (padded * (k // 4 * 3 + k // 64 * 2) if want else 0), (rows, n, k)
+    assert lib.svdq_gemm_w4a4_act_scratch_bytes(None) == 0
+
+
 def test_ops_refuse_cpu_tensors_loudly():
     from nunchaku_rocm_amd import ops
 

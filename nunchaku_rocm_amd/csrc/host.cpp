@@ -112,13 +112,14 @@ PyObject *quantize_buffers(PyObject *, PyObject *const *a, Py_ssize_t n) {
 }
 
 // quantize(args, input, output, oscales, lora_down, lora_down_t, lora_act_out, smooth, stats, scale, shift, norm_eps, out_blocked):
-// no GLU or GELU, signed; norm with one scale and shift for all rows
+// no GLU or GELU, signed; norm_eps None: no norm, else one with one scale and shift for all rows
 PyObject *quantize(PyObject *, PyObject *const *a, Py_ssize_t n) {
     if (n != 13) return no();
     Reader r;
     Tensor x, out, sc, down, downt, la, smooth, stats, scale, shift;
     long blocked;
-    const double eps = PyFloat_Check(a[11]) ? PyFloat_AS_DOUBLE(a[11]) : -1.0;
+    const bool norm = a[11] != Py_None;
+    const double eps = !norm ? 0.0 : PyFloat_Check(a[11]) ? PyFloat_AS_DOUBLE(a[11]) : -1.0;
     if (!r.get(a[1], x) || !r.get(a[2], out) || !r.get(a[3], sc) || !r.get(a[4], down, true) || !r.get(a[5], downt, true) || !r.get(a[6], la, true) ||
         !r.get(a[7], smooth, true) || !r.get(a[8], stats, true) || !r.get(a[9], scale, true) || !r.get(a[10], shift, true) || !r.done() ||
         !flag(a[12], blocked) || blocked < 0 || blocked > 3 || eps < 0.0)
@@ -140,7 +141,7 @@ PyObject *quantize(PyObject *, PyObject *const *a, Py_ssize_t n) {
     }
     if (smooth.defined() && (smooth.scalar_type() != T || !smooth.is_contiguous() || smooth.numel() != K)) return no();
     int64_t stride = 1, batch = 0;
-    if (scale.defined() || shift.defined()) {
+    if (norm) {
         if (!scale.defined() || !shift.defined() || scale.scalar_type() != T || shift.scalar_type() != T || scale.dim() < 1 || scale.dim() > 2 ||
             scale.dim() != shift.dim() || scale.numel() != K || shift.numel() != K || scale.size(-1) != K || shift.size(-1) != K)
             return no();
@@ -149,7 +150,7 @@ PyObject *quantize(PyObject *, PyObject *const *a, Py_ssize_t n) {
         if (scale.strides() != shift.strides() || stride < 1 || !fits(stride) || !fits(batch) || (stats.defined() ? stats.scalar_type() != at::kFloat || stats.dim() != 2 || stats.size(0) != M ||
                                                                                                  stats.size(1) != 2 || !stats.is_contiguous() : !(eps > 0.0)))
             return no();
-    } else if (stats.defined()) {
+    } else if (scale.defined() || shift.defined() || stats.defined()) {
         return no();
     }
     Block<svdq_quantize_args> b(a[0]);
@@ -170,7 +171,7 @@ PyObject *quantize(PyObject *, PyObject *const *a, Py_ssize_t n) {
     q.norm_scale = ptr(scale), q.norm_shift = ptr(shift);
     q.norm_ld = (int32_t)batch, q.norm_stride = (int32_t)stride;
     q.out_blocked = blocked >= 2 ? 2 : (int32_t)blocked, q.scales_blocked = blocked == 3;
-    q.norm_eps = scale.defined() && !stats.defined() ? (float)eps : 0.0f;
+    q.norm_eps = norm && !stats.defined() ? (float)eps : 0.0f;
     Py_RETURN_TRUE;
 }
 

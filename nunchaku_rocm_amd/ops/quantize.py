@@ -102,10 +102,10 @@ def quantize_w4a4_act_fuse_lora(
         # the ordinary call, checked in native code; anything else is left to what follows
         down = (None, None) if lora_down is None else _prep.made_lora_down(lora_down)
         if down is not None:
-            scale, shift, stats = (None, None, None) if norm is None else (norm[0], norm[1], norm[2] if len(norm) > 2 else None)
+            scale, shift, stats, eps = (None,) * 4 if norm is None else (norm[0], norm[1], norm[2] if len(norm) > 2 else None, norm_eps)
             args = _lib.QuantizeArgs()
             if _lib.host().quantize(args, input, output, oscales, lora_down, down[0], lora_act_out, smooth, stats, scale, shift,
-                                    norm_eps, int(out_blocked)):  # fmt: skip
+                                    eps, int(out_blocked)):  # fmt: skip
                 own = _stats_first(args, input.device)  # noqa: F841 (kept until the launch)
                 _lib.check(_lib.load().svdq_quantize_act(args, _lib.stream_of(input)))
                 return output, oscales, lora_act_out

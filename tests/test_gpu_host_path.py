@@ -174,6 +174,19 @@ def test_attention_blocks(dev, calls, B, H, q, kv, d, dtype):
     assert outs[0].shape == outs[1].shape and outs[0].stride() == outs[1].stride() and torch.equal(outs[0], outs[1])
 
 
+def test_norm_without_scale_or_shift(dev):
+    """A norm whose scale and shift are missing is refused, not quantized without the norm."""
+    from nunchaku_rocm_amd import ops
+
+    x = torch.randn(16, 512, device=dev).to(torch.bfloat16)
+    v = torch.ones(512, device=dev, dtype=x.dtype)
+    buf = (torch.zeros(16, 256, dtype=torch.uint8, device=dev), torch.zeros(8, 16, dtype=x.dtype, device=dev))
+    ops.quantize_w4a4_act_fuse_lora(x, *buf, norm=(v, v))
+    for norm in ((None, None), (None, None, None), (v, None), (None, v), (None, None, ops.layer_norm_stats(x))):
+        with pytest.raises((AttributeError, TypeError)):
+            ops.quantize_w4a4_act_fuse_lora(x, *buf, norm=norm)
+
+
 def test_what_is_left_to_python(dev):
     """Not the ordinary case: declined, and the block is not touched."""
     from nunchaku_rocm_amd import _lib

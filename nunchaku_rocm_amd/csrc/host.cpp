@@ -119,10 +119,10 @@ PyObject *quantize(PyObject *, PyObject *const *a, Py_ssize_t n) {
     Tensor x, out, sc, down, downt, la, smooth, stats, scale, shift;
     long blocked;
     const bool norm = a[11] != Py_None;
-    const double eps = !norm ? 0.0 : PyFloat_Check(a[11]) ? PyFloat_AS_DOUBLE(a[11]) : -1.0;
+    const float eps = !norm ? 0.0f : PyFloat_Check(a[11]) ? (float)PyFloat_AS_DOUBLE(a[11]) : -1.0f;  // (as the block holds it)
     if (!r.get(a[1], x) || !r.get(a[2], out) || !r.get(a[3], sc) || !r.get(a[4], down, true) || !r.get(a[5], downt, true) || !r.get(a[6], la, true) ||
         !r.get(a[7], smooth, true) || !r.get(a[8], stats, true) || !r.get(a[9], scale, true) || !r.get(a[10], shift, true) || !r.done() ||
-        !flag(a[12], blocked) || blocked < 0 || blocked > 3 || eps < 0.0)
+        !flag(a[12], blocked) || blocked < 0 || blocked > 3 || eps < 0.0f)
         return no();
     if (x.dim() != 2 || !is16(x.scalar_type()) || x.stride(1) != 1 || x.stride(0) % 8 || !al(x, 16)) return no();
     const auto T = x.scalar_type();
@@ -148,7 +148,7 @@ PyObject *quantize(PyObject *, PyObject *const *a, Py_ssize_t n) {
         stride = scale.stride(-1);
         batch = scale.dim() == 2 ? scale.stride(0) : K * stride;  // (one batch: not looked at)
         if (scale.strides() != shift.strides() || stride < 1 || !fits(stride) || !fits(batch) || (stats.defined() ? stats.scalar_type() != at::kFloat || stats.dim() != 2 || stats.size(0) != M ||
-                                                                                                 stats.size(1) != 2 || !stats.is_contiguous() : !(eps > 0.0)))
+                                                                                                 stats.size(1) != 2 || !stats.is_contiguous() : !(eps > 0.0f)))
             return no();
     } else if (scale.defined() || shift.defined() || stats.defined()) {
         return no();
@@ -171,7 +171,7 @@ PyObject *quantize(PyObject *, PyObject *const *a, Py_ssize_t n) {
     q.norm_scale = ptr(scale), q.norm_shift = ptr(shift);
     q.norm_ld = (int32_t)batch, q.norm_stride = (int32_t)stride;
     q.out_blocked = blocked >= 2 ? 2 : (int32_t)blocked, q.scales_blocked = blocked == 3;
-    q.norm_eps = norm && !stats.defined() ? (float)eps : 0.0f;
+    q.norm_eps = norm && !stats.defined() ? eps : 0.0f;
     Py_RETURN_TRUE;
 }
 

@@ -797,6 +797,10 @@ extern "C" int svdq_quantize_act(const svdq_quantize_args *args, void *stream) {
         set_error("svdq_quantize_act: dtype %d", a.dtype);
         return SVDQ_E_INVALID;
     }
+    if (!(a.norm_eps >= 0.0f)) {
+        set_error("svdq_quantize_act: norm_eps=%g is neither positive nor 0 (off)", (double)a.norm_eps);
+        return SVDQ_E_INVALID;
+    }
     if (has_norm(a)) {
         if (a.prologue != SVDQ_PRE_NONE) {
             set_error("svdq_quantize_act: the norm prologue cannot be combined with the GLU / GELU prologue");

@@ -2,6 +2,8 @@
 
 from __future__ import annotations
 
+import ctypes
+
 import torch
 
 from .. import _lib
@@ -30,11 +32,12 @@ def layer_norm_stats(input: torch.Tensor, eps: float = 1e-6) -> torch.Tensor:
 
 def _norm_args(norm, inp: torch.Tensor, M: int, K: int, eps: float):
     """``norm = (scale, shift[, stats])`` -> (stats, scale, shift, rows_per_batch, ld, stride) for the C call; no stats: the
-    quantizer computes them itself or :func:`_stats_first` does (except for an ``eps`` of 0, which the C call reads as none).  scale and shift are used
+    quantizer computes them itself or :func:`_stats_first` does (except for an ``eps`` of 0 in
+    32 bits, which the C call reads as none).  scale and shift are used
     where they lie when they share their strides (as the slices of one adaLN projection do)."""
     scale, shift = norm[0], norm[1]
     stats = norm[2] if len(norm) > 2 else None
-    if stats is None and not eps > 0:
+    if stats is None and not ctypes.c_float(eps).value > 0:
         stats = layer_norm_stats(inp, eps)
     if scale.dim() == 1:
         scale, shift = scale[None], shift[None]

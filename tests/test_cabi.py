@@ -62,6 +62,9 @@ def test_invalid_arguments_are_rejected_without_launch(lib):
     q = _lib.QuantizeArgs(x=16, out=16, scales=16, M=4, K=100, ld_x=100, ld_out=50, ld_scales=4)
     assert lib.svdq_quantize_act(q, None) == _lib.E_INVALID
     assert b"multiple of 64" in lib.svdq_last_error()
+    for eps in (-1e-6, float("nan")):
+        q = _lib.QuantizeArgs(x=16, out=16, scales=16, M=4, K=64, ld_x=64, ld_out=32, ld_scales=4, norm_scale=16, norm_shift=16, norm_stride=1, norm_eps=eps)
+        assert lib.svdq_quantize_act(q, None) == _lib.E_INVALID and b"norm_eps" in lib.svdq_last_error()
     with pytest.raises(ValueError):
         _lib.check(_lib.E_INVALID)
     g = _lib.GemmArgs(act=16, wgt=16, ascales=16, wscales=16, out=16, M=8, N=8, K=96, ld_act=48, ld_wgt=48)

@@ -215,6 +215,23 @@ def test_statistics_inside_the_quantizer(dev, M, K, R, dtype):
         assert torch.equal(own[2][:M], given[2][:M])
 
 
+@pytest.mark.parametrize("eps", [1e-50, 1e-46, 1e-44])
+def test_norm_with_an_eps_that_32_bits_lose(dev, eps):
+    """The norm is applied, with the eps that 32 bits hold, by native and Python checks alike."""
+    from nunchaku_rocm_amd import ops
+
+    x = (torch.randn(33, 512, device=dev) * 3 + 1).to(torch.bfloat16)
+    scale, shift = torch.rand(512, device=dev).to(x.dtype) + 0.5, torch.rand(512, device=dev).to(x.dtype)
+    want = ops.quantize_w4a4_act_fuse_lora(x, norm=(scale, shift, ops.layer_norm_stats(x, eps)))
+    out = [ops.quantize_w4a4_act_fuse_lora(x, norm=(scale, shift), norm_eps=eps)]
+    buf = torch.zeros_like(want[0]), torch.zeros_like(want[1])
+    out.append(ops.quantize_w4a4_act_fuse_lora(x, *buf, norm=(scale, shift), norm_eps=eps))
+    plain = ops.quantize_w4a4_act_fuse_lora(x)
+    torch.cuda.synchronize()
+    for q, s, _ in out:
+        assert torch.equal(q, want[0]) and torch.equal(s, want[1]) and not torch.equal(q, plain[0])
+
+
 @pytest.mark.parametrize("M,K,R,launches", [(4096, 128, 64, 1), (4097, 128, 64, 2), (17, 4096, 32, 1), (17, 4160, 32, 2), (512, 192, 256, 1), (530, 192, 256, 2)])
 def test_statistics_in_a_launch_of_their_own(dev, monkeypatch, M, K, R, launches):
     """Where a statistics launch in front is the faster way it is made, by native and Python checks alike; the bits are the same."""

@@ -69,6 +69,16 @@ bool flag(PyObject *o, long &v) { v = PyLong_Check(o) ? PyLong_AsLong(o) : -1; r
 // an allocation goes through torch.empty's Python surface when somebody listens there
 bool listened() { return at::impl::PythonTorchFunctionTLS::stack_len() > 0; }
 
+// An allocation may wait for the device, and with somebody else's allocator for another Python thread: not under the interpreter's lock.
+struct Unlocked {
+    PyThreadState *state = PyEval_SaveThread();
+    ~Unlocked() { PyEval_RestoreThread(state); }
+};
+Tensor empty(at::IntArrayRef size, const at::Device &device, at::ScalarType type) {
+    const Unlocked unlocked;
+    return at::empty(size, at::TensorOptions().device(device).dtype(type));
+}
+
 // same_source((version, storage, place, shape, stride), tensor): _prep._same_source; None where it cannot tell
 PyObject *same_source(PyObject *, PyObject *const *a, Py_ssize_t n) {
     if (n != 2 || !PyTuple_Check(a[0]) || PyTuple_GET_SIZE(a[0]) != 5 || !THPStorage_Check(PyTuple_GET_ITEM(a[0], 1))) Py_RETURN_NONE;
@@ -100,9 +110,8 @@ PyObject *quantize_buffers(PyObject *, PyObject *const *a, Py_ssize_t n) {
         rank < 0 || x.size(1) % 64)
         return no();
     const int64_t rows = (x.size(0) + pad - 1) / pad * pad, k = x.size(1);
-    const auto opt = at::TensorOptions().device(x.device());
-    const Tensor q = at::empty({rows, blocked >= 2 ? k * 3 / 4 : k / 2}, opt.dtype(at::kByte)), s = at::empty({k / 64, rows}, opt.dtype(x.scalar_type())),
-                 l = at::empty({rows, rank}, opt.dtype(at::kFloat));
+    const Tensor q = empty({rows, blocked >= 2 ? k * 3 / 4 : k / 2}, x.device(), at::kByte), s = empty({k / 64, rows}, x.device(), x.scalar_type()),
+                 l = empty({rows, rank}, x.device(), at::kFloat);
     PyObject *out = PyTuple_New(3);
     if (!out) return nullptr;
     PyTuple_SET_ITEM(out, 0, THPVariable_Wrap(q));
@@ -256,7 +265,7 @@ PyObject *gemm(PyObject *, PyObject *const *a, Py_ssize_t n) {
     if (!R2) Py_RETURN_TRUE;
     g.lora_down_t = ptr(downt), g.lora_act_out = (float *)lo.data_ptr(), g.ld_lora_act_out = (int32_t)lo.stride(0);
     g.lora_down_blocked = ptr(downb);
-    const Tensor scratch = at::empty({(N + 127) / 128 * M * R2}, at::TensorOptions().device(act.device()).dtype(at::kFloat));
+    const Tensor scratch = empty({(N + 127) / 128 * M * R2}, act.device(), at::kFloat);
     g.scratch = (float *)scratch.data_ptr();
     return THPVariable_Wrap(scratch);
 }
@@ -281,7 +290,7 @@ PyObject *gemv(PyObject *, PyObject *const *a, Py_ssize_t n) {
         return no();
     Block<svdq_awq_gemv_args> b(a[0]);
     if (!b.ok) return no();
-    const Tensor out = at::empty({m, nn}, at::TensorOptions().device(x.device()).dtype(T));
+    const Tensor out = empty({m, nn}, x.device(), T);
     *b = svdq_awq_gemv_args{ptr(x), (const int32_t *)ptr(w), ptr(s), ptr(z), out.data_ptr(), (int32_t)m, (int32_t)nn, (int32_t)k, (int32_t)x.stride(0),
                             (int32_t)s.stride(0), (int32_t)nn, code(T)};
     PyObject *res = PyTuple_New(2);
@@ -310,7 +319,7 @@ PyObject *attention(PyObject *, PyObject *const *a, Py_ssize_t n) {
     }
     Block<svdq_attention_args> b(a[0]);
     if (!b.ok) return no();
-    const Tensor out = at::empty({B, Tq, H * D}, at::TensorOptions().device(q.device()).dtype(q.scalar_type()));
+    const Tensor out = empty({B, Tq, H * D}, q.device(), q.scalar_type());
     svdq_attention_args &g = *b;
     g = svdq_attention_args{};
     g.q = ptr(q), g.k = ptr(k), g.v = ptr(v), g.o = out.data_ptr();

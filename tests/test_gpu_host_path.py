@@ -187,6 +187,34 @@ def test_norm_without_scale_or_shift(dev):
             ops.quantize_w4a4_act_fuse_lora(x, *buf, norm=norm)
 
 
+def test_allocations_let_other_threads_run(dev):
+    """While the native code allocates, another Python thread gets the interpreter's lock, as inside torch.empty.  (The lock changes hands
+    only where it is let go of: no switches by time here.)"""
+    import sys
+    import threading
+
+    from nunchaku_rocm_amd import _lib
+
+    host, gate, ran = _lib.host(), threading.Lock(), []
+    x = torch.zeros(16, 2048, device=dev, dtype=torch.bfloat16)
+    gate.acquire()
+    thread = threading.Thread(target=lambda: (gate.acquire(), ran.append(1)))
+    torch.cuda.empty_cache()  # the allocation asks the device for memory, which takes long enough for a thread to wake up
+    thread.start()
+    old = sys.getswitchinterval()
+    sys.setswitchinterval(60.0)
+    try:
+        gate.release()
+        buffers = host.quantize_buffers(x, 0, 1 << 23, 0)  # 8 GB of codes
+        during = list(ran)
+    finally:
+        sys.setswitchinterval(old)
+        thread.join()
+    assert buffers is not False and during == [1]
+    del buffers
+    torch.cuda.empty_cache()
+
+
 def test_what_is_left_to_python(dev):
     """Not the ordinary case: declined, and the block is not touched."""
     from nunchaku_rocm_amd import _lib

@@ -44,7 +44,8 @@ def host_command(out: str) -> list[str]:
     from torch.utils.cpp_extension import include_paths, library_paths
 
     flags = [f"-I{p}" for p in (*include_paths(), sysconfig.get_paths()["include"])] + [f"-L{p}" for p in library_paths()]
-    return [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+    compiler = os.environ.get("CXX") or shutil.which("g++") or os.path.join(os.path.dirname(os.path.realpath(hipcc())), "amdclang++")
+    return [compiler, f'-DSVDQ_TORCH_VERSION="{torch.__version__}"', "-O2", "-std=c++17", "-fPIC", "-shared", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
             *flags, os.path.join(CSRC, "host.cpp"), "-lc10", "-ltorch_cpu", "-ltorch_python", "-o", out]  # fmt: skip
 
 

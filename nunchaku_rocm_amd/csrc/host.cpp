@@ -11,6 +11,8 @@
 #include <Python.h>
 
 #include <cmath>
+#include <cstring>
+#include <string>
 
 #include <ATen/ATen.h>
 #include <ATen/PythonTorchFunctionTLS.h>
@@ -347,7 +349,18 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", nullptr, -1, methods, null
 
 }  // namespace
 
+// The tensors' layout and the interpreter's are those of the headers this was compiled with: under others it does not load.
 PyMODINIT_FUNC PyInit__host(void) {
+    const std::string python = std::to_string(PY_MAJOR_VERSION) + "." + std::to_string(PY_MINOR_VERSION) + ".";
+    if (std::strncmp(Py_GetVersion(), python.c_str(), python.size()) != 0)
+        return PyErr_Format(PyExc_ImportError, "built for Python %s, this is %s", PY_VERSION, Py_GetVersion());
+    PyObject *torch = PyImport_ImportModule("torch"), *version = torch ? PyObject_GetAttrString(torch, "__version__") : nullptr;
+    Py_XDECREF(torch);
+    const char *text = version ? PyUnicode_AsUTF8(version) : nullptr;
+    const bool same = text && std::strcmp(text, SVDQ_TORCH_VERSION) == 0;
+    if (text && !same) PyErr_Format(PyExc_ImportError, "built for torch %s, this is %s", SVDQ_TORCH_VERSION, text);
+    Py_XDECREF(version);
+    if (!same) return nullptr;
     PyObject *m = PyModule_Create(&module);
     if (m) PyModule_AddIntConstant(m, "ABI_VERSION", SVDQ_ABI_VERSION);
     return m;

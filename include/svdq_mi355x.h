@@ -265,7 +265,9 @@ int svdq_split_weight_planes(const void *wgt, const void *wscales, void *planes,
                              int32_t ld_wscales, int32_t dtype, void *stream);
 size_t svdq_weight_planes_bytes(int32_t N, int32_t K);
 
-/* Bytes of `scratch` needed by a requantizing epilogue with LoRA-down (0 when R2 == 0). */
+/* Bytes of `scratch` needed by a requantizing epilogue with LoRA-down (0 when R2 == 0): one (M, R2) fp32 partial product for
+ * every SVDQ_LORA_PART_COLS columns. */
+#define SVDQ_LORA_PART_COLS 128
 size_t svdq_gemm_w4a4_scratch_bytes(int32_t M, int32_t N, int32_t R2, int32_t epilogue);
 
 /*

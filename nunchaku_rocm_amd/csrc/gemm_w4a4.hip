@@ -1021,6 +1021,7 @@ extern "C" size_t svdq_gemm_w4a4_act_scratch_bytes(const svdq_gemm_args *args) {
 
 extern "C" size_t svdq_gemm_w4a4_scratch_bytes(int32_t M, int32_t N, int32_t R2, int32_t epilogue) {
     if (R2 <= 0 || (epilogue != SVDQ_EPI_GELU_QUANT && epilogue != SVDQ_EPI_SWIGLU_QUANT)) return 0;
+    static_assert(BN == SVDQ_LORA_PART_COLS, "callers size the scratch memory by the header");
     return (size_t)((N + BN - 1) / BN) * (size_t)M * (size_t)R2 * sizeof(float);
 }
 

@@ -267,7 +267,7 @@ PyObject *gemm(PyObject *, PyObject *const *a, Py_ssize_t n) {
     if (!R2) Py_RETURN_TRUE;
     g.lora_down_t = ptr(downt), g.lora_act_out = (float *)lo.data_ptr(), g.ld_lora_act_out = (int32_t)lo.stride(0);
     g.lora_down_blocked = ptr(downb);
-    const Tensor scratch = empty({(N + 127) / 128 * M * R2}, act.device(), at::kFloat);
+    const Tensor scratch = empty({(N + SVDQ_LORA_PART_COLS - 1) / SVDQ_LORA_PART_COLS * M * R2}, act.device(), at::kFloat);
     g.scratch = (float *)scratch.data_ptr();
     return THPVariable_Wrap(scratch);
 }

@@ -144,6 +144,35 @@ def test_gemm_blocks(dev, calls, epilogue, blocked, rank, bias, dtype):
     assert a == b and len(a) == 1 and taken == [True]
 
 
+@pytest.mark.parametrize("M,N,R2,swiglu", [(16, 128, 16, False), (160, 1024, 48, True), (272, 1152, 32, False)])
+def test_scratch_memory_is_what_the_library_asks_for(dev, monkeypatch, M, N, R2, swiglu):
+    from nunchaku_rocm_amd import _lib, ops
+    from nunchaku_rocm_amd.ops import gemm as G
+
+    k, nq, dtype = 128, N // 2 if swiglu else N, torch.bfloat16
+    byte = lambda *s: torch.zeros(*s, dtype=torch.uint8, device=dev)  # noqa: E731
+    val = lambda *s: torch.ones(*s, dtype=dtype, device=dev)  # noqa: E731
+    kw = dict(act=byte(M, k // 2), wgt=byte(N, k // 2), ascales=val(k // 64, M), wscales=val(k // 64, N), fuse_swiglu=swiglu, qout=byte(M, nq // 2),
+              oscales=val(nq // 64, M), lora_down=val(nq, R2), lora_act_out=torch.empty(M, R2, device=dev))  # fmt: skip
+    native, made = _lib.host(), []
+
+    class Host:
+        def __getattr__(self, name):
+            return getattr(native, name)
+
+        def gemm(self, *a):
+            made.append(native.gemm(*a))
+            return made[-1]
+
+    monkeypatch.setattr(_lib, "host", lambda: Host())
+    monkeypatch.setattr(G, "USE_WEIGHT_PLANES", "all")
+    for _ in range(3):
+        ops.svdq_gemm_w4a4_cuda(**kw)
+        torch.cuda.synchronize()
+    epilogue = _lib.EPI_SWIGLU_QUANT if swiglu else _lib.EPI_GELU_QUANT
+    assert made and made[-1].nbytes == _lib.load().svdq_gemm_w4a4_scratch_bytes(M, N, R2, epilogue)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("m,bias", [(1, True), (8, False), (32, True)])
 def test_gemv_blocks(dev, calls, m, bias, dtype):

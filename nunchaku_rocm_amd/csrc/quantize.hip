@@ -229,7 +229,8 @@ __global__ __launch_bounds__(Q_WAVES * 64, QR == 32 ? 1 : (NORM ? 4 : 2)) void q
 #pragma unroll
         for (int h = 0; h < NH; h++) {
             const int mr = min(m0 + Q_ROWS * h + ml, a.M - 1);
-            const float2 st = a.norm_stats ? *(const float2 *)(a.norm_stats + 2 * mr) : lds_st[Q_ROWS * h + ml];
+            // (given statistics are floats anywhere: not read as an 8-byte pair)
+            const float2 st = a.norm_stats ? make_float2(a.norm_stats[2 * mr], a.norm_stats[2 * mr + 1]) : lds_st[Q_ROWS * h + ml];
             n_mean[h] = st.x;
             n_rstd[h] = st.y;
         }
@@ -540,7 +541,7 @@ __global__ __launch_bounds__(256) void row_stats_kernel(const uint16_t *x, float
     const uint16_t *row[1] = {x + (long)m * ld_x};
     float2 st[1];
     row_moments<T, 1, 16>(row, K, eps, lane, st);
-    if (lane == 0) *(float2 *)(stats + 2 * m) = st[0];
+    if (lane == 0) stats[2 * m] = st[0].x, stats[2 * m + 1] = st[0].y;  // (4-byte aligned)
 }
 
 // one wavefront per row; the rounded results stay in registers (packed) for the statistics, so the row is read once

@@ -215,6 +215,23 @@ def test_statistics_inside_the_quantizer(dev, M, K, R, dtype):
         assert torch.equal(own[2][:M], given[2][:M])
 
 
+@pytest.mark.parametrize("M,K", [(1, 64), (33, 512), (17, 8256)])
+def test_statistics_at_any_float(dev, M, K):
+    """Row statistics are written and read where they lie: four bytes of alignment are enough."""
+    from nunchaku_rocm_amd import _lib, ops
+
+    x = (torch.randn(M, K, device=dev) * 3 + 1).to(torch.bfloat16)
+    scale, shift = torch.rand(K, device=dev).to(x.dtype) + 0.5, torch.rand(K, device=dev).to(x.dtype)
+    want = ops.layer_norm_stats(x)
+    buf = torch.full((2 * M + 2,), -7.0, device=dev)
+    stats = buf[1:-1].view(M, 2)
+    assert stats.data_ptr() % 8 == 4
+    _lib.check(_lib.load().svdq_row_stats(x.data_ptr(), stats.data_ptr(), M, K, K, _lib.dtype_code(x.dtype), 1e-6, _lib.stream_of(x)))
+    assert torch.equal(stats, want) and buf[0] == buf[-1] == -7.0
+    for a, b in zip(*(ops.quantize_w4a4_act_fuse_lora(x, norm=(scale, shift, s))[:2] for s in (stats, want))):
+        assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
+
+
 @pytest.mark.parametrize("eps", [1e-50, 1e-46, 1e-44])
 def test_norm_with_an_eps_that_32_bits_lose(dev, eps):
     """The norm is applied, with the eps that 32 bits hold, by native and Python checks alike."""

@@ -1084,10 +1084,6 @@ static int gemm_w4a4_checked(const svdq_gemm_args &a, void *stream) {
         set_error("svdq_gemm_w4a4: LoRA rows must be 16-byte aligned");
         return SVDQ_E_INVALID;
     }
-    if (a.R > 0 && a.ld_lora_up >= 1 << 26) {  // 32 rows are fetched with 32-bit offsets
-        set_error("svdq_gemm_w4a4: lora_up row stride %d is too large for 32-bit offsets", a.ld_lora_up);
-        return SVDQ_E_UNSUPPORTED;
-    }
     if (a.bias && ((uintptr_t)a.bias & 7)) {
         set_error("svdq_gemm_w4a4: bias must be 8-byte aligned");
         return SVDQ_E_INVALID;

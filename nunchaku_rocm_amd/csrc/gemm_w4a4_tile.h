@@ -96,6 +96,9 @@ __device__ inline void tile_ids(int tiles_m, int tiles_n, int &pid_m, int &pid_n
     pid_n = (id % band) / gm;
 }
 
+// Row strides of lora_up below this: the offsets of 32 of its rows fit 32 bits.
+constexpr int LORA_UP_LD32 = 1 << 26;
+
 // Epilogue operands every wavefront of the tile needs, fetched global -> LDS next to stage 0: the tile's 128 bias
 // values, the first 32 ranks of lora_up and (Q/K norm + RoPE epilogue, Q and K tiles) the head's 128 norm weights.
 // (Buffer loads: next to a global_load_lds in flight the compiler waits for every load before the first register load's
@@ -117,7 +120,17 @@ __device__ inline void fetch_epilogue_operands(const svdq_gemm_args &a, uint8_t 
             const int r0 = min(n0 + blk * 32, a.N - 1);         // the block's first row: its rows are 32-bit offsets from there
             const __amdgpu_buffer_rsrc_t r = g_buffer((const uint16_t *)a.lora_up + (size_t)r0 * a.ld_lora_up);
             const uint32_t row = (uint32_t)(min(n0 + blk * 32 + l32, a.N - 1) - r0);
-            if (16 * c < a.R) g_load16_lds(r, sepi + q * BLK_BYTES, row * 2u * (uint32_t)a.ld_lora_up + (uint32_t)(32 * c + 16 * half), 0);
+            if (16 * c >= a.R) continue;
+            if (a.ld_lora_up < LORA_UP_LD32) {
+                g_load16_lds(r, sepi + q * BLK_BYTES, row * 2u * (uint32_t)a.ld_lora_up + (uint32_t)(32 * c + 16 * half), 0);
+            } else {  // rows too far apart: one by one (a lane's 16 bytes land at its place whoever else is masked off; through registers
+                      // the fp8 loop's kernels spill up to three more)
+#pragma unroll 1
+                for (int i32 = 0; i32 < 32; i32++)
+                    if (l32 == i32)
+                        g_load16_lds(g_buffer((const uint16_t *)a.lora_up + (size_t)min(r0 + i32, a.N - 1) * a.ld_lora_up), sepi + q * BLK_BYTES,
+                                     (uint32_t)(32 * c + 16 * half), 0);
+            }
         }
     }
 }

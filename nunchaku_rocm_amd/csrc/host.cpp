@@ -220,7 +220,7 @@ PyObject *gemm(PyObject *, PyObject *const *a, Py_ssize_t n) {
     const int64_t R = la.defined() && up.defined() ? (up.dim() == 2 ? up.size(1) : -1) : 0;
     if (R < 0) return no();
     if (R && (la.dim() != 2 || la.scalar_type() != at::kFloat || up.scalar_type() != T || up.size(0) < N || la.size(0) < M || la.size(1) < R || la.stride(1) != 1 ||
-              up.stride(1) != 1 || !fits(la.stride(0)) || up.stride(0) >= 1 << 26))
+              up.stride(1) != 1 || !fits(la.stride(0)) || !fits(up.stride(0))))
         return no();
     if (ablk && (!act.is_contiguous() || M % 32 || !al(act, 16))) return no();
     if (ablk == 3 && (K % 512 || !as.is_contiguous() || as.size(0) != G || as.size(1) != M || !al(as, 16))) return no();

@@ -274,8 +274,6 @@ def svdq_gemm_w4a4_cuda(
     if out2d is not None and out2d.stride(1) != 1:
         raise ValueError("out not row-major")
 
-    if R and lora_up.stride(0) >= 1 << 26:  # the kernels fetch 32 of its rows with 32-bit offsets
-        lora_up = lora_up[:N].contiguous()
     planes = working_copy(wgt, wscales)
     if act_blocked:
         if planes is None:
@@ -313,7 +311,7 @@ def svdq_gemm_w4a4_cuda(
         act_blocked=min(act_blocked, ACT_CODES_F6),
         ascales_blocked=int(act_blocked == ACT_CODES_F6_SCALES),
     )
-    keep = [planes, lora_up]  # tensors that must outlive the launch call
+    keep = [planes]  # tensors that must outlive the launch call
     lib = _lib.load()
     if want_qk:
         rot_key = rotary_emb  # the caller's tensor: what the re-laid-out copy is cached under

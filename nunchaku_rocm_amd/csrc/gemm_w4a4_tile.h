@@ -121,7 +121,7 @@ __device__ inline void fetch_epilogue_operands(const svdq_gemm_args &a, uint8_t 
             const __amdgpu_buffer_rsrc_t r = g_buffer((const uint16_t *)a.lora_up + (size_t)r0 * a.ld_lora_up);
             const uint32_t row = (uint32_t)(min(n0 + blk * 32 + l32, a.N - 1) - r0);
             if (16 * c >= a.R) continue;
-            if (a.ld_lora_up < LORA_UP_LD32) {
+            if (__builtin_expect(a.ld_lora_up < LORA_UP_LD32, 1)) {
                 g_load16_lds(r, sepi + q * BLK_BYTES, row * 2u * (uint32_t)a.ld_lora_up + (uint32_t)(32 * c + 16 * half), 0);
             } else {  // rows too far apart: one by one (a lane's 16 bytes land at its place whoever else is masked off; through registers
                       // the fp8 loop's kernels spill up to three more)

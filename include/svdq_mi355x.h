@@ -201,8 +201,8 @@ int svdq_gemm_w4a4(const svdq_gemm_args *args, void *stream);
 
 /* How many bytes svdq_gemm_w4a4 wants behind args->act_scratch; 0 where it reads the activations as they are.  Not zero where
  * the launch is long enough that re-laying-out its activations first (one pass over them) and running the fp6 x fp6 loop is
- * the faster way.  Without the memory the launch runs all the same.  Host arithmetic on the sizes; no counterpart in the
- * reference. */
+ * the faster way.  Without the memory the launch runs all the same; unsigned codes then give the same bits, signed ones may
+ * differ in the last one (the nibble-fed loop takes them as a + 8 and a - 7 with 16-bit offset terms, and never splits their K).  Host arithmetic on the sizes; no counterpart in the reference. */
 size_t svdq_gemm_w4a4_act_scratch_bytes(const svdq_gemm_args *args);
 
 /*
@@ -233,9 +233,9 @@ size_t svdq_lora_down_blocked_bytes(int32_t N, int32_t R2);
  * software-pipelined steps (a workgroup on its own runs faster); svdq_gemm_w4a4 picks by the number of tiles and CUs, K and
  * the epilogue.  This overrides the choice for the whole process: -1 = by size (default), 0 = for full CUs, 1 = two per CU.
  * For tuning and tests; results of the two are bit-identical.  By default launches with few rows (unsigned activations or
- * fp6 codes) go to a third kernel that splits K over wavefronts and adds the groups up in another order, so the last bit of
- * a row's output may depend on how many rows the launch has (the same launch gives the same bits every time); forced
- * builds do not.  No counterpart in the reference. */
+ * fp6 codes) go to a third kernel that splits K over wavefronts and adds the groups up in another order, and signed nibbles with
+ * act_scratch run as fp6 codes where svdq_gemm_w4a4_act_scratch_bytes is not 0, so the last bit of a row's output may depend on how
+ * many rows the launch has (the same launch gives the same bits every time); forced builds do neither.  No counterpart in the reference. */
 int svdq_gemm_w4a4_set_variant(int32_t variant);
 /* Over how many wavefronts (8 or 4) svdq_gemm_w4a4 splits K for `args` on a device of `cus` compute units (0: this one's);
  * 0 = not split.  Host arithmetic on the sizes; for tests.  No counterpart in the reference. */
@@ -276,7 +276,7 @@ size_t svdq_gemm_w4a4_scratch_bytes(int32_t M, int32_t N, int32_t R2, int32_t ep
  * sums go to a buffer of SVDQ_STATIC_SCRATCH_BYTES built into the library (one per GPU, held until the process
  * ends).  Returns SVDQ_E_UNSUPPORTED when svdq_gemm_w4a4_scratch_bytes(M, N, R2, epilogue) exceeds it.  Calls no
  * hipMalloc / hipFree.  All calls on one GPU share the buffer: calls that overlap in time on one GPU (two streams) race;
- * calls on one stream are ordered.  Results are bit-identical to svdq_gemm_w4a4's.
+ * calls on one stream are ordered.  Results are bit-identical to svdq_gemm_w4a4's for the same `args` (act_scratch included).
  */
 #define SVDQ_STATIC_SCRATCH_BYTES (16u << 20)
 int svdq_gemm_w4a4_static_scratch(const svdq_gemm_args *args, void *stream);

@@ -46,7 +46,8 @@ ACT_CODES_F6_SCALES = 3
 # True sends the requantizing epilogues' LoRA-down partial sums to the buffer built into the library
 # (svdq_gemm_w4a4_static_scratch) instead of a torch allocation per call: for callers that may not allocate, e.g. while
 # a HIP graph is being captured.  The buffer holds 16 MiB (about M * N / 128 * R2 * 4 bytes are needed) and is shared
-# by every call on the GPU, so calls on two streams must not overlap.
+# by every call on the GPU, so calls on two streams must not overlap.  Activations that arrive as nibbles are then read as they are
+# whatever the launch's size (no allocation: svdq_gemm_args.act_scratch), which for signed ones may be another last bit.
 STATIC_SCRATCH = False
 
 
@@ -94,14 +95,12 @@ GELU_SHIFT = 0.171875
 
 
 def _act_scratch(args, device: torch.device) -> torch.Tensor | None:
-    """Memory in which a long launch re-lays-out activations that arrive as nibbles, where it wants some (set in ``args``)."""
+    """Memory in which a long launch re-lays-out activations that arrive as nibbles, where it wants some (set in ``args``).  Where there
+    is none the call fails: the launch would run without it, but with other last bits for signed codes."""
     nbytes = _lib.load().svdq_gemm_w4a4_act_scratch_bytes(args)
     if not nbytes:
         return None
-    try:
-        t = torch.empty(nbytes, dtype=torch.uint8, device=device)
-    except torch.OutOfMemoryError:  # the launch runs without it
-        return None
+    t = torch.empty(nbytes, dtype=torch.uint8, device=device)
     args.act_scratch = t.data_ptr()
     return t
 

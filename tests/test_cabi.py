@@ -123,6 +123,24 @@ def test_when_nibbles_are_relaid_out(lib):
     assert lib.svdq_gemm_w4a4_act_scratch_bytes(None) == 0
 
 
+def test_no_memory_for_relaid_out_nibbles_is_an_error(lib, monkeypatch):
+    """What a call computes does not depend on whether an allocation succeeds."""
+    from nunchaku_rocm_amd import _lib
+    from nunchaku_rocm_amd.ops import gemm as G
+
+    args = _lib.GemmArgs(wgt_planes=16, M=256, actual_m=256, N=3072, K=3072, R=32)
+    t = G._act_scratch(args, torch.device("cpu"))
+    assert t.nbytes == lib.svdq_gemm_w4a4_act_scratch_bytes(args) and args.act_scratch == t.data_ptr()
+
+    def none_left(*args, **kw):
+        raise torch.OutOfMemoryError("none left")
+
+    monkeypatch.setattr(torch, "empty", none_left)
+    with pytest.raises(torch.OutOfMemoryError):
+        G._act_scratch(args, torch.device("cpu"))
+    assert G._act_scratch(_lib.GemmArgs(wgt_planes=16, M=256, actual_m=256, N=3072, K=512, R=32), torch.device("cpu")) is None
+
+
 def test_ops_refuse_cpu_tensors_loudly():
     from nunchaku_rocm_amd import ops
 

@@ -668,7 +668,7 @@ static int quantize_grid_y(const svdq_quantize_args &a, int row_blocks, int rows
     if (a.R == 0) return 1;
     const int chunks = (a.R + Q_RCHUNK - 1) / Q_RCHUNK, cus = device_cus();
     // (with a prologue the workgroups that only project compute it a second time: only where half the CUs would idle
-    // anyway.  Norm prologue, K = 3072, R = 32, with half of the CUs / all of them as the limit: M = 512 11.0 / 11.0 us, 1024 13.6 /
+    // anyway.  That was the better limit while the row statistics had a launch of their own; all of the CUs is now.  Norm prologue, K = 3072, R = 32, with half of the CUs / all of them as the limit: M = 512 11.0 / 11.0 us, 1024 13.6 /
     // 12.0, 2048 15.3 / 14.2, 4096 16.7 / 16.2, 4608 23.2 / 22.7)
     const bool prologue = has_norm(a) || a.prologue != SVDQ_PRE_NONE;
     const int limit = prologue ? cus / 2 : cus + (rows == 32 ? cus / 8 : 0);

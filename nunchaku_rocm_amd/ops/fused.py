@@ -17,7 +17,8 @@ def _row_block(pad_size: int) -> int:
     """What the buffers between the two GEMMs are padded to.  fc1's epilogue requantizes every row of its buffers, so rows up to
     ``pad_size`` are computed for nobody; the kernels ask for whole blocks of 32 only.  us per call, 256 / 32 (bf16,
     K = 3072, hidden 12288): SwiGLU 32 rows 67.3 / 53.1, 333 rows 97.0 / 91.9, 1100 rows 188 / 183, GELU 2100 rows 217 / 211;
-    K = 1536, hidden 6144: GELU 32 rows 38.5 / 34.7, 600 rows 47.8 / 44.1; multiples of 256 as before."""
+    K = 1536, hidden 6144: GELU 32 rows 38.5 / 34.7, 600 rows 47.8 / 44.1; multiples of 256 as before.
+    (Fewer rows may bring in the kernel that splits K: the last bits of a row's sums are then that kernel's.)"""
     return 32 if pad_size > 0 and pad_size % 32 == 0 else pad_size
 
 

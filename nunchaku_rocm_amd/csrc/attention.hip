@@ -24,8 +24,8 @@
 //    (ds_read_b64_tr_b16: sixteen lanes pass the addresses of four rows x 16 columns and lane l receives column l
 //    of the four rows), two reads per operand.
 //  * 256 threads = 4 wavefronts of 32 queries, two workgroups per CU; Q stays in registers (pre-scaled), the output
-//    accumulator is D / 2 registers.  A tile is processed as two 32-key halves so that the softmax instructions of one
-//    half sit between the matrix instructions of the other (see the pipeline comment in the kernel).
+//    accumulator is D / 2 registers.  The keys are walked 32 at a time in a software pipeline: the products of the next and
+//    of the previous 32 keys are issued beside the softmax of the current ones (see the comment in the kernel).
 //  * Workgroups of one head run on one XCD (when the head count is a multiple of 8), so K and V of a head are
 //    fetched into one L2 only.
 #include <type_traits>
@@ -178,170 +178,175 @@ __global__ __launch_bounds__(256, 2) void attention_kernel(svdq_attention_args a
 #pragma unroll
     for (int i = 0; i < 16; i++) cinit[i] = 0.0f;
 
-    const int nblk = (a.Tkv + AT_BK - 1) / AT_BK;
-    // Software pipeline.  Tile t lives in stage t & 1 and is handled as two halves of 32 keys, each a complete online-
-    // softmax step, so that the softmax arithmetic of one half is issued between the matrix instructions of the other:
-    //   (A) S0 = K[0:32] Q^T                            + V^T operand reads (keys 0..31)
-    //   (B) S1 = K[32:64] Q^T         ||  softmax(S0)   + V^T operand reads (keys 32..63)
-    //   (C) O^T += V^T[:, 0:32] P0^T  ||  softmax(S1)
-    //       barrier: tile t + 1 has landed for everybody, nobody reads tile t any more
-    //   (D) O^T += V^T[:, 32:64] P1^T                   + K operand reads of tile t + 1, loads of tile t + 2 into
-    //                                                     the stage tile t has left
-    // The compiler is kept from regrouping the slots (one matrix instruction plus its share of the rest).
+    const int nblk = (a.Tkv + AT_BK - 1) / AT_BK, nhalf = (a.Tkv + 31) / 32;
+    // Software pipeline over halves of 32 keys.  Iteration j issues three independent strands side by side:
+    //   S(j + 1) = K[j + 1] Q^T      |  softmax of S(j)  |      O^T += V^T[j - 1] P(j - 1)^T
+    // in 2 NC slots of one matrix instruction, its share of the softmax and the read that refills the operand registers it
+    // has just used with the operand of RING matrix instructions of its strand later.  Stage t & 1 holds V of tile t and K of
+    // tile t + 1; the operands are read from it between the middle of tile t's first iteration, where a barrier releases it and
+    // the other stage begins to fill, and the middle of tile t + 1's.  The compiler is kept from regrouping the slots.
+    // Before, the softmax of a half stood beside one product only, with nothing beside the row maximum and the exponentials in
+    // half of the slots, and a tile's operands filled 128 registers a phase ahead (now 32).  Same bits; us before / now (bf16):
+    // D = 128, 24 heads x 4608 253 / 232, 28 x 4608 270 / 254, 24 x 2000 58 / 52; D = 64, 40 x 4096 172 / 166.  Of 271 us (28 heads, a
+    // slower board) the V^T reads are 42, the tile loads 30, the K reads 14, the exponentials 12; matrix instructions alone run at
+    // 1.8 PFLOP/s on random data (1.86 GHz), which is 167 us.
+    // Priority: the second iteration of a tile goes first (s_setprio), which keeps the two wavefronts of a SIMD out of step: 242 / 236.
+    constexpr int RING = NC / 2;
+    static_assert(NC == 2 * NDT, "as many matrix instructions per half in either product");
 #pragma unroll
-    for (int j = 0; j < LOADS; j++) issue_k(0, smem0, j);
+    for (int j = 0; j < LOADS; j++) issue_k(0, smem1, j);  // K of tile 0: read before the first barrier in the loop
 #pragma unroll
     for (int j = 0; j < LOADS; j++) issue_v(0, smem0, j);
-    {
-        const int t1 = min(1, nblk - 1);
 #pragma unroll
-        for (int j = 0; j < LOADS; j++) issue_k(t1, smem1, j);
-#pragma unroll
-        for (int j = 0; j < LOADS; j++) issue_v(t1, smem1, j);
-    }
-    __builtin_amdgcn_s_waitcnt(waitcnt_imm(2 * LOADS, 15));  // tile 0 (the older half of the loads)
+    for (int j = 0; j < LOADS; j++) issue_k(min(1, nblk - 1), smem0, j);
+    // V of half -1: zeros (the keys that are read of it: the last sixteen rows of the stage's V)
+    if (tid < 16 * G::KCH) *(v4i *)(smem1 + G::KT_BYTES + 48 * G::KROW + 16 * tid) = (v4i){0, 0, 0, 0};
+    __builtin_amdgcn_s_waitcnt(waitcnt_imm(2 * LOADS, 0));
     __builtin_amdgcn_s_barrier();
-    v4i rk[2 * NC], rv[4 * NDT];  // rk[NC t + c]: K rows 32 t.., chunk c;  rv[4 dt + c]: V^T rows 32 dt.., 16-key chunk c
+    v4i rk[RING], rv[RING];  // operand c of a half in c % RING; of V^T operand c: rows 32 (c % NDT).., 16-key chunk c / NDT
+    v16f sc[2];
+    {
+        v4i k0[NC];
 #pragma unroll
-    for (int c = 0; c < NC; c++) {
-        rk[c] = *(const v4i *)(smem0 + koff[c]);
-        rk[NC + c] = *(const v4i *)(smem0 + 32 * G::KROW + koff[c]);
+        for (int c = 0; c < NC; c++) k0[c] = *(const v4i *)(smem1 + koff[c]);
+#pragma unroll
+        for (int c = 0; c < NC; c++) sc[0] = mfma32_16bit<T>(k0[c], qop[c], c == 0 ? cinit : sc[0]);
     }
+#pragma unroll
+    for (int c = 0; c < RING; c++) rk[c] = *(const v4i *)(smem1 + 32 * G::KROW + koff[c]), rv[c] = (v4i){0, 0, 0, 0};
+    v4i pop[2][2];  // [parity of the half][16-key chunk]: P^T operand = accumulator quads 2 cc, 2 cc + 1 of S
+#pragma unroll
+    for (int c = 0; c < 2; c++) pop[1][c] = (v4i){0, 0, 0, 0};
 
-    float shift, alpha, rs;  // rs: this half's row sum, at the new reference
     auto max3 = [](float x, float y, float z) {
         float r;
         asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(x), "v"(y), "v"(z));
         return r;
     };
-    // row maximum of one half (16 scores of this lane, 16 of lane ^ 32) relative to the bias; when it exceeds the
-    // allowance: shift = how far the reference moves, alpha = the factor that moves the accumulator there (0 before the
-    // first keys).  Returns whether any lane of the wavefront moved.
-    auto row_max = [&](const v16f &sv) -> bool {
-        float mx = max3(sv[0], sv[1], sv[2]);
-#pragma unroll
-        for (int i = 3; i < 15; i += 2) mx = max3(mx, sv[i], sv[i + 1]);
-        mx = max3(mx, sv[15], sv[15]);
-        const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
-        mx = max3(__uint_as_float(sw[0]), __uint_as_float(sw[1]), __uint_as_float(sw[1]));
-        const bool need = mx > gap + AT_LAZY;
-        shift = need ? mx : 0.0f;
-        alpha = __builtin_amdgcn_exp2f(need ? gap - mx : 0.0f);
-        gap = need ? 0.0f : gap;
-        return __builtin_amdgcn_ballot_w64(need) != 0;
-    };
-    auto shift16 = [&](v16f &sv) {
-#pragma unroll
-        for (int i = 0; i < 16; i++) sv[i] -= shift;
-    };
-    // four scores -> two packed P values; the row sum adds what the matrix instruction will see (the rounded P)
-    auto exp4 = [&](const v16f &sv, int i0, v4i &pw, int e0) {
-        float p[4];
-#pragma unroll
-        for (int e = 0; e < 4; e++) p[e] = __builtin_amdgcn_exp2f(sv[i0 + e]);
-        pw[e0] = (int)pack2<T>(p[0], p[1]);
-        pw[e0 + 1] = (int)pack2<T>(p[2], p[3]);
-        rs = T::sum2((uint32_t)pw[e0], rs);
-        rs = T::sum2((uint32_t)pw[e0 + 1], rs);
-    };
-    // the reference moved: accumulator and row sum to the new reference, later scores start from the new bias
-    auto rescale = [&]() {
-        l_run *= alpha;
-#pragma unroll
-        for (int dt = 0; dt < G::NDT; dt++)
-#pragma unroll
-            for (int i = 0; i < 16; i++) acc_o[dt][i] *= alpha;
-        shift16(cinit);
-    };
-
-    auto tile = [&](auto par_tag, int blk) {  // tile blk, which lives in stage par_tag
-        constexpr int PAR = decltype(par_tag)::value;
-        uint8_t *st = PAR ? smem1 : smem0;
-        const uint8_t *sn = PAR ? smem0 : smem1;
-        const int nxt = min(blk + 2, nblk - 1);  // past the end: the last tile again, into a stage nobody reads
-        const bool ragged = blk == nblk - 1 && (a.Tkv & (AT_BK - 1));
-        v16f s0, s1;
-        v4i pop[4];  // P^T operand: chunk cc of half t = accumulator quads 2 cc, 2 cc + 1 of S_t
-
-        // ---- (A) ---------------------------------------------------------------------------------------------------------
-#pragma unroll
-        for (int c = 0; c < NC; c++) {
-            s0 = mfma32_16bit<T>(rk[c], qop[c], c == 0 ? cinit : s0);
-            rv[4 * (c % NDT) + c / NDT] = read_v(st, c % NDT, c / NDT);  // chunks 0, 1: keys 0..31
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        if (ragged) {  // keys past the end count as -inf
+    auto iteration = [&](auto half_tag, auto stage_tag, int blk) {  // half half_tag of tile blk, which lives in stage stage_tag
+        constexpr int H = decltype(half_tag)::value, PAR = decltype(stage_tag)::value, NU = 2 * NC;
+        const uint8_t *st = PAR ? smem1 : smem0;
+        uint8_t *other = PAR ? smem0 : smem1;  // the stage before this one, then the next
+        v16f &cur = sc[H], &nxt = sc[H ^ 1];
+        const int key0 = blk * AT_BK + 32 * H;
+        if (key0 + 32 > a.Tkv) {  // keys past the end count as -inf
 #pragma unroll
             for (int i = 0; i < 16; i++)
-                if (blk * AT_BK + 8 * (i >> 2) + 4 * half + (i & 3) >= a.Tkv) s0[i] = -INFINITY;
+                if (key0 + 8 * (i >> 2) + 4 * half + (i & 3) >= a.Tkv) cur[i] = -INFINITY;
         }
-
-        // ---- (B) ---------------------------------------------------------------------------------------------------------
-        bool moved = false;
+        float mx, shift = 0.0f, alpha = 1.0f, rs = 0.0f;  // rs: this half's row sum, at the new reference
+        bool need = false, moved = false;
+        // the softmax in sixteen pieces: row maximum of the half (16 scores of this lane, 16 of lane ^ 32) relative to the bias;
+        // when it exceeds the allowance, shift = how far the reference moves, alpha = the factor that moves the accumulator there
+        // (0 before the first keys); then two scores at a time to packed P values, whose rounded sum is the row sum's share
+        auto piece = [&](int v) {
+            if (v == 0) {
+                mx = max3(cur[0], cur[1], cur[2]);
+                mx = max3(mx, cur[3], cur[4]);
+            } else if (v < 4) {
+                mx = max3(mx, cur[4 * v + 1], cur[4 * v + 2]);
+                mx = max3(mx, cur[4 * v + 3], cur[v == 3 ? 15 : 4 * v + 4]);
+            } else if (v == 4) {
+                const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
+                mx = max3(__uint_as_float(sw[0]), __uint_as_float(sw[1]), __uint_as_float(sw[1]));
+                need = mx > gap + AT_LAZY;
+                moved = __builtin_amdgcn_ballot_w64(need) != 0;
+            } else if (v == 5) {
+                if (moved) {
+                    shift = need ? mx : 0.0f;
+                    alpha = __builtin_amdgcn_exp2f(need ? gap - mx : 0.0f);
+                    gap = need ? 0.0f : gap;
 #pragma unroll
-        for (int c = 0; c < NC; c++) {
-            s1 = mfma32_16bit<T>(rk[NC + c], qop[c], c == 0 ? cinit : s1);
-            rv[4 * (c % NDT) + 2 + c / NDT] = read_v(st, c % NDT, 2 + c / NDT);  // keys 32..63
-            if (c == 0) {
-                moved = row_max(s0);
-                rs = 0.0f;
-                if (moved) shift16(s0);
+                    for (int i = 0; i < 16; i++) cur[i] -= shift;
+                }
+            } else if (v < 14) {
+                const int k = v - 6;
+                uint32_t p = pack2<T>(__builtin_amdgcn_exp2f(cur[2 * k]), __builtin_amdgcn_exp2f(cur[2 * k + 1]));
+                asm volatile("" : "+v"(p));  // (not moved to its use in the next iteration)
+                pop[H][k >> 2][k & 3] = (int)p;
+                rs = T::sum2(p, rs);
             }
+        };
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_setprio(H);
 #pragma unroll
-            for (int j = 0; j < 4; j++)  // the four exp slices go with slots 1 .. 4 (the last slot takes what is left)
-                if (c == (1 + j < NC - 1 ? 1 + j : NC - 1)) exp4(s0, 4 * j, pop[j >> 1], 2 * (j & 1));
+        for (int u = 0; u < NU; u++) {
+            const int c = u >> 1, r = c % RING;
+#pragma unroll
+            for (int v = u * 16 / NU; v < (u + 1) * 16 / NU; v++) piece(v);
+            __builtin_amdgcn_sched_barrier(0);
+            const bool early = c < RING;
+            if (H == 0 && u == NC) {  // my loads of this stage have landed, my reads of the other are done
+                __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, 0));
+                __builtin_amdgcn_s_barrier();
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if ((u & 1) == 0) {
+                nxt = mfma32_16bit<T>(rk[r], qop[c], c == 0 ? cinit : nxt);
+                if (early)  // the rest of half j + 1, then the first operands of half j + 2
+                    rk[r] = *(const v4i *)((H ? st : other + 32 * G::KROW) + koff[c + RING]);
+                else
+                    rk[r] = *(const v4i *)(st + H * (32 * G::KROW) + koff[c - RING]);
+            } else {
+                acc_o[c % NDT] = mfma32_16bit<T>(rv[r], pop[H ^ 1][c / NDT], acc_o[c % NDT]);
+                if (early)  // the rest of half j - 1, then the first operands of half j
+                    rv[r] = read_v(H ? st : other, (c + RING) % NDT, 2 * (H ^ 1) + (c + RING) / NDT);
+                else
+                    rv[r] = read_v(st, (c - RING) % NDT, 2 * H + (c - RING) / NDT);
+            }
+            if (H == 0 && u >= NC && u - NC < 2 * LOADS) {
+                if (u & 1)
+                    issue_k(min(blk + 2, nblk - 1), other, (u - NC) >> 1);
+                else
+                    issue_v(min(blk + 1, nblk - 1), other, (u - NC) >> 1);
+            }
             __builtin_amdgcn_sched_barrier(0);
         }
-        if (moved) {
-            shift16(s1);  // computed from the old bias
-            rescale();
+        if (moved) {  // accumulator, row sum and the scores already computed to the new reference, later ones start from it
+            l_run *= alpha;
+#pragma unroll
+            for (int dt = 0; dt < NDT; dt++)
+#pragma unroll
+                for (int i = 0; i < 16; i++) acc_o[dt][i] *= alpha;
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                nxt[i] -= shift;
+                cinit[i] -= shift;
+            }
         }
         l_run += rs;
-        if (ragged) {
-#pragma unroll
-            for (int i = 0; i < 16; i++)
-                if (blk * AT_BK + 32 + 8 * (i >> 2) + 4 * half + (i & 3) >= a.Tkv) s1[i] = -INFINITY;
-        }
         __builtin_amdgcn_sched_barrier(0);
-
-        // ---- (C) ---------------------------------------------------------------------------------------------------------
+    };
+    const std::integral_constant<int, 0> I0;
+    const std::integral_constant<int, 1> I1;
+    auto last_pv = [&](const uint8_t *st, auto half_tag) {  // O^T += V^T P^T of the last half
+        constexpr int H = decltype(half_tag)::value;
 #pragma unroll
         for (int c = 0; c < NC; c++) {
-            acc_o[c % NDT] = mfma32_16bit<T>(rv[4 * (c % NDT) + c / NDT], pop[c / NDT], acc_o[c % NDT]);
-            if (c == 0) {
-                moved = row_max(s1);
-                rs = 0.0f;
-                if (moved) shift16(s1);
-            }
-#pragma unroll
-            for (int j = 0; j < 4; j++)
-                if (c == (1 + j < NC - 1 ? 1 + j : NC - 1)) exp4(s1, 4 * j, pop[2 + (j >> 1)], 2 * (j & 1));
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        if (moved) rescale();
-        l_run += rs;
-        __builtin_amdgcn_sched_barrier(0);
-        __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, 0));  // my loads of tile blk + 1 have landed, my reads of tile blk are done
-        __builtin_amdgcn_s_barrier();
-        __builtin_amdgcn_sched_barrier(0);
-
-        // ---- (D) ---------------------------------------------------------------------------------------------------------
-#pragma unroll
-        for (int c = 0; c < NC; c++) {
-            acc_o[c % NDT] = mfma32_16bit<T>(rv[4 * (c % NDT) + 2 + c / NDT], pop[2 + c / NDT], acc_o[c % NDT]);
-            rk[2 * c] = *(const v4i *)(sn + ((2 * c) / NC) * (32 * G::KROW) + koff[(2 * c) % NC]);
-            rk[2 * c + 1] = *(const v4i *)(sn + ((2 * c + 1) / NC) * (32 * G::KROW) + koff[(2 * c + 1) % NC]);
-            if (c & 1) issue_k(nxt, st, c >> 1); else issue_v(nxt, st, c >> 1);
-            __builtin_amdgcn_sched_barrier(0);
+            const v4i v = c < RING ? rv[c % RING] : read_v(st, c % NDT, 2 * H + c / NDT);
+            acc_o[c % NDT] = mfma32_16bit<T>(v, pop[H][c / NDT], acc_o[c % NDT]);
         }
     };
     {
         int blk = 0;
-        for (; blk + 1 < nblk; blk += 2) {
-            tile(std::integral_constant<int, 0>{}, blk);
-            tile(std::integral_constant<int, 1>{}, blk + 1);
+        for (; 2 * blk + 4 <= nhalf; blk += 2) {
+            iteration(I0, I0, blk);
+            iteration(I1, I0, blk);
+            iteration(I0, I1, blk + 1);
+            iteration(I1, I1, blk + 1);
         }
-        if (blk < nblk) tile(std::integral_constant<int, 0>{}, blk);
+        const int left = nhalf - 2 * blk;  // 0 .. 3
+        if (left >= 1) iteration(I0, I0, blk);
+        if (left >= 2) iteration(I1, I0, blk);
+        if (left == 3) iteration(I0, I1, blk + 1);
+        if (left == 0)
+            last_pv(smem1, I1);
+        else if (left == 1)
+            last_pv(smem0, I0);
+        else if (left == 2)
+            last_pv(smem0, I1);
+        else
+            last_pv(smem1, I0);
     }
 
     // ---- O = O^T / l, staged through LDS so that rows leave as 256-byte segments -------------------------------------

@@ -185,3 +185,20 @@ def test_full_size_invariants(dev):
     # each output row is a convex combination of value rows
     vmax = v.float().abs().amax(dim=2)  # (B, H, D)
     assert bool((base.view(B, T, H, D).float().abs() <= vmax[:, None] * (1 + 2**-6)).all())
+
+
+@pytest.mark.parametrize("D", [128, 64])
+@pytest.mark.parametrize("Tkv", [1, 31, 32, 33, 64, 65, 96, 97, 128, 129, 160, 161, 192, 193, 224, 256, 257])
+def test_ends_of_the_key_pipeline(dev, Tkv, D):
+    """Key counts around every way in which the pipeline over halves of 32 keys ends; an infinite value reaches its own column
+    only (what the pipeline multiplies before the first and behind the last half must not meet it)."""
+    print(f"case Tkv={Tkv} D={D}", flush=True)
+    q, k, v = _inputs(1, 3, 70, Tkv, torch.float16, seed=Tkv, D=D)
+    out = _run(dev, q, k, v, D**-0.5)
+    assert O.max_rel_err(out, O.attention_fp16(q, k, v, D**-0.5)) <= TOL
+    v[0, 1, Tkv - 1, 5] = float("inf")
+    spoilt = _run(dev, q, k, v, D**-0.5)
+    assert (spoilt[0, :, D + 5] == float("inf")).all()
+    keep = torch.ones(3 * D, dtype=torch.bool)
+    keep[D + 5] = False
+    assert torch.equal(spoilt[..., keep], out[..., keep])

@@ -840,7 +840,7 @@ template <typename T, bool U>
 static void launch_gemm_f8(const svdq_gemm_args &a, hipStream_t s) {
     const bool two = two_workgroups_per_cu((long)((a.M + BM - 1) / BM) * ((a.N + BN - 1) / BN));
     if (const int wavefronts = split_of(a, cu_count())) {
-        launch_gemm_split(a, wavefronts, s);
+        launch_gemm_split(a, wavefronts, cu_count(), s);
         return;
     }
     if (a.act_blocked == 2) {  // fp6 codes carry their sign: one instantiation for signed and unsigned activations

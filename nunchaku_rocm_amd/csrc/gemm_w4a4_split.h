@@ -9,7 +9,7 @@ namespace svdq {
 // act_blocked == 2.
 int split_wavefronts(const svdq_gemm_args &a, int cus);
 
-// The launch, for `wavefronts` = 4 or 8; `a` has passed svdq_gemm_w4a4's checks and has rows to write.
-void launch_gemm_split(const svdq_gemm_args &a, int wavefronts, hipStream_t s);
+// The launch on a device of `cus` compute units, for `wavefronts` = 4 or 8; `a` has passed svdq_gemm_w4a4's checks and has rows to write.
+void launch_gemm_split(const svdq_gemm_args &a, int wavefronts, int cus, hipStream_t s);
 
 }  // namespace svdq

@@ -197,3 +197,45 @@ def test_qk_norm_rope(dev, splits, tokens, heads, K, wavefronts, dtype):
     assert torch.equal(a, b)
     # each side within one rounding of values that differ in the order of the K / 64 group terms
     assert ((a.float() - tiles.float()).abs() <= tiles.float().abs() * (2.0**-7 if dtype == torch.bfloat16 else 2.0**-10) + 1e-4).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,K,N", [(65, 1280, 16640), (65, 1280, 16384), (33, 1344, 18440), (160, 3072, 8192)])
+def test_rows_of_a_workgroup(dev, splits, M, K, N, dtype):
+    """Workgroups of 64 rows up to one per CU (256 at 65 x 16384 on 256 CUs), beyond that (260) of 32; a last workgroup of one row,
+    a second row block without rows and a column half past N."""
+    print(f"case M={M} K={K} N={N} {dtype}", flush=True)
+    mod = _module(dev, K, N, 32, dtype)
+    x = O.make_activations(M, K, seed=M, dtype=dtype).to(dev)[None]
+    canary = torch.full((M + 8, N), 7.0, dtype=dtype, device=dev)
+    with torch.no_grad():
+        tiles, a, b = _both(lambda: mod(x, output=canary[:M]).clone(), splits, [4])
+    assert torch.equal(a, b) and (canary[M:] == 7.0).all()
+    # as in test_split_against_tiles
+    bound = tiles.float().abs() * (2.0**-7 if dtype == torch.bfloat16 else 2.0**-10) + 2 * (K // 64) * 2.0**-24 * _abs_terms(mod, x) + 1e-6
+    assert ((a.float() - tiles.float()).abs() <= bound).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(40, 136, 512), (333, 4104, 1536), (65, 16640, 1536)])
+def test_hand_over_forms_give_the_same_bits(dev, splits, M, N, K):
+    """Unsigned activations with ordinary scales: the same sums in the same order in every form."""
+    from nunchaku_rocm_amd import ops
+    from nunchaku_rocm_amd.layout import block_activations, block_activations_f6, block_scales
+
+    print(f"case M={M} N={N} K={K}", flush=True)
+    rows = -(-M // 32) * 32
+    g = torch.Generator().manual_seed(M)
+    act = torch.randint(0, 256, (rows, K // 2), dtype=torch.uint8, generator=g)
+    asc = (torch.rand(K // 64, rows, generator=g) * 0.1 + 0.01).to(torch.bfloat16)
+    wgt = torch.nn.Parameter(torch.randint(0, 256, (N, K // 2), dtype=torch.uint8, generator=g).view(torch.int8).to(dev), requires_grad=False)
+    wsc = (torch.rand(K // 64, N, generator=g) * 0.02 + 0.005).to(torch.bfloat16).to(dev)
+    f6 = block_activations_f6(act, True)
+    results = []
+    for sent, scales, blocked in ((act, asc, 0), (block_activations(act), asc, 1), (f6, asc, 2), (f6, block_scales(asc), 3)):
+        out = torch.empty(M, N, dtype=torch.bfloat16, device=dev)
+        ops.svdq_gemm_w4a4_cuda(act=sent.to(dev), wgt=wgt, out=out, ascales=scales.to(dev), wscales=wsc, act_unsigned=True, act_blocked=blocked)
+        results.append(out.cpu())
+    assert len(set(splits)) == 1 and splits[0] in (4, 8)
+    assert all(torch.equal(r, results[0]) for r in results[1:])

@@ -23,7 +23,7 @@
 //    barrier per 64 keys; the V^T operand comes out of the V tile through the transposing LDS read of gfx950
 //    (ds_read_b64_tr_b16: sixteen lanes pass the addresses of four rows x 16 columns and lane l receives column l
 //    of the four rows), two reads per operand.
-//  * 256 threads = 4 wavefronts of 32 queries, two workgroups per CU; Q stays in registers (pre-scaled), the output
+//  * Four wavefronts of 32 queries, two workgroups per CU, or eight and one (wide_queries); Q stays in registers (pre-scaled), the output
 //    accumulator is D / 2 registers.  The keys are walked 32 at a time in a software pipeline: the products of the next and
 //    of the previous 32 keys are issued beside the softmax of the current ones (see the comment in the kernel).
 //  * Workgroups of one head run on one XCD (when the head count is a multiple of 8), so K and V of a head are
@@ -34,7 +34,7 @@
 
 namespace svdq {
 
-constexpr int AT_BQ = 128, AT_BK = 64;     // queries per workgroup, keys per tile
+constexpr int AT_BK = 64;  // keys per tile
 
 // Geometry for head dimension D (128 or 64).  K and V tiles are [key][2 D bytes]; every block load moves 1 KB
 // (64 lanes x 16 bytes) = whole rows; 16-byte chunks are XOR-swizzled by the row so that the operand reads touch every
@@ -44,7 +44,7 @@ constexpr int AT_BQ = 128, AT_BK = 64;     // queries per workgroup, keys per ti
 // different 32-byte slots of the 256 bytes the banks span, so the 64-byte quarter of a row is swizzled by row & 3
 // (256-byte rows) or the 64-byte half by row / 2 & 1 (128-byte rows, where rows r and r + 1 already differ by half
 // the banks).
-template <int D>
+template <int D, int WAVES>
 struct AtGeo {
     static constexpr int NC = D / 16;               // 16-wide k chunks of q k^T = matrix instructions per 32-key half
     static constexpr int NDT = D / 32;              // 32-row d tiles of O^T
@@ -53,7 +53,7 @@ struct AtGeo {
     static constexpr int KT_BYTES = AT_BK * KROW;   // K tile
     static constexpr int VT_BYTES = KT_BYTES;       // V tile
     static constexpr int STAGE = KT_BYTES + VT_BYTES;
-    static constexpr int LOADS = KT_BYTES / 1024 / 4;  // block loads per wavefront and tile, of K and of V alike
+    static constexpr int LOADS = KT_BYTES / 1024 / WAVES;  // block loads per wavefront and tile, of K and of V alike
     static constexpr int OPITCH = 2 * D + 16;       // staged output row
     __host__ __device__ static constexpr int kswz(int row) { return KROW == 256 ? (row & 15) : ((row >> 1) & 7); }
     __host__ __device__ static constexpr int vswz(int row) { return KROW == 256 ? ((row & 3) << 2) : (((row >> 1) & 1) << 2); }
@@ -78,14 +78,15 @@ __device__ inline v2i32 at_read_tr(const uint8_t *p) {
 }
 constexpr float AT_LAZY = 8.0f;                 // the accumulator is rescaled when a row maximum grew by more than this
 
-template <typename T, int D>
-__global__ __launch_bounds__(256, 2) void attention_kernel(svdq_attention_args a, int ntile, int xcd_heads) {
-    using G = AtGeo<D>;
+template <typename T, int D, int WAVES>
+__global__ __launch_bounds__(64 * WAVES, 2) void attention_kernel(svdq_attention_args a, int ntile, int xcd_heads) {
+    using G = AtGeo<D, WAVES>;
+    constexpr int AT_BQ = 32 * WAVES;  // queries per workgroup
     constexpr int NC = G::NC, NDT = G::NDT, LOADS = G::LOADS;
     // Two separate LDS objects, one per stage, and a main loop unrolled over them: the compiler then knows that a tile
     // load into one stage cannot touch what is being read from the other.  With one object and a run-time stage offset
     // it made every LDS read wait for all loads in flight, i.e. for the tile that was requested just before.
-    static_assert(AT_BQ == 128 && 64 * G::OPITCH <= G::STAGE, "the output tile is staged as two halves of 64 rows, one per stage");
+    static_assert(WAVES % 4 == 0 && 64 * G::OPITCH <= G::STAGE, "the output tile is staged as two halves of 64 rows, one per stage");
     __shared__ __align__(16) uint8_t smem0[G::STAGE];
     __shared__ __align__(16) uint8_t smem1[G::STAGE];
 
@@ -187,7 +188,7 @@ __global__ __launch_bounds__(256, 2) void attention_kernel(svdq_attention_args a
     // the other stage begins to fill, and the middle of tile t + 1's.  The compiler is kept from regrouping the slots.
     // Before, the softmax of a half stood beside one product only, with nothing beside the row maximum and the exponentials in
     // half of the slots, and a tile's operands filled 128 registers a phase ahead (now 32).  Same bits; us before / now (bf16):
-    // D = 128, 24 heads x 4608 253 / 232, 28 x 4608 270 / 254, 24 x 2000 58 / 52; D = 64, 40 x 4096 172 / 166.  Of 271 us (28 heads, a
+    // workgroups of 128 queries; D = 128, 24 heads x 4608 253 / 232, 28 x 4608 270 / 254, 24 x 2000 58 / 52; D = 64, 40 x 4096 172 / 166.  Of 271 us (28 heads, a
     // slower board) the V^T reads are 42, the tile loads 30, the K reads 14, the exponentials 12; matrix instructions alone run at
     // 1.8 PFLOP/s on random data (1.86 GHz), which is 167 us.
     // Priority: the second iteration of a tile goes first (s_setprio), which keeps the two wavefronts of a SIMD out of step: 242 / 236.
@@ -294,6 +295,7 @@ __global__ __launch_bounds__(256, 2) void attention_kernel(svdq_attention_args a
                 else
                     rv[r] = read_v(st, (c - RING) % NDT, 2 * H + (c - RING) / NDT);
             }
+            static_assert(2 * LOADS <= NC, "the block loads fit the second half of an iteration");
             if (H == 0 && u >= NC && u - NC < 2 * LOADS) {
                 if (u & 1)
                     issue_k(min(blk + 2, nblk - 1), other, (u - NC) >> 1);
@@ -353,32 +355,59 @@ __global__ __launch_bounds__(256, 2) void attention_kernel(svdq_attention_args a
     l_run += __shfl_xor(l_run, 32);
     const float inv = 1.0f / (l_run == 0.0f ? 1.0f : l_run);
     __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, 0));  // the redundant last tile load has landed
-    __syncthreads();
-#pragma unroll
-    for (int dt = 0; dt < NDT; dt++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            uint2 w;
-            w.x = pack2<T>(acc_o[dt][4 * j] * inv, acc_o[dt][4 * j + 1] * inv);
-            w.y = pack2<T>(acc_o[dt][4 * j + 2] * inv, acc_o[dt][4 * j + 3] * inv);
-            *(uint2 *)((wave < 2 ? smem0 : smem1) + ((wave & 1) * 32 + l32) * G::OPITCH + (32 * dt + 8 * j + 4 * half) * 2) = w;
-        }
-    __syncthreads();
     uint16_t *op = (uint16_t *)a.o + (long)b * a.sob + (long)h * D;
-    constexpr int OCH = D / 8, OROWS = 256 / OCH;  // 16-byte chunks per output row, rows per pass
+    constexpr int OCH = D / 8, OROWS = 64 * WAVES / OCH;  // 16-byte chunks per output row, rows per pass
     const int c = tid % OCH;
 #pragma unroll
-    for (int pass = 0; pass < AT_BQ / OROWS; pass++) {
-        const int row = pass * OROWS + tid / OCH, q = q0 + row;
-        if (q < a.Tq) *(v4i *)(op + (long)q * a.som + 8 * c) = *(const v4i *)((row < 64 ? smem0 : smem1) + (row & 63) * G::OPITCH + c * 16);
+    for (int part = 0; part < WAVES / 4; part++) {  // 128 rows at a time
+        __syncthreads();
+        if (WAVES == 4 || wave >> 2 == part) {
+#pragma unroll
+            for (int dt = 0; dt < NDT; dt++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    uint2 w;
+                    w.x = pack2<T>(acc_o[dt][4 * j] * inv, acc_o[dt][4 * j + 1] * inv);
+                    w.y = pack2<T>(acc_o[dt][4 * j + 2] * inv, acc_o[dt][4 * j + 3] * inv);
+                    *(uint2 *)((wave & 2 ? smem1 : smem0) + ((wave & 1) * 32 + l32) * G::OPITCH + (32 * dt + 8 * j + 4 * half) * 2) = w;
+                }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int pass = 0; pass < 128 / OROWS; pass++) {
+            const int row = pass * OROWS + tid / OCH, q = q0 + 128 * part + row;
+            if (q < a.Tq) *(v4i *)(op + (long)q * a.som + 8 * c) = *(const v4i *)((row < 64 ? smem0 : smem1) + (row & 63) * G::OPITCH + c * 16);
+        }
     }
 }
 
-template <typename T, int D>
+// Whether workgroups of 256 queries (eight wavefronts, one workgroup to a CU) are the faster ones than two of 128 to a CU: they fetch a
+// tile of K and V once for eight wavefronts and not for four, which at head dimension 128 is 2 to 7 % of a launch.  A round of them
+// counts 0.97 of a round of two workgroups of 128, and one workgroup of 128 alone on a CU 0.565 (28 heads x 4608: 504 workgroups of
+// 256 252.8 us, 1008 of 128 258.7; 7 heads, 252 of 128 73, 126 of 256 93).  With few keys a launch is mostly beginnings and ends of
+// workgroups, which two to a CU hide from each other: beyond one round 77 keys 1.00 to 1.16 of the time, 512 1.02 to 1.10, 2500 0.96
+// to 0.97; within one, 256 keys at 480 workgroups of 128 1.015, at 432 0.99.  us, 128 / 256 queries (bf16): 24 x 4608 234 / 225, 24 x 2000
+// 52.5 / 49.9, 24 x 8192 672 / 658, 10 x 4608 112 / 108, 20 x 3000 87.8 / 87.0.  Head dimension 64: 40 x 4096 169 / 192.
+static bool wide_queries(const svdq_attention_args &a, int cus) {
+    const long wg4 = (long)((a.Tq + 127) / 128) * a.H * a.B, wg8 = (long)((a.Tq + 255) / 256) * a.H * a.B;
+    const long deep = (wg4 + cus - 1) / cus, rounds = (wg8 + cus - 1) / cus;  // workgroups of 128 on the fullest CU
+    if (0.97 * (double)rounds >= (double)(deep / 2) + (deep % 2 ? 0.565 : 0.0)) return false;
+    return rounds > 1 ? a.Tkv >= 2048 : a.Tkv >= 1024 || 4 * wg4 <= 7L * cus;
+}
+
+template <typename T, int D, int WAVES>
 static void launch_attention(const svdq_attention_args &a, hipStream_t s) {
-    const int ntile = (a.Tq + AT_BQ - 1) / AT_BQ;
-    const int xcd_heads = (a.B * a.H) % 8 == 0;
-    hipLaunchKernelGGL((attention_kernel<T, D>), dim3((unsigned)(ntile * a.H * a.B)), dim3(256), 0, s, a, ntile, xcd_heads);
+    const int ntile = (a.Tq + 32 * WAVES - 1) / (32 * WAVES), xcd_heads = (a.B * a.H) % 8 == 0;
+    hipLaunchKernelGGL((attention_kernel<T, D, WAVES>), dim3((unsigned)(ntile * a.H * a.B)), dim3(64 * WAVES), 0, s, a, ntile, xcd_heads);
+}
+template <typename T>
+static void launch_attention(const svdq_attention_args &a, hipStream_t s) {
+    if (a.D == 64)
+        launch_attention<T, 64, 4>(a, s);
+    else if (wide_queries(a, cu_count()))
+        launch_attention<T, 128, 8>(a, s);
+    else
+        launch_attention<T, 128, 4>(a, s);
 }
 
 }  // namespace svdq
@@ -416,7 +445,7 @@ extern "C" int svdq_attention_fp16(const svdq_attention_args *args, void *stream
     if (a.Tq == 0) return SVDQ_OK;
     const int Tpad = (a.Tkv + AT_BK - 1) / AT_BK * AT_BK;
     if (((size_t)Tpad * a.svn + a.D) * 2 >= ((size_t)1 << 31) || ((size_t)Tpad * a.skn + a.D) * 2 >= ((size_t)1 << 31) ||
-        (size_t)a.B * a.H * ((a.Tq + AT_BQ - 1) / AT_BQ) >= ((size_t)1 << 31)) {
+        (size_t)a.B * a.H * ((a.Tq + 127) / 128) >= ((size_t)1 << 31)) {
         set_error("svdq_attention_fp16: Tq=%d Tkv=%d key / value stride %lld / %lld: too large for 32-bit tile offsets", a.Tq, a.Tkv,
                   (long long)a.skn, (long long)a.svn);
         return SVDQ_E_UNSUPPORTED;
@@ -426,16 +455,9 @@ extern "C" int svdq_attention_fp16(const svdq_attention_args *args, void *stream
         return SVDQ_E_INVALID;
     }
     hipStream_t s = (hipStream_t)stream;
-    if (a.D == 128) {
-        if (a.dtype == SVDQ_BF16)
-            launch_attention<BF16, 128>(a, s);
-        else
-            launch_attention<FP16, 128>(a, s);
-    } else {
-        if (a.dtype == SVDQ_BF16)
-            launch_attention<BF16, 64>(a, s);
-        else
-            launch_attention<FP16, 64>(a, s);
-    }
+    if (a.dtype == SVDQ_BF16)
+        launch_attention<BF16>(a, s);
+    else
+        launch_attention<FP16>(a, s);
     return check_launch("svdq_attention_fp16");
 }

@@ -7,7 +7,7 @@
 // add, clamp, low nibble first.  The LoRA-down product consumes the raw 16-bit activations (before shift and
 // smoothing) on the 16x16x32 MFMA with fp32 accumulation.
 //
-// Work split: one workgroup = 16 (or 32) rows x all of K, eight wavefronts taking scale groups round-robin with two
+// Work split: one workgroup = 16 (or 32) rows x all of K, eight (or, with the norm prologue, sixteen) wavefronts taking scale groups round-robin with two
 // groups in flight each; on the grid's second axis, one workgroup row per chunk of 32 LoRA ranks and, where CUs are
 // left over, up to three rows that only quantize a slice of the groups each.  A group's operands (16 rows x 128 bytes of activations, 32 ranks x 128 bytes of the transposed
 // LoRA-down weight (R, K)) are fetched straight into LDS (buffer_load_dwordx4 ... lds: with a 64-bit address per load, as
@@ -22,6 +22,8 @@
 // the same bytes in its lanes' order, or the same integers as fp6 codes in that order (from the hardware's float -> fp6
 // conversion), with the scales in that order as well.
 #include <algorithm>
+#include <climits>
+#include <type_traits>
 
 #include "svdq_common.h"
 
@@ -31,7 +33,6 @@
 namespace svdq {
 
 constexpr int Q_ROWS = 16;         // rows of one MFMA pass; a workgroup takes QR = 16 or 32 rows (one or two passes)
-constexpr int Q_WAVES = 8;
 constexpr int Q_ROW_BYTES = 128;  // one scale group of one row (64 x 16 bit)
 constexpr int Q_RCHUNK = 32;  // LoRA ranks per pass over the row block
 constexpr int Q_STATS_K = 4096;  // longest row whose statistics the norm prologue computes from registers (two rows to a wavefront)
@@ -127,8 +128,8 @@ __device__ __forceinline__ void row_moments(const uint16_t *const (&row)[NR], in
     for (int n = 0; n < NR; n++) out[n] = make_float2(mean[n], 1.0f / sqrtf(wave_sum(q[n]) / (float)K + eps));
 }
 
-template <typename T, bool UNSIGNED, int PRE, bool HAS_LORA, bool HAS_SMOOTH, bool NORM, int QR>
-__global__ __launch_bounds__(Q_WAVES * 64, QR == 32 ? 1 : (NORM ? 4 : 2)) void quantize_act_kernel(svdq_quantize_args a) {
+template <typename T, bool UNSIGNED, int PRE, bool HAS_LORA, bool HAS_SMOOTH, bool NORM, int QR, int WAVES>
+__global__ __launch_bounds__(WAVES * 64, QR == 32 ? 1 : (NORM ? 4 : 2)) void quantize_act_kernel(svdq_quantize_args a, int split_from, int share) {
     constexpr bool GLU = PRE == SVDQ_PRE_GLU, GELU = PRE == SVDQ_PRE_GELU;
     constexpr int NH = QR / Q_ROWS;  // 16-row halves of the row block: each LoRA-down tile read serves all of them
     // per wavefront: two activation stages (16 rows, + the gate tile with GLU) and one LoRA-down tile (32 ranks), 128
@@ -138,26 +139,31 @@ __global__ __launch_bounds__(Q_WAVES * 64, QR == 32 ? 1 : (NORM ? 4 : 2)) void q
     constexpr int WAVE_BYTES = L_OFF + (HAS_LORA ? Q_RCHUNK * Q_ROW_BYTES : 0);
     // the cross-wave sum after the loop keeps each wavefront's partial products in that wavefront's own (then idle) stages
     static_assert(!HAS_LORA || Q_RCHUNK * (QR + 1) * 4 <= WAVE_BYTES, "partial products do not fit the wavefront's stages");
-    __shared__ __align__(16) uint8_t smem[Q_WAVES * WAVE_BYTES];
-    __shared__ float lds_rs[Q_WAVES][64];
+    __shared__ __align__(16) uint8_t smem[WAVES * WAVE_BYTES];
+    __shared__ float lds_rs[WAVES][64];
     __shared__ float2 lds_st[NORM ? QR : 1];  // (mean, rstd) of the workgroup's rows
-    __shared__ float lds_ns[NORM ? Q_WAVES : 1][64], lds_nh[NORM ? Q_WAVES : 1][64];
+    __shared__ float lds_ns[NORM ? WAVES : 1][64], lds_nh[NORM ? WAVES : 1][64];
     auto lds_acc = [&](int w) { return (float (*)[QR + 1])(smem + w * WAVE_BYTES); };  // [Q_RCHUNK][QR + 1] of wavefront w
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform: keep it in an SGPR
     const int ml = lane & 15;
     const int kq = lane >> 4;
-    const int m0 = blockIdx.x * QR;
+    // Row block, and place on the grid's second axis.  From row block split_from on `share` workgroups of the first axis share a block,
+    // as if they were the second axis of a grid of its own: the last one projects, the others quantize.
+    const bool shared = HAS_LORA && QR == Q_ROWS && (int)blockIdx.x >= split_from;
+    const int over = (int)blockIdx.x - split_from, part = over / share;
+    const int bx = shared ? split_from + part : (int)blockIdx.x, by = shared ? over - part * share : (int)blockIdx.y;
+    const int m0 = bx * QR;
     const int ngroups = a.K / GROUP;
     // The grid's second axis: nq >= 0 workgroup rows that only quantize, each its own slice of the groups (a shorter chain
     // of group steps per wavefront where CUs would otherwise idle), then one row per chunk of 32 ranks.
     const int rchunks = (a.R + Q_RCHUNK - 1) / Q_RCHUNK;
-    const int nq = HAS_LORA ? max((int)gridDim.y - rchunks, 0) : 0;
-    const bool qonly = (int)blockIdx.y < nq;
-    const int g_lo = qonly ? (ngroups * (int)blockIdx.y) / nq : 0, g_hi = qonly ? (ngroups * ((int)blockIdx.y + 1)) / nq : ngroups;
-    const int gw = g_lo + wave;  // this wavefront's groups: gw + Q_WAVES * i < g_hi
-    const int nmy = max((g_hi - gw + Q_WAVES - 1) / Q_WAVES, 0);
+    const int nq = HAS_LORA ? max((shared ? share : (int)gridDim.y) - rchunks, 0) : 0;
+    const bool qonly = by < nq;
+    const int g_lo = qonly ? (ngroups * by) / nq : 0, g_hi = qonly ? (ngroups * (by + 1)) / nq : ngroups;
+    const int gw = g_lo + wave;  // this wavefront's groups: gw + WAVES * i < g_hi
+    const int nmy = max((g_hi - gw + WAVES - 1) / WAVES, 0);
     // Block loads: lane l of load i fetches chunk (l % 8) ^ (l / 8) of tile row 8 i + l / 8 into LDS slot l of that
     // load's 1 KB, i.e. tile[row][chunk ^ (row & 7)].  Rows >= M re-read row M - 1 and ranks >= R rank R - 1 (valid
     // memory; nothing is stored for them).  Addresses = uniform base + 32-bit lane offset (+ uniform group step).
@@ -175,7 +181,8 @@ __global__ __launch_bounds__(Q_WAVES * 64, QR == 32 ? 1 : (NORM ? 4 : 2)) void q
     const uint32_t outoff = (uint32_t)ml * a.ld_out + kq * 8;
     uint16_t *__restrict__ scales = (uint16_t *)a.scales + (size_t)gw * a.ld_scales + m0;
     // scales_blocked: the eight scales of groups 8 j .. 8 j + 7 of a row side by side (16 bytes), 32 rows to a 512-byte block:
-    // group gw + 8 i of row m at ((m / 32) * (ngroups / 8) + gw / 8 + i) * 256 + (m % 32) * 8 + gw % 8
+    // group gw + WAVES i of row m at ((m / 32) * (ngroups / 8) + gw / 8 + WAVES / 8 i) * 256 + (m % 32) * 8 + gw % 8
+    static_assert(WAVES % 8 == 0, "a wavefront's groups have the same place in their block of eight");
     uint16_t *__restrict__ const scalesb = (uint16_t *)a.scales + ((size_t)(m0 >> 5) * (ngroups >> 3) + (gw >> 3)) * 256 + (gw & 7);
     // out_blocked: the 32 packed bytes of (row, group) go where the GEMM's lane (row % 32, half) of that 32-row block and
     // group finds them, [32-row block][group][64 lanes x 16 bytes]: this lane's 8 bytes are half kq / 2, offset 8 (kq % 2)
@@ -203,7 +210,7 @@ __global__ __launch_bounds__(Q_WAVES * 64, QR == 32 ? 1 : (NORM ? 4 : 2)) void q
         f6o16[h] = kq == 0 ? 16u * r + 4u : kq == 1 ? 16u * r + 6u : kq == 2 ? 1024u + 8u * r : 1024u + 8u * r + 2u;
     }
     const uint32_t f6d32 = kq < 3 ? 512u : 256u, f6d16 = kq < 2 ? 512u : 256u;  // from kh = 0 to kh = 1
-    constexpr int GSTEP = Q_WAVES * GROUP;  // elements between consecutive groups of one wavefront
+    constexpr int GSTEP = WAVES * GROUP;  // elements between consecutive groups of one wavefront
     const float qmax = UNSIGNED ? 15.0f : 7.0f;
     const float rmagic = UNSIGNED ? RNE_MAGIC : RNE_MAGIC + 8.0f;  // signed codes are packed as c + 8, then ^ 8
     const bool has_shift = a.shift != 0.0f;
@@ -214,15 +221,18 @@ __global__ __launch_bounds__(Q_WAVES * 64, QR == 32 ? 1 : (NORM ? 4 : 2)) void q
         if (a.norm_stats == nullptr) {
             // the statistics of the workgroup's own rows, two to a wavefront, by the code (and with the bits) of
             // row_stats_kernel: the rows are about to be read anyway, the second time from L2 (when it is the faster way: stats_first)
-            static_assert(Q_ROWS == 2 * Q_WAVES, "two rows of a half to a wavefront");
+            constexpr int NR = Q_ROWS / WAVES;  // rows of a half to a wavefront
 #pragma unroll
             for (int h = 0; h < NH; h++) {
-                const uint16_t *row[2];
-                float2 st[2];
+                const uint16_t *row[NR];
+                float2 st[NR];
 #pragma unroll
-                for (int n = 0; n < 2; n++) row[n] = (const uint16_t *)a.x + (size_t)min(m0 + Q_ROWS * h + 2 * wave + n, a.M - 1) * a.ld_x;
-                row_moments<T, 2, Q_STATS_K / 512>(row, a.K, a.norm_eps, lane, st);
-                if (lane == 0) lds_st[Q_ROWS * h + 2 * wave] = st[0], lds_st[Q_ROWS * h + 2 * wave + 1] = st[1];
+                for (int n = 0; n < NR; n++) row[n] = (const uint16_t *)a.x + (size_t)min(m0 + Q_ROWS * h + NR * wave + n, a.M - 1) * a.ld_x;
+                row_moments<T, NR, Q_STATS_K / 512>(row, a.K, a.norm_eps, lane, st);
+                if (lane == 0) {
+#pragma unroll
+                    for (int n = 0; n < NR; n++) lds_st[Q_ROWS * h + NR * wave + n] = st[n];
+                }
             }
             __syncthreads();
         }
@@ -246,7 +256,7 @@ __global__ __launch_bounds__(Q_WAVES * 64, QR == 32 ? 1 : (NORM ? 4 : 2)) void q
     // then run side by side on different CUs instead of one after the other in every wavefront).
     {
         const bool split = nq > 0;
-        const int rc = max((int)blockIdx.y - nq, 0);
+        const int rc = max(by - nq, 0);
         const bool do_lora = HAS_LORA && !qonly;
         v4f acc0[NH], acc1[NH];
 #pragma unroll
@@ -262,8 +272,8 @@ __global__ __launch_bounds__(Q_WAVES * 64, QR == 32 ? 1 : (NORM ? 4 : 2)) void q
         const bool do_quant = split ? qonly : rc == 0;
 
         constexpr int NX = (GLU ? 4 : 2) * NH;  // block loads of one activation stage
-        auto group_off = [&](int i) {  // byte offset of group wave + Q_WAVES * i in a row; past the end: the last group
-            return (uint32_t)min(gw + Q_WAVES * i, ngroups - 1) * (GROUP * 2);
+        auto group_off = [&](int i) {  // byte offset of group wave + WAVES * i in a row; past the end: the last group
+            return (uint32_t)min(gw + WAVES * i, ngroups - 1) * (GROUP * 2);
         };
         auto issue_x = [&](int i, QVecs &qv) {
             const uint32_t k0 = group_off(i);
@@ -439,11 +449,11 @@ __global__ __launch_bounds__(Q_WAVES * 64, QR == 32 ? 1 : (NORM ? 4 : 2)) void q
                 if (row_ok) {
                     if (kq == 0) {
                         if (a.scales_blocked)
-                            scalesb[(size_t)i * 256 + ((m0 + Q_ROWS * h + ml) & 31) * 8] = T::from_f32(scale);
+                            scalesb[(size_t)i * (WAVES / 8 * 256) + ((m0 + Q_ROWS * h + ml) & 31) * 8] = T::from_f32(scale);
                         else
-                            (scales + (size_t)i * Q_WAVES * a.ld_scales)[Q_ROWS * h + ml] = T::from_f32(scale);
+                            (scales + (size_t)i * WAVES * a.ld_scales)[Q_ROWS * h + ml] = T::from_f32(scale);
                     }
-                    uint8_t *blk = f6base + (size_t)(gw + Q_WAVES * i) * 1536;
+                    uint8_t *blk = f6base + (size_t)(gw + WAVES * i) * 1536;
 #pragma unroll
                     for (int e = 0; e < 2; e++) {
                         const uint32_t d32 = (kq & 1) ? __builtin_amdgcn_alignbit(phi[e], plo[e], 16) : plo[e];
@@ -473,11 +483,11 @@ __global__ __launch_bounds__(Q_WAVES * 64, QR == 32 ? 1 : (NORM ? 4 : 2)) void q
             if (row_ok) {
                 if (kq == 0) {
                     if (a.scales_blocked)
-                        scalesb[(size_t)i * 256 + ((m0 + Q_ROWS * h + ml) & 31) * 8] = T::from_f32(scale);
+                        scalesb[(size_t)i * (WAVES / 8 * 256) + ((m0 + Q_ROWS * h + ml) & 31) * 8] = T::from_f32(scale);
                     else
-                        (scales + (size_t)i * Q_WAVES * a.ld_scales)[Q_ROWS * h + ml] = T::from_f32(scale);
+                        (scales + (size_t)i * WAVES * a.ld_scales)[Q_ROWS * h + ml] = T::from_f32(scale);
                 }
-                uint8_t *dst = a.out_blocked ? bout[h] + (size_t)(gw + Q_WAVES * i) * 1024
+                uint8_t *dst = a.out_blocked ? bout[h] + (size_t)(gw + WAVES * i) * 1024
                                              : outbase + (size_t)i * (GSTEP / 2) + (uint32_t)(Q_ROWS * h) * a.ld_out + outoff;
                 *(uint2 *)dst = make_uint2(w0, w1);
             }
@@ -521,11 +531,11 @@ __global__ __launch_bounds__(Q_WAVES * 64, QR == 32 ? 1 : (NORM ? 4 : 2)) void q
                     mine[16 + 4 * kq + i][Q_ROWS * h + ml] = acc1[h][i];
                 }
             __syncthreads();
-            for (int o = threadIdx.x; o < QR * Q_RCHUNK; o += Q_WAVES * 64) {
+            for (int o = threadIdx.x; o < QR * Q_RCHUNK; o += WAVES * 64) {
                 const int mm = o / Q_RCHUNK, r = o % Q_RCHUNK;
                 float s = lds_acc(0)[r][mm];
 #pragma unroll
-                for (int w = 1; w < Q_WAVES; w++) s += lds_acc(w)[r][mm];
+                for (int w = 1; w < WAVES; w++) s += lds_acc(w)[r][mm];
                 if (m0 + mm < a.M && rc * Q_RCHUNK + r < a.R)
                     a.lora_act[(size_t)(m0 + mm) * a.ld_lora_act + rc * Q_RCHUNK + r] = s;
             }
@@ -635,6 +645,29 @@ __global__ void transpose_kr_kernel(const uint16_t *in, uint16_t *out, int K, in
 
 static bool has_norm(const svdq_quantize_args &a) { return a.norm_stats || a.norm_eps > 0.0f; }
 
+static int device_cus() {
+    static int cus = 0;
+    if (!cus) {
+        int dev = 0, n = 0;
+        cus = hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0 ? n : 256;
+    }
+    return cus;
+}
+
+// Workgroups that share each of the row blocks behind the last whole round of one 16-row workgroup to a CU (1: none do).  A round that
+// is nearly empty otherwise takes as long as a full one: its workgroups run beside another on a few CUs while the rest idle.  Four to
+// a block where all of them find a CU to themselves, three up to a third of the CUs: us, before / now (K = 3072, R = 32, bf16; norm
+// prologue with its own statistics | with given ones | without): 4100 rows 20.6 / 16.9 | 17.1 / 13.4 | 15.6 / 11.3, 4608 21.9 / 18.8 |
+// 18.5 / 15.6 | 14.1 / 13.0, 5120 22.4 / 21.5 | 18.5 / 15.5 | 14.3 / 13.7, 5400 22.8 / 22.2 | 18.6 / 15.7 | 14.6 / 14.0, 8704 34.9 / 31.7 |
+// 26.2 / 22.4 | 22.0 / 19.5.  Two to a block (5632 rows 22.9 / 24.0 | 19.0 / 17.6 | 14.8 / 14.4, K = 4096 10240 46.2 / 47.8 | 33.6 / 35.2 | 28.9 /
+// 29.6) do not pay for the prologue that both compute.
+static int quantize_share(const svdq_quantize_args &a) {
+    const int blocks = (a.M + Q_ROWS - 1) / Q_ROWS, cus = device_cus(), left = blocks % cus;
+    if (a.R == 0 || a.R > Q_RCHUNK || blocks <= cus || left == 0 || a.prologue != SVDQ_PRE_NONE) return 1;
+    const int share = std::min({4, cus / left, a.K / GROUP});
+    return share >= 3 ? share : 1;
+}
+
 // Rows per workgroup.  A workgroup streams 4 KB of LoRA-down weight per group whatever its number of rows, and the
 // vector memory pipe of a CU is what that traffic is bound by: with 16-row workgroups, M = 4608 puts two of them on 32 of
 // the 256 CUs and the launch waits for those.  32-row workgroups (one LoRA-down tile read for two MFMA passes; a longer
@@ -645,16 +678,8 @@ static int quantize_rows_per_workgroup(const svdq_quantize_args &a) {
     if (a.R == 0 || a.prologue != SVDQ_PRE_NONE) return Q_ROWS;
     if (has_norm(a)) return Q_ROWS;  // twice the arithmetic per value: 23.2 against 25.2 us at M = 4608, 27.5 against 28.3 at 8192
     const int wg16 = (a.M + 15) / 16;
+    if (quantize_share(a) > 1) return Q_ROWS;
     return (wg16 > Q32_ABOVE && wg16 <= Q32_UPTO) ? 32 : Q_ROWS;
-}
-
-static int device_cus() {
-    static int cus = 0;
-    if (!cus) {
-        int dev = 0, n = 0;
-        cus = hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0 ? n : 256;
-    }
-    return cus;
 }
 
 // Second grid axis: one workgroup row per chunk of 32 ranks, plus rows that only quantize where that still leaves about
@@ -667,11 +692,10 @@ static int device_cus() {
 static int quantize_grid_y(const svdq_quantize_args &a, int row_blocks, int rows) {
     if (a.R == 0) return 1;
     const int chunks = (a.R + Q_RCHUNK - 1) / Q_RCHUNK, cus = device_cus();
-    // (with a prologue the workgroups that only project compute it a second time: only where half the CUs would idle
-    // anyway.  That was the better limit while the row statistics had a launch of their own; all of the CUs is now.  Norm prologue, K = 3072, R = 32, with half of the CUs / all of them as the limit: M = 512 11.0 / 11.0 us, 1024 13.6 /
-    // 12.0, 2048 15.3 / 14.2, 4096 16.7 / 16.2, 4608 23.2 / 22.7)
-    const bool prologue = has_norm(a) || a.prologue != SVDQ_PRE_NONE;
-    const int limit = prologue ? cus / 2 : cus + (rows == 32 ? cus / 8 : 0);
+    // (with a GLU or GELU prologue the workgroups that only project compute it a second time: only where half the CUs would idle
+    // anyway.  With the norm prologue, of sixteen wavefronts, up to all of the CUs: K = 3072, R = 32, limits of a half / all of them 1024
+    // rows 11.5 / 10.6 us, 1201 12.7 / 10.7, 2048 13.3 / 12.3; R = 128 512 rows 12.5 / 10.4)
+    const int limit = has_norm(a) ? cus : a.prologue != SVDQ_PRE_NONE ? cus / 2 : cus + (rows == 32 ? cus / 8 : 0);
     if (row_blocks * (chunks + 1) > limit) return chunks;
     const int nq = std::min({3, limit / row_blocks - chunks, a.K / GROUP});
     return chunks + std::max(nq, 1);
@@ -692,27 +716,44 @@ static bool stats_first(const svdq_quantize_args &a) {
 
 template <typename T, bool U, int G, bool NORM>
 static void launch_quantize3(const svdq_quantize_args &a, hipStream_t s) {
-    const dim3 block(Q_WAVES * 64);
     const bool lora = a.R > 0, sm = a.smooth != nullptr;
     if constexpr (G == SVDQ_PRE_NONE) {
         if (quantize_rows_per_workgroup(a) == 32) {
             const dim3 grid((a.M + 31) / 32, quantize_grid_y(a, (a.M + 31) / 32, 32));
             if (sm)
-                hipLaunchKernelGGL((quantize_act_kernel<T, U, G, true, true, NORM, 32>), grid, block, 0, s, a);
+                hipLaunchKernelGGL((quantize_act_kernel<T, U, G, true, true, NORM, 32, 8>), grid, dim3(512), 0, s, a, INT_MAX, 1);
             else
-                hipLaunchKernelGGL((quantize_act_kernel<T, U, G, true, false, NORM, 32>), grid, block, 0, s, a);
+                hipLaunchKernelGGL((quantize_act_kernel<T, U, G, true, false, NORM, 32, 8>), grid, dim3(512), 0, s, a, INT_MAX, 1);
             return;
         }
     }
-    const dim3 grid((a.M + Q_ROWS - 1) / Q_ROWS, quantize_grid_y(a, (a.M + Q_ROWS - 1) / Q_ROWS, Q_ROWS));
-    if (lora && sm)
-        hipLaunchKernelGGL((quantize_act_kernel<T, U, G, true, true, NORM, 16>), grid, block, 0, s, a);
-    else if (lora)
-        hipLaunchKernelGGL((quantize_act_kernel<T, U, G, true, false, NORM, 16>), grid, block, 0, s, a);
-    else if (sm)
-        hipLaunchKernelGGL((quantize_act_kernel<T, U, G, false, true, NORM, 16>), grid, block, 0, s, a);
-    else
-        hipLaunchKernelGGL((quantize_act_kernel<T, U, G, false, false, NORM, 16>), grid, block, 0, s, a);
+    const dim3 full((a.M + Q_ROWS - 1) / Q_ROWS, quantize_grid_y(a, (a.M + Q_ROWS - 1) / Q_ROWS, Q_ROWS));
+    auto go = [&](auto wtag) {
+        constexpr int W = decltype(wtag)::value;
+        const dim3 block(W * 64);
+        const int share = W == 16 ? 1 : quantize_share(a), split_from = share > 1 ? (int)full.x / device_cus() * device_cus() : INT_MAX;
+        const dim3 grid = share > 1 ? dim3(split_from + share * (full.x - split_from)) : full;
+        if (lora && sm)
+            hipLaunchKernelGGL((quantize_act_kernel<T, U, G, true, true, NORM, 16, W>), grid, block, 0, s, a, split_from, share);
+        else if (lora)
+            hipLaunchKernelGGL((quantize_act_kernel<T, U, G, true, false, NORM, 16, W>), grid, block, 0, s, a, split_from, share);
+        else if (sm)
+            hipLaunchKernelGGL((quantize_act_kernel<T, U, G, false, true, NORM, 16, W>), grid, block, 0, s, a, split_from, share);
+        else
+            hipLaunchKernelGGL((quantize_act_kernel<T, U, G, false, false, NORM, 16, W>), grid, block, 0, s, a, split_from, share);
+    };
+    if constexpr (NORM) {
+        // One workgroup to a CU at most: sixteen wavefronts, whose chains of group steps are half as long and of which each takes the
+        // statistics of one row.  us, eight / sixteen (K = 3072, R = 32): 333 rows 10.3 / 9.8, 1201 14.0 / 12.7, 4096 15.8 / 15.0; K = 4096: 1201
+        // rows 17.1 / 15.3.  Two of them do not fit a CU's LDS (4608 rows 22.4 / 26.1), and without the prologue they are slower (1024 rows
+        // 5.4 / 6.3).  Short rows: with given statistics K = 1024 512 rows 4.6 / 5.0, 4096 6.3 / 6.5, K = 1536 1024 rows 6.5 / 5.9 (the line is the
+        // same with its own, for the same bits).
+        if (a.K >= 1536 && (long)full.x * full.y <= device_cus()) {
+            go(std::integral_constant<int, 16>{});
+            return;
+        }
+    }
+    go(std::integral_constant<int, 8>{});
 }
 
 template <typename T, bool U, int G>

@@ -355,3 +355,45 @@ def test_full_size_invariants(dev):
     codes = O.unpack_int4(q0.cpu(), True).view(M, K // 64, 64)
     nz = s0.cpu().t().float() != 0
     assert bool((codes.abs().amax(dim=2)[nz] == 7).all()) and int(codes.min()) >= -7
+
+
+@pytest.mark.parametrize("norm", [False, True, "given"])
+@pytest.mark.parametrize("M,K,R", [(333, 2048, 64), (1201, 3072, 48), (2048, 1536, 32), (2064, 1536, 32), (4096, 1536, 16), (2048, 1472, 32), (4097, 256, 32), (4100, 192, 32), (4112, 128, 32), (5120, 320, 32),
+                                   (5136, 512, 16), (5456, 256, 32), (5457, 256, 32), (8208, 512, 32), (4112, 256, 48)])  # fmt: skip
+def test_row_blocks_behind_the_last_whole_round(dev, M, K, R, norm):
+    """On 256 CUs: sixteen wavefronts with the norm prologue up to one workgroup to a CU (4096 rows; 2048: with rows that only quantize)
+    from K = 1536 on, four (to 5120 rows) and three (to 5456) workgroups to a block of the rest, not with fewer groups than that
+    (192) or a second chunk of ranks -- against the same rows, normalised before, a few blocks at a time, which take none of these routes."""
+    from nunchaku_rocm_amd import ops
+    from nunchaku_rocm_amd.layout import block_scales
+
+    print(f"case M={M} K={K} R={R} norm={norm}", flush=True)
+    g = torch.Generator().manual_seed(M + K)
+    T = torch.bfloat16
+    x = O.make_activations(M, K, seed=M, dtype=T).to(dev)
+    down, smooth = (torch.randn(K, R, generator=g) * 0.02).to(T).to(dev), (torch.rand(K, generator=g) + 0.5).to(T).to(dev)
+    scale, shift = (1 + 0.3 * torch.randn(K, generator=g)).to(T).to(dev), (0.2 * torch.randn(K, generator=g)).to(T).to(dev)
+    vecs, xm = None, x
+    if norm:
+        stats = ops.layer_norm_stats(x)
+        vecs = (scale, shift, stats) if norm == "given" else (scale, shift)
+        xm = ((x.float() - stats[:, :1]) * stats[:, 1:]).to(T)
+        xm = ((xm.float() * scale.float()).to(T).float() + shift.float()).to(T)
+
+    def run(rows, blocked, norm=None):
+        return ops.svdq_quantize_w4a4_act_fuse_lora_cuda(rows, lora_down=down, smooth=smooth, norm=norm, pad_size=32, out_blocked=blocked)
+
+    unblocked = None
+    for blocked in (0, 2, 3) if K % 512 == 0 else (0, 2):
+        codes, scales, la = run(x, blocked, vecs)
+        if blocked == 3:
+            full = M // 32 * 32
+            assert torch.equal(scales.view(-1)[: full * K // 64].cpu(), block_scales(unblocked.cpu()).view(-1)[: full * K // 64])
+        unblocked = scales
+        for i in range(0, M, 1024):
+            n = min(1024, M - i)
+            c, s, a = run(xm[i : i + n], blocked)
+            whole = n // 32 * 32 if blocked else n  # (rows of the padding are not written)
+            assert torch.equal(codes[i : i + whole], c[:whole]) and (blocked == 3 or torch.equal(scales[:, i : i + n], s[:, :n]))
+            # fp32 sums of K products in another order
+            assert ((la[i : i + n] - a[:n]).abs() <= K * 2.0**-23 * (xm[i : i + n].float().abs().amax() * down.float().abs().sum(0)) + 1e-6).all()

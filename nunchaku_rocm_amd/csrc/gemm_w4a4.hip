@@ -988,13 +988,15 @@ extern "C" int svdq_gemm_w4a4_split_wavefronts(const svdq_gemm_args *args, int32
 // us as they are / re-laid-out (bf16, signed, rank 32):
 //   few rows (K split over wavefronts), eight of them: as long as there are fewer rows than K: 256 x 3072 K = 1024 10.8 / 9.8, K = 3072 22.4 /
 //     14.1, K = 512 7.9 / 8.8;  K = 1024, 1024 columns, 512 rows 11.3 / 10.6, 1024 rows 11.4 / 11.5;  K = 2048, 256 columns, 3072 rows 17.5 / 18.1
-//   four: up to K / 4 rows: K = 2048, 256 x 6144 16.8 / 15.7, 1024 x 1536 17.1 / 18.1;  K = 3072, 512 x 3072 22.5 / 20.0, 1344 x 1536 23.1 /
-//     23.8;  from K = 4096 up to 2 K / 3: K = 4608, 1344 x 1536 32.9 / 28.8, 8192 x 256 1.06 of the time
-//   more than two 128-row tiles to a CU: K = 2048, 1536 x 6144 33.2 / 29.0, 8192 x 1536 37.2 / 38.7;  K = 3072, 4608 x 9216 168 / 132, 8192 x 1536
-//     52.7 / 48.5, 16384 x 1024 0.92, 32768 x 512 1.04;  K = 1536, 8192 x 1536 29.6 / 31.7;  fewer: K = 3072, 1536 x 3072 32.1 / 31.4, 1024 x 3072
-//     22.7 / 24.5
-//   K = 6144: 768 x 3072 41.7 / 40.1, 4608 x 3072 117 / 93, 3072 x 1536 (288 tiles) 59.0 / 55.1, 2048 x 1536 (192) 42.4 / 43.8;  K = 12288, 2048 x
-//     1536 78.2 / 73.4
+//   four (quantizer and GEMM together, re-laid-out / as they are): up to K / 4 rows: K = 1536 333 x 3072 0.87, 256 x 4608 0.89, 512 x 4608 1.01;  K = 2048
+//     768 x 1536 0.86, 1536 x 1536 1.02;  from K = 3584 up to 2 K / 3: K = 3584 1024 x 1536 0.77, 1344 x 1536 0.76, 6144 x 512
+//     1.08;  K = 4608 4096 x 512 0.83, 6144 x 512 1.06
+//   more than two 128-row tiles to a CU (together, as above): K = 1024 3072 x 4608 0.90, 1344 x 6144 0.92, 1024 x 9216 0.91, 4096 x 3072 1.03;  K = 1536 3072
+//     x 3072 0.91, 2048 x 4608 0.91, 4608 columns and more 0.80 to 0.93, 8192 x 1536 0.95, 4096 x 2048 1.08;  K = 2048 8192 x 1536 0.95;  unsigned K = 1024
+//     1024 x 9216 0.96, 4096 0.91, K = 1536 3072 x 3072 0.96
+//   more than one: K = 3584 1344 x 3072 0.90, 3072 x 1536 0.92, 333 x 12288 0.89;  K = 4608 1344 x 3072 0.88;  unsigned 0.95 to 0.98;  one at most: K = 3584
+//     512 x 4608 0.97, 768 x 3072 1.00;  K = 3072 1536 x 3072 0.91, 768 x 3072 1.01, 512 x 4608 0.99 (the line lies above them)
+//   K = 6144: 768 x 3072 41.7 / 40.1, 4608 x 3072 117 / 93, 2048 x 1536 (192 tiles) 42.4 / 43.8;  K = 12288, 2048 x 1536 78.2 / 73.4
 // Unsigned activations of few rows split their K as they are (split_of); beyond those 1536 x 9216 at K = 3072 58.4 / 51.2.  (The
 // grid of the pass is two-dimensional: 2^20 rows keep it inside 65536.)
 static size_t act_scratch_bytes(const svdq_gemm_args &a, int cus) {
@@ -1008,9 +1010,10 @@ static size_t act_scratch_bytes(const svdq_gemm_args &a, int cus) {
     bool pays;
     switch (split_wavefronts(b, cus)) {
         case 8: pays = K >= 1024 && rows < K; break;
-        case 4: pays = K >= 2048 && (K >= 4096 ? 3 * rows <= 2 * K : 4 * rows <= K); break;
+        case 4: pays = K >= 1536 && (K >= 3584 ? 3 * rows <= 2 * K : 4 * rows <= K); break;
         default:
-            pays = N >= 1024 && ((tiles > 2L * cus && K >= (N >= 2048 ? 2048 : 3072)) || (K >= 6144 && (tiles > cus || K * N >= 1 << 24)));
+            pays = N >= 1024 && ((tiles > 2L * cus && K >= (N >= 4608 ? 1024 : N >= 3072 ? 1536 : N >= 2048 ? 2048 : 3072)) || (K >= 3584 && tiles > cus) ||
+                                 (K >= 6144 && K * N >= 1 << 24));
     }
     if (!pays) return 0;
     const size_t padded = (size_t)((a.M + 31) / 32 * 32);

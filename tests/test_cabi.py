@@ -123,6 +123,18 @@ def test_when_nibbles_are_relaid_out(lib):
     assert lib.svdq_gemm_w4a4_act_scratch_bytes(None) == 0
 
 
+def test_lines_of_the_pass_over_nibbles(lib):
+    """256 CUs, signed codes: both sides of the lines in K, in rows and in columns."""
+    from nunchaku_rocm_amd import _lib
+
+    for rows, n, k, want in (
+        (384, 3072, 1536, 1), (385, 3072, 1536, 0), (2048, 1024, 3584, 1), (4096, 512, 3584, 0), (333, 12288, 3584, 1), (256, 16384, 3584, 0), (333, 12288, 3072, 0),
+        (4608, 3072, 1536, 1), (4608, 2944, 1536, 0), (4608, 4608, 1024, 1), (4608, 4480, 1024, 0), (4608, 9216, 512, 0),
+    ):  # fmt: skip
+        nbytes = lib.svdq_gemm_w4a4_act_scratch_bytes(_lib.GemmArgs(wgt_planes=16, M=rows, actual_m=rows, N=n, K=k, R=32))
+        assert bool(nbytes) == bool(want), (rows, n, k)
+
+
 def test_no_memory_for_relaid_out_nibbles_is_an_error(lib, monkeypatch):
     """What a call computes does not depend on whether an allocation succeeds."""
     from nunchaku_rocm_amd import _lib

@@ -672,8 +672,9 @@ static int quantize_share(const svdq_quantize_args &a) {
 // vector memory pipe of a CU is what that traffic is bound by: with 16-row workgroups, M = 4608 puts two of them on 32 of
 // the 256 CUs and the launch waits for those.  32-row workgroups (one LoRA-down tile read for two MFMA passes; a longer
 // chain per wavefront, 12 us even for one workgroup per CU) are faster where the 16-row grid needs between one and two
-// workgroups per CU: 13.4 against 14.2 us at M = 4608, 14.6 against 15.5 at 6144, 16.2 against 16.7 at 8192 (K = 3072,
-// R = 32); below and above that range the 16-row kernel wins.
+// workgroups per CU and too many blocks are left behind the last whole round for them to be shared (quantize_share; 4608 rows 13.0 us
+// shared, 14.1 with 32-row workgroups): 14.6 against 15.5 us at M = 6144, 16.2 against 16.7 at 8192 (K = 3072, R = 32); below and above
+// that range the 16-row kernel wins.
 static int quantize_rows_per_workgroup(const svdq_quantize_args &a) {
     if (a.R == 0 || a.prologue != SVDQ_PRE_NONE) return Q_ROWS;
     if (has_norm(a)) return Q_ROWS;  // twice the arithmetic per value: 23.2 against 25.2 us at M = 4608, 27.5 against 28.3 at 8192

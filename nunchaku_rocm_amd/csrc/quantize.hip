@@ -7,8 +7,8 @@
 // add, clamp, low nibble first.  The LoRA-down product consumes the raw 16-bit activations (before shift and
 // smoothing) on the 16x16x32 MFMA with fp32 accumulation.
 //
-// Work split: one workgroup = 16 (or 32) rows x all of K, eight (or, with the norm prologue, sixteen) wavefronts taking scale groups round-robin with two
-// groups in flight each; on the grid's second axis, one workgroup row per chunk of 32 LoRA ranks and, where CUs are
+// Work split: one workgroup = 16 (or 32) rows x all of K, eight wavefronts taking scale groups round-robin with two groups in flight each (sixteen
+// in workgroups that only quantize behind the norm prologue); on the grid's second axis, one workgroup row per chunk of 32 LoRA ranks and, where CUs are
 // left over, up to three rows that only quantize a slice of the groups each.  A group's operands (16 rows x 128 bytes of activations, 32 ranks x 128 bytes of the transposed
 // LoRA-down weight (R, K)) are fetched straight into LDS (buffer_load_dwordx4 ... lds: with a 64-bit address per load, as
 // global_load_lds, the norm prologue's launch took 17.0 instead of 15.7 us at 4096 x 3072) by loads whose 64 lanes cover eight
@@ -35,6 +35,7 @@ namespace svdq {
 constexpr int Q_ROWS = 16;         // rows of one MFMA pass; a workgroup takes QR = 16 or 32 rows (one or two passes)
 constexpr int Q_ROW_BYTES = 128;  // one scale group of one row (64 x 16 bit)
 constexpr int Q_RCHUNK = 32;  // LoRA ranks per pass over the row block
+constexpr int Q_CHAINS = 8;   // partial sums of a lora_act value: that of groups c, c + 8, .. in order for c = 0 .. 7, added up in order
 constexpr int Q_STATS_K = 4096;  // longest row whose statistics the norm prologue computes from registers (two rows to a wavefront)
 constexpr int Q32_ABOVE = 256, Q32_UPTO = 512;  // number of 16-row workgroups for which 32-row workgroups are used instead
 
@@ -139,7 +140,11 @@ __global__ __launch_bounds__(WAVES * 64, QR == 32 ? 1 : (NORM ? 4 : 2)) void qua
     constexpr int WAVE_BYTES = L_OFF + (HAS_LORA ? Q_RCHUNK * Q_ROW_BYTES : 0);
     // the cross-wave sum after the loop keeps each wavefront's partial products in that wavefront's own (then idle) stages
     static_assert(!HAS_LORA || Q_RCHUNK * (QR + 1) * 4 <= WAVE_BYTES, "partial products do not fit the wavefront's stages");
-    __shared__ __align__(16) uint8_t smem[WAVES * WAVE_BYTES];
+    // A workgroup that projects takes its groups with eight wavefronts also where it has sixteen (the others take part in the row
+    // statistics): a row's lora_act is the same sums in the same order whatever rows stand beside it.
+    constexpr bool WIDE = HAS_LORA && WAVES > Q_CHAINS;
+    static_assert(!HAS_LORA || WAVES % Q_CHAINS == 0, "a wavefront to a partial sum");
+    __shared__ __align__(16) uint8_t smem[WIDE ? (WAVES * L_OFF > Q_CHAINS * WAVE_BYTES ? WAVES * L_OFF : Q_CHAINS * WAVE_BYTES) : WAVES * WAVE_BYTES];
     __shared__ float lds_rs[WAVES][64];
     __shared__ float2 lds_st[NORM ? QR : 1];  // (mean, rstd) of the workgroup's rows
     __shared__ float lds_ns[NORM ? WAVES : 1][64], lds_nh[NORM ? WAVES : 1][64];
@@ -162,8 +167,9 @@ __global__ __launch_bounds__(WAVES * 64, QR == 32 ? 1 : (NORM ? 4 : 2)) void qua
     const int nq = HAS_LORA ? max((shared ? share : (int)gridDim.y) - rchunks, 0) : 0;
     const bool qonly = by < nq;
     const int g_lo = qonly ? (ngroups * by) / nq : 0, g_hi = qonly ? (ngroups * (by + 1)) / nq : ngroups;
-    const int gw = g_lo + wave;  // this wavefront's groups: gw + WAVES * i < g_hi
-    const int nmy = max((g_hi - gw + WAVES - 1) / WAVES, 0);
+    const int gwaves = WIDE && !qonly ? Q_CHAINS : WAVES;  // wavefronts that take groups
+    const int gw = g_lo + wave;                            // this wavefront's groups: gw + gwaves * i < g_hi
+    const int nmy = wave < gwaves ? max((g_hi - gw + gwaves - 1) / gwaves, 0) : 0;
     // Block loads: lane l of load i fetches chunk (l % 8) ^ (l / 8) of tile row 8 i + l / 8 into LDS slot l of that
     // load's 1 KB, i.e. tile[row][chunk ^ (row & 7)].  Rows >= M re-read row M - 1 and ranks >= R rank R - 1 (valid
     // memory; nothing is stored for them).  Addresses = uniform base + 32-bit lane offset (+ uniform group step).
@@ -175,13 +181,13 @@ __global__ __launch_bounds__(WAVES * 64, QR == 32 ? 1 : (NORM ? 4 : 2)) void qua
     for (int i = 0; i < 2 * NH; i++) xdma[i] = (uint32_t)(min(m0 + 8 * i + drow, a.M - 1) - m0) * a.ld_x * 2 + dchunk * 16;
     // read-back: lane (m, q) takes chunks 2 q and 2 q + 1 of tile row m (and of row m + 16 of the LoRA-down tile)
     const int rd_lo = ml * Q_ROW_BYTES + (((2 * kq) ^ (ml & 7)) * 16), rd_hi = ml * Q_ROW_BYTES + (((2 * kq + 1) ^ (ml & 7)) * 16);
-    uint8_t *const wbase = smem + wave * WAVE_BYTES;
+    uint8_t *const wbase = smem + wave * (WIDE && qonly ? L_OFF : WAVE_BYTES);
     const uint16_t *__restrict__ smooth = (const uint16_t *)a.smooth;
     uint8_t *__restrict__ outbase = (uint8_t *)a.out + (size_t)m0 * a.ld_out + gw * (GROUP / 2);
     const uint32_t outoff = (uint32_t)ml * a.ld_out + kq * 8;
     uint16_t *__restrict__ scales = (uint16_t *)a.scales + (size_t)gw * a.ld_scales + m0;
     // scales_blocked: the eight scales of groups 8 j .. 8 j + 7 of a row side by side (16 bytes), 32 rows to a 512-byte block:
-    // group gw + WAVES i of row m at ((m / 32) * (ngroups / 8) + gw / 8 + WAVES / 8 i) * 256 + (m % 32) * 8 + gw % 8
+    // group gw + gwaves i of row m at ((m / 32) * (ngroups / 8) + gw / 8 + gwaves / 8 i) * 256 + (m % 32) * 8 + gw % 8
     static_assert(WAVES % 8 == 0, "a wavefront's groups have the same place in their block of eight");
     uint16_t *__restrict__ const scalesb = (uint16_t *)a.scales + ((size_t)(m0 >> 5) * (ngroups >> 3) + (gw >> 3)) * 256 + (gw & 7);
     // out_blocked: the 32 packed bytes of (row, group) go where the GEMM's lane (row % 32, half) of that 32-row block and
@@ -210,7 +216,6 @@ __global__ __launch_bounds__(WAVES * 64, QR == 32 ? 1 : (NORM ? 4 : 2)) void qua
         f6o16[h] = kq == 0 ? 16u * r + 4u : kq == 1 ? 16u * r + 6u : kq == 2 ? 1024u + 8u * r : 1024u + 8u * r + 2u;
     }
     const uint32_t f6d32 = kq < 3 ? 512u : 256u, f6d16 = kq < 2 ? 512u : 256u;  // from kh = 0 to kh = 1
-    constexpr int GSTEP = WAVES * GROUP;  // elements between consecutive groups of one wavefront
     const float qmax = UNSIGNED ? 15.0f : 7.0f;
     const float rmagic = UNSIGNED ? RNE_MAGIC : RNE_MAGIC + 8.0f;  // signed codes are packed as c + 8, then ^ 8
     const bool has_shift = a.shift != 0.0f;
@@ -219,7 +224,7 @@ __global__ __launch_bounds__(WAVES * 64, QR == 32 ? 1 : (NORM ? 4 : 2)) void qua
     const uint16_t *__restrict__ nscale = nullptr, *__restrict__ nshift = nullptr;
     if (NORM) {
         if (a.norm_stats == nullptr) {
-            // the statistics of the workgroup's own rows, two to a wavefront, by the code (and with the bits) of
+            // the statistics of the workgroup's own rows, one or two to a wavefront, by the code (and with the bits) of
             // row_stats_kernel: the rows are about to be read anyway, the second time from L2 (when it is the faster way: stats_first)
             constexpr int NR = Q_ROWS / WAVES;  // rows of a half to a wavefront
 #pragma unroll
@@ -272,8 +277,8 @@ __global__ __launch_bounds__(WAVES * 64, QR == 32 ? 1 : (NORM ? 4 : 2)) void qua
         const bool do_quant = split ? qonly : rc == 0;
 
         constexpr int NX = (GLU ? 4 : 2) * NH;  // block loads of one activation stage
-        auto group_off = [&](int i) {  // byte offset of group wave + WAVES * i in a row; past the end: the last group
-            return (uint32_t)min(gw + WAVES * i, ngroups - 1) * (GROUP * 2);
+        auto group_off = [&](int i) {  // byte offset of group wave + gwaves * i in a row; past the end: the last group
+            return (uint32_t)min(gw + gwaves * i, ngroups - 1) * (GROUP * 2);
         };
         auto issue_x = [&](int i, QVecs &qv) {
             const uint32_t k0 = group_off(i);
@@ -449,11 +454,11 @@ __global__ __launch_bounds__(WAVES * 64, QR == 32 ? 1 : (NORM ? 4 : 2)) void qua
                 if (row_ok) {
                     if (kq == 0) {
                         if (a.scales_blocked)
-                            scalesb[(size_t)i * (WAVES / 8 * 256) + ((m0 + Q_ROWS * h + ml) & 31) * 8] = T::from_f32(scale);
+                            scalesb[(size_t)(i * gwaves) * 32 + ((m0 + Q_ROWS * h + ml) & 31) * 8] = T::from_f32(scale);
                         else
-                            (scales + (size_t)i * WAVES * a.ld_scales)[Q_ROWS * h + ml] = T::from_f32(scale);
+                            (scales + (size_t)i * gwaves * a.ld_scales)[Q_ROWS * h + ml] = T::from_f32(scale);
                     }
-                    uint8_t *blk = f6base + (size_t)(gw + WAVES * i) * 1536;
+                    uint8_t *blk = f6base + (size_t)(gw + gwaves * i) * 1536;
 #pragma unroll
                     for (int e = 0; e < 2; e++) {
                         const uint32_t d32 = (kq & 1) ? __builtin_amdgcn_alignbit(phi[e], plo[e], 16) : plo[e];
@@ -483,12 +488,12 @@ __global__ __launch_bounds__(WAVES * 64, QR == 32 ? 1 : (NORM ? 4 : 2)) void qua
             if (row_ok) {
                 if (kq == 0) {
                     if (a.scales_blocked)
-                        scalesb[(size_t)i * (WAVES / 8 * 256) + ((m0 + Q_ROWS * h + ml) & 31) * 8] = T::from_f32(scale);
+                        scalesb[(size_t)(i * gwaves) * 32 + ((m0 + Q_ROWS * h + ml) & 31) * 8] = T::from_f32(scale);
                     else
-                        (scales + (size_t)i * WAVES * a.ld_scales)[Q_ROWS * h + ml] = T::from_f32(scale);
+                        (scales + (size_t)i * gwaves * a.ld_scales)[Q_ROWS * h + ml] = T::from_f32(scale);
                 }
-                uint8_t *dst = a.out_blocked ? bout[h] + (size_t)(gw + WAVES * i) * 1024
-                                             : outbase + (size_t)i * (GSTEP / 2) + (uint32_t)(Q_ROWS * h) * a.ld_out + outoff;
+                uint8_t *dst = a.out_blocked ? bout[h] + (size_t)(gw + gwaves * i) * 1024
+                                             : outbase + (size_t)(i * gwaves) * (GROUP / 2) + (uint32_t)(Q_ROWS * h) * a.ld_out + outoff;
                 *(uint2 *)dst = make_uint2(w0, w1);
             }
             }  // halves
@@ -500,9 +505,11 @@ __global__ __launch_bounds__(WAVES * 64, QR == 32 ? 1 : (NORM ? 4 : 2)) void qua
         // group's LoRA-down tile, the activations two groups on), then compute from the registers.
         QVecs sm_a = {0, 0, 0}, sm_b = {0, 0, 0};
         Ops ops;
-        issue_x(0, sm_a);
-        issue_l(0);
-        issue_x(1, sm_b);
+        if (!WIDE || wave < gwaves) {
+            issue_x(0, sm_a);
+            issue_l(0);
+            issue_x(1, sm_b);
+        }
         auto step = [&](int i, QVecs &sm) {
             // group i's activations and LoRA-down tile have landed: the loads issued after them are at least the NX
             // block loads of group i + 1's activations
@@ -522,20 +529,22 @@ __global__ __launch_bounds__(WAVES * 64, QR == 32 ? 1 : (NORM ? 4 : 2)) void qua
 
         if (do_lora) {
             // fixed-order sum of the wavefronts' partial products (this wavefront is done with its own stages)
-            float (*mine)[QR + 1] = lds_acc(wave);
+            if (!WIDE || wave < Q_CHAINS) {
+                float (*mine)[QR + 1] = lds_acc(wave);
 #pragma unroll
-            for (int h = 0; h < NH; h++)
+                for (int h = 0; h < NH; h++)
 #pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    mine[4 * kq + i][Q_ROWS * h + ml] = acc0[h][i];
-                    mine[16 + 4 * kq + i][Q_ROWS * h + ml] = acc1[h][i];
-                }
+                    for (int i = 0; i < 4; i++) {
+                        mine[4 * kq + i][Q_ROWS * h + ml] = acc0[h][i];
+                        mine[16 + 4 * kq + i][Q_ROWS * h + ml] = acc1[h][i];
+                    }
+            }
             __syncthreads();
             for (int o = threadIdx.x; o < QR * Q_RCHUNK; o += WAVES * 64) {
                 const int mm = o / Q_RCHUNK, r = o % Q_RCHUNK;
                 float s = lds_acc(0)[r][mm];
 #pragma unroll
-                for (int w = 1; w < WAVES; w++) s += lds_acc(w)[r][mm];
+                for (int w = 1; w < Q_CHAINS; w++) s += lds_acc(w)[r][mm];
                 if (m0 + mm < a.M && rc * Q_RCHUNK + r < a.R)
                     a.lora_act[(size_t)(m0 + mm) * a.ld_lora_act + rc * Q_RCHUNK + r] = s;
             }
@@ -744,12 +753,14 @@ static void launch_quantize3(const svdq_quantize_args &a, hipStream_t s) {
             hipLaunchKernelGGL((quantize_act_kernel<T, U, G, false, false, NORM, 16, W>), grid, block, 0, s, a, split_from, share);
     };
     if constexpr (NORM) {
-        // One workgroup to a CU at most: sixteen wavefronts, whose chains of group steps are half as long and of which each takes the
-        // statistics of one row.  us, eight / sixteen (K = 3072, R = 32): 333 rows 10.3 / 9.8, 1201 14.0 / 12.7, 4096 15.8 / 15.0; K = 4096: 1201
-        // rows 17.1 / 15.3.  Two of them do not fit a CU's LDS (4608 rows 22.4 / 26.1), and without the prologue they are slower (1024 rows
-        // 5.4 / 6.3).  Short rows: with given statistics K = 1024 512 rows 4.6 / 5.0, 4096 6.3 / 6.5, K = 1536 1024 rows 6.5 / 5.9 (the line is the
-        // same with its own, for the same bits).
-        if (a.K >= 1536 && (long)full.x * full.y <= device_cus()) {
+        // One workgroup to a CU at most: sixteen wavefronts, each of which takes the statistics of one row instead of two, and half the groups of
+        // a workgroup that only quantizes (one that projects gives its groups to eight of them: Q_CHAINS).  us, eight / sixteen (K = 3072,
+        // R = 32, bf16), its own statistics: 333 rows 10.5 / 10.2, 2048 13.2 / 12.4, 2560 14.6 / 14.3, 4096 15.3 / 15.3; K = 4096: 2048 16.6 / 15.1.  With given ones only where
+        // one workgroup quantizes beside those that project: 2048 rows 10.5 / 9.8, but 333 rows (three) 7.7 / 7.8.  Short rows: given, K = 1024 512 rows
+        // 4.6 / 5.0, K = 1536 1536 rows 6.7 / 6.2.  Two of them do not fit a CU's registers (4608 rows 22.4 / 26.1); without the prologue they are slower (1024
+        // rows 5.4 / 6.3).
+        const int chunks = (a.R + Q_RCHUNK - 1) / Q_RCHUNK;
+        if (a.K >= 1536 && (long)full.x * full.y <= device_cus() && (!lora || !a.norm_stats || (int)full.y == chunks + 1)) {
             go(std::integral_constant<int, 16>{});
             return;
         }

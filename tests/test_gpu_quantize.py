@@ -395,5 +395,37 @@ def test_row_blocks_behind_the_last_whole_round(dev, M, K, R, norm):
             c, s, a = run(xm[i : i + n], blocked)
             whole = n // 32 * 32 if blocked else n  # (rows of the padding are not written)
             assert torch.equal(codes[i : i + whole], c[:whole]) and (blocked == 3 or torch.equal(scales[:, i : i + n], s[:, :n]))
-            # fp32 sums of K products in another order
-            assert ((la[i : i + n] - a[:n]).abs() <= K * 2.0**-23 * (xm[i : i + n].float().abs().amax() * down.float().abs().sum(0)) + 1e-6).all()
+            assert torch.equal(la[i : i + n], a[:n])
+    # fp32 sums of K products, 32 at a time
+    exact, terms = xm.double() @ down.double(), xm.double().abs() @ down.double().abs()
+    assert ((la[:M].double() - exact).abs() <= (K // 32 + 8) * 2.0**-24 * terms).all()
+
+
+@pytest.mark.parametrize("given", [False, True])
+@pytest.mark.parametrize("K,R", [(1536, 32), (3072, 48), (4096, 128)])
+def test_low_rank_state_of_a_row_whatever_stands_beside_it(dev, K, R, given):
+    """Two batches with scale and shift of their own, in launches of one row block to several for each CU: eight and sixteen wavefronts, row
+    blocks shared or not, one to three workgroups that quantize beside those that project."""
+    from nunchaku_rocm_amd import ops
+
+    g = torch.Generator().manual_seed(K)
+    T = torch.bfloat16
+    x = O.make_activations(2 * 4608, K, seed=K, dtype=T).to(dev)
+    down = (torch.randn(K, R, generator=g) * 0.02).to(T).to(dev)
+    scale, shift = (1 + 0.3 * torch.randn(2, K, generator=g)).to(T).to(dev), (0.2 * torch.randn(2, K, generator=g)).to(T).to(dev)
+    stats = ops.layer_norm_stats(x)
+    first = None
+    for rows in (16, 336, 512, 640, 1024, 2048, 4608):  # of a batch
+        print(f"case K={K} R={R} rows={rows} given={given}", flush=True)
+        both = torch.cat([x[:rows], x[4608 : 4608 + rows]])
+        vecs = (scale, shift, torch.cat([stats[:rows], stats[4608 : 4608 + rows]])) if given else (scale, shift)
+        _, _, la = ops.svdq_quantize_w4a4_act_fuse_lora_cuda(both, lora_down=down, norm=vecs, pad_size=32, out_blocked=2)
+        head = torch.cat([la[:16], la[rows : rows + 16]])
+        first = head if first is None else first
+        assert torch.equal(head, first)
+    xm = torch.cat([x[:16], x[4608:4624]])
+    st = torch.cat([stats[:16], stats[4608:4624]])
+    xm = ((xm.float() - st[:, :1]) * st[:, 1:]).to(T).view(2, 16, K)
+    xm = ((xm.float() * scale[:, None].float()).to(T).float() + shift[:, None].float()).to(T).view(32, K)
+    exact, terms = xm.double() @ down.double(), xm.double().abs() @ down.double().abs()
+    assert ((first.double() - exact).abs() <= (K // 32 + 8) * 2.0**-24 * terms).all()

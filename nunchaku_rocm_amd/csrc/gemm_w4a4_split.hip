@@ -206,14 +206,15 @@ __global__ __launch_bounds__(WAVES * 64, 2) void gemm_w4a4_split_kernel(svdq_gem
 // wavefront's next stage), and scales come for two stages at a time: the lanes of one half hold the scales of a stage, those of the other
 // half the scales of the wavefront's next one, and the activation side is zero in the half whose stage it is not.  (One load per
 // stage and scale, of lanes that all hold the same: 512 x 3072, K = 12288 40.2 us, 29.0 without scales.)
-// us, 32-row workgroups / these (bf16, rank 32, fp6 codes with blocked scales): K = 3072: 512 x 3072 15.8 / 12.8, 333 x 4096 15.2 / 12.3,
-// 64 x 18432 17.5 / 13.7; K = 12288: 333 x 3072 40.2 / 31.8, 512 x 3072 41.5 / 31.9; K = 2048: 1000 x 2048 12.5 / 10.5.  Of the 31.9 the
-// matrix instructions and FMAs alone are 20, launch, exchange and epilogue 6.
+// us, 32-row workgroups / these (bf16, rank 32, fp6 codes with blocked scales): K = 3072: 512 x 3072 14.8 / 11.4, 333 x 4096 14.7 / 11.4,
+// 64 x 18432 17.4 / 13.1; K = 12288: 333 x 3072 40.4 / 31.0, 512 x 3072 41.4 / 31.2; K = 2048: 1000 x 2048 12.1 / 9.5.  Of the 31.2 the
+// matrix instructions and FMAs alone are 20.  Partial sums added pairwise by half of the wavefronts, then a quarter, with three barriers
+// instead of two: 512 x 3072 at K = 3072 12.1, at K = 12288 31.9.
 template <typename T, int EPI, bool F6ACT, bool SB>
 __global__ __launch_bounds__(512, 2) void gemm_w4a4_split64_kernel(svdq_gemm_args a, int tiles_m) {
     static_assert(F6ACT || !SB, "blocked scales come with fp6 codes");
     constexpr int RB = 2, CB = 2, WC = NBN / CB, KS = 8 / WC;  // blocks of a wavefront, column halves, wavefronts that split K
-    __shared__ __align__(16) uint8_t sred[(KS / 2) * RB * NBN * SK_BLOCK_BYTES];
+    __shared__ __align__(16) uint8_t sred[KS * RB * NBN * SK_BLOCK_BYTES];  // [wavefront along K][row block][column block]
     __shared__ __align__(16) uint8_t sepi[EPI_LDS_BYTES];
 
     const int tid = threadIdx.x, lane = tid & 63;
@@ -374,40 +375,38 @@ __global__ __launch_bounds__(512, 2) void gemm_w4a4_split64_kernel(svdq_gemm_arg
         if (left >= 3) stage(I0, I1, i + 2);
     }
 
-    // ---- partial sums: four wavefronts of a column half to two to one, then a row block to a wavefront
+    // ---- partial sums: every wavefront adds up one block, in the order of gemm_w4a4_split_kernel (of column block bn: wavefront bn's
+    // first, then the others'), so that an output has the same bits as there; then a row block to a wavefront
     auto slot = [&](int k, int r, int b) { return sred + ((k * RB + r) * NBN + b) * SK_BLOCK_BYTES + lane * 16; };
-    auto put = [&](int k) {
 #pragma unroll
-        for (int rb = 0; rb < RB; rb++)
+    for (int rb = 0; rb < RB; rb++)
 #pragma unroll
-            for (int bn = 0; bn < CB; bn++) {
-                uint8_t *p = slot(k, rb, wc * CB + bn);
+        for (int bn = 0; bn < CB; bn++) {
+            uint8_t *p = slot(ks, rb, wc * CB + bn);
 #pragma unroll
-                for (int j = 0; j < 4; j++) *(v4f *)(p + j * 1024) = (v4f){acc[rb][bn][4 * j], acc[rb][bn][4 * j + 1], acc[rb][bn][4 * j + 2], acc[rb][bn][4 * j + 3]};
-            }
-    };
-#pragma unroll
-    for (int d = KS / 2; d >= 1; d >>= 1) {
-        if (ks >= d && ks < 2 * d) put(ks - d);
-        if (d == KS / 2) __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, 0));  // this wavefront's share of the epilogue operands has landed
-        __syncthreads();
-        if (ks < d) {
-#pragma unroll
-            for (int rb = 0; rb < RB; rb++)
-#pragma unroll
-                for (int bn = 0; bn < CB; bn++) {
-                    const uint8_t *p = slot(ks, rb, wc * CB + bn);
-#pragma unroll
-                    for (int j = 0; j < 4; j++) {
-                        const v4f t = *(const v4f *)(p + j * 1024);
-#pragma unroll
-                        for (int e = 0; e < 4; e++) acc[rb][bn][4 * j + e] += t[e];
-                    }
-                }
+            for (int j = 0; j < 4; j++) *(v4f *)(p + j * 1024) = (v4f){acc[rb][bn][4 * j], acc[rb][bn][4 * j + 1], acc[rb][bn][4 * j + 2], acc[rb][bn][4 * j + 3]};
         }
-        if (d > 1) __syncthreads();
+    __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, 0));  // (also: this wavefront's share of the epilogue operands has landed)
+    __syncthreads();
+    {
+        static_assert(KS == RB * CB && KS == NBN, "a block to a wavefront, a wavefront along K that a column block's sum begins with");
+        const int rb = ks / CB, b = wc * CB + ks % CB;
+        v4f sum[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) sum[j] = *(const v4f *)(slot(b, rb, b) + j * 1024);
+#pragma unroll
+        for (int v = 0; v < KS - 1; v++) {
+            const uint8_t *p = slot(v < b ? v : v + 1, rb, b);
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const v4f t = *(const v4f *)(p + j * 1024);
+#pragma unroll
+                for (int e = 0; e < 4; e++) sum[j][e] += t[e];
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++) *(v4f *)(slot(0, rb, b) + j * 1024) = sum[j];
     }
-    if (ks == 0) put(0);  // where this wavefront alone has just read
     __syncthreads();
     if (wave >= RB || m0 + 32 * wave >= a.M) return;
     v16f mine[NBN];

@@ -239,3 +239,30 @@ def test_hand_over_forms_give_the_same_bits(dev, splits, M, N, K):
         results.append(out.cpu())
     assert len(set(splits)) == 1 and splits[0] in (4, 8)
     assert all(torch.equal(r, results[0]) for r in results[1:])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("form", ["fp6 and scales", "fp6", "nibbles"])
+@pytest.mark.parametrize("M,K", [(65, 1536), (90, 2560), (96, 4608)])
+def test_rows_of_a_workgroup_leave_the_sums_alone(dev, splits, M, K, form, dtype):
+    """16640 columns are 260 workgroups of 64 rows, more than 256 CUs, and run as 32-row ones; the first 16384 alone are 256 and do not: the same
+    bits in either."""
+    from nunchaku_rocm_amd import ops
+    from nunchaku_rocm_amd.layout import block_activations_f6, block_scales
+
+    print(f"case M={M} K={K} {form} {dtype}", flush=True)
+    g = torch.Generator().manual_seed(M + K)
+    act = torch.randint(0, 256, (96, K // 2), dtype=torch.uint8, generator=g)
+    asc = (torch.rand(K // 64, 96, generator=g) * 0.1 + 0.01).to(dtype)
+    wgt = torch.randint(0, 256, (16640, K // 2), dtype=torch.uint8, generator=g).view(torch.int8)
+    wsc = (torch.rand(K // 64, 16640, generator=g) * 0.02 + 0.005).to(dtype)
+    nibbles, blocked = form == "nibbles", {"fp6 and scales": 3, "fp6": 2, "nibbles": 0}[form]
+    sent, scales = (act if nibbles else block_activations_f6(act, False)).to(dev), (block_scales(asc) if blocked == 3 else asc).to(dev)
+    out = []
+    for n in (16640, 16384):
+        out.append(torch.empty(M, n, dtype=dtype, device=dev))
+        param = torch.nn.Parameter(wgt[:n].contiguous().to(dev), requires_grad=False)
+        ops.svdq_gemm_w4a4_cuda(act=sent, wgt=param, out=out[-1], ascales=scales, wscales=wsc[:, :n].contiguous().to(dev), act_unsigned=nibbles, act_blocked=blocked)
+    assert splits == [4, 4]
+    assert torch.equal(out[0][:, :16384], out[1])

@@ -992,10 +992,12 @@ extern "C" int svdq_gemm_w4a4_split_wavefronts(const svdq_gemm_args *args, int32
 //     768 x 1536 0.86, 1536 x 1536 1.02;  from K = 3584 up to 2 K / 3: K = 3584 1024 x 1536 0.77, 1344 x 1536 0.76, 6144 x 512
 //     1.08;  K = 4608 4096 x 512 0.83, 6144 x 512 1.06
 //   more than two 128-row tiles to a CU (together, as above): K = 1024 3072 x 4608 0.90, 1344 x 6144 0.92, 1024 x 9216 0.91, 4096 x 3072 1.03;  K = 1536 3072
-//     x 3072 0.91, 2048 x 4608 0.91, 4608 columns and more 0.80 to 0.93, 8192 x 1536 0.95, 4096 x 2048 1.08;  K = 2048 8192 x 1536 0.95;  unsigned K = 1024
-//     1024 x 9216 0.96, 4096 0.91, K = 1536 3072 x 3072 0.96
-//   more than one: K = 3584 1344 x 3072 0.90, 3072 x 1536 0.92, 333 x 12288 0.89;  K = 4608 1344 x 3072 0.88;  unsigned 0.95 to 0.98;  one at most: K = 3584
-//     512 x 4608 0.97, 768 x 3072 1.00;  K = 3072 1536 x 3072 0.91, 768 x 3072 1.01, 512 x 4608 0.99 (the line lies above them)
+//     x 3072 0.91, 2048 x 4608 0.91, 4608 columns and more 0.80 to 0.93, 8192 x 1536 0.95, 4096 x 2048 1.08;  K = 2048 8192 x 1536 0.95;  unsigned K = 1536
+//     3072 x 3072 0.94, K = 1024 more than three to a CU 0.86 to 0.97, up to three 2048 x 6144 1.02, 1024 x 12288 1.03, 1152 x 9216 1.00
+//   more than one: K = 3584 1344 x 3072 0.90, 3072 x 1536 0.92, 333 x 12288 0.89;  K = 4608 1344 x 3072 0.88;  many rows, below K = 6144: 4608 x 1536 0.97, 4608 x 1024
+//     0.96, 8192 x 1024 1.04;  unsigned 0.93 to 0.99 up to 3072 rows, 4096 x 1536 1.02, 4096 x 2048 1.04, 4608 x 1536 1.03 to 1.06, 8192 x 1024 1.07 (220
+//     launches of the lines for K below 6144, two thirds of them in fp16);  one at most: K = 3584 512 x 4608 0.97, 768 x 3072 1.00;  K = 3072 1536 x 3072 0.91, 768 x
+//     3072 1.01, 512 x 4608 0.99 (the line lies above them)
 //   K = 6144: 768 x 3072 41.7 / 40.1, 4608 x 3072 117 / 93, 2048 x 1536 (192 tiles) 42.4 / 43.8;  K = 12288, 2048 x 1536 78.2 / 73.4
 // Unsigned activations of few rows split their K as they are (split_of); beyond those 1536 x 9216 at K = 3072 58.4 / 51.2.  (The
 // grid of the pass is two-dimensional: 2^20 rows keep it inside 65536.)
@@ -1012,8 +1014,8 @@ static size_t act_scratch_bytes(const svdq_gemm_args &a, int cus) {
         case 8: pays = K >= 1024 && rows < K; break;
         case 4: pays = K >= 1536 && (K >= 3584 ? 3 * rows <= 2 * K : 4 * rows <= K); break;
         default:
-            pays = N >= 1024 && ((tiles > 2L * cus && K >= (N >= 4608 ? 1024 : N >= 3072 ? 1536 : N >= 2048 ? 2048 : 3072)) || (K >= 3584 && tiles > cus) ||
-                                 (K >= 6144 && K * N >= 1 << 24));
+            pays = N >= 1024 && ((tiles > (K < 1536 && a.act_unsigned ? 3L : 2L) * cus && K >= (N >= 4608 ? 1024 : N >= 3072 ? 1536 : N >= 2048 ? 2048 : 3072)) ||
+                                 (K >= 3584 && tiles > cus && (K >= 6144 || rows <= (a.act_unsigned ? 3072 : 4608))) || (K >= 6144 && K * N >= 1 << 24));
     }
     if (!pays) return 0;
     const size_t padded = (size_t)((a.M + 31) / 32 * 32);

@@ -129,9 +129,22 @@ def test_lines_of_the_pass_over_nibbles(lib):
 
     for rows, n, k, want in (
         (384, 3072, 1536, 1), (385, 3072, 1536, 0), (2048, 1024, 3584, 1), (4096, 512, 3584, 0), (333, 12288, 3584, 1), (256, 16384, 3584, 0), (333, 12288, 3072, 0),
-        (4608, 3072, 1536, 1), (4608, 2944, 1536, 0), (4608, 4608, 1024, 1), (4608, 4480, 1024, 0), (4608, 9216, 512, 0),
+        (4608, 3072, 1536, 1), (4608, 2944, 1536, 0), (4608, 4608, 1024, 1), (4608, 4480, 1024, 0), (4608, 9216, 512, 0), (4608, 1536, 3584, 1),
+        (4736, 1536, 3584, 0), (8192, 1024, 4608, 0), (8192, 1024, 6144, 1),
     ):  # fmt: skip
         nbytes = lib.svdq_gemm_w4a4_act_scratch_bytes(_lib.GemmArgs(wgt_planes=16, M=rows, actual_m=rows, N=n, K=k, R=32))
+        assert bool(nbytes) == bool(want), (rows, n, k)
+
+
+def test_unsigned_nibbles_that_the_pass_would_slow_down_stay(lib):
+    """256 CUs: K = 1024 up to three 128-row tiles to a CU, many rows of one to two tiles to a CU."""
+    from nunchaku_rocm_amd import _lib
+
+    for rows, n, k, want in (
+        (2048, 6144, 1024, 0), (1024, 12288, 1024, 0), (2176, 6144, 1024, 1), (1152, 9216, 1024, 0), (1344, 9216, 1024, 1), (3072, 1536, 3584, 1), (3200, 1536, 3584, 0),
+        (4096, 2048, 4096, 0), (8192, 1024, 4608, 0), (1536, 3072, 3584, 1), (3072, 3072, 1536, 1),
+    ):  # fmt: skip
+        nbytes = lib.svdq_gemm_w4a4_act_scratch_bytes(_lib.GemmArgs(wgt_planes=16, M=rows, actual_m=rows, N=n, K=k, R=32, act_unsigned=1))
         assert bool(nbytes) == bool(want), (rows, n, k)
 
 

@@ -22,7 +22,6 @@
 // the same bytes in its lanes' order, or the same integers as fp6 codes in that order (from the hardware's float -> fp6
 // conversion), with the scales in that order as well.
 #include <algorithm>
-#include <climits>
 #include <type_traits>
 
 #include "svdq_common.h"
@@ -130,7 +129,7 @@ __device__ __forceinline__ void row_moments(const uint16_t *const (&row)[NR], in
 }
 
 template <typename T, bool UNSIGNED, int PRE, bool HAS_LORA, bool HAS_SMOOTH, bool NORM, int QR, int WAVES>
-__global__ __launch_bounds__(WAVES * 64, QR == 32 ? 1 : (NORM ? 4 : 2)) void quantize_act_kernel(svdq_quantize_args a, int split_from, int share) {
+__global__ __launch_bounds__(WAVES * 64, QR == 32 ? 1 : (NORM ? 4 : 2)) void quantize_act_kernel(svdq_quantize_args a, int split_from, int rows) {
     constexpr bool GLU = PRE == SVDQ_PRE_GLU, GELU = PRE == SVDQ_PRE_GELU;
     constexpr int NH = QR / Q_ROWS;  // 16-row halves of the row block: each LoRA-down tile read serves all of them
     // per wavefront: two activation stages (16 rows, + the gate tile with GLU) and one LoRA-down tile (32 ranks), 128
@@ -154,22 +153,28 @@ __global__ __launch_bounds__(WAVES * 64, QR == 32 ? 1 : (NORM ? 4 : 2)) void qua
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform: keep it in an SGPR
     const int ml = lane & 15;
     const int kq = lane >> 4;
-    // Row block, and place on the grid's second axis.  From row block split_from on `share` workgroups of the first axis share a block,
-    // as if they were the second axis of a grid of its own: the last one projects, the others quantize.
-    const bool shared = HAS_LORA && QR == Q_ROWS && (int)blockIdx.x >= split_from;
-    const int over = (int)blockIdx.x - split_from, part = over / share;
-    const int bx = shared ? split_from + part : (int)blockIdx.x, by = shared ? over - part * share : (int)blockIdx.y;
+    // Row block, and place on the grid's second axis, which has `rows` workgroups; or, with split_from >= 0, from row block split_from on
+    // `rows` = 3 or 4 workgroups of the first axis share a block, as if they were the second axis of a grid of its own: the last one projects,
+    // the others quantize.  (A division by `rows` and the grid's size from its hidden argument, behind a wait of its own, took 0.1 us of
+    // every launch.)
+    const bool sharing = HAS_LORA && QR == Q_ROWS && split_from >= 0, shared = sharing && (int)blockIdx.x >= split_from;
+    int bx = blockIdx.x, by = blockIdx.y;
+    if (shared) {
+        const unsigned over = blockIdx.x - (unsigned)split_from, part = rows == 4 ? over / 4u : over / 3u;
+        bx = split_from + (int)part;
+        by = (int)(over - part * (unsigned)rows);
+    }
     const int m0 = bx * QR;
     const int ngroups = a.K / GROUP;
     // The grid's second axis: nq >= 0 workgroup rows that only quantize, each its own slice of the groups (a shorter chain
     // of group steps per wavefront where CUs would otherwise idle), then one row per chunk of 32 ranks.
     const int rchunks = (a.R + Q_RCHUNK - 1) / Q_RCHUNK;
-    const int nq = HAS_LORA ? max((shared ? share : (int)gridDim.y) - rchunks, 0) : 0;
+    const int nq = HAS_LORA ? max((sharing && !shared ? 1 : rows) - rchunks, 0) : 0;
     const bool qonly = by < nq;
     const int g_lo = qonly ? (ngroups * by) / nq : 0, g_hi = qonly ? (ngroups * (by + 1)) / nq : ngroups;
     const int gwaves = WIDE && !qonly ? Q_CHAINS : WAVES;  // wavefronts that take groups
     const int gw = g_lo + wave;                            // this wavefront's groups: gw + gwaves * i < g_hi
-    const int nmy = wave < gwaves ? max((g_hi - gw + gwaves - 1) / gwaves, 0) : 0;
+    const int nmy = !WIDE || wave < gwaves ? max((g_hi - gw + gwaves - 1) / gwaves, 0) : 0;
     // Block loads: lane l of load i fetches chunk (l % 8) ^ (l / 8) of tile row 8 i + l / 8 into LDS slot l of that
     // load's 1 KB, i.e. tile[row][chunk ^ (row & 7)].  Rows >= M re-read row M - 1 and ranks >= R rank R - 1 (valid
     // memory; nothing is stored for them).  Addresses = uniform base + 32-bit lane offset (+ uniform group step).
@@ -674,7 +679,7 @@ static int quantize_share(const svdq_quantize_args &a) {
     const int blocks = (a.M + Q_ROWS - 1) / Q_ROWS, cus = device_cus(), left = blocks % cus;
     if (a.R == 0 || a.R > Q_RCHUNK || blocks <= cus || left == 0 || a.prologue != SVDQ_PRE_NONE) return 1;
     const int share = std::min({4, cus / left, a.K / GROUP});
-    return share >= 3 ? share : 1;
+    return share >= 3 ? share : 1;  // (the kernel divides by three or four)
 }
 
 // Rows per workgroup.  A workgroup streams 4 KB of LoRA-down weight per group whatever its number of rows, and the
@@ -731,9 +736,9 @@ static void launch_quantize3(const svdq_quantize_args &a, hipStream_t s) {
         if (quantize_rows_per_workgroup(a) == 32) {
             const dim3 grid((a.M + 31) / 32, quantize_grid_y(a, (a.M + 31) / 32, 32));
             if (sm)
-                hipLaunchKernelGGL((quantize_act_kernel<T, U, G, true, true, NORM, 32, 8>), grid, dim3(512), 0, s, a, INT_MAX, 1);
+                hipLaunchKernelGGL((quantize_act_kernel<T, U, G, true, true, NORM, 32, 8>), grid, dim3(512), 0, s, a, -1, (int)grid.y);
             else
-                hipLaunchKernelGGL((quantize_act_kernel<T, U, G, true, false, NORM, 32, 8>), grid, dim3(512), 0, s, a, INT_MAX, 1);
+                hipLaunchKernelGGL((quantize_act_kernel<T, U, G, true, false, NORM, 32, 8>), grid, dim3(512), 0, s, a, -1, (int)grid.y);
             return;
         }
     }
@@ -741,16 +746,17 @@ static void launch_quantize3(const svdq_quantize_args &a, hipStream_t s) {
     auto go = [&](auto wtag) {
         constexpr int W = decltype(wtag)::value;
         const dim3 block(W * 64);
-        const int share = W == 16 ? 1 : quantize_share(a), split_from = share > 1 ? (int)full.x / device_cus() * device_cus() : INT_MAX;
+        const int share = W == 16 ? 1 : quantize_share(a), split_from = share > 1 ? (int)full.x / device_cus() * device_cus() : -1;
         const dim3 grid = share > 1 ? dim3(split_from + share * (full.x - split_from)) : full;
+        const int rows = share > 1 ? share : (int)full.y;
         if (lora && sm)
-            hipLaunchKernelGGL((quantize_act_kernel<T, U, G, true, true, NORM, 16, W>), grid, block, 0, s, a, split_from, share);
+            hipLaunchKernelGGL((quantize_act_kernel<T, U, G, true, true, NORM, 16, W>), grid, block, 0, s, a, split_from, rows);
         else if (lora)
-            hipLaunchKernelGGL((quantize_act_kernel<T, U, G, true, false, NORM, 16, W>), grid, block, 0, s, a, split_from, share);
+            hipLaunchKernelGGL((quantize_act_kernel<T, U, G, true, false, NORM, 16, W>), grid, block, 0, s, a, split_from, rows);
         else if (sm)
-            hipLaunchKernelGGL((quantize_act_kernel<T, U, G, false, true, NORM, 16, W>), grid, block, 0, s, a, split_from, share);
+            hipLaunchKernelGGL((quantize_act_kernel<T, U, G, false, true, NORM, 16, W>), grid, block, 0, s, a, split_from, rows);
         else
-            hipLaunchKernelGGL((quantize_act_kernel<T, U, G, false, false, NORM, 16, W>), grid, block, 0, s, a, split_from, share);
+            hipLaunchKernelGGL((quantize_act_kernel<T, U, G, false, false, NORM, 16, W>), grid, block, 0, s, a, split_from, rows);
     };
     if constexpr (NORM) {
         // One workgroup to a CU at most: sixteen wavefronts, each of which takes the statistics of one row instead of two, and half the groups of

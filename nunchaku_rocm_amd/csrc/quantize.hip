@@ -699,18 +699,17 @@ static int quantize_rows_per_workgroup(const svdq_quantize_args &a) {
 
 // Second grid axis: one workgroup row per chunk of 32 ranks, plus rows that only quantize where that still leaves about
 // one workgroup per CU: quantizing and projecting then run side by side on different CUs (K = 3072, R = 32: 6.4
-// against 7.9 us at M = 512, 7.1 against 8.5 at 2048, 12.3 against 13.4 at 4608 with 32-row workgroups; slower once the
-// CUs are taken: 9.9 against 9.5 us at M = 4096, 17.2 against 14.5 at 6144).  While CUs are left over, up to three such
+// against 7.9 us at M = 512, 7.1 against 8.5 at 2048; slower once the CUs are taken: 9.9 against 9.5 us at M = 4096, 17.2 against 14.5 at
+// 6144, and with 32-row workgroups at K = 64 and 128 5.7 against 4.6 at 4608).  While CUs are left over, up to three such
 // rows share the groups between them: a wavefront's chain of group steps gets shorter (M = 1024: 7.8 -> 5.1 us with
-// three, M = 512: 7.6 -> 4.9; slower again beyond one workgroup per CU: M = 1024 with four 6.4 us, M = 4608 with two
-// 14.2 against 12.8).
-static int quantize_grid_y(const svdq_quantize_args &a, int row_blocks, int rows) {
+// three, M = 512: 7.6 -> 4.9; slower again beyond one workgroup per CU: M = 1024 with four 6.4 us).
+static int quantize_grid_y(const svdq_quantize_args &a, int row_blocks) {
     if (a.R == 0) return 1;
     const int chunks = (a.R + Q_RCHUNK - 1) / Q_RCHUNK, cus = device_cus();
     // (with a GLU or GELU prologue the workgroups that only project compute it a second time: only where half the CUs would idle
     // anyway.  With the norm prologue, of sixteen wavefronts, up to all of the CUs: K = 3072, R = 32, limits of a half / all of them 1024
     // rows 11.5 / 10.6 us, 1201 12.7 / 10.7, 2048 13.3 / 12.3; R = 128 512 rows 12.5 / 10.4)
-    const int limit = has_norm(a) ? cus : a.prologue != SVDQ_PRE_NONE ? cus / 2 : cus + (rows == 32 ? cus / 8 : 0);
+    const int limit = has_norm(a) ? cus : a.prologue != SVDQ_PRE_NONE ? cus / 2 : cus;
     if (row_blocks * (chunks + 1) > limit) return chunks;
     const int nq = std::min({3, limit / row_blocks - chunks, a.K / GROUP});
     return chunks + std::max(nq, 1);
@@ -734,7 +733,7 @@ static void launch_quantize3(const svdq_quantize_args &a, hipStream_t s) {
     const bool lora = a.R > 0, sm = a.smooth != nullptr;
     if constexpr (G == SVDQ_PRE_NONE) {
         if (quantize_rows_per_workgroup(a) == 32) {
-            const dim3 grid((a.M + 31) / 32, quantize_grid_y(a, (a.M + 31) / 32, 32));
+            const dim3 grid((a.M + 31) / 32, quantize_grid_y(a, (a.M + 31) / 32));
             if (sm)
                 hipLaunchKernelGGL((quantize_act_kernel<T, U, G, true, true, NORM, 32, 8>), grid, dim3(512), 0, s, a, -1, (int)grid.y);
             else
@@ -742,7 +741,7 @@ static void launch_quantize3(const svdq_quantize_args &a, hipStream_t s) {
             return;
         }
     }
-    const dim3 full((a.M + Q_ROWS - 1) / Q_ROWS, quantize_grid_y(a, (a.M + Q_ROWS - 1) / Q_ROWS, Q_ROWS));
+    const dim3 full((a.M + Q_ROWS - 1) / Q_ROWS, quantize_grid_y(a, (a.M + Q_ROWS - 1) / Q_ROWS));
     auto go = [&](auto wtag) {
         constexpr int W = decltype(wtag)::value;
         const dim3 block(W * 64);

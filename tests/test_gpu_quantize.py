@@ -359,11 +359,11 @@ def test_full_size_invariants(dev):
 
 @pytest.mark.parametrize("norm", [False, True, "given"])
 @pytest.mark.parametrize("M,K,R", [(333, 2048, 64), (1201, 3072, 48), (2048, 1536, 32), (2064, 1536, 32), (4096, 1536, 16), (2048, 1472, 32), (4097, 256, 32), (4100, 192, 32), (4112, 128, 32), (5120, 320, 32),
-                                   (5136, 512, 16), (5456, 256, 32), (5457, 256, 32), (8208, 512, 32), (4112, 256, 48)])  # fmt: skip
+                                   (5136, 512, 16), (5456, 256, 32), (5457, 256, 32), (8208, 512, 32), (4112, 256, 48), (4608, 64, 32)])  # fmt: skip
 def test_row_blocks_behind_the_last_whole_round(dev, M, K, R, norm):
     """On 256 CUs: sixteen wavefronts with the norm prologue up to one workgroup to a CU (4096 rows; 2048: with rows that only quantize)
-    from K = 1536 on, four (to 5120 rows) and three (to 5456) workgroups to a block of the rest, not with fewer groups than that
-    (192) or a second chunk of ranks -- against the same rows, normalised before, a few blocks at a time, which take none of these routes."""
+    from K = 1536 on, four (to 5120 rows) and three (to 5456) workgroups to a block of the rest, three where there are three groups (192),
+    none with fewer (128, 64) or a second chunk of ranks -- against the same rows, normalised before, a few blocks at a time, which take none of these routes."""
     from nunchaku_rocm_amd import ops
     from nunchaku_rocm_amd.layout import block_scales
 

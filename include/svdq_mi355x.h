@@ -368,6 +368,9 @@ typedef struct {
 } svdq_attention_args;
 
 int svdq_attention_fp16(const svdq_attention_args *args, void *stream);
+/* Queries to a workgroup (128 or 256) with which svdq_attention_fp16 runs `args` on a device of `cus` compute units (0: this
+ * one's); the bits are the same.  Host arithmetic on the sizes; for tests.  No counterpart in the reference. */
+int svdq_attention_queries(const svdq_attention_args *args, int32_t cus);
 
 /*
  * Checkpoint ingestion.  The published SVDQuant int4 checkpoints hold every tensor of a quantized linear pre-shuffled

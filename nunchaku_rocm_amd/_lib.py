@@ -52,6 +52,7 @@ EXPORTS = (
     "svdq_awq_gemm_w4a16",
     "svdq_awq_gemm_tile",
     "svdq_attention_fp16",
+    "svdq_attention_queries",
     "svdq_unpack_mma_weight",
     "svdq_unpack_mma_scale",
     "svdq_unpack_mma_lowrank",
@@ -165,6 +166,7 @@ def load() -> ctypes.CDLL:
     lib.svdq_awq_gemm_w4a16.argtypes = [ctypes.POINTER(AwqGemvArgs), _i32, _vp]
     lib.svdq_awq_gemm_tile.argtypes = [_i32, _i32, _i32]
     lib.svdq_attention_fp16.argtypes = [ctypes.POINTER(AttentionArgs), _vp]
+    lib.svdq_attention_queries.argtypes = [ctypes.POINTER(AttentionArgs), _i32]
     lib.svdq_unpack_mma_weight.argtypes = [_vp, _vp, _i32, _i32, _i32, _vp]
     lib.svdq_unpack_mma_scale.argtypes = [_vp, _vp, _i32, _i32, _i32, _vp]
     lib.svdq_unpack_mma_lowrank.argtypes = [_vp, _vp, _i32, _i32, _i32, _i32, _vp]

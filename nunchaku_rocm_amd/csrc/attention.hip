@@ -389,6 +389,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attention_kernel(svdq_attention
 // to 0.97; within one, 256 keys at 480 workgroups of 128 1.015, at 432 0.99.  us, 128 / 256 queries (bf16): 24 x 4608 234 / 225, 24 x 2000
 // 52.5 / 49.9, 24 x 8192 672 / 658, 10 x 4608 112 / 108, 20 x 3000 87.8 / 87.0.  Head dimension 64: 40 x 4096 169 / 192.
 static bool wide_queries(const svdq_attention_args &a, int cus) {
+    if (a.D != 128) return false;
     const long wg4 = (long)((a.Tq + 127) / 128) * a.H * a.B, wg8 = (long)((a.Tq + 255) / 256) * a.H * a.B;
     const long deep = (wg4 + cus - 1) / cus, rounds = (wg8 + cus - 1) / cus;  // workgroups of 128 on the fullest CU
     if (0.97 * (double)rounds >= (double)(deep / 2) + (deep % 2 ? 0.565 : 0.0)) return false;
@@ -402,17 +403,21 @@ static void launch_attention(const svdq_attention_args &a, hipStream_t s) {
 }
 template <typename T>
 static void launch_attention(const svdq_attention_args &a, hipStream_t s) {
-    if (a.D == 64)
-        launch_attention<T, 64, 4>(a, s);
-    else if (wide_queries(a, cu_count()))
+    if (wide_queries(a, cu_count()))
         launch_attention<T, 128, 8>(a, s);
-    else
+    else if (a.D == 128)
         launch_attention<T, 128, 4>(a, s);
+    else
+        launch_attention<T, 64, 4>(a, s);
 }
 
 }  // namespace svdq
 
 using namespace svdq;
+
+extern "C" int svdq_attention_queries(const svdq_attention_args *args, int32_t cus) {
+    return args && args->B > 0 && args->H > 0 && args->Tq > 0 && wide_queries(*args, cus > 0 ? cus : cu_count()) ? 256 : 128;
+}
 
 extern "C" int svdq_attention_fp16(const svdq_attention_args *args, void *stream) {
     if (!args) {

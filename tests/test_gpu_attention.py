@@ -205,20 +205,35 @@ def test_ends_of_the_key_pipeline(dev, Tkv, D):
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("B,H,Tq,Tkv", [(1, 40, 1100, 70), (2, 20, 1025, 1), (1, 24, 1500, 1100), (1, 9, 3584, 1100), (1, 43, 1537, 2048)])
-def test_workgroups_of_256_queries(dev, B, H, Tq, Tkv, dtype):
-    """Launches that are large enough for them on 256 CUs (and one past their first round) against the same heads a few at a
-    time, which are not: the same bits; the last workgroup has rows of its first or of neither half only."""
-    from nunchaku_rocm_amd import ops
+@pytest.mark.parametrize(
+    "B,H,Tq,Tkv,queries",
+    [
+        (1, 40, 1100, 70, 256),  # one round on 256 CUs; rows of the last workgroup's first half only
+        (2, 20, 1025, 1, 256),  # one row
+        (1, 24, 1500, 1100, 256),
+        (1, 24, 4500, 2049, 256),  # two rounds, the last key alone in its tile; a partial last workgroup
+        (1, 40, 4609, 2150, 256),  # three
+        (1, 24, 4500, 2047, 128),  # too few keys for several rounds
+        (1, 9, 3584, 1100, 128),  # a CU to each workgroup of 128
+        (1, 43, 1537, 2048, 128),  # an odd number of them on the fullest
+    ],
+)
+def test_workgroups_of_256_queries(dev, B, H, Tq, Tkv, queries, dtype):
+    """Both sides of the rule's lines against the same heads a few at a time, which run as workgroups of 128: the same bits."""
+    from nunchaku_rocm_amd import _lib, ops
 
     print(f"case {B}x{H}x{Tq}x{Tkv} {dtype}", flush=True)
+    chosen = lambda h: _lib.load().svdq_attention_queries(_lib.AttentionArgs(B=B, H=h, Tq=Tq, Tkv=Tkv, D=128), 0)  # noqa: E731
+    assert chosen(H) == queries
     q, k, v = (t.to(dev) for t in _inputs(B, H, Tq, Tkv, dtype, seed=Tq))
     o = torch.full((B, Tq + 3, H * 128), 7.0, dtype=dtype, device=dev)
     ops.attention_fp16(q, k, v, o[:, :Tq], 128**-0.5)
     assert (o[:, Tq:] == 7.0).all()
     step = max(1, 256 // (B * -(-Tq // 128)))
     for h in range(0, H, step):
-        few = torch.full((B, Tq, min(step, H - h) * 128), float("nan"), dtype=dtype, device=dev)
+        heads = min(step, H - h)
+        assert chosen(heads) == 128
+        few = torch.full((B, Tq, heads * 128), float("nan"), dtype=dtype, device=dev)
         ops.attention_fp16(q[:, h : h + step], k[:, h : h + step], v[:, h : h + step], few, 128**-0.5)
         assert torch.equal(o[:, :Tq, h * 128 : h * 128 + few.shape[2]], few)
     exact = torch.softmax(q[0, -1].float() @ k[0, -1].float().t().contiguous() * 128**-0.5, dim=-1) @ v[0, -1].float()

@@ -266,3 +266,35 @@ def test_rows_of_a_workgroup_leave_the_sums_alone(dev, splits, M, K, form, dtype
         ops.svdq_gemm_w4a4_cuda(act=sent, wgt=param, out=out[-1], ascales=scales, wscales=wsc[:, :n].contiguous().to(dev), act_unsigned=nibbles, act_blocked=blocked)
     assert splits == [4, 4]
     assert torch.equal(out[0][:, :16384], out[1])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,rel", [(torch.bfloat16, 1.5e-3), (torch.float16, 3.5e-4)])
+@pytest.mark.parametrize("K", [320, 512])
+def test_epilogues_of_32_row_workgroups(dev, splits, K, dtype, rel):
+    """Four wavefronts along K of 64-rank launches with 260 and 273 workgroups: K up to 896 stays with 32 rows to a workgroup (some wavefronts have one
+    stage, at K = 320 one has none).  Bounds as in test_requantizing_epilogues and test_qk_norm_rope."""
+    from nunchaku_rocm_amd import ops
+    from nunchaku_rocm_amd.flux_shaped import flux_ids, rope_table
+
+    print(f"case K={K} {dtype}", flush=True)
+    x = O.make_activations(400, K, seed=K, dtype=dtype).to(dev)[None]
+    glu = _module(dev, K, 2560, 64, dtype), _module(dev, 1280, K, 64, dtype)
+    ops.interleave_swiglu_linear_(glu[0])
+    for fn, fc1, fc2, bar in (
+        (ops.fused_gelu_mlp, _module(dev, K, 2560, 64, dtype), _module(dev, 2560, K, 64, dtype, unsigned=True), rel),
+        (ops.fused_swiglu_mlp, *glu, 3 * rel),
+    ):
+        splits.clear()
+        with torch.no_grad():
+            tiles, a, b = _both(lambda: fn(x, fc1, fc2), splits, [4, 8])
+        assert torch.equal(a, b)
+        assert ((a.double() - tiles.double()).norm() / tiles.double().norm()).item() <= bar
+    mod = _module(dev, K, 3 * 7 * 128, 64, dtype)
+    norm = torch.nn.RMSNorm(128, eps=1e-6, device=dev, dtype=dtype).requires_grad_(False)
+    rot = rope_table(flux_ids(0, 1, 400, device=dev), (16, 56, 56), 10000.0)
+    splits.clear()
+    with torch.no_grad():
+        tiles, a, b = _both(lambda: ops.fused_qkv_norm_rottary(x, mod, norm, norm, rot), splits, [4])
+    assert torch.equal(a, b)
+    assert ((a.float() - tiles.float()).abs() <= tiles.float().abs() * (2.0**-7 if dtype == torch.bfloat16 else 2.0**-10) + 1e-4).all()

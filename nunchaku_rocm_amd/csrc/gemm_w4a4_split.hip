@@ -227,7 +227,7 @@ __global__ __launch_bounds__(512, 2) void gemm_w4a4_split64_kernel(svdq_gemm_arg
     const int pid_m = id % tiles_m, pid_n = id / tiles_m;
     const int m0 = pid_m * 32 * RB, n0 = pid_n * BN;
     const int G = a.K / GROUP, nst = (G + 1) / 2;
-    const int count = (nst - ks + KS - 1) / KS;  // this wavefront's stages (none where K is short)
+    const int count = (nst - ks + KS - 1) / KS;  // this wavefront's stages, two at least (split64_takes)
 
     // column blocks past N and row blocks past M re-read the last one (their outputs are never stored)
     const int blast = (a.N + 31) / 32 - 1, b0 = min(n0 / 32 + wc * CB, blast);
@@ -345,35 +345,31 @@ __global__ __launch_bounds__(512, 2) void gemm_w4a4_split64_kernel(svdq_gemm_arg
     };
     const std::integral_constant<int, 0> I0;
     const std::integral_constant<int, 1> I1;
-    if (count > 0) {
-        load_scales(0, 0);
+    load_scales(0, 0);
 #pragma unroll
-        for (int gg = 0; gg < 2; gg++) {
+    for (int gg = 0; gg < 2; gg++) {
 #pragma unroll
-            for (int rb = 0; rb < RB; rb++) load_a(0, gg, rb);
+        for (int rb = 0; rb < RB; rb++) load_a(0, gg, rb);
 #pragma unroll
-            for (int bn = 0; bn < CB; bn++) {
-                load_w(0, bn, gg);
-                if (gg == 0) load_w(0, bn, 2);
-            }
+        for (int bn = 0; bn < CB; bn++) {
+            load_w(0, bn, gg);
+            if (gg == 0) load_w(0, bn, 2);
         }
     }
     if (wave < NWAVES) fetch_epilogue_operands<EPI>(a, sepi, n0, wave, lane);
-    if (count > 0) {
-        S[0] = scales(0, 0, 0);
-        P[0] = group(0);
-        int i = 0;
-        for (; i + 3 < count; i += 4) {
-            stage(I0, I0, i);
-            stage(I1, I0, i + 1);
-            stage(I0, I1, i + 2);
-            stage(I1, I1, i + 3);
-        }
-        const int left = count - i;  // 0 .. 3
-        if (left >= 1) stage(I0, I0, i);
-        if (left >= 2) stage(I1, I0, i + 1);
-        if (left >= 3) stage(I0, I1, i + 2);
+    S[0] = scales(0, 0, 0);
+    P[0] = group(0);
+    int i = 0;
+    for (; i + 3 < count; i += 4) {
+        stage(I0, I0, i);
+        stage(I1, I0, i + 1);
+        stage(I0, I1, i + 2);
+        stage(I1, I1, i + 3);
     }
+    const int left = count - i;  // 0 .. 3
+    if (left >= 1) stage(I0, I0, i);
+    if (left >= 2) stage(I1, I0, i + 1);
+    if (left >= 3) stage(I0, I1, i + 2);
 
     // ---- partial sums: every wavefront adds up one block, in the order of gemm_w4a4_split_kernel (of column block bn: wavefront bn's
     // first, then the others'), so that an output has the same bits as there; then a row block to a wavefront
@@ -467,7 +463,8 @@ static void launch_split64(const svdq_gemm_args &a, int tiles_m, hipStream_t s) 
 }
 
 // Workgroups of 64 rows, of those launches that split K over four wavefronts, where all of them find a CU of their own (beyond that the
-// 32-row ones, two to a CU, divide the rows better) and a wavefront has two stages: with one the refills in it are for nothing.  Time against
+// 32-row ones, two to a CU, divide the rows better) and every wavefront has two stages (with one the refills in it are for nothing; the
+// kernel relies on it).  Time against
 // the 32-row workgroups over 687 launches of 64 to 2048 rows, both types, PLAIN | GELU at rank 128: K = 128 1.00 to 1.06 | 1.00 to 1.03, 512
 // 1.08 to 1.15 | 1.02 to 1.06, 1024 0.89 to 0.92 | 0.86 to 0.95, 3072 0.78 to 0.84 | 0.79 to 0.90, 12288 0.75 to 0.81 | 0.75 to 0.81.
 static bool split64_takes(const svdq_gemm_args &a, int cus) {

@@ -186,11 +186,10 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attention_kernel(svdq_attention
     // has just used with the operand of RING matrix instructions of its strand later.  Stage t & 1 holds V of tile t and K of
     // tile t + 1; the operands are read from it between the middle of tile t's first iteration, where a barrier releases it and
     // the other stage begins to fill, and the middle of tile t + 1's.  The compiler is kept from regrouping the slots.
-    // Before, the softmax of a half stood beside one product only, with nothing beside the row maximum and the exponentials in
-    // half of the slots, and a tile's operands filled 128 registers a phase ahead (now 32).  Same bits; us before / now (bf16):
-    // workgroups of 128 queries; D = 128, 24 heads x 4608 253 / 232, 28 x 4608 270 / 254, 24 x 2000 58 / 52; D = 64, 40 x 4096 172 / 166.  Of 271 us (28 heads, a
-    // slower board) the V^T reads are 42, the tile loads 30, the K reads 14, the exponentials 12; matrix instructions alone run at
-    // 1.8 PFLOP/s on random data (1.86 GHz), which is 167 us.
+    // What bounds it is power.  us with the softmax beside one of the two products only / this way (bf16, workgroups of 128 queries): D = 128, 24
+    // heads x 4608 253 / 232, 24 x 2000 58 / 52; D = 64, 40 x 4096 172 / 166.  Scores of the next tile that are there when the reference moves
+    // get the difference subtracted; started anew from the new bias (the last bit of a few outputs in a million) keys whose size
+    // grows along the sequence took 280 instead of 263.
     // Priority: the second iteration of a tile goes first (s_setprio), which keeps the two wavefronts of a SIMD out of step: 242 / 236.
     constexpr int RING = NC / 2;
     static_assert(NC == 2 * NDT, "as many matrix instructions per half in either product");

@@ -6,24 +6,25 @@
 // activations give the same bits.  (Signed nibbles need the offset correction and stay with the tiles.)  Same arithmetic as
 // gemm_w4a4_f8_kernel (per group one fp6 x fp6 or fp6 x fp8 matrix instruction = the exact integer dot product, one 16-bit
 // matrix instruction = the product of the two scales, one fp32 FMA per output); only the order of the fp32 sums over groups
-// differs (a partial sum per wavefront).  Against 64-bit sums it is the closer one: of 512 x 3072 outputs in fp16 (K = 3072)
-// 989 are not the correctly rounded value, 1086 with the tiles; K = 12288, 333 rows: 1053 and 1366.
+// differs (a partial sum per wavefront; the same order with 32 and 64 rows to a workgroup).  Against 64-bit sums it is the closer one: of 512 x 3072
+// outputs in fp16 (K = 3072) 989 are not the correctly rounded value, 1086 with the tiles; K = 12288, 333 rows: 1053 and 1366.
 //
 // Why: with 128 x 128 tiles a prompt's 512 rows give a 3072-wide layer 96 workgroups on 256 CUs, each alone on its CU with
 // one wavefront per SIMD and a barrier per 128 k.  Here the same layer has 384 workgroups and a wavefront runs a quarter of
 // K (an eighth where no CU gets a second workgroup).  A CU with two workgroups, or with one of eight wavefronts, has two
 // wavefronts per SIMD.  Between one and two of them per CU most launches run as half as many workgroups of 64 rows (split64_takes).
-// What bounds it: every workgroup streams its own copy of the weight tile from L2 (there is no second row block in the
-// workgroup to share it with), in all about 11 TB/s at K = 12288 and 512 rows, the rate the tiles' loop is delivered at too and
-// less than half of 64 bytes per clock and CU.  That is why large launches stay with the tiles.  The epilogue is wavefront
-// 0's alone; the others have ended.
+// What bounds the 32-row form: every workgroup streams its own copy of the weight tile from L2 (there is no second row block in it to
+// share it with), in all about 11 TB/s at K = 12288 and 512 rows, the rate the tiles' loop is delivered at too and less than half of 64
+// bytes per clock and CU.  That is why large launches stay with the tiles.  The epilogue is one wavefront's for each row block; the
+// others have ended.
 //
 //  * Nothing is shared between the wavefronts of a workgroup inside the loop, so weights go straight to registers (they lie
 //    in the matrix instruction's lane order) and there is neither LDS nor a barrier in it; a stage (two groups) is
-//    requested one stage ahead: 16 KB in flight per wavefront.
-//  * Wavefront w takes stages w, w + WAVES, ...: the workgroup reads a contiguous stretch of the weight at a time.
-//  * The partial tiles meet in LDS: wavefront w < 4 adds up column block w in a fixed order (the result does not depend on
-//    timing), the sums go to wavefront 0, which owns the whole 32 x 128 tile for the epilogue as in the other kernels.
+//    requested one stage ahead: 16 KB in flight per wavefront (32 rows).
+//  * Wavefront w of those along K takes stages w, w + WAVES, ...: the workgroup reads a contiguous stretch of the weight at a time.
+//  * The partial tiles meet in LDS: one wavefront (w < 4 for column block w with 32 rows, each of the eight with 64) adds up a 32 x 32 block in a
+//    fixed order (the result does not depend on timing); the sums of a row block go to one wavefront, which owns its whole
+//    32 x 128 tile for the epilogue as in the other kernels.
 //  * Workgroups of one column tile are neighbours on one XCD, so that a weight tile is fetched into one L2.
 #include <algorithm>
 #include <type_traits>

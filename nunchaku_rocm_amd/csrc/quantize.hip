@@ -674,7 +674,7 @@ static int device_cus() {
 // prologue with its own statistics | with given ones | without): 4100 rows 20.6 / 16.9 | 17.1 / 13.4 | 15.6 / 11.3, 4608 21.9 / 18.8 |
 // 18.5 / 15.6 | 14.1 / 13.0, 5120 22.4 / 21.5 | 18.5 / 15.5 | 14.3 / 13.7, 5400 22.8 / 22.2 | 18.6 / 15.7 | 14.6 / 14.0, 8704 34.9 / 31.7 |
 // 26.2 / 22.4 | 22.0 / 19.5.  Two to a block (5632 rows 22.9 / 24.0 | 19.0 / 17.6 | 14.8 / 14.4, K = 4096 10240 46.2 / 47.8 | 33.6 / 35.2 | 28.9 /
-// 29.6) do not pay for the prologue that both compute.
+// 29.6) do not pay for the prologue that both compute.  Shorter rows: K = 192 to 2048, 4100 to 16400 rows 0.70 to 1.00 of the time.
 static int quantize_share(const svdq_quantize_args &a) {
     const int blocks = (a.M + Q_ROWS - 1) / Q_ROWS, cus = device_cus(), left = blocks % cus;
     if (a.R == 0 || a.R > Q_RCHUNK || blocks <= cus || left == 0 || a.prologue != SVDQ_PRE_NONE) return 1;
@@ -707,8 +707,8 @@ static int quantize_grid_y(const svdq_quantize_args &a, int row_blocks) {
     if (a.R == 0) return 1;
     const int chunks = (a.R + Q_RCHUNK - 1) / Q_RCHUNK, cus = device_cus();
     // (with a GLU or GELU prologue the workgroups that only project compute it a second time: only where half the CUs would idle
-    // anyway.  With the norm prologue, of sixteen wavefronts, up to all of the CUs: K = 3072, R = 32, limits of a half / all of them 1024
-    // rows 11.5 / 10.6 us, 1201 12.7 / 10.7, 2048 13.3 / 12.3; R = 128 512 rows 12.5 / 10.4)
+    // anyway.  With the norm prologue up to all of the CUs, half / all of them (K = 3072, R = 32, eight / sixteen wavefronts): 1201 rows 13.7 / 10.7 us,
+    // 2048 14.2 / 12.4; K = 128 to 1472, eight wavefronts, R = 32 to 128: 0.83 to 0.96 of the time where it changes the grid)
     const int limit = has_norm(a) ? cus : a.prologue != SVDQ_PRE_NONE ? cus / 2 : cus;
     if (row_blocks * (chunks + 1) > limit) return chunks;
     const int nq = std::min({3, limit / row_blocks - chunks, a.K / GROUP});

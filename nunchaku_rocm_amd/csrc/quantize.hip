@@ -35,7 +35,7 @@ constexpr int Q_ROWS = 16;         // rows of one MFMA pass; a workgroup takes Q
 constexpr int Q_ROW_BYTES = 128;  // one scale group of one row (64 x 16 bit)
 constexpr int Q_RCHUNK = 32;  // LoRA ranks per pass over the row block
 constexpr int Q_CHAINS = 8;   // partial sums of a lora_act value: that of groups c, c + 8, .. in order for c = 0 .. 7, added up in order
-constexpr int Q_STATS_K = 4096;  // longest row whose statistics the norm prologue computes from registers (two rows to a wavefront)
+constexpr int Q_STATS_K = 4096;  // longest row whose statistics the norm prologue computes from registers (one or two rows to a wavefront)
 constexpr int Q32_ABOVE = 256, Q32_UPTO = 512;  // number of 16-row workgroups for which 32-row workgroups are used instead
 
 // sum_j (0x4B400000 << 4 j) mod 2^32: what eight magic-biased codes add up to besides their nibbles
